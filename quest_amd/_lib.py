@@ -1,4 +1,5 @@
-"""ctypes binding of libquest_hip.so (the C ABI declared in include/quest_hip.h).
+"""ctypes binding of libquest_hip.so (the C ABI declared in include/quest_hip.h), and the native host module over it
+(`host`, csrc/host.cpp) that the hot calls go through.
 
 There is no fallback: if the shared library is missing or an entry point returns an error the
 caller gets a RuntimeError.
@@ -77,6 +78,21 @@ def load() -> ctypes.CDLL:
             fn.restype = _RESTYPES.get(name, ctypes.c_int)
         _lib = lib
     return _lib
+
+
+class _NotBuilt:
+    def __init__(self, why):
+        self._why = why
+
+    def __getattr__(self, name):
+        raise RuntimeError(f'quest_amd/_host.so cannot be loaded ({self._why}): build it first (python -m quest_amd.build). '
+                           'quest_amd has no fallback path.')
+
+
+try:
+    from . import _host as host
+except ImportError as e:                   # the builder imports this package before there is anything to load
+    host = _NotBuilt(e)
 
 
 def check(status: int, what: str) -> None:

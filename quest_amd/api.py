@@ -5,6 +5,9 @@ kernels reached through the C ABI of libquest_hip.so.  Differences, all additive
   * float16 is accepted wherever the reference asserts bfloat16;
   * `hadamard128` and `hadamard_quantize_int4` are new (the fused activation kernel);
   * the 4:8-sparse entry points raise NotImplementedError (NVIDIA sparse tensor cores only).
+
+The hot calls first go to the native host path (csrc/host.cpp), which checks and launches in one step; it declines (None,
+nothing launched) whatever is not the plain case, and the statement below it then runs or raises.
 """
 from __future__ import annotations
 
@@ -13,7 +16,7 @@ import ctypes
 import torch
 
 from . import _lib
-from ._lib import DTYPE_CODE, check, ptr, require_gpu, stream_of
+from ._lib import DTYPE_CODE, check, host, ptr, require_gpu, stream_of
 
 _FLOAT16S = (torch.bfloat16, torch.float16)
 HADAMARD_ENTRY = 181. / 2048.        # bf16(2**-3.5) == fp16(2**-3.5): what the reference's matrix holds
@@ -33,6 +36,10 @@ def fused_matmul_dequantize_int4_int4t_bf16(
 
     `workspace` (not in the reference): a uint8 tensor from `gemm_workspace`, which lets up to 16 tokens split K across
     workgroups; the result is the same bit for bit.  One workspace serves any number of calls on one stream."""
+    if workspace is None:
+        done = host.gemm(mat_a, mat_b, vec_a_add, vec_b_add, vec_a_mul, vec_b_mul, out)
+        if done is not None:
+            return done
     if out is None:
         out = torch.empty(mat_a.size(0), mat_b.size(0), dtype=vec_a_mul.dtype, device=mat_a.device)
     assert mat_a.dtype == torch.uint8 and mat_b.dtype == torch.uint8 and vec_a_add.dtype == torch.int32 and vec_b_add.dtype == torch.int32
@@ -194,6 +201,9 @@ def matmul_int4_int4t_int32(
         out: torch.Tensor = None,
 ) -> torch.Tensor:
     """gemm-quest/quest/__init__.py:23-33."""
+    done = host.matmul_int32(mat_a, mat_b, out)
+    if done is not None:
+        return done
     if out is None:
         out = torch.empty(mat_a.size(0), mat_b.size(0), dtype=torch.int32, device=mat_a.device)
     assert mat_a.dtype == torch.uint8 and mat_b.dtype == torch.uint8 and out.dtype == torch.int32
@@ -224,6 +234,9 @@ def find_scale_int4(
         scale: torch.Tensor = None,
 ) -> torch.Tensor:
     """gemm-quest/quest/__init__.py:87-96."""
+    done = host.find_scale(x, scale)
+    if done is not None:
+        return done
     if scale is None:
         scale = torch.empty(x.size(0), 1, dtype=x.dtype, device=x.device)
     assert x.dtype in _FLOAT16S and scale.dtype == x.dtype
@@ -245,6 +258,8 @@ def quantize_int4(
         do_dequantize: bool = False,
 ) -> tuple[torch.Tensor, torch.Tensor | None, torch.Tensor | None, torch.Tensor | None]:
     """gemm-quest/quest/__init__.py:99-114.  Outputs passed as None are not produced."""
+    if host.quantize(x, scale, x_int, x_int_packed, x_int_row_sum, do_dequantize):
+        return x, x_int, x_int_packed, x_int_row_sum
     assert x.dtype in _FLOAT16S and scale.dtype == x.dtype
     assert x_int is None or x_int.dtype == torch.int8
     assert x_int_packed is None or x_int_packed.dtype == torch.uint8
@@ -272,6 +287,9 @@ def add_mul_vv(
         mat_d: torch.Tensor = None,
 ) -> torch.Tensor:
     """gemm-quest/quest/__init__.py:117-130."""
+    done = host.add_mul_vv(vec_a_add, vec_a_mul, vec_b_add, vec_b_mul, mat_c, mat_d)
+    if done is not None:
+        return done
     if mat_d is None:
         mat_d = torch.empty(mat_c.shape, dtype=vec_a_mul.dtype, device=mat_c.device)
     assert vec_a_add.dtype == torch.int32 and vec_b_add.dtype == torch.int32 and mat_c.dtype == torch.int32
@@ -292,6 +310,9 @@ def hadamard128(x: torch.Tensor, out: torch.Tensor = None, scale: float = HADAMA
     """Block-128 Walsh-Hadamard transform along the last dimension.  scale=181/2048 is the
     activation transform of linear_forward (gemm-quest/benchmarks/utils.py:17,89-90),
     scale=2**-3.5 the weight transform of preprocess_weight (utils.py:38-39).  out may be x."""
+    done = host.hadamard128(x, out, float(scale))
+    if done is not None:
+        return done
     if out is None:
         out = torch.empty_like(x)
     assert x.dtype in _FLOAT16S and out.dtype == x.dtype and out.shape == x.shape
@@ -321,8 +342,12 @@ def hadamard_quantize_int4(
     (scale = max|x| / 7.5 + 1e-8).  from_fp32: scale and codes from the transform's fp32 output (the arithmetic of the
     reference's evaluation-side fake quantiser, src/eval_hswag.py:201-214) instead of from the dtype-rounded tensor.
     Returns (scale, x_int_packed, x_int_row_sum)."""
-    m, k = x.shape
     rule = {'gaussian': 0, 'absmax': 1}[scale_rule] | (4 if from_fp32 else 0)
+    if x_had is None:
+        done = host.hadamard_quantize(x, scale, x_int_packed, x_int_row_sum, float(hadamard_scale), rule)
+        if done is not None:
+            return done
+    m, k = x.shape
     if scale is None:
         scale = torch.empty(m, 1, dtype=x.dtype, device=x.device)
     if x_int_packed is None:

@@ -1,4 +1,5 @@
-"""Builds quest_amd/libquest_hip.so for gfx950 with hipcc (no torch headers, no pybind).
+"""Builds quest_amd/libquest_hip.so for gfx950 with hipcc (the C ABI: no torch headers, no pybind) and
+quest_amd/_host.so, the CPython module over it (csrc/host.cpp: torch's C++ tensors, no device code), with the host compiler.
 
     python -m quest_amd.build
 """
@@ -7,12 +8,14 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB_PATH = os.path.join(HERE, 'libquest_hip.so')
+HOST_PATH = os.path.join(HERE, '_host.so')
 SOURCES = ['rowops.hip', 'hadamard_mfma.hip', 'gemm.hip', 'gemm_big.hip', 'gemm_small.hip', 'gemm_staged.hip',
            'gemm_decode.hip', 'gemm_e2m3.hip', 'capi.hip']
 
@@ -36,8 +39,17 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(err, file=sys.stderr)
 
 
+def _host_command(out: str) -> list[str]:
+    import torch
+    root = os.path.dirname(torch.__file__)
+    return [os.environ.get('CXX', 'g++'), '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
+            '-isystem', os.path.join(root, 'include'), '-isystem', '/opt/rocm/include', '-isystem', sysconfig.get_paths()['include'],
+            os.path.join(CSRC, 'host.cpp'), '-o', out, '-L' + os.path.join(root, 'lib'), '-lc10', '-lc10_hip', '-ltorch_cpu',
+            '-ltorch_python', '-L' + HERE, '-l:libquest_hip.so', '-Wl,-rpath,$ORIGIN']
+
+
 def build(verbose: bool = False, extra_flags: list[str] | None = None, jobs: int = 4) -> str:
-    """Compiles every source to an object (up to `jobs` at a time) and links the shared library."""
+    """Compiles every source to an object (up to `jobs` at a time), links the shared library, then the host module."""
     hipcc = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
     flags = [f for f in FLAGS if f != '-shared'] + list(extra_flags or [])
     with tempfile.TemporaryDirectory(prefix='quest_hip_build_') as tmp:
@@ -47,6 +59,7 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None, jobs: int
             for fut in [pool.submit(_run, c, verbose) for c in cmds]:
                 fut.result()
         _run([hipcc, '--offload-arch=gfx950', '-shared', '-fPIC', *objs, '-o', LIB_PATH], verbose)
+    _run(_host_command(HOST_PATH), verbose)
     return LIB_PATH
 
 

@@ -1,0 +1,475 @@
+// Host side of the hot calls in native code: argument checks, output and scratch allocation, stream lookup and the launches
+// of libquest_hip.so, as a CPython module over torch's C++ tensors.
+//
+// Why: a layer at a handful of tokens is 7 us of GPU work in two launches, and its Python host path (asserts, ctypes
+// conversions, device context, one allocation per output) took 36 us per call, so every small call ran at the speed of the
+// interpreter.  The same checks and launches from here take 6-8 us, most of it the two launches.
+//
+// Contract of every function: either the call is the plain case -- exact torch tensors on one GPU, contiguous, right types
+// and sizes, accepted by the library -- and everything is launched, or None comes back with nothing launched and the
+// caller's Python statement of the same call runs, which raises what there is to raise.  Nothing is cached between calls.
+#include <Python.h>
+
+#include <ATen/core/Tensor.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <ATen/ops/empty.h>
+#include <ATen/ops/scaled_dot_product_attention.h>
+#include <c10/core/DeviceGuard.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/quest_hip.h"
+
+namespace {
+
+constexpr float kHadamardEntry = 181.f / 2048.f;      // bf16(2^-3.5) == fp16(2^-3.5)
+
+// ---- arguments ------------------------------------------------------------------------------------------------------
+// Collects what the arguments of one call have in common and whether every one of them is as expected.
+struct Args {
+    bool ok = true;
+    c10::Device dev{c10::DeviceType::CPU};
+    at::Tensor none;                  // stands for an argument that is no tensor
+    const at::Tensor *tensor(PyObject *o) {
+        if (!THPVariable_CheckExact(o)) {
+            ok = false;
+            return &none;
+        }
+        const at::Tensor &t = THPVariable_Unpack(o);
+        if (!t.is_cuda() || !t.is_contiguous() || t.numel() == 0) {
+            ok = false;
+        } else if (dev.is_cpu()) {
+            dev = t.device();
+        } else if (t.device() != dev) {
+            ok = false;
+        }
+        return &t;
+    }
+    const at::Tensor *tensor(PyObject *o, at::ScalarType type, int64_t numel) {
+        const at::Tensor *t = tensor(o);
+        if (ok && (t->scalar_type() != type || t->numel() != numel)) ok = false;
+        return t;
+    }
+    const at::Tensor *matrix(PyObject *o, at::ScalarType type, int64_t rows, int64_t cols) {
+        const at::Tensor *t = tensor(o);
+        if (ok && (t->scalar_type() != type || t->dim() != 2 || t->size(0) != rows || t->size(1) != cols)) ok = false;
+        return t;
+    }
+};
+
+bool is_half(at::ScalarType t) { return t == at::kBFloat16 || t == at::kHalf; }
+int dtype_code(at::ScalarType t) { return t == at::kBFloat16 ? QUEST_DTYPE_BF16 : QUEST_DTYPE_FP16; }
+bool fits_int(int64_t v) { return v > 0 && v <= 0x7fffffff; }
+void *stream_of(c10::Device dev) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream(); }
+at::Tensor make(at::IntArrayRef sizes, at::ScalarType type, c10::Device dev) {
+    return at::empty(sizes, at::TensorOptions().dtype(type).device(dev));
+}
+PyObject *wrap(at::Tensor t) { return THPVariable_Wrap(std::move(t)); }
+PyObject *declined() { Py_RETURN_NONE; }
+PyObject *ref(PyObject *o) {
+    Py_INCREF(o);
+    return o;
+}
+int64_t up(int64_t bytes) { return (bytes + 255) & ~(int64_t)255; }
+
+// One activation's codes in a single scratch allocation: packed nibbles, row sums and scales, or E2M3 tiles and scales.
+struct Codes {
+    at::Tensor hold;
+    uint8_t *codes = nullptr;         // packed nibbles or tiles
+    int32_t *row_sum = nullptr;
+    void *scale = nullptr;
+    bool tiles = false;
+    Codes(int64_t m, int64_t k, bool as_tiles, c10::Device dev) : tiles(as_tiles) {
+        const int64_t body = up(as_tiles ? (int64_t)quest_e2m3_tiles_bytes((int)m, (int)k) : m * (k / 2));
+        const int64_t sums = as_tiles ? 0 : up(4 * m);
+        hold = make({body + sums + 2 * m}, at::kByte, dev);
+        codes = (uint8_t *)hold.data_ptr();
+        row_sum = as_tiles ? nullptr : (int32_t *)(codes + body);
+        scale = codes + body + sums;
+    }
+};
+
+// ---- linear(x, w_packed, w_scale, w_add, w_tiles, bias, had_scale, out) ---------------------------------------------
+// The W4A4 linear layer: activation kernel, GEMM, bias.  x (..., K); w_tiles: None, or the weight's E2M3 tiles when the
+// FP6 kernel is wanted; out: None or the (M, N) result to fill.
+PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 8) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *x = args.tensor(a[0]);
+    if (!args.ok || !is_half(x->scalar_type()) || x->dim() < 1) return declined();
+    const at::ScalarType type = x->scalar_type();
+    const int64_t k = x->size(-1), m = x->numel() / k;
+    const at::Tensor *w = args.tensor(a[1]);
+    if (!args.ok || w->scalar_type() != at::kByte || w->dim() != 2 || w->size(1) * 2 != k) return declined();
+    const int64_t n = w->size(0);
+    if (!fits_int(m) || !fits_int(k) || !fits_int(n)) return declined();
+    const at::Tensor *w_scale = args.tensor(a[2], type, n);
+    const at::Tensor *w_add = args.tensor(a[3], at::kInt, n);
+    const bool tiles = a[4] != Py_None;
+    const at::Tensor *w_tiles = tiles ? args.tensor(a[4], at::kByte, (int64_t)quest_e2m3_tiles_bytes((int)n, (int)k)) : nullptr;
+    const at::Tensor *bias = a[5] == Py_None ? nullptr : args.tensor(a[5], type, n);
+    const double had_scale = PyFloat_AsDouble(a[6]);
+    const at::Tensor *given = a[7] == Py_None ? nullptr : args.matrix(a[7], type, m, n);
+    if (!args.ok) return declined();
+
+    const c10::DeviceGuard guard(args.dev);
+    void *st = stream_of(args.dev);
+    const int dt = dtype_code(type);
+    Codes q(m, k, tiles, args.dev);
+    int rc = tiles ? quest_hadamard_quantize_e2m3(x->data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, (int)k, (int)m, (float)had_scale, dt, st)
+                   : quest_hadamard_quantize_int4(x->data_ptr(), q.scale, q.codes, q.row_sum, nullptr, (int)k, (int)m, (float)had_scale, dt, st);
+    if (rc != QUEST_OK) return declined();
+    at::Tensor out;
+    if (given != nullptr) {
+        out = *given;
+    } else {
+        c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
+        shape.back() = n;
+        out = make(shape, type, args.dev);
+    }
+    rc = tiles ? quest_fused_matmul_dequantize_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), (int)m, (int)k, (int)n, dt, st)
+               : quest_fused_matmul_dequantize_int4_int4t(out.data_ptr(), q.codes, (const uint8_t *)w->data_ptr(), q.row_sum,
+                                                          (const int32_t *)w_add->data_ptr(), q.scale, w_scale->data_ptr(), (int)m, (int)k, (int)n, dt, st);
+    if (rc != QUEST_OK) return declined();
+    if (bias != nullptr) out.add_(*bias);
+    return given != nullptr ? ref(a[7]) : wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- gemm(mat_a, mat_b, a_add, b_add, a_mul, b_mul, out) ------------------------------------------------------------
+PyObject *gemm(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 7) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *x = args.tensor(a[0]), *w = args.tensor(a[1]);
+    if (!args.ok || x->scalar_type() != at::kByte || w->scalar_type() != at::kByte || x->dim() != 2 || w->dim() != 2 ||
+        x->size(1) != w->size(1))
+        return declined();
+    const int64_t m = x->size(0), n = w->size(0), k = w->size(1) * 2;
+    if (!fits_int(m) || !fits_int(k) || !fits_int(n)) return declined();
+    const at::Tensor *a_add = args.tensor(a[2], at::kInt, m), *b_add = args.tensor(a[3], at::kInt, n);
+    const at::Tensor *a_mul = args.tensor(a[4]);
+    if (!args.ok || !is_half(a_mul->scalar_type()) || a_mul->numel() != m) return declined();
+    const at::ScalarType type = a_mul->scalar_type();
+    const at::Tensor *b_mul = args.tensor(a[5], type, n);
+    const at::Tensor *given = a[6] == Py_None ? nullptr : args.matrix(a[6], type, m, n);
+    if (!args.ok) return declined();
+    const c10::DeviceGuard guard(args.dev);
+    at::Tensor out = given != nullptr ? *given : make({m, n}, type, args.dev);
+    const int rc = quest_fused_matmul_dequantize_int4_int4t(out.data_ptr(), (const uint8_t *)x->data_ptr(), (const uint8_t *)w->data_ptr(),
+                                                            (const int32_t *)a_add->data_ptr(), (const int32_t *)b_add->data_ptr(),
+                                                            a_mul->data_ptr(), b_mul->data_ptr(), (int)m, (int)k, (int)n, dtype_code(type), stream_of(args.dev));
+    if (rc != QUEST_OK) return declined();
+    return given != nullptr ? ref(a[6]) : wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- matmul_int32(mat_a, mat_b, out) --------------------------------------------------------------------------------
+PyObject *matmul_int32(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 3) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *x = args.tensor(a[0]), *w = args.tensor(a[1]);
+    if (!args.ok || x->scalar_type() != at::kByte || w->scalar_type() != at::kByte || x->dim() != 2 || w->dim() != 2 ||
+        x->size(1) != w->size(1))
+        return declined();
+    const int64_t m = x->size(0), n = w->size(0), k = w->size(1) * 2;
+    if (!fits_int(m) || !fits_int(k) || !fits_int(n)) return declined();
+    const at::Tensor *given = a[2] == Py_None ? nullptr : args.matrix(a[2], at::kInt, m, n);
+    if (!args.ok) return declined();
+    const c10::DeviceGuard guard(args.dev);
+    at::Tensor out = given != nullptr ? *given : make({m, n}, at::kInt, args.dev);
+    const int rc = quest_matmul_int4_int4t_int32((int32_t *)out.data_ptr(), (const uint8_t *)x->data_ptr(), (const uint8_t *)w->data_ptr(),
+                                                 (int)m, (int)k, (int)n, stream_of(args.dev));
+    if (rc != QUEST_OK) return declined();
+    return given != nullptr ? ref(a[2]) : wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- hadamard_quantize(x, scale, packed, row_sum, had_scale, rule) -> (scale, packed, row_sum) ------------------------
+// scale, packed and row_sum: None or the tensor to fill.
+PyObject *hadamard_quantize(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 6) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *x = args.tensor(a[0]);
+    if (!args.ok || !is_half(x->scalar_type()) || x->dim() != 2) return declined();
+    const at::ScalarType type = x->scalar_type();
+    const int64_t m = x->size(0), k = x->size(1);
+    if (!fits_int(m) || !fits_int(k)) return declined();
+    at::Tensor scale, packed, row_sum;
+    if (a[1] != Py_None) scale = *args.tensor(a[1], type, m);
+    if (a[2] != Py_None) packed = *args.matrix(a[2], at::kByte, m, k / 2);
+    if (a[3] != Py_None) row_sum = *args.tensor(a[3], at::kInt, m);
+    const double had_scale = PyFloat_AsDouble(a[4]);
+    const long rule = PyLong_AsLong(a[5]);
+    if (!args.ok) return declined();
+    const c10::DeviceGuard guard(args.dev);
+    if (!scale.defined()) scale = make({m, 1}, type, args.dev);
+    if (!packed.defined()) packed = make({m, k / 2}, at::kByte, args.dev);
+    if (!row_sum.defined()) row_sum = make({m, 1}, at::kInt, args.dev);
+    const int rc = quest_hadamard_quantize_int4_rule(x->data_ptr(), scale.data_ptr(), (uint8_t *)packed.data_ptr(), (int32_t *)row_sum.data_ptr(),
+                                                     nullptr, (int)k, (int)m, (float)had_scale, (int)rule, dtype_code(type), stream_of(args.dev));
+    if (rc != QUEST_OK) return declined();
+    PyObject *t = PyTuple_New(3);
+    if (t == nullptr) return nullptr;
+    PyTuple_SET_ITEM(t, 0, a[1] != Py_None ? ref(a[1]) : wrap(std::move(scale)));
+    PyTuple_SET_ITEM(t, 1, a[2] != Py_None ? ref(a[2]) : wrap(std::move(packed)));
+    PyTuple_SET_ITEM(t, 2, a[3] != Py_None ? ref(a[3]) : wrap(std::move(row_sum)));
+    return t;
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- hadamard128(x, out, had_scale) ----------------------------------------------------------------------------------
+PyObject *hadamard128(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 3) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *x = args.tensor(a[0]);
+    if (!args.ok || !is_half(x->scalar_type()) || x->dim() < 1) return declined();
+    const int64_t k = x->size(-1), rows = x->numel() / k;
+    at::Tensor out;
+    if (a[1] != Py_None) out = *args.tensor(a[1], x->scalar_type(), x->numel());
+    if (!args.ok || (out.defined() && out.sizes() != x->sizes()) || !fits_int(k) || !fits_int(rows)) return declined();
+    const c10::DeviceGuard guard(args.dev);
+    if (!out.defined()) out = make(x->sizes(), x->scalar_type(), args.dev);
+    const int rc = quest_hadamard128(out.data_ptr(), x->data_ptr(), (int)k, (int)rows, (float)PyFloat_AsDouble(a[2]), dtype_code(x->scalar_type()), stream_of(args.dev));
+    if (rc != QUEST_OK) return declined();
+    return a[1] != Py_None ? ref(a[1]) : wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- find_scale(x, scale) --------------------------------------------------------------------------------------------
+PyObject *find_scale(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 2) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *x = args.tensor(a[0]);
+    if (!args.ok || !is_half(x->scalar_type()) || x->dim() != 2) return declined();
+    const int64_t m = x->size(0), k = x->size(1);
+    at::Tensor scale;
+    if (a[1] != Py_None) scale = *args.tensor(a[1], x->scalar_type(), m);
+    if (!args.ok || !fits_int(m) || !fits_int(k)) return declined();
+    const c10::DeviceGuard guard(args.dev);
+    if (!scale.defined()) scale = make({m, 1}, x->scalar_type(), args.dev);
+    const int rc = quest_find_scale_int4(scale.data_ptr(), x->data_ptr(), (int)k, (int)m, dtype_code(x->scalar_type()), stream_of(args.dev));
+    if (rc != QUEST_OK) return declined();
+    return a[1] != Py_None ? ref(a[1]) : wrap(std::move(scale));
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- quantize(x, scale, x_int, packed, row_sum, do_dequantize) -> True -----------------------------------------------
+PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 6) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *x = args.tensor(a[0]);
+    if (!args.ok || !is_half(x->scalar_type()) || x->dim() != 2) return declined();
+    const int64_t m = x->size(0), k = x->size(1);
+    const at::Tensor *scale = args.tensor(a[1], x->scalar_type(), m);
+    const at::Tensor *x_int = a[2] == Py_None ? nullptr : args.matrix(a[2], at::kChar, m, k);
+    const at::Tensor *packed = a[3] == Py_None ? nullptr : args.matrix(a[3], at::kByte, m, k / 2);
+    const at::Tensor *row_sum = a[4] == Py_None ? nullptr : args.tensor(a[4], at::kInt, m);
+    if (!args.ok || !fits_int(m) || !fits_int(k)) return declined();
+    const c10::DeviceGuard guard(args.dev);
+    const int rc = quest_quantize_int4(x->data_ptr(), scale->data_ptr(), x_int ? (int8_t *)x_int->data_ptr() : nullptr,
+                                       packed ? (uint8_t *)packed->data_ptr() : nullptr, row_sum ? (int32_t *)row_sum->data_ptr() : nullptr,
+                                       (int)k, (int)m, PyObject_IsTrue(a[5]) == 1, dtype_code(x->scalar_type()), stream_of(args.dev));
+    if (rc != QUEST_OK) return declined();
+    Py_RETURN_TRUE;
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- add_mul_vv(a_add, a_mul, b_add, b_mul, mat_c, mat_d) -------------------------------------------------------------
+PyObject *add_mul_vv(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 6) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *c = args.tensor(a[4]);
+    if (!args.ok || c->scalar_type() != at::kInt || c->dim() != 2) return declined();
+    const int64_t m = c->size(0), n = c->size(1);
+    const at::Tensor *a_mul = args.tensor(a[1]);
+    if (!args.ok || !is_half(a_mul->scalar_type()) || a_mul->numel() != m) return declined();
+    const at::ScalarType type = a_mul->scalar_type();
+    const at::Tensor *a_add = args.tensor(a[0], at::kInt, m), *b_add = args.tensor(a[2], at::kInt, n), *b_mul = args.tensor(a[3], type, n);
+    const at::Tensor *given = a[5] == Py_None ? nullptr : args.matrix(a[5], type, m, n);
+    if (!args.ok || !fits_int(m) || !fits_int(n)) return declined();
+    const c10::DeviceGuard guard(args.dev);
+    at::Tensor out = given != nullptr ? *given : make({m, n}, type, args.dev);
+    const int rc = quest_add_mul_vv(out.data_ptr(), (const int32_t *)a_add->data_ptr(), a_mul->data_ptr(), (const int32_t *)b_add->data_ptr(),
+                                    b_mul->data_ptr(), (const int32_t *)c->data_ptr(), (int)m, (int)n, dtype_code(type), stream_of(args.dev));
+    if (rc != QUEST_OK) return declined();
+    return given != nullptr ? ref(a[5]) : wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// ---- block(x, branch, freqs, n_head, norm1, eps1, norm2, eps2, qkv, o, gate_up, glu, down, tiles) ---------------------
+// One producer-fused decoder block (LlamaBlock.forward_fused with every option at its default): x (B, T, C) is the residual
+// stream, updated in place; branch: None, or the previous block's MLP output still to be added.  qkv, o, gate_up, glu, down:
+// (packed, scale, add, tiles or None) of the projections, glu the row-interleaved gate / up weights; tiles: which of the
+// four GEMMs (bit 0 qkv, 1 o, 2 gate_up, 3 down) run on E2M3 tiles.  Returns True, or the block's MLP output when it is
+// still to be added.
+struct Linear {
+    const at::Tensor *packed, *scale, *add, *tiles;
+    int n, k;
+    bool take(Args &args, PyObject *t, at::ScalarType type, bool want_tiles) {
+        if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 4) return args.ok = false;
+        packed = args.tensor(PyTuple_GET_ITEM(t, 0));
+        if (!args.ok || packed->scalar_type() != at::kByte || packed->dim() != 2 || !fits_int(packed->size(0)) ||
+            !fits_int(packed->size(1) * 2))
+            return args.ok = false;
+        n = (int)packed->size(0);
+        k = (int)packed->size(1) * 2;
+        scale = args.tensor(PyTuple_GET_ITEM(t, 1), type, n);
+        add = args.tensor(PyTuple_GET_ITEM(t, 2), at::kInt, n);
+        tiles = want_tiles ? args.tensor(PyTuple_GET_ITEM(t, 3), at::kByte, (int64_t)quest_e2m3_tiles_bytes(n, k)) : nullptr;
+        return args.ok;
+    }
+};
+
+void launched(int rc, const char *what) {
+    TORCH_CHECK(rc == QUEST_OK, what, " failed with status ", rc, ": ", quest_status_string(rc));
+}
+
+// the GEMM of a projection on quantised activations: dst = product, or dst += product with the two roundings of x + y
+void project(const Linear &w, const Codes &q, at::Tensor &dst, int m, int dt, void *st, bool add_to_dst = false) {
+    if (q.tiles) {
+        auto *f = add_to_dst ? quest_fused_matmul_dequantize_add_e2m3 : quest_fused_matmul_dequantize_e2m3;
+        launched(f(dst.data_ptr(), q.codes, w.tiles->data_ptr(), q.scale, w.scale->data_ptr(), m, w.k, w.n, dt, st), "projection");
+    } else {
+        auto *f = add_to_dst ? quest_fused_matmul_dequantize_add_int4_int4t : quest_fused_matmul_dequantize_int4_int4t;
+        launched(f(dst.data_ptr(), q.codes, (const uint8_t *)w.packed->data_ptr(), q.row_sum, (const int32_t *)w.add->data_ptr(),
+                   q.scale, w.scale->data_ptr(), m, w.k, w.n, dt, st), "projection");
+    }
+}
+
+Codes quantised(const at::Tensor &x, int m, int k, bool tiles, c10::Device dev, int dt, void *st) {
+    Codes q(m, k, tiles, dev);
+    launched(tiles ? quest_hadamard_quantize_e2m3(x.data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, k, m, kHadamardEntry, dt, st)
+                   : quest_hadamard_quantize_int4(x.data_ptr(), q.scale, q.codes, q.row_sum, nullptr, k, m, kHadamardEntry, dt, st),
+             "activation kernel");
+    return q;
+}
+
+Codes normed(at::Tensor &x, const at::Tensor *branch, const at::Tensor &weight, double eps, int m, int k, bool tiles, c10::Device dev,
+             int dt, void *st) {
+    Codes q(m, k, tiles, dev);
+    int rc;
+    if (branch == nullptr)
+        rc = tiles ? quest_rmsnorm_hadamard_quantize_e2m3(x.data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, nullptr, k, m, kHadamardEntry, dt, st)
+                   : quest_rmsnorm_hadamard_quantize_int4(x.data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, q.row_sum, nullptr, nullptr, k, m, kHadamardEntry, dt, st);
+    else
+        rc = tiles ? quest_add_rmsnorm_hadamard_quantize_e2m3(x.data_ptr(), branch->data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, k, m, kHadamardEntry, dt, st)
+                   : quest_add_rmsnorm_hadamard_quantize_int4(x.data_ptr(), branch->data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, q.row_sum, k, m, kHadamardEntry, dt, st);
+    launched(rc, "norm kernel");
+    return q;
+}
+
+PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 14) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *xp = args.tensor(a[0]);
+    if (!args.ok || !is_half(xp->scalar_type()) || xp->dim() != 3) return declined();
+    const at::ScalarType type = xp->scalar_type();
+    const int64_t b = xp->size(0), t = xp->size(1), c64 = xp->size(2);
+    if (!fits_int(b * t) || !fits_int(3 * c64)) return declined();
+    const int m = (int)(b * t), c = (int)c64;
+    const at::Tensor *branch = a[1] == Py_None ? nullptr : args.tensor(a[1], type, xp->numel());
+    const long n_head = PyLong_AsLong(a[3]);
+    if (n_head <= 0 || c % n_head != 0) return declined();
+    const int head_dim = (int)(c / n_head);
+    const at::Tensor *freqs = args.tensor(a[2], at::kFloat, t * (head_dim / 2) * 2);
+    const at::Tensor *norm1 = args.tensor(a[4], type, c), *norm2 = args.tensor(a[6], type, c);
+    const double eps1 = PyFloat_AsDouble(a[5]), eps2 = PyFloat_AsDouble(a[7]);
+    const long tiles = PyLong_AsLong(a[13]);
+    Linear qkv, o, gate_up, glu, down;
+    if (!args.ok || PyErr_Occurred() || !qkv.take(args, a[8], type, tiles & 1) || !o.take(args, a[9], type, tiles & 2) ||
+        !gate_up.take(args, a[10], type, false) || !glu.take(args, a[11], type, tiles & 4) || !down.take(args, a[12], type, tiles & 8))
+        return declined();
+    const int hidden = down.k;
+    if (qkv.k != c || qkv.n != 3 * c || o.k != c || o.n != c || gate_up.k != c || gate_up.n != 2 * hidden || glu.k != c || glu.n != 2 * hidden ||
+        down.n != c || (c & 127) != 0 || (hidden & 127) != 0 || c > 32768 || hidden > 32768 || (hidden & 3) != 0 || (head_dim & 7) != 0)
+        return declined();
+
+    const c10::DeviceGuard guard(args.dev);
+    void *st = stream_of(args.dev);
+    const int dt = dtype_code(type);
+    at::Tensor x = *xp;
+
+    // norm -> q, k, v with q and k rotated
+    at::Tensor heads = make({m, 3 * c}, type, args.dev);
+    {
+        const Codes q = normed(x, branch, *norm1, eps1, m, c, qkv.tiles != nullptr, args.dev, dt, st);
+        const float *f = (const float *)freqs->data_ptr();
+        int rc = q.tiles ? (t >= 32 && head_dim % 32 == 0
+                                ? quest_fused_matmul_dequantize_rope_e2m3(heads.data_ptr(), q.codes, qkv.tiles->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st)
+                                : QUEST_ERR_UNSUPPORTED)
+                         : quest_fused_matmul_dequantize_rope_int4_int4t(heads.data_ptr(), q.codes, (const uint8_t *)qkv.packed->data_ptr(), q.row_sum, (const int32_t *)qkv.add->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st);
+        if (rc == QUEST_ERR_UNSUPPORTED || rc == QUEST_ERR_BAD_SHAPE) {        // nothing was launched: the two calls
+            project(qkv, q, heads, m, dt, st);
+            rc = quest_rope_interleaved(heads.data_ptr(), f, m, (int)t, 3 * c, 2 * c, head_dim, dt, st);
+        }
+        launched(rc, "QKV projection");
+    }
+    // causal attention
+    const int64_t row = 3 * c64;
+    const auto part = [&](int64_t i) { return heads.as_strided({b, n_head, t, head_dim}, {t * row, head_dim, row, 1}, i * c64); };
+    const at::Tensor y = at::scaled_dot_product_attention(part(0), part(1), part(2), {}, 0.0, true);
+    const at::Tensor core = y.transpose(1, 2).contiguous();
+    // output projection: into the residual stream where its GEMM can add
+    bool has_att = false;
+    at::Tensor att;
+    {
+        const Codes q = quantised(core, m, c, o.tiles != nullptr, args.dev, dt, st);
+        if (q.tiles || quest_fused_matmul_dequantize_add_available(m, c, c, st)) {
+            project(o, q, x, m, dt, st, true);
+        } else {
+            has_att = true;
+            att = make({m, c}, type, args.dev);
+            project(o, q, att, m, dt, st);
+        }
+    }
+    // norm -> gated unit -> its codes
+    const bool down_tiles = down.tiles != nullptr;
+    Codes act(m, hidden, down_tiles, args.dev);
+    {
+        const Codes q = normed(x, has_att ? &att : nullptr, *norm2, eps2, m, c, glu.tiles != nullptr, args.dev, dt, st);
+        if (!q.tiles && m <= 64) {
+            // the weight-streaming GEMM has no gated epilogue: gate and up side by side, the product inside the quantiser
+            at::Tensor both = make({m, 2 * hidden}, type, args.dev);
+            project(gate_up, q, both, m, dt, st);
+            launched(down_tiles ? quest_silu_mul_hadamard_quantize_e2m3(both.data_ptr(), act.scale, act.codes, nullptr, hidden, m, kHadamardEntry, dt, st)
+                                : quest_silu_mul_hadamard_quantize_int4(both.data_ptr(), act.scale, act.codes, act.row_sum, nullptr, nullptr, hidden, m, kHadamardEntry, dt, st),
+                     "gated unit");
+        } else {
+            at::Tensor gated = make({m, hidden}, type, args.dev);
+            launched(q.tiles ? quest_fused_matmul_dequantize_swiglu_e2m3(gated.data_ptr(), q.codes, glu.tiles->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st)
+                             : quest_fused_matmul_dequantize_swiglu_int4_int4t(gated.data_ptr(), q.codes, (const uint8_t *)glu.packed->data_ptr(), q.row_sum, (const int32_t *)glu.add->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st),
+                     "gated projection");
+            launched(down_tiles ? quest_hadamard_quantize_e2m3(gated.data_ptr(), act.scale, act.codes, nullptr, nullptr, nullptr, hidden, m, kHadamardEntry, dt, st)
+                                : quest_hadamard_quantize_int4(gated.data_ptr(), act.scale, act.codes, act.row_sum, nullptr, hidden, m, kHadamardEntry, dt, st),
+                     "activation kernel");
+        }
+    }
+    if (down_tiles || quest_fused_matmul_dequantize_add_available(m, hidden, c, st)) {
+        project(down, act, x, m, dt, st, true);
+        Py_RETURN_TRUE;
+    }
+    at::Tensor mlp = make({b, t, c64}, type, args.dev);
+    project(down, act, mlp, m, dt, st);
+    return wrap(std::move(mlp));
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef kMethods[] = {
+#define QUEST_FN(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
+    QUEST_FN(linear), QUEST_FN(gemm), QUEST_FN(matmul_int32), QUEST_FN(hadamard_quantize), QUEST_FN(hadamard128), QUEST_FN(find_scale), QUEST_FN(quantize), QUEST_FN(add_mul_vv), QUEST_FN(block),
+#undef QUEST_FN
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", "Native host path of quest_amd's hot calls.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&kModule); }

@@ -145,6 +145,13 @@ def linear_forward(activation, w_int_packed, w_scale, w_add, w_meta_e=None, out=
     if w_meta_e is not None:
         raise NotImplementedError('4:8-sparse weights are not part of this build')
     m, k, n = activation.size(0), activation.size(1), w_int_packed.size(0)
+    if w_tiles is not None and not prefers_e2m3(m, k, n):
+        w_tiles = None
+    if (_a_scale is None and _a_int_packed is None and _a_int_row_sum is None and _a_tiles is None
+            and not (quantize_from_fp32 and use_hadamard) and activation.dim() == 2):
+        done = quest.host.linear(activation, w_int_packed, w_scale, w_add, w_tiles, None, HADAMARD_ENTRY if use_hadamard else 0., out)
+        if done is not None:
+            return done
     dtype, device = activation.dtype, activation.device
     if out is None:
         out = torch.empty(m, n, dtype=dtype, device=device)
@@ -153,7 +160,7 @@ def linear_forward(activation, w_int_packed, w_scale, w_add, w_meta_e=None, out=
             activation, _a_scale, _a_int_packed, _a_int_row_sum, hadamard_scale=WEIGHT_HADAMARD_SCALE, from_fp32=True)
         return quest.fused_matmul_dequantize_int4_int4t_bf16(mat_a=a_int_packed, mat_b=w_int_packed, vec_a_add=a_int_row_sum,
                                                              vec_b_add=w_add, vec_a_mul=a_scale, vec_b_mul=w_scale, out=out)
-    if w_tiles is not None and prefers_e2m3(m, k, n):
+    if w_tiles is not None:
         a_scale, a_tiles = quest.hadamard_quantize_e2m3(activation, _a_scale, _a_tiles,
                                                         hadamard_scale=HADAMARD_ENTRY if use_hadamard else 0.)
         return quest.fused_matmul_dequantize_e2m3(a_tiles, w_tiles, a_scale, w_scale, k, out)
@@ -294,6 +301,15 @@ class Linear4bit(nn.Module):
         return y
 
     def forward(self, x) -> torch.Tensor:
+        n = self.weight.size(0)
+        if not self.use_noop and not self.quantize_from_fp32 and x.dim() > 0:
+            k = x.size(-1)
+            held = self._buffers
+            tiles = self.w_tiles() if prefers_e2m3(x.numel() // max(k, 1), k, n) else None
+            y = quest.host.linear(x, held['w_int_packed'], held['w_scale'], held['w_add'], tiles, self.bias,
+                                  HADAMARD_ENTRY if self.use_hadamard else 0., None)
+            if y is not None:
+                return y
         lead, n = x.shape[:-1], self.weight.size(0)
         rows = x.contiguous().view(-1, x.size(-1))
         if self.use_noop:

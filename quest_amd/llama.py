@@ -208,8 +208,11 @@ class LlamaBlock(nn.Module):
         added it already."""
         b, t, c = x.shape
         m = b * t
-        x2 = x.view(m, c)
         hidden = self.mlp.c_proj.weight.size(1)
+        done = self._forward_native(x, freqs_cis, branch, m, c, hidden)
+        if done is not None:
+            return x, (None if done is True else done)
+        x2 = x.view(m, c)
         # each producer writes the operand form its GEMM runs fastest on: E2M3 tiles for the FP6 kernel, or packed
         # nibbles and row sums for the INT8 kernels (same codes, same output bits either way)
         rotated = False
@@ -292,6 +295,34 @@ class LlamaBlock(nn.Module):
             return x, None
         y = self.mlp.c_proj.forward_tiles(*q) if down_tiles else self.mlp.c_proj.forward_quantized(*q)
         return x, y.view(b, t, c)
+
+
+    def _forward_native(self, x, freqs_cis, branch, m, c, hidden):
+        """`forward_fused` as one call of the native host path (the same kernels in the same order; at 37 tokens the
+        twelve launches of a block cost 240 us from Python and about 50 from there).  None, with nothing launched, where
+        an option is not at its default: the statement in Python then runs."""
+        attn, mlp = self.attn, self.mlp
+        linears = (attn.c_attn, attn.c_proj, mlp.w12, mlp.c_proj)
+        if not (mlp.glu is not None and attn.fused_rope and harness.GEMM_ADDS_RESIDUAL and harness.GEMM_ADDS_RESIDUAL_PACKED
+                and harness.GEMM_ROTATES_QK):
+            return None
+        for w in linears:
+            if not (type(w) is harness.Linear4bit and w.bias is None and w.use_hadamard and not w.use_noop
+                    and not w.quantize_from_fp32):
+                return None
+        tiles = (harness.prefers_e2m3(m, c, 3 * c) | harness.prefers_e2m3(m, c, c) << 1
+                 | harness.prefers_e2m3(m, c, 2 * hidden) << 2 | harness.prefers_e2m3(m, hidden, c) << 3)
+        if tiles & 4 and mlp.glu_tiles is None:
+            mlp.glu_tiles = harness.weight_tiles(mlp.glu[0])
+        qkv, o, both, down = (w._buffers for w in linears)
+        return quest.host.block(
+            x, branch, freqs_cis, attn.n_head, self.ln_1.weight, float(self.ln_1.eps), self.ln_2.weight, float(self.ln_2.eps),
+            (qkv['w_int_packed'], qkv['w_scale'], qkv['w_add'], attn.c_attn.w_tiles() if tiles & 1 else None),
+            (o['w_int_packed'], o['w_scale'], o['w_add'], attn.c_proj.w_tiles() if tiles & 2 else None),
+            (both['w_int_packed'], both['w_scale'], both['w_add'], None),
+            (*mlp.glu, mlp.glu_tiles),
+            (down['w_int_packed'], down['w_scale'], down['w_add'], mlp.c_proj.w_tiles() if tiles & 8 else None),
+            tiles)
 
 
 class Llama(nn.Module):

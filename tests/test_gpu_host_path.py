@@ -1,0 +1,64 @@
+"""The native host path (csrc/host.cpp) against the Python statements it stands in for: the same bits, the same errors.
+Declining every call makes the Python statements run."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda:0'
+
+
+class _DeclinesAll:
+    def __getattr__(self, _name):
+        return lambda *_: None
+
+
+@pytest.fixture
+def python_path(monkeypatch):
+    from quest_amd import api
+    return lambda: monkeypatch.setattr(api, 'host', _DeclinesAll())
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('lead,k,n,hadamard,bias', [((1,), 256, 64, True, False), ((3, 5), 384, 72, True, True), ((70,), 160, 33, False, True),
+                                                    ((512,), 2048, 8448, True, False), ((512,), 2048, 8448, False, True)])
+def test_linear_native_equals_python(python_path, dtype, lead, k, n, hadamard, bias):
+    from quest_amd import harness
+    g = torch.Generator(device=DEV).manual_seed(5)
+    w = (torch.randn(n, k, device=DEV, generator=g) * 0.02).to(dtype)
+    x = torch.randn(*lead, k, device=DEV, generator=g).to(dtype)
+    layer = harness.Linear4bit.from_weight(w, torch.randn(n, device=DEV, generator=g).to(dtype) if bias else None, use_hadamard=hadamard)
+    got = layer(x)
+    strided = layer(x.repeat_interleave(2, -1)[..., ::2])          # not contiguous: the native path declines
+    python_path()
+    want = layer(x)
+    assert got.shape == (*lead, n)
+    assert torch.equal(got, want) and torch.equal(strided, want)
+
+
+@pytest.mark.parametrize('batch,seq', [(1, 1), (1, 37), (3, 64), (2, 512)])
+def test_block_native_equals_python(python_path, batch, seq):
+    """Small, mid-sized and large-tile kernels, the packed and the tile form of the codes (hidden 2816, 256-wide tiles)."""
+    from quest_amd import llama
+    torch.manual_seed(3)
+    with torch.device(DEV):
+        net = llama.Llama(llama.LlamaConfig(n_layer=2, n_embd=2048, n_head=16, vocab_size=512)).to(torch.bfloat16).eval()
+        ids = torch.randint(0, 512, (batch, seq))
+    net = llama.quantize_model(net, 'int4', fuse_producers=True)
+    with torch.no_grad():
+        got = net(ids, all_logits=True)['logits']
+        python_path()
+        want = net(ids, all_logits=True)['logits']
+    assert torch.equal(got, want)
+
+
+def test_declined_calls_raise_as_before():
+    import quest_amd as quest
+    x = torch.zeros(4, 256, dtype=torch.bfloat16, device=DEV)
+    with pytest.raises(AssertionError):
+        quest.hadamard128(x, torch.empty(4, 128, dtype=torch.bfloat16, device=DEV))
+    with pytest.raises(AssertionError):
+        quest.find_scale_int4(x[:, ::2])
+    with pytest.raises(RuntimeError):
+        quest.find_scale_int4(x.view(-1)[4:1028 - 4].view(4, 255)[:, :252].contiguous()[:, :4].contiguous())
+    with pytest.raises(RuntimeError):
+        quest.quantize_int4(x, torch.ones(4, 1, dtype=torch.bfloat16, device='cpu'))
