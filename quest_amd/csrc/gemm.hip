@@ -12,10 +12,10 @@
 // This file holds the checks, the choice of kernel by shape and the C entry points; all kernels give bit-identical
 // results:
 //   gemm_decode.hip   gemm_w4a4_decode_kernel   a handful of tokens: the weights are streamed once;
-//   gemm_small.hip    gemm_w4a4_small_kernel    K % 256 == 0, a few hundred tokens: 64 x 64 or 128 x 128 tiles, K split
-//                                               inside the workgroup;
-//   gemm_big.hip      gemm_w4a4_big_kernel      K % 128 == 0: the prefill kernel, persistent 256 x 256 or 256 x 128 tiles;
-//   gemm_staged.hip   gemm_w4a4_staged_kernel   K % 32 == 0 (and scale vectors that are not 4-byte aligned): operands
+//   gemm_small.hip    gemm_w4a4_small_kernel    a few hundred tokens: 64 x 64 or 128 x 128 tiles, K split inside the
+//                                               workgroup;
+//   gemm_big.hip      gemm_w4a4_big_kernel      the prefill kernel, persistent 256 x 256 or 256 x 128 tiles;
+//   gemm_staged.hip   gemm_w4a4_staged_kernel   large problems whose scale vectors are not 4-byte aligned: operands
 //                                               staged through registers into int8 LDS tiles.
 #include "gemm_tiles.h"
 
@@ -44,8 +44,7 @@ static int gemm_check(const void *out, const uint8_t *a, const uint8_t *b, int M
 // small tile of 64 tokens per 64 channels from N > 4096 on (measured at N = 4608 .. 11264, K = 2048 and 4096: 8.3 -> 5.4 us,
 // 11.2 -> 7.6 us; at N = 4096 the weight-streaming kernel is 0.6 to 1.2 us faster), 17 to 32 tokens from N > 8192 on (up to
 // 2 x faster at N from 8192 to 28672).
-static int small_tile_shape(int M, int K, int N, int cus) {
-    if ((K & 255) != 0) return 0;
+static int small_tile_shape(int M, int N, int cus) {
     if (M <= 64) return (M > 32 ? N > 4096 : (M > 16 && N > 8192)) ? 64 : 0;
     const long tiles = (long)((M + 63) / 64) * ((N + 63) / 64);
     const long per_cu = (tiles + cus - 1) / cus;
@@ -63,9 +62,8 @@ static int small_tile_shape(int M, int K, int N, int cus) {
 static int gemm_launch_large(int out_kind, bool glu, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add,
                              const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, int cus,
                              hipStream_t st, const RopeArgs *rope = nullptr, bool add = false) {
-    const int small_shape = small_tile_shape(M, K, N, cus);
+    const int small_shape = add ? 0 : small_tile_shape(M, N, cus);       // the small tiles do not add into their output
     const int epi = add ? kEpiAdd : rope != nullptr ? kEpiRope : glu ? kEpiGlu : kEpiPlain;
-    if (small_shape != 0 && add) return QUEST_ERR_UNSUPPORTED;           // the small tiles do not add into their output
     if (small_shape != 0) return launch_gemm_small(out_kind, epi, small_shape, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st, rope);
     const int units = (N + 31) / 32;
     const int per_group = units >= 8 ? units / 8 : units;
@@ -80,20 +78,14 @@ static int gemm_launch(int out_kind, void *out, const uint8_t *a, const uint8_t 
                        const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st) {
     // the device is asked for its CU count once per call, and only where a rule below uses it (not for a handful of tokens)
     const int cus = M > 64 ? device_cu_count(st) : 0;
-    const int small_shape = small_tile_shape(M, K, N, cus);
+    const int small_shape = small_tile_shape(M, N, cus);
     if (small_shape != 0) return launch_gemm_small(out_kind, kEpiPlain, small_shape, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
-    // a handful of tokens: the weight-streaming kernel
-    // (up to 64 of them unless the small tiles took the call above; where K rules those out, up to 128 while its
-    // N / 16 workgroups still run as one round: twice as fast as large tiles that would be half empty)
-    if (M <= 64 || (M <= 128 && N <= 8192)) {
-        const int rc = launch_gemm_decode(out_kind, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
-        if (rc != QUEST_ERR_UNSUPPORTED) return rc;
-    }
+    // a handful of tokens (unless the small tiles took the call above): the weight-streaming kernel
+    if (M <= 64) return launch_gemm_decode(out_kind, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
     // the large-tile kernel fetches the 16-bit scale vectors two per dword: 4-byte aligned vectors
-    if ((K & 127) == 0 && M > 64 && aligned(b_mul, 4) && aligned(a_mul, 4))
+    if (aligned(b_mul, 4) && aligned(a_mul, 4))
         return gemm_launch_large(out_kind, false, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, cus, st);
-    // K % 128 != 0, or scale vectors at odd element offsets (a sliced tensor): the register-staged kernel reads them
-    // element by element
+    // scale vectors at odd element offsets (a sliced tensor): the register-staged kernel reads them element by element
     return launch_gemm_staged(out_kind, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
 }
 
@@ -215,7 +207,7 @@ extern "C" int quest_fused_matmul_dequantize_rope_int4_int4t(void *mat_d, const 
         return QUEST_ERR_BAD_SHAPE;
     if (!aligned(freqs_cis, 16)) return QUEST_ERR_ALIGNMENT;
     // the large-tile and the small-tile kernels have this epilogue (the sizes the plain entry point hands to them)
-    if ((size_k & 127) != 0 || size_m <= 64 || (size_m <= 128 && size_n <= 8192) || !aligned(vec_b_mul, 4) || !aligned(vec_a_mul, 4) ||
+    if ((size_k & 127) != 0 || size_m <= 64 || !aligned(vec_b_mul, 4) || !aligned(vec_a_mul, 4) ||
         !aligned(mat_d, 16))
         return QUEST_ERR_UNSUPPORTED;
     const RopeArgs rope = {freqs_cis, seq_len, rot_cols, head_dim};
@@ -224,9 +216,10 @@ extern "C" int quest_fused_matmul_dequantize_rope_int4_int4t(void *mat_d, const 
                              (hipStream_t)stream, &rope);
 }
 
-// Whether quest_fused_matmul_dequantize_add_int4_int4t runs this size in one launch (the large-tile kernel takes it)
+// Whether quest_fused_matmul_dequantize_add_int4_int4t runs this size in one launch.  Only the large-tile kernel adds into
+// its output; it does so where the small tiles would not be the faster kernel on whole stages (K % 256 == 0).
 static bool add_gemm_applies(int M, int K, int N, int cus) {
-    return (K & 127) == 0 && M > 64 && !(M <= 128 && N <= 8192) && small_tile_shape(M, K, N, cus) == 0;
+    return (K & 127) == 0 && M > 64 && !(M <= 128 && N <= 8192) && ((K & 255) != 0 || small_tile_shape(M, N, cus) == 0);
 }
 
 extern "C" int quest_fused_matmul_dequantize_add_available(int size_m, int size_k, int size_n, void *stream) {

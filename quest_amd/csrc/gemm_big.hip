@@ -1,4 +1,4 @@
-// Large-tile persistent packed-INT4 x packed-INT4 GEMM (K % 128 == 0): the prefill path.  Same arithmetic and outputs
+// Large-tile persistent packed-INT4 x packed-INT4 GEMM (K % 32 == 0): the prefill path.  Same arithmetic and outputs
 // as the other GEMM kernels (gemm-quest/quest/matmul_kernel.cu:8-63 and
 // gemm-quest/quest/fused_matmul_dequantize_kernel.cu:4-57 of the reference, with the functor
 // gemm-quest/include/symmetric/epilogue/thread/linear_combination_dequant.h:122-185).
@@ -62,6 +62,17 @@ __device__ __forceinline__ void loader_offsets(Loader &l, const Cursor &ld, int 
     l.off_c = (uint32_t)(ld.ch0 + l.wave * C::kChnRowsPerWave + row) * (uint32_t)l.kbytes + chunk * 16;
 }
 
+// A last stage that is not whole (K % 128 != 0): the lanes whose chunk lies past the end of its token row fetch from beyond
+// the buffer, which leaves zeros in LDS, and a zero token code cancels whatever the channel side holds there.  Applied
+// to the cursor's offset when it reaches that stage (its next tile sets the offset anew), so that the loads themselves
+// carry no test.
+__device__ __forceinline__ void loader_end_of_row(Loader &l, const Cursor &ld, int lane) {
+    if (ld.kt == l.nk - 1 && (l.kbytes & (kRowB - 1)) != 0) {
+        const int chunk = (lane & 3) ^ ((lane >> 4) & 3);
+        if (ld.kt * kRowB + chunk * 16 >= l.kbytes) l.off_t = 0x80000000u;
+    }
+}
+
 // The load cursor's stage goes into the next LDS slot as kLoads instructions per wave (loader_one: four of
 // 16 token rows, then those of 16 channel rows), issued a few MFMAs apart because each takes the CU's address path about
 // half an MFMA; loader_end then advances the cursor (into the next tile when this one is done; when nothing is
@@ -80,19 +91,20 @@ __device__ __forceinline__ void loader_one(const Loader &l, const Cursor &ld, ui
             l.wgt, (__attribute__((address_space(3))) void *)(sb + kTileB + (l.wave * C::kChnRowsPerWave + (j - 4) * 16) * kRowB), 16,
             l.off_c, kb + (j - 4) * step, 0, 0);
 }
-template <typename C>
+template <typename C, bool TAIL>
 __device__ __forceinline__ void loader_end(Loader &l, Cursor &ld) {
     l.issued++;
     if (++ld.kt == l.nk) {
         cursor_next_tile<C::kMaxUnits>(ld);
         if (ld.valid) loader_offsets<C>(l, ld, fresh_lane_id()); else ld.kt = l.nk - 1;
     }
+    if constexpr (TAIL) loader_end_of_row(l, ld, fresh_lane_id());
 }
-template <typename C>
+template <typename C, bool TAIL>
 __device__ __forceinline__ void loader_issue(Loader &l, Cursor &ld, uint8_t *lds) {
 #pragma unroll
     for (int j = 0; j < C::kLoads; j++) loader_one<C>(l, ld, lds, j);
-    loader_end<C>(l, ld);
+    loader_end<C, TAIL>(l, ld);
 }
 
 // at most kLoads * (kStages - 3) + extra younger memory operations may still be in flight
@@ -185,6 +197,7 @@ __device__ __forceinline__ void big_tile(uint8_t *lds, Cursor &ld, Loader &ldr, 
     constexpr bool GLU = EPI == kEpiGlu;
     constexpr bool ROPE = EPI == kEpiRope;
     constexpr bool ADD = EPI == kEpiAdd;
+    constexpr bool TAIL = EPI == kEpiPlain;      // (the other epilogues are for K % 128 == 0)
     static_assert(EPI == kEpiPlain || OUT != OUT_INT32, "epilogues on 16-bit outputs only");
     constexpr int NAX = NA > 0 ? NA : 1;
     // Lane coordinates are derived afresh in every phase (here, in the loader's cursor step, in the epilogue): a value
@@ -197,7 +210,7 @@ __device__ __forceinline__ void big_tile(uint8_t *lds, Cursor &ld, Loader &ldr, 
     const int tok_in_tile = TB == 4 ? (wave >> 1) * 128 : wave * 64;
     const int li = lane & 31;
     const int lg = lane >> 5;
-    const int nk = K / 128;
+    const int nk = (K + 127) / 128;
 
     // operand reads: row li of a 32-row sub-tile; the 16-byte chunk 2 j + lg of its 64-byte stage row (k-pair j)
     const int rd_t = (tok_in_tile + li) * kRowB;
@@ -256,10 +269,10 @@ __device__ __forceinline__ void big_tile(uint8_t *lds, Cursor &ld, Loader &ldr, 
             pp.clock = (unsigned)__builtin_amdgcn_s_memtime();       // read one stage later: never waited for
         }
     };
-    auto dma = [&](int j) { if (j < C::kLoads) loader_one<C>(ldr, ld, lds, j); else loader_end<C>(ldr, ld); };
+    auto dma = [&](int j) { if (j < C::kLoads) loader_one<C>(ldr, ld, lds, j); else loader_end<C, TAIL>(ldr, ld); };
     auto no_sync = []() {};
     if constexpr (NA == 0) {
-        for (int kt = 0; kt < nk; kt++) { sync(); loader_issue<C>(ldr, ld, lds); pp.it++; }
+        for (int kt = 0; kt < nk; kt++) { sync(); loader_issue<C, TAIL>(ldr, ld, lds); pp.it++; }
     } else {
         Frags u0, u1;
         {   // prologue: the first k-pair of the tile's first stage (landed: the previous synchronisation saw to it)
@@ -522,6 +535,7 @@ gemm_w4a4_big_kernel(void *__restrict__ out, const uint8_t *__restrict__ act, co
     // asm cuts the value loose from threadIdx, which would otherwise be kept (and spilled) to derive it again
     int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     asm volatile("" : "+s"(wave));
+    constexpr bool TAIL = EPI == kEpiPlain;
     const int wc = wave & 1;                     // channel half this wave multiplies
     const int kbytes = K >> 1;
 
@@ -543,14 +557,15 @@ gemm_w4a4_big_kernel(void *__restrict__ out, const uint8_t *__restrict__ act, co
     ldr.aadd = __builtin_amdgcn_make_buffer_rsrc((void *)a_add, 0, M * 4, 0x00020000);
     ldr.amul = __builtin_amdgcn_make_buffer_rsrc((void *)a_mul, 0, (M * 2 + 2) & ~3, 0x00020000);
     ldr.kbytes = kbytes;
-    ldr.nk = K / 128;
+    ldr.nk = (K + 127) / 128;
     ldr.wave = wave;
     ldr.issued = 0;
     loader_offsets<C>(ldr, ld, fresh_lane_id());
+    if constexpr (TAIL) loader_end_of_row(ldr, ld, fresh_lane_id());
 
     // ---- pipeline prologue: stages 0 .. kStages - 2 in flight, stage 0 landed
 #pragma unroll
-    for (int s = 0; s < C::kStages - 1; s++) loader_issue<C>(ldr, ld, lds);
+    for (int s = 0; s < C::kStages - 1; s++) loader_issue<C, TAIL>(ldr, ld, lds);
     wait_vmcnt_imm<C::kLoads * (C::kStages - 2)>();
     plain_barrier();
     Pipe pp;
@@ -616,7 +631,7 @@ static int launch_shape(bool duo, void *out, const uint8_t *a, const uint8_t *b,
 int launch_gemm_big(int out_kind, int epi, bool duo, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add,
                     const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, int cus, hipStream_t st,
                     const RopeArgs *rope_args) {
-    if ((K & 127) != 0 || cus <= 0 || (epi != kEpiPlain && out_kind == OUT_INT32)) return QUEST_ERR_UNSUPPORTED;
+    if ((K & (epi == kEpiPlain ? 31 : 127)) != 0 || cus <= 0 || (epi != kEpiPlain && out_kind == OUT_INT32)) return QUEST_ERR_UNSUPPORTED;
     if (epi == kEpiRope && rope_args == nullptr) return QUEST_ERR_NULL_POINTER;
     const RopeArgs rope = epi == kEpiRope ? *rope_args : RopeArgs{nullptr, 32, 0, 32};
 #define QUEST_BIG_EPI(E)                                                                                                            \

@@ -1,4 +1,4 @@
-// Packed-INT4 x packed-INT4 GEMM for a handful of tokens (M <= 128): the weight matrix is streamed
+// Packed-INT4 x packed-INT4 GEMM for a handful of tokens (M <= 64): the weight matrix is streamed
 // from HBM exactly once and that stream is the whole cost, so the kernel is laid out around it.
 //
 // Same arithmetic and outputs as the large GEMM (gemm-quest/quest/matmul_kernel.cu:8-63 and
@@ -41,7 +41,7 @@ __device__ __forceinline__ void split16(const v4i &p, v4i &even, v4i &odd) {
 
 // TM = token tiles of 16 (M <= 16 TM)
 template <int OUT, int TM>
-__global__ void __launch_bounds__(64 * kWaves, TM == 1 ? 8 : TM == 2 ? 4 : TM == 4 ? 2 : 1)
+__global__ void __launch_bounds__(64 * kWaves, TM == 1 ? 8 : TM == 2 ? 4 : 2)
 gemm_w4a4_decode_kernel(void *__restrict__ out, const uint8_t *__restrict__ act, const uint8_t *__restrict__ wgt,
                         const int32_t *__restrict__ a_add, const int32_t *__restrict__ b_add,
                         const uint16_t *__restrict__ a_mul, const uint16_t *__restrict__ b_mul, int M, int N, int K) {
@@ -94,10 +94,11 @@ gemm_w4a4_decode_kernel(void *__restrict__ out, const uint8_t *__restrict__ act,
             const int cb = c * kChunkB;
 #pragma unroll
             for (int hlf = 0; hlf < 2; hlf++) {
-                // a piece past the end of the row (chunk index too large, or the second half of a 64-byte tail) reads as zero
+                // a piece past the end of the row (chunk index too large, or a tail) reads as zero; the weights' lanes look at
+                // their own 16 bytes of it, and a zero weight cancels whatever the tokens hold there
                 const bool in_row = c < n_chunks && cb + 64 * hlf < row_b;
                 const uint32_t shift = (uint32_t)(cb + 64 * hlf);
-                wq[i][hlf] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, (int)(in_row ? w_off + shift : dead), 0, 0));
+                wq[i][hlf] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wr, (int)(c < n_chunks && cb + 64 * hlf + g * 16 < row_b ? w_off + shift : dead), 0, 0));
 #pragma unroll
                 for (int t = 0; t < TM; t++)
                     aq[i][t][hlf] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ar, (int)(in_row ? a_off[t] + shift : dead), 0, 0));
@@ -323,8 +324,7 @@ static int launch_out(void *out, const uint8_t *a, const uint8_t *b, const int32
                       const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st) {
     if (M <= 16) launch_tm<OUT, 1>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
     else if (M <= 32) launch_tm<OUT, 2>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
-    else if (M <= 64) launch_tm<OUT, 4>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
-    else launch_tm<OUT, 8>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
+    else launch_tm<OUT, 4>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
     return launch_status();
 }
 
@@ -375,10 +375,10 @@ int launch_gemm_decode_splitk(int out_kind, void *out, const uint8_t *a, const u
     return launch_status();
 }
 
-// The weight-streaming kernel applies to M <= 128 and K a multiple of 128 (whole 64-byte pieces); QUEST_ERR_UNSUPPORTED otherwise.
+// The weight-streaming kernel applies to M <= 64 and K a multiple of 32 (whole 16-byte pieces); QUEST_ERR_UNSUPPORTED otherwise.
 int launch_gemm_decode(int out_kind, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add,
                        const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st) {
-    if (M > 128 || (K & 127) != 0 || !aligned(a, 16) || !aligned(b, 16)) return QUEST_ERR_UNSUPPORTED;
+    if (M > 64 || (K & 31) != 0 || !aligned(a, 16) || !aligned(b, 16)) return QUEST_ERR_UNSUPPORTED;
     switch (out_kind) {
         case OUT_BF16: return decode::launch_out<OUT_BF16>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
         case OUT_FP16: return decode::launch_out<OUT_FP16>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);

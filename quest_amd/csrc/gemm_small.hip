@@ -1,4 +1,4 @@
-// Small-tile packed-INT4 x packed-INT4 GEMM (K % 256 == 0): a few hundred tokens.  Same arithmetic and outputs as the
+// Small-tile packed-INT4 x packed-INT4 GEMM (K % 32 == 0): a few hundred tokens.  Same arithmetic and outputs as the
 // other GEMM kernels (gemm-quest/quest/matmul_kernel.cu:8-63 and gemm-quest/quest/fused_matmul_dequantize_kernel.cu:4-57
 // of the reference).
 //
@@ -12,6 +12,9 @@
 // large-tile kernel: packed bytes HBM -> LDS by direct loads (stages of 256 k = two sub-stages of 64-byte rows,
 // each wave bringing 16 token or channel rows), 16 packed bytes per lane per k-pair, split into the int8 vectors of
 // 16 * even-k and 16 * odd-k nibbles for two MFMA k-steps.
+// K need not be whole stages: in the last stage the lanes whose 16-byte chunk lies past the end of its token row fetch
+// from beyond the buffer, which leaves zeros in LDS, and a zero token code cancels whatever the channel side holds
+// there.  (K = 1376, M = 333, N = 4096, fp16: 57 us on the register-staged kernel.)
 #include "gemm_tiles.h"
 
 namespace quest {
@@ -68,7 +71,7 @@ gemm_w4a4_small_kernel(void *__restrict__ out, const uint8_t *__restrict__ act, 
     if (ct >= tiles_c) return;                                   // uniform: the whole workgroup
     const int tok0 = tt * S::kTok, ch0 = ct * S::kChn;
     const int kbytes = K >> 1;
-    const int nk = K / 256;
+    const int nk = (K + 255) / 256;
 
     // ---- loads: waves 0-3 bring the token rows, waves 4-7 the channel rows of each sub-stage, kLoads groups of 16 each
     const bool ld_tok = wave < 4;
@@ -78,15 +81,24 @@ gemm_w4a4_small_kernel(void *__restrict__ out, const uint8_t *__restrict__ act, 
     const int ld_row0 = (wave & 3) * S::kLoads * 16;
     const uint32_t voff = (uint32_t)((ld_tok ? tok0 : ch0) + ld_row0 + (lane >> 2)) * (uint32_t)kbytes +
                           (uint32_t)(((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+    // the same two offsets for the last stage
+    uint32_t voff_end[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const bool past = ld_tok && (nk - 1) * 128 + h * 64 + ((lane & 3) ^ ((lane >> 4) & 3)) * 16 >= kbytes;
+        voff_end[h] = past ? 0x80000000u : voff;                 // operands are smaller than 2^31 bytes
+    }
     uint8_t *const dst0 = lds + (ld_tok ? 0 : S::kTok * kRowB) + ld_row0 * kRowB;
     auto issue = [&](int kt, int slot) {
+        const bool end = kt == nk - 1;
+        const uint32_t v0 = end ? voff_end[0] : voff, v1 = end ? voff_end[1] : voff;
 #pragma unroll
         for (int j = 0; j < S::kLoads; j++) {
             uint8_t *d = dst0 + slot * S::kStageB + j * 16 * kRowB;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void *)d, 16,
-                                                     voff + (uint32_t)(j * 16 * kbytes), kt * 128, 0, 0);
+                                                     v0 + (uint32_t)(j * 16 * kbytes), kt * 128, 0, 0);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void *)(d + S::kHalfB), 16,
-                                                     voff + (uint32_t)(j * 16 * kbytes), kt * 128 + 64, 0, 0);
+                                                     v1 + (uint32_t)(j * 16 * kbytes), kt * 128 + 64, 0, 0);
         }
     };
 
@@ -276,7 +288,7 @@ static int launch_shape(int shape, void *out, const uint8_t *a, const uint8_t *b
 int launch_gemm_small(int out_kind, int epi, int shape, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add,
                       const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st,
                       const RopeArgs *rope_args) {
-    if ((K & 255) != 0 || (shape != 64 && shape != 128) || (epi != kEpiPlain && out_kind == OUT_INT32)) return QUEST_ERR_UNSUPPORTED;
+    if ((K & 31) != 0 || (shape != 64 && shape != 128) || (epi != kEpiPlain && out_kind == OUT_INT32)) return QUEST_ERR_UNSUPPORTED;
     if (epi == kEpiRope && (rope_args == nullptr || (N & 7) != 0 || !aligned(out, 16))) return QUEST_ERR_UNSUPPORTED;
     const RopeArgs rope = epi == kEpiRope ? *rope_args : RopeArgs{nullptr, 32, 0, 32};
 #define QUEST_SMALL_EPI(E)                                                                                                   \

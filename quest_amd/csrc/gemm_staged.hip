@@ -1,5 +1,5 @@
-// Register-staged packed-INT4 x packed-INT4 GEMM: the path for K % 128 != 0 (K % 32 == 0) and for scale vectors that
-// are not 4-byte aligned.  Same arithmetic and outputs as the other GEMM kernels (gemm-quest/quest/matmul_kernel.cu:8-63
+// Register-staged packed-INT4 x packed-INT4 GEMM (K % 32 == 0): the path for large problems whose scale vectors are not
+// 4-byte aligned.  Same arithmetic and outputs as the other GEMM kernels (gemm-quest/quest/matmul_kernel.cu:8-63
 // and gemm-quest/quest/fused_matmul_dequantize_kernel.cu:4-57 of the reference).
 //
 // A workgroup of four waves owns a 256-token x 256-channel tile; each wave a 128 x 128

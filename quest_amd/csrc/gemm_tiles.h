@@ -97,13 +97,13 @@ __device__ __forceinline__ void split16(const v4i &p, v4i &even, v4i &odd) {
     }
 }
 
-// gemm_big.hip: the large-tile kernel (K % 128 == 0, 4-byte aligned scale vectors); `duo` picks two workgroups of
+// gemm_big.hip: the large-tile kernel (K % 32 == 0, or 128 with an epilogue; 4-byte aligned scale vectors); `duo` picks two workgroups of
 // 256 x 128 tiles per CU instead of one of 256 x 256, `epi` the epilogue (kEpiPlain, or on 16-bit outputs kEpiGlu or
 // kEpiRope with its arguments in `rope`), `cus` the device's CU count (the persistent grid's size)
 int launch_gemm_big(int out_kind, int epi, bool duo, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add,
                     const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, int cus, hipStream_t st,
                     const RopeArgs *rope = nullptr);
-// gemm_small.hip: tiles of `shape` x `shape` (64 or 128), K % 256 == 0; `epi` as above
+// gemm_small.hip: tiles of `shape` x `shape` (64 or 128), K % 32 == 0; `epi` as above
 int launch_gemm_small(int out_kind, int epi, int shape, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add,
                       const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st,
                       const RopeArgs *rope = nullptr);
