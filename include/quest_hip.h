@@ -296,7 +296,7 @@ int quest_fused_matmul_dequantize_add_available(int size_m, int size_k, int size
  * before it is stored (`self.c_attn(x)` followed by `apply_rotary_emb(q, k, freqs_cis)`, src/models/llama.py:134-140 and
  * 43-62, in one launch), on packed codes: arguments and limits as quest_fused_matmul_dequantize_rope_e2m3 below.  The
  * large-tile and the small-tile kernels have this epilogue: QUEST_ERR_UNSUPPORTED (nothing launched) for the sizes the plain
- * entry point gives to another kernel (size_m <= 64, size_m <= 128 with size_n <= 8192, size_k % 128 != 0, scale vectors or
+ * entry point gives to another kernel (size_m <= 64, size_k % 128 != 0, scale vectors or
  * output not 4- / 16-byte aligned) -- make the two calls then.
  */
 int quest_fused_matmul_dequantize_rope_int4_int4t(void *mat_d, const uint8_t *mat_a, const uint8_t *mat_b,
@@ -354,6 +354,29 @@ int quest_add_rmsnorm_hadamard_quantize_e2m3(void *x, const void *branch, const 
                                              float had_scale, int dtype, void *stream);
 int quest_silu_mul_hadamard_quantize_e2m3(const void *gate_up, void *scale, void *x_tiles, void *x_act, int group_size,
                                           int batch_size, float had_scale, int dtype, void *stream);
+
+/*
+ * A weight (size_n, size_k) dtype packed for the GEMMs above: w_scale (size_n), w_int_packed (size_n, size_k / 2) and
+ * w_add (size_n) int32 = row sum of the codes + size_k / 2, in one pass (preprocess_weight, benchmarks/utils.py:20-53).  had_scale,
+ * scale_rule and limits as in quest_hadamard_quantize_int4_rule.
+ */
+int quest_pack_weight_int4(const void *weight, void *w_scale, uint8_t *w_int_packed, int32_t *w_add, int size_k, int size_n,
+                           float had_scale, int scale_rule, int dtype, void *stream);
+
+/*
+ * RMSNorm of n_rows rows of `cols` elements, row_stride elements apart (the last position of every sequence of a (B, T, C)
+ * tensor: x = its first such row, row_stride = T * C): out (n_rows, cols) = norm of x, or of dtype(x + branch) when branch is
+ * given (src/models/llama.py:65-77, 175-176).  cols and row_stride even, pointers 4-byte aligned.
+ */
+int quest_rmsnorm_rows(void *out, const void *x, const void *branch, const void *norm_weight, float eps, int n_rows,
+                       long row_stride, int cols, int dtype, void *stream);
+
+/*
+ * out (size_m, size_n) dtype = x (size_m, size_k) * weight (size_n, size_k)^T in 16-bit floats with fp32 accumulation: the dense
+ * language-model head (src/models/llama.py:253-262) on a few rows.  size_m <= 64 (QUEST_ERR_UNSUPPORTED above), size_k % 64
+ * == 0, x and weight 16-byte aligned.
+ */
+int quest_dense_rows(void *out, const void *x, const void *weight, int size_m, int size_k, int size_n, int dtype, void *stream);
 
 #ifdef __cplusplus
 }

@@ -304,10 +304,11 @@ int launch_gemm_decode_splitk(int out_kind, void *out, const uint8_t *a, const u
 size_t gemm_decode_workspace_bytes(int K, int N);
 
 // hadamard_mfma.hip: the matrix-core fused activation kernel, optionally with the producer of the activation in
-// front (pre: 0 none, 1 RMSNorm, 2 SiLU(gate) * up); QUEST_ERR_UNSUPPORTED when it does not apply
+// front (pre: 0 none, 1 RMSNorm, 2 SiLU(gate) * up); sum_bias is added to every row sum.  QUEST_ERR_UNSUPPORTED when it does
+// not apply
 int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, float eps, void *scale, uint8_t *packed,
                                   int32_t *row_sum, void *x_had, void *pre_out, int K, int M, float had_scale, int dtype,
-                                  hipStream_t st, const void *add_in = nullptr, void *sum_out = nullptr, uint8_t *tiles = nullptr);
+                                  hipStream_t st, const void *add_in = nullptr, void *sum_out = nullptr, uint8_t *tiles = nullptr, int sum_bias = 0);
 
 inline int check_dtype(int dtype) { return dtype == QUEST_DTYPE_BF16 || dtype == QUEST_DTYPE_FP16; }
 inline int aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }

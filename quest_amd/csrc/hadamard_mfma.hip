@@ -117,7 +117,7 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
                               uint16_t *__restrict__ scale, uint32_t *__restrict__ packed, int32_t *__restrict__ row_sum,
                               uint16_t *__restrict__ x_had, uint16_t *__restrict__ pre_out, const uint16_t *add_in,
                               uint16_t *sum_out, uint8_t *__restrict__ tiles, int xcd_chunk, int K, int M, int ldx,
-                              uint32_t entry_bits, float eps) {
+                              uint32_t entry_bits, float eps, int sum_bias) {
     static_assert(WPR == 1 || G == 32, "rows shared by waves: whole waves");
     using Sh = Shape<WPR, G, TL>;
     constexpr int kRows = Sh::kRows;
@@ -455,7 +455,7 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
 #pragma unroll
             for (int w = 0; w < WPR; w++) t += part_sum[row_local * WPR + w];
         }
-        if (writer) row_sum[row] = t;
+        if (writer) row_sum[row] = t + sum_bias;
     }
 }
 
@@ -491,6 +491,7 @@ struct Args {
     uint32_t bits;
     float eps;
     hipStream_t st;
+    int sum_bias;
     int cus;                   // compute units of the device (only looked at when tiles are written)
 };
 
@@ -506,7 +507,7 @@ static void launch_shape_as(const Args &a) {
     hq::hadamard_quantize_mfma_kernel<DT, WPR, G, PRE, TL><<<dim3(grid), dim3(64 * Sh::kWaves), 0, a.st>>>(
         (const uint16_t *)a.x, (const uint16_t *)a.norm_w, (uint16_t *)a.scale, (uint32_t *)a.packed, a.row_sum,
         (uint16_t *)a.x_had, (uint16_t *)a.pre_out, (const uint16_t *)a.add_in, (uint16_t *)a.sum_out, a.tiles, xcd_chunk,
-        a.K, a.M, a.ldx, a.bits, a.eps);
+        a.K, a.M, a.ldx, a.bits, a.eps, a.sum_bias);
 }
 
 // Tiles go through the workgroup's LDS where a workgroup of eight (four) rows fits -- rows of 8 to 96 blocks -- and where
@@ -573,7 +574,7 @@ static void launch_dtype(int pre, const Args &a) {
 // with x a (M, 2 K) tensor.  tiles: the codes as E2M3 tiles (M rows; besides or instead of packed nibbles).
 int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, float eps, void *scale, uint8_t *packed,
                                   int32_t *row_sum, void *x_had, void *pre_out, int K, int M, float had_scale, int dtype,
-                                  hipStream_t st, const void *add_in, void *sum_out, uint8_t *tiles) {
+                                  hipStream_t st, const void *add_in, void *sum_out, uint8_t *tiles, int sum_bias) {
     uint32_t bits = 0;
     // (had_scale == 0: no transform; the kernel then only moves the chunks between lanes)
     if (K > 32768 || (K & 127) || had_scale < 0.f || !representable16(had_scale, dtype, &bits)) return QUEST_ERR_UNSUPPORTED;
@@ -595,7 +596,7 @@ int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, fl
         };
         const Args a = {at(x, ldx, es), norm_w, at(scale, 1, es), (uint8_t *)at(packed, K / 2, 1), (int32_t *)at(row_sum, 1, 4),
                         at(x_had, K, es), at(pre_out, K, es), at(add_in, K, es), at(sum_out, K, es),
-                        tiles == nullptr ? nullptr : tiles + (size_t)(r0 / 32) * (size_t)(K / 64) * 1536, K, rows, ldx, bits, eps, st, cus};
+                        tiles == nullptr ? nullptr : tiles + (size_t)(r0 / 32) * (size_t)(K / 64) * 1536, K, rows, ldx, bits, eps, st, sum_bias, cus};
         if (dtype == QUEST_DTYPE_BF16) launch_dtype<0>(pre, a);
         else launch_dtype<1>(pre, a);
     }

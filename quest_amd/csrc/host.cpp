@@ -221,6 +221,30 @@ PyObject *hadamard_quantize(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
+// ---- pack_weight(weight, had_scale, rule) -> (packed, scale, add) ------------------------------------------------------
+PyObject *pack_weight(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 3) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *w = args.tensor(a[0]);
+    if (!args.ok || !is_half(w->scalar_type()) || w->dim() != 2) return declined();
+    const at::ScalarType type = w->scalar_type();
+    const int64_t n = w->size(0), k = w->size(1);
+    if (!fits_int(n) || !fits_int(k)) return declined();
+    const c10::DeviceGuard guard(args.dev);
+    at::Tensor packed = make({n, k / 2}, at::kByte, args.dev), scale = make({n, 1}, type, args.dev), add = make({n, 1}, at::kInt, args.dev);
+    const int rc = quest_pack_weight_int4(w->data_ptr(), scale.data_ptr(), (uint8_t *)packed.data_ptr(), (int32_t *)add.data_ptr(), (int)k, (int)n,
+                                          (float)PyFloat_AsDouble(a[1]), (int)PyLong_AsLong(a[2]), dtype_code(type), stream_of(args.dev));
+    if (rc != QUEST_OK) return declined();
+    PyObject *t = PyTuple_New(3);
+    if (t == nullptr) return nullptr;
+    PyTuple_SET_ITEM(t, 0, wrap(std::move(packed)));
+    PyTuple_SET_ITEM(t, 1, wrap(std::move(scale)));
+    PyTuple_SET_ITEM(t, 2, wrap(std::move(add)));
+    return t;
+    END_HANDLE_TH_ERRORS
+}
+
 // ---- hadamard128(x, out, had_scale) ----------------------------------------------------------------------------------
 PyObject *hadamard128(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (n_args != 3) return declined();
@@ -463,9 +487,37 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
+// ---- last_logits(x, branch, norm_w, eps, head_w) -> (B, 1, V) ----------------------------------------------------------
+// Final norm and language-model head for the last position of every sequence of x (B, T, C); branch: None, or what is still to be
+// added to x.
+PyObject *last_logits(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    if (n_args != 5) return declined();
+    HANDLE_TH_ERRORS
+    Args args;
+    const at::Tensor *x = args.tensor(a[0]);
+    if (!args.ok || !is_half(x->scalar_type()) || x->dim() != 3) return declined();
+    const at::ScalarType type = x->scalar_type();
+    const int64_t b = x->size(0), t = x->size(1), c = x->size(2);
+    const at::Tensor *branch = a[1] == Py_None ? nullptr : args.tensor(a[1], type, x->numel());
+    const at::Tensor *norm_w = args.tensor(a[2], type, c), *head = args.tensor(a[4]);
+    const double eps = PyFloat_AsDouble(a[3]);
+    if (!args.ok || head->scalar_type() != type || head->dim() != 2 || head->size(1) != c || b > 64 || (c & 63) != 0 || !fits_int(head->size(0)))
+        return declined();
+    const c10::DeviceGuard guard(args.dev);
+    void *st = stream_of(args.dev);
+    const int64_t v = head->size(0), last = (t - 1) * c * 2;
+    at::Tensor normed = make({b, c}, type, args.dev), logits = make({b, 1, v}, type, args.dev);
+    int rc = quest_rmsnorm_rows(normed.data_ptr(), (const uint8_t *)x->data_ptr() + last, branch ? (const uint8_t *)branch->data_ptr() + last : nullptr,
+                                norm_w->data_ptr(), (float)eps, (int)b, (long)(t * c), (int)c, dtype_code(type), st);
+    if (rc == QUEST_OK) rc = quest_dense_rows(logits.data_ptr(), normed.data_ptr(), head->data_ptr(), (int)b, (int)c, (int)v, dtype_code(type), st);
+    if (rc != QUEST_OK) return declined();
+    return wrap(std::move(logits));
+    END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef kMethods[] = {
 #define QUEST_FN(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
-    QUEST_FN(linear), QUEST_FN(gemm), QUEST_FN(matmul_int32), QUEST_FN(hadamard_quantize), QUEST_FN(hadamard128), QUEST_FN(find_scale), QUEST_FN(quantize), QUEST_FN(add_mul_vv), QUEST_FN(block),
+    QUEST_FN(linear), QUEST_FN(gemm), QUEST_FN(matmul_int32), QUEST_FN(hadamard_quantize), QUEST_FN(pack_weight), QUEST_FN(hadamard128), QUEST_FN(find_scale), QUEST_FN(quantize), QUEST_FN(add_mul_vv), QUEST_FN(block), QUEST_FN(last_logits),
 #undef QUEST_FN
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", "Native host path of quest_amd's hot calls.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -19,17 +19,31 @@ namespace quest {
 // lane xor 1, 2, 4, 8.  Each butterfly is (a, b) -> (a + b, a - b) with `a` the element at the
 // lower index, so the result is the same bit pattern as the textbook in-place loop.
 // ---------------------------------------------------------------------------------------------
-template <int M>
-__device__ __forceinline__ void fwht_lane_stage(float (&v)[8], uint32_t sign) {
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        float other = lane_xor_f<M>(v[e]);
-        float self = __uint_as_float(__float_as_uint(v[e]) ^ sign);   // -own on the upper lane
-        v[e] = self + other;                                            // lower: a + b, upper: a - b
-    }
-}
+// One stage across lanes for the chunk's eight values: v <- v + sign * v[partner], one DPP multiply-add each (sign = -1 on the
+// upper lane of a pair, whose difference so comes out negated: b - a for a - b; the caller turns it back once for all
+// stages).  sign * v is exact, so every value is the textbook sum or difference, rounded once.  The leading s_nop covers
+// the two wait states a DPP read needs after the write of its register, which the compiler does not track through asm.
+#define QUEST_FWHT_STAGE(CTRL)                                                                                                    \
+    asm("s_nop 1\n\t"                                                                                                             \
+        "v_fmac_f32_dpp %0, %0, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %1, %1, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %2, %2, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %3, %3, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %4, %4, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %5, %5, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %6, %6, %8 " CTRL " row_mask:0xf bank_mask:0xf\n\t"                                                       \
+        "v_fmac_f32_dpp %7, %7, %8 " CTRL " row_mask:0xf bank_mask:0xf"                                                           \
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])                          \
+        : "v"(sign))
 
-__device__ __forceinline__ void fwht128_chunk(float (&v)[8], int lane) {
+// Which of the 16 chunks of its block a lane works on: chunk lane % 16 with its two low bits flipped on the lanes whose bit 2
+// is set.  The chunk at distance 4 is then eight lanes' mirror image (row_half_mirror), a DPP move like the other distances,
+// where lane xor 4 would be a trip through the LDS crossbar.
+__device__ __forceinline__ int fwht_chunk_of(int i) { return i ^ ((i & 4) != 0 ? 3 : 0); }
+
+// The unscaled transform of a block whose lanes hold the chunks above, with `factor` as what the results have yet to be
+// multiplied by: had_scale, negated on the lanes whose values the stages left negated (scaled() below).
+__device__ __forceinline__ void fwht128_chunk(float (&v)[8], int lane, float had_scale, float &factor) {
 #pragma unroll
     for (int h = 1; h < 8; h <<= 1) {
 #pragma unroll
@@ -41,11 +55,20 @@ __device__ __forceinline__ void fwht128_chunk(float (&v)[8], int lane) {
             }
         }
     }
-    fwht_lane_stage<1>(v, (lane & 1) ? 0x80000000u : 0u);
-    fwht_lane_stage<2>(v, (lane & 2) ? 0x80000000u : 0u);
-    fwht_lane_stage<4>(v, (lane & 4) ? 0x80000000u : 0u);
-    fwht_lane_stage<8>(v, (lane & 8) ? 0x80000000u : 0u);
+    const int c = fwht_chunk_of(lane);
+    float sign = (c & 1) ? -1.f : 1.f;
+    QUEST_FWHT_STAGE("quad_perm:[1,0,3,2]");
+    sign = (c & 2) ? -1.f : 1.f;
+    QUEST_FWHT_STAGE("quad_perm:[2,3,0,1]");
+    sign = (c & 4) ? -1.f : 1.f;
+    QUEST_FWHT_STAGE("row_half_mirror");
+    sign = (c & 8) ? -1.f : 1.f;
+    QUEST_FWHT_STAGE("row_ror:8");
+    factor = (__builtin_popcount(c & 15) & 1) ? -had_scale : had_scale;
 }
+
+// A product that turns no zero negative: a difference of equals is +0 in the textbook order, whatever lane it was taken on.
+__device__ __forceinline__ float scaled(float v, float factor) { return __builtin_fmaf(v, factor, 0.f); }
 
 template <int DT>
 __device__ __forceinline__ void unpack8(const uint4 &raw, float (&v)[8]) {
@@ -80,55 +103,63 @@ __device__ __forceinline__ uint32_t pack_nibbles8(const float (&q)[8], int &sum)
 // ---------------------------------------------------------------------------------------------
 // Fused Hadamard + scale + quantise + pack: one workgroup per row, NCHUNK 16-byte chunks per
 // thread, the row lives in registers between its single read and its writes.
+// Vector instructions bound it, not memory: at about 34 per element it took 36.5 us for bf16 [11008, 4096] (113 MB, 3.1 TB/s);
+// with the DPP multiply-add stages, the clamp-free quantiser and the dot-product row sum it is about 16.
+// FP32 (QUEST_QUANT_FROM_FP32): scale and codes come from the transform's fp32 output and the unrounded scale -- the
+// arithmetic of the reference's evaluation-side fake quantiser (src/eval_hswag.py:201-214), which never holds the
+// rotated tensor in 16 bits -- instead of from the dtype-rounded tensor the inference path materialises.
 // ---------------------------------------------------------------------------------------------
-template <int DT, int NCHUNK, int BLOCK>
+template <int DT, int NCHUNK, int BLOCK, bool FP32>
 __global__ void __launch_bounds__(BLOCK)
 hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ scale,
                          uint32_t *__restrict__ packed, int32_t *__restrict__ row_sum,
-                         uint16_t *__restrict__ x_had, int K, float had_scale, int scale_rule) {
+                         uint16_t *__restrict__ x_had, int K, float had_scale, int scale_rule, int sum_bias) {
     __shared__ float slots_f[BLOCK / 64];
     __shared__ int slots_i[BLOCK / 64];
     const int row = blockIdx.x;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int nchunks = K >> 3;
+    const int chunk0 = had_scale != 0.f ? fwht_chunk_of(tid) : tid;         // blocks of 16 chunks: a row holds whole ones
     const uint4 *xr = reinterpret_cast<const uint4 *>(x + (size_t)row * K);
-    // QUEST_QUANT_FROM_FP32: scale and codes come from the transform's fp32 output and the unrounded scale -- the
-    // arithmetic of the reference's evaluation-side fake quantiser (src/eval_hswag.py:201-214), which never holds the
-    // rotated tensor in 16 bits -- instead of from the dtype-rounded tensor the inference path materialises
-    const bool from_fp32 = (scale_rule & QUEST_QUANT_FROM_FP32) != 0;
-    scale_rule &= ~QUEST_QUANT_FROM_FP32;
+    const bool absmax = scale_rule == QUEST_SCALE_ABSMAX;
 
     uint4 raw[NCHUNK];
 #pragma unroll
     for (int i = 0; i < NCHUNK; i++) {
-        const int c = i * BLOCK + tid;
+        const int c = i * BLOCK + chunk0;
         raw[i] = (c < nchunks) ? xr[c] : make_uint4(0, 0, 0, 0);
     }
 
-    float y[NCHUNK][8];
+    float y[FP32 ? NCHUNK : 1][8];
     float sumsq = 0.f, amax = 0.f;
 #pragma unroll
     for (int i = 0; i < NCHUNK; i++) {
-        unpack8<DT>(raw[i], y[i]);
+        float (&v)[8] = y[FP32 ? i : 0];
+        unpack8<DT>(raw[i], v);
         if (had_scale != 0.f) {
-            fwht128_chunk(y[i], lane);
+            float factor;
+            fwht128_chunk(v, lane, had_scale, factor);
 #pragma unroll
-            for (int e = 0; e < 8; e++) y[i][e] *= had_scale;
-            raw[i] = pack8<DT>(y[i]);           // the transform's output exists only in dtype ...
-            if (!from_fp32) unpack8<DT>(raw[i], y[i]);     // ... unless the caller asks for the fp32 one to be quantised
+            for (int e = 0; e < 8; e++) v[e] = scaled(v[e], factor);
+            raw[i] = make_uint4(pack2_rounded_products<DT>(v[0], v[1]), pack2_rounded_products<DT>(v[2], v[3]),
+                                pack2_rounded_products<DT>(v[4], v[5]), pack2_rounded_products<DT>(v[6], v[7]));
+            if (!FP32) unpack8<DT>(raw[i], v);  // the transform's output exists only in dtype
         }
+        // the squares of 16-bit floats are exact in fp32: the multiply-add rounds as multiply and add would (the fp32
+        // transform's squares are not, and stay separate)
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            sumsq += y[i][e] * y[i][e];         // squares of 16-bit floats are exact in fp32
-            amax = fmaxf(amax, fabsf(y[i][e]));
+        for (int e = 0; e < 8; e++) sumsq = FP32 ? sumsq + v[e] * v[e] : __builtin_fmaf(v[e], v[e], sumsq);
+        if (absmax) {                           // uniform
+#pragma unroll
+            for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
         }
     }
     if (x_had != nullptr) {
         uint4 *hr = reinterpret_cast<uint4 *>(x_had + (size_t)row * K);
 #pragma unroll
         for (int i = 0; i < NCHUNK; i++) {
-            const int c = i * BLOCK + tid;
+            const int c = i * BLOCK + chunk0;
             if (c < nchunks) hr[c] = raw[i];
         }
     }
@@ -136,7 +167,7 @@ hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ 
     // QUEST_SCALE_GAUSSIAN: the reference's rule from the row's mean square; QUEST_SCALE_ABSMAX: the row's largest
     // magnitude sits 7.5 steps out (a maximum is exact whatever the order, so this scale has no rounding slack)
     float s32;
-    if (scale_rule == QUEST_SCALE_ABSMAX) {
+    if (absmax) {
         const float m = block_max_f<BLOCK>(amax, slots_f);
         s32 = __fadd_rn(__fdiv_rn(m, 7.5f), kScaleEps);
     } else {
@@ -145,27 +176,45 @@ hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ 
     }
     const uint32_t s16 = from_f32<DT>(s32);
     if (tid == 0) scale[row] = (uint16_t)s16;
-    const float s = from_fp32 ? s32 : to_f32<DT>(s16);
+    const float s = FP32 ? s32 : to_f32<DT>(s16);
 
     if (packed == nullptr && row_sum == nullptr) return;
-    const float inv = quant_inv(s);
     int isum = 0;
-#pragma unroll
-    for (int i = 0; i < NCHUNK; i++) {
-        float q[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) q[e] = quant_code_inv(y[i][e], inv);
-        int csum = 0;
-        const uint32_t w = pack_nibbles8(q, csum);
-        const int c = i * BLOCK + tid;
+    auto put = [&](int i, uint32_t w) {
+        const int c = i * BLOCK + chunk0;
         if (c < nchunks) {                      // chunks past the row's end are padding
-            isum += csum;
+            isum = __builtin_amdgcn_sdot8((int)w, 0x11111111, isum, false);
             if (packed != nullptr) packed[(size_t)row * nchunks + c] = w;
+        }
+    };
+    if (!FP32 && quant_fast_ok(s)) {            // uniform: everything but degenerate rows
+        const float inv28 = quant_inv28(s);
+#pragma unroll
+        for (int i = 0; i < NCHUNK; i++) {
+            const uint32_t d[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
+            uint32_t w = 0;
+#pragma unroll
+            for (int p = 3; p >= 0; p--) {
+                w = push_top_nibble(w, quant_top_nibble_half<DT, 1>(d[p], inv28));
+                w = push_top_nibble(w, quant_top_nibble_half<DT, 0>(d[p], inv28));
+            }
+            put(i, w);
+        }
+    } else {
+        const float inv = quant_inv(s);
+#pragma unroll
+        for (int i = 0; i < NCHUNK; i++) {
+            float v[8], q[8];
+            if constexpr (!FP32) unpack8<DT>(raw[i], v);
+#pragma unroll
+            for (int e = 0; e < 8; e++) q[e] = quant_code_inv(FP32 ? y[FP32 ? i : 0][e] : v[e], inv);
+            int unused = 0;
+            put(i, pack_nibbles8(q, unused));
         }
     }
     if (row_sum != nullptr) {
         const int t = block_sum_i<BLOCK>(isum, slots_i);
-        if (tid == 0) row_sum[row] = t;
+        if (tid == 0) row_sum[row] = t + sum_bias;
     }
 }
 
@@ -178,13 +227,15 @@ hadamard128_kernel(uint16_t *__restrict__ y, const uint16_t *__restrict__ x, lon
     const int lane = threadIdx.x & 63;
     // 16 consecutive chunks (= threads) make one block; the grid strides in multiples of 256 threads
     for (long c = (long)blockIdx.x * 256 + threadIdx.x; c < nchunks_total; c += (long)gridDim.x * 256) {
-        uint4 raw = reinterpret_cast<const uint4 *>(x)[c];
-        float v[8];
+        const long mine = (c & ~15L) + fwht_chunk_of((int)(c & 15));         // c is block-aligned up to the lane's part
+        uint4 raw = reinterpret_cast<const uint4 *>(x)[mine];
+        float v[8], factor;
         unpack8<DT>(raw, v);
-        fwht128_chunk(v, lane);
+        fwht128_chunk(v, lane, had_scale, factor);
 #pragma unroll
-        for (int e = 0; e < 8; e++) v[e] *= had_scale;
-        reinterpret_cast<uint4 *>(y)[c] = pack8<DT>(v);
+        for (int e = 0; e < 8; e++) v[e] = scaled(v[e], factor);
+        reinterpret_cast<uint4 *>(y)[mine] = make_uint4(pack2_rounded_products<DT>(v[0], v[1]), pack2_rounded_products<DT>(v[2], v[3]),
+                                                        pack2_rounded_products<DT>(v[4], v[5]), pack2_rounded_products<DT>(v[6], v[7]));
     }
 }
 
@@ -294,11 +345,12 @@ add_mul_vv_kernel(uint16_t *__restrict__ d, const int32_t *__restrict__ a_add, c
 // ---------------------------------------------------------------------------------------------
 template <int DT>
 static int launch_hadamard_quantize(const void *x, void *scale, uint8_t *packed, int32_t *row_sum, void *x_had,
-                                    int K, int M, float had_scale, int scale_rule, hipStream_t st) {
+                                    int K, int M, float had_scale, int scale_rule, hipStream_t st, int sum_bias = 0) {
     const int nchunks = K >> 3;
+    const bool fp32 = (scale_rule & QUEST_QUANT_FROM_FP32) != 0;
 #define QUEST_HQ(NCH, BLK)                                                                              \
-    hadamard_quantize_kernel<DT, NCH, BLK><<<dim3(M), dim3(BLK), 0, st>>>(                              \
-        (const uint16_t *)x, (uint16_t *)scale, (uint32_t *)packed, row_sum, (uint16_t *)x_had, K, had_scale, scale_rule)
+    (fp32 ? hadamard_quantize_kernel<DT, NCH, BLK, true> : hadamard_quantize_kernel<DT, NCH, BLK, false>)<<<dim3(M), dim3(BLK), 0, st>>>( \
+        (const uint16_t *)x, (uint16_t *)scale, (uint32_t *)packed, row_sum, (uint16_t *)x_had, K, had_scale, scale_rule & ~QUEST_QUANT_FROM_FP32, sum_bias)
     if (nchunks <= 256) QUEST_HQ(1, 256);
     else if (nchunks <= 512) QUEST_HQ(2, 256);
     else if (nchunks <= 1024) QUEST_HQ(4, 256);
@@ -458,34 +510,9 @@ extern "C" int quest_hadamard128(void *y, const void *x, int group_size, int bat
     return launch_status();
 }
 
-extern "C" int quest_hadamard_quantize_int4(const void *x, void *scale, uint8_t *x_int_packed, int32_t *x_int_row_sum,
-                                            void *x_had, int group_size, int batch_size, float had_scale, int dtype,
-                                            void *stream) {
-    forget_stale_error();
-    if (!x || !scale) return QUEST_ERR_NULL_POINTER;
-    if (!check_dtype(dtype)) return QUEST_ERR_BAD_DTYPE;
-    // the transform works on blocks of 128; without it (had_scale == 0) a row only has to be whole 16-byte chunks
-    if (group_size <= 0 || batch_size <= 0 || (group_size & (had_scale != 0.f ? 127 : 7))) return QUEST_ERR_BAD_SHAPE;
-    if (!aligned(x, 16) || !aligned(x_had, 16) || !aligned(x_int_packed, 4)) return QUEST_ERR_ALIGNMENT;
-    hipStream_t st = (hipStream_t)stream;
-    // rows of up to 32768 with a Hadamard entry the dtype holds exactly: matrix cores; anything else: butterflies
-    const int rc = launch_hadamard_quantize_mfma(0, x, nullptr, 0.f, scale, x_int_packed, x_int_row_sum, x_had, nullptr,
-                                                 group_size, batch_size, had_scale, dtype, st);
-    if (rc != QUEST_ERR_UNSUPPORTED) return rc;
-    if (dtype == QUEST_DTYPE_BF16)
-        return launch_hadamard_quantize<0>(x, scale, x_int_packed, x_int_row_sum, x_had, group_size, batch_size, had_scale,
-                                           QUEST_SCALE_GAUSSIAN, st);
-    return launch_hadamard_quantize<1>(x, scale, x_int_packed, x_int_row_sum, x_had, group_size, batch_size, had_scale,
-                                       QUEST_SCALE_GAUSSIAN, st);
-}
-
-extern "C" int quest_hadamard_quantize_int4_rule(const void *x, void *scale, uint8_t *x_int_packed, int32_t *x_int_row_sum,
-                                                 void *x_had, int group_size, int batch_size, float had_scale,
-                                                 int scale_rule, int dtype, void *stream) {
-    forget_stale_error();
-    if (scale_rule == QUEST_SCALE_GAUSSIAN)
-        return quest_hadamard_quantize_int4(x, scale, x_int_packed, x_int_row_sum, x_had, group_size, batch_size, had_scale,
-                                            dtype, stream);
+// sum_bias is added to every row sum that is written
+static int hadamard_quantize_any(const void *x, void *scale, uint8_t *x_int_packed, int32_t *x_int_row_sum, void *x_had,
+                                 int group_size, int batch_size, float had_scale, int scale_rule, int dtype, hipStream_t st, int sum_bias) {
     if ((scale_rule & ~QUEST_QUANT_FROM_FP32) != QUEST_SCALE_ABSMAX && (scale_rule & ~QUEST_QUANT_FROM_FP32) != QUEST_SCALE_GAUSSIAN)
         return QUEST_ERR_BAD_SHAPE;
     if (!x || !scale) return QUEST_ERR_NULL_POINTER;
@@ -493,12 +520,38 @@ extern "C" int quest_hadamard_quantize_int4_rule(const void *x, void *scale, uin
     // the transform works on blocks of 128; without it (had_scale == 0) a row only has to be whole 16-byte chunks
     if (group_size <= 0 || batch_size <= 0 || (group_size & (had_scale != 0.f ? 127 : 7))) return QUEST_ERR_BAD_SHAPE;
     if (!aligned(x, 16) || !aligned(x_had, 16) || !aligned(x_int_packed, 4)) return QUEST_ERR_ALIGNMENT;
-    hipStream_t st = (hipStream_t)stream;
-    if (dtype == QUEST_DTYPE_BF16)
-        return launch_hadamard_quantize<0>(x, scale, x_int_packed, x_int_row_sum, x_had, group_size, batch_size, had_scale,
-                                           scale_rule, st);
-    return launch_hadamard_quantize<1>(x, scale, x_int_packed, x_int_row_sum, x_had, group_size, batch_size, had_scale,
-                                       scale_rule, st);
+    if (scale_rule == QUEST_SCALE_GAUSSIAN) {
+        // rows of up to 32768 with a Hadamard entry the dtype holds exactly: matrix cores; anything else: butterflies
+        const int rc = launch_hadamard_quantize_mfma(0, x, nullptr, 0.f, scale, x_int_packed, x_int_row_sum, x_had, nullptr,
+                                                     group_size, batch_size, had_scale, dtype, st, nullptr, nullptr, nullptr, sum_bias);
+        if (rc != QUEST_ERR_UNSUPPORTED) return rc;
+    }
+    auto *f = dtype == QUEST_DTYPE_BF16 ? launch_hadamard_quantize<0> : launch_hadamard_quantize<1>;
+    return f(x, scale, x_int_packed, x_int_row_sum, x_had, group_size, batch_size, had_scale, scale_rule, st, sum_bias);
+}
+
+extern "C" int quest_hadamard_quantize_int4(const void *x, void *scale, uint8_t *x_int_packed, int32_t *x_int_row_sum,
+                                            void *x_had, int group_size, int batch_size, float had_scale, int dtype,
+                                            void *stream) {
+    forget_stale_error();
+    return hadamard_quantize_any(x, scale, x_int_packed, x_int_row_sum, x_had, group_size, batch_size, had_scale, QUEST_SCALE_GAUSSIAN,
+                                 dtype, (hipStream_t)stream, 0);
+}
+
+extern "C" int quest_hadamard_quantize_int4_rule(const void *x, void *scale, uint8_t *x_int_packed, int32_t *x_int_row_sum,
+                                                 void *x_had, int group_size, int batch_size, float had_scale,
+                                                 int scale_rule, int dtype, void *stream) {
+    forget_stale_error();
+    return hadamard_quantize_any(x, scale, x_int_packed, x_int_row_sum, x_had, group_size, batch_size, had_scale, scale_rule, dtype,
+                                 (hipStream_t)stream, 0);
+}
+
+extern "C" int quest_pack_weight_int4(const void *weight, void *w_scale, uint8_t *w_int_packed, int32_t *w_add, int size_k, int size_n,
+                                      float had_scale, int scale_rule, int dtype, void *stream) {
+    forget_stale_error();
+    if (!w_int_packed || !w_add) return QUEST_ERR_NULL_POINTER;
+    return hadamard_quantize_any(weight, w_scale, w_int_packed, w_add, nullptr, size_k, size_n, had_scale, scale_rule, dtype,
+                                 (hipStream_t)stream, size_k / 2);
 }
 
 extern "C" int quest_rmsnorm_hadamard_quantize_int4(const void *x, const void *norm_weight, float eps, void *scale,

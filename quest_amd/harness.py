@@ -119,6 +119,10 @@ def preprocess_weight(weight: torch.Tensor, use_sparse: bool = False, use_hadama
     if use_sparse:
         raise NotImplementedError('4:8-sparse weights are not part of this build')
     weight = weight.contiguous()
+    rule = {'rms': 'gaussian', 'absmax': 'absmax'}[w_scale_mode]
+    done = quest.host.pack_weight(weight, WEIGHT_HADAMARD_SCALE if use_hadamard else 0., {'gaussian': 0, 'absmax': 1}[rule] | (4 if quantize_from_fp32 else 0))
+    if done is not None:
+        return *done, None
     n, k = weight.shape
     w_scale = torch.empty(n, 1, dtype=weight.dtype, device=weight.device)
     w_int_packed = torch.empty(n, k // 2, dtype=torch.uint8, device=weight.device)
@@ -127,7 +131,7 @@ def preprocess_weight(weight: torch.Tensor, use_sparse: bool = False, use_hadama
     # (w_scale_mode: 'rms' is the reference's rule, 'absmax' puts the row's largest magnitude at the grid's edge)
     quest.hadamard_quantize_int4(weight, w_scale, w_int_packed, w_int_row_sum,
                                  hadamard_scale=WEIGHT_HADAMARD_SCALE if use_hadamard else 0.,
-                                 scale_rule={'rms': 'gaussian', 'absmax': 'absmax'}[w_scale_mode], from_fp32=quantize_from_fp32)
+                                 scale_rule=rule, from_fp32=quantize_from_fp32)
     w_add = w_int_row_sum + k // 2
     return w_int_packed, w_scale, w_add, None
 

@@ -353,6 +353,11 @@ class Llama(nn.Module):
 
     def hidden_states(self, idx: torch.Tensor) -> torch.Tensor:
         """Everything up to and including the final norm: (B, T) ids -> (B, T, d)."""
+        x, branch = self._stream(idx)
+        return self.transformer.ln_f(x if branch is None else x + branch)
+
+    def _stream(self, idx: torch.Tensor):
+        """(B, T) ids -> the residual stream after the last block (B, T, d) and the branch still to be added to it, or None."""
         t = idx.size(1)
         assert t <= self.config.sequence_length
         x = self.transformer.wte(idx)
@@ -367,15 +372,21 @@ class Llama(nn.Module):
                 if branch is not None:
                     x, branch = x + branch, None
                 x = block(x, freqs_cis)
-        if branch is not None:
-            x = x + branch
-        return self.transformer.ln_f(x)
+        return x, branch
 
     def forward(self, idx: torch.Tensor, all_logits: bool = False) -> dict:
         """Logits of the last position (llama.py:253-262, the reference's inference default) or of all positions."""
-        x = self.hidden_states(idx)
-        logits = self.lm_head(x) if all_logits else self.lm_head(x[:, -1:, :])      # a slice: index lists copy from the host
-        return {'logits': logits}
+        if all_logits:
+            return {'logits': self.lm_head(self.hidden_states(idx))}
+        # one position per sequence: norm and head read those rows only
+        x, branch = self._stream(idx)
+        norm, head = self.transformer.ln_f, self.lm_head
+        if not torch.is_grad_enabled() and type(head) is nn.Linear and head.bias is None:
+            logits = quest.host.last_logits(x, branch, norm.weight, float(norm.eps), head.weight)
+            if logits is not None:
+                return {'logits': logits}
+        x = x[:, -1:, :]                               # a slice: index lists copy from the host
+        return {'logits': head(norm(x if branch is None else x + branch[:, -1:, :]))}
 
 
 def _pack(linear: nn.Linear, use_hadamard: bool, use_noop: bool, from_fp32: bool = False) -> harness.Linear4bit:
