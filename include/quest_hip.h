@@ -356,6 +356,15 @@ int quest_silu_mul_hadamard_quantize_e2m3(const void *gate_up, void *scale, void
                                           int batch_size, float had_scale, int dtype, void *stream);
 
 /*
+ * The fused GEMM with the layer's bias (size_n, dtype) in its epilogue: mat_d = dtype(dtype(product) + bias), the two roundings of
+ * `y = gemm(...); y += bias` (benchmarks/bench_e2e.py:67-69).  Arguments and limits of the plain entry
+ * point; the bias 16-byte aligned.
+ */
+int quest_fused_matmul_dequantize_bias_e2m3(void *mat_d, const void *a_tiles, const void *b_tiles, const void *vec_a_mul,
+                                            const void *vec_b_mul, const void *bias, int size_m, int size_k, int size_n, int dtype,
+                                            void *stream);
+
+/*
  * A weight (size_n, size_k) dtype packed for the GEMMs above: w_scale (size_n), w_int_packed (size_n, size_k / 2) and
  * w_add (size_n) int32 = row sum of the codes + size_k / 2, in one pass (preprocess_weight, benchmarks/utils.py:20-53).  had_scale,
  * scale_rule and limits as in quest_hadamard_quantize_int4_rule.

@@ -24,6 +24,7 @@
 // units: 4 x 4 accumulators of 32 x 32 in the AGPR half of a lone wave's 512 registers.  Six LDS slots of one
 // 64-k step (24 KiB: 8 token and 8 channel fragments) form the pipeline: while step s is multiplied from registers,
 // the fragments of step s + 1 are read from LDS and the direct loads of step s + 6 are issued.
+#include "e2m3_epilogue.h"
 #include "gemm_schedule.h"
 
 namespace quest {
@@ -171,7 +172,8 @@ __device__ __forceinline__ void tile(uint8_t *lds, Cursor &ld, Loader &ldr, Pipe
                                      int tok0, int ch0, int unit0, int width, const RopeArgs &rope) {
     constexpr int DT = OUT;
     constexpr bool GLU = EPI == kEpiGlu;
-    constexpr bool ADD = EPI == kEpiAdd;
+    constexpr bool BIAS = EPI == kEpiBias;
+    constexpr bool ADD = EPI == kEpiAdd || BIAS;      // something is added to the rounded product
     constexpr bool ROPE = EPI == kEpiRope;
     constexpr int NAX = NA > 0 ? NA : 1;
     const int wave = ldr.wave;                                      // scalar
@@ -271,7 +273,7 @@ __device__ __forceinline__ void tile(uint8_t *lds, Cursor &ld, Loader &ldr, Pipe
         auto convert_and_store = [&](auto guarded_tag) {
             constexpr bool kGuard = decltype(guarded_tag)::value;
             // kEpiAdd: what the output holds under this lane's sixteen-byte pieces, fetched one channel unit ahead of
-            // the arithmetic that needs it (eight pieces per unit)
+            // the arithmetic that needs it (eight pieces per unit); kEpiBias: the bias of their channels
             uint4 res[2][8];
             auto fetch_unit = [&](int a, int par) {
 #pragma unroll
@@ -280,7 +282,9 @@ __device__ __forceinline__ void tile(uint8_t *lds, Cursor &ld, Loader &ldr, Pipe
                     for (int pr = 0; pr < 2; pr++) {
                         const bool ok = !kGuard || (tok0 + tok_e + b * 32 + li_e < M && ch0 + (unit0 + a) * 32 + (2 * pr + lg_e) * 8 < N);
                         res[par][b * 2 + pr] = make_uint4(0, 0, 0, 0);
-                        if (ok) res[par][b * 2 + pr] = *reinterpret_cast<const uint4 *>(out_lane + ((size_t)b * 32 * n_out + a * kOutPerUnit) * 2 + (2 * pr + lg_e) * 16);
+                        const uint8_t *from = BIAS ? reinterpret_cast<const uint8_t *>(rope.bias + ch0 + (unit0 + a) * 32)
+                                                   : out_lane + ((size_t)b * 32 * n_out + a * kOutPerUnit) * 2;
+                        if (ok) res[par][b * 2 + pr] = *reinterpret_cast<const uint4 *>(from + (2 * pr + lg_e) * 16);
                     }
             };
             if constexpr (ADD) fetch_unit(0, 0);
@@ -342,11 +346,7 @@ __device__ __forceinline__ void tile(uint8_t *lds, Cursor &ld, Loader &ldr, Pipe
                                 if (ch0 + cl < rope.rot_cols) o = rope_turn<DT>(o, cs[pr]);
                             }
                             if constexpr (ADD) {
-                                const uint4 r = res[a & 1][b * 2 + pr];
-                                auto add2 = [](uint32_t p, uint32_t q) {
-                                    return pack2_rounded_products<DT>(__fadd_rn(lo_f32<DT>(q), lo_f32<DT>(p)), __fadd_rn(hi_f32<DT>(q), hi_f32<DT>(p)));
-                                };
-                                o = make_uint4(add2(o.x, r.x), add2(o.y, r.y), add2(o.z, r.z), add2(o.w, r.w));
+                                o = add_eight<DT>(o, res[a & 1][b * 2 + pr]);
                             }
                             *reinterpret_cast<uint4 *>(dst + (2 * pr + lg_e) * 16) = o;
                         }
@@ -373,7 +373,7 @@ __device__ __forceinline__ void tile(uint8_t *lds, Cursor &ld, Loader &ldr, Pipe
                     uint16_t *dst = reinterpret_cast<uint16_t *>(out) + (size_t)tok * N + ch0 + cl;
                     uint32_t o = from_f32<DT>(__fmul_rn(__fadd_rn(s, s), rhs));
                     if constexpr (ADD) {
-                        float sum = __fadd_rn(to_f32<DT>(*dst), to_f32<DT>((uint16_t)o));
+                        float sum = __fadd_rn(to_f32<DT>(BIAS ? rope.bias[ch0 + cl] : *dst), to_f32<DT>((uint16_t)o));
                         asm volatile("" : "+v"(sum));
                         o = from_f32<DT>(sum);
                     }
@@ -486,8 +486,8 @@ __global__ void __launch_bounds__(256) int4_to_e2m3_tiles_kernel(uint8_t *__rest
 }  // namespace e2m3
 
 template <int EPI>
-static int launch_e2m3(int dtype, void *out, const uint8_t *a, const uint8_t *b, const void *a_mul, const void *b_mul, int M,
-                       int K, int N, int cus, hipStream_t st, RopeArgs rope = RopeArgs{nullptr, 1, 0, 2}) {
+static int launch_large(int dtype, void *out, const uint8_t *a, const uint8_t *b, const void *a_mul, const void *b_mul, int M,
+                        int K, int N, int cus, hipStream_t st, const RopeArgs &rope) {
     long grid = 0;
     const Schedule sch = make_schedule(M, N, e2m3::kMaxUnits, 1, cus, &grid, e2m3::kTokSplit);
     if (dtype == QUEST_DTYPE_BF16)
@@ -497,6 +497,45 @@ static int launch_e2m3(int dtype, void *out, const uint8_t *a, const uint8_t *b,
         e2m3::gemm_e2m3_kernel<OUT_FP16, EPI><<<dim3((unsigned)grid), dim3(256), 0, st>>>(
             out, a, b, (const uint16_t *)a_mul, (const uint16_t *)b_mul, M, N, K, sch, rope);
     return launch_status();
+}
+
+// The tile shapes of the two kernels for smaller problems, with what a launch takes in us: fixed + rounds (stage K / 128 + tile) +
+// weights (per MB of weight tiles), rounds = tiles per CU, rounded up.  Fitted to 240 sizes (M from 20 to 3000, K from 1024 to 11008,
+// N from 1024 to 22016, weights rotating through several copies): the shape with the smallest estimate is within 0.9 % of
+// always picking the fastest one in total time, within 16 % on every single size.
+struct Shape {
+    bool split;
+    int tf, cf;
+    float fixed, stage, tile, weights;
+};
+static constexpr Shape kShapes[] = {
+    {false, 8, 4, -1.41f, 0.4260f, 9.85f, 0.036f}, {false, 4, 6, -1.00f, 0.3598f, 8.35f, 0.028f}, {false, 4, 4, 0.26f, 0.2965f, 5.47f, 0.015f},
+    {false, 4, 2, 2.72f, 0.2207f, 1.35f, -0.013f}, {false, 2, 4, 3.13f, 0.2150f, 1.32f, 0.018f},  {false, 2, 2, 2.88f, 0.1393f, 0.79f, 0.020f},
+    {true, 1, 1, 2.31f, 0.0568f, 1.10f, 0.044f},   {true, 1, 2, 2.28f, 0.0772f, 1.13f, 0.053f},   {true, 2, 2, 2.22f, 0.1246f, 1.30f, 0.018f},
+    {true, 4, 2, 0.37f, 0.1900f, 4.62f, -0.014f}};
+
+// Up to half a 256 x 256 tile per CU the smaller tiles are the faster ones (1.01 to 4 x at all of those sizes); from 129 tiles on the
+// 256 x 256 kernel is, by 5 to 40 %.
+static const Shape *smaller_shape(int M, int K, int N, int cus) {
+    if (2L * ((M + 255) / 256) * ((N + 255) / 256) > cus) return nullptr;
+    const Shape *best = nullptr;
+    float best_us = 0.f;
+    for (const Shape &s : kShapes) {
+        const long tiles = (long)((M + 32 * s.tf - 1) / (32 * s.tf)) * ((N + 32 * s.cf - 1) / (32 * s.cf));
+        const float us = s.fixed + (float)((tiles + cus - 1) / cus) * (s.stage * (float)(K / 128) + s.tile) + s.weights * 0.75e-6f * (float)N * (float)K;
+        if (best == nullptr || us < best_us) { best = &s; best_us = us; }
+    }
+    return best;
+}
+
+template <int EPI>
+static int launch_e2m3(int dtype, void *out, const uint8_t *a, const uint8_t *b, const void *a_mul, const void *b_mul, int M,
+                       int K, int N, hipStream_t st, const RopeArgs &rope = RopeArgs{nullptr, 1, 0, 2}) {
+    const int cus = device_cu_count(st);
+    const Shape *s = smaller_shape(M, K, N, cus);
+    if (s == nullptr) return launch_large<EPI>(dtype, out, a, b, a_mul, b_mul, M, K, N, cus, st, rope);
+    const Epilogue epi = {EPI, (const uint16_t *)a_mul, (const uint16_t *)b_mul, rope};
+    return (s->split ? launch_gemm_e2m3_split : launch_gemm_e2m3_mid)(dtype, s->tf, s->cf, out, a, b, M, K, N, epi, st);
 }
 
 static size_t tiles_bytes(int rows, int K) { return (size_t)((rows + 31) / 32) * (size_t)(K / 64) * e2m3::kFragB; }
@@ -542,7 +581,7 @@ extern "C" int quest_fused_matmul_dequantize_e2m3(void *mat_d, const void *a_til
     const int rc = e2m3_gemm_check(mat_d, a_tiles, b_tiles, vec_a_mul, vec_b_mul, size_m, size_k, size_n, dtype);
     if (rc != QUEST_OK) return rc;
     return launch_e2m3<kEpiPlain>(dtype, mat_d, (const uint8_t *)a_tiles, (const uint8_t *)b_tiles, vec_a_mul, vec_b_mul, size_m,
-                              size_k, size_n, device_cu_count((hipStream_t)stream), (hipStream_t)stream);
+                              size_k, size_n, (hipStream_t)stream);
 }
 
 extern "C" int quest_fused_matmul_dequantize_add_e2m3(void *mat_d, const void *a_tiles, const void *b_tiles, const void *vec_a_mul,
@@ -552,7 +591,19 @@ extern "C" int quest_fused_matmul_dequantize_add_e2m3(void *mat_d, const void *a
     const int rc = e2m3_gemm_check(mat_d, a_tiles, b_tiles, vec_a_mul, vec_b_mul, size_m, size_k, size_n, dtype);
     if (rc != QUEST_OK) return rc;
     return launch_e2m3<kEpiAdd>(dtype, mat_d, (const uint8_t *)a_tiles, (const uint8_t *)b_tiles, vec_a_mul, vec_b_mul, size_m,
-                                      size_k, size_n, device_cu_count((hipStream_t)stream), (hipStream_t)stream);
+                                      size_k, size_n, (hipStream_t)stream);
+}
+
+extern "C" int quest_fused_matmul_dequantize_bias_e2m3(void *mat_d, const void *a_tiles, const void *b_tiles, const void *vec_a_mul,
+                                                       const void *vec_b_mul, const void *bias, int size_m, int size_k, int size_n,
+                                                       int dtype, void *stream) {
+    forget_stale_error();
+    const int rc = e2m3_gemm_check(mat_d, a_tiles, b_tiles, vec_a_mul, vec_b_mul, size_m, size_k, size_n, dtype);
+    if (rc != QUEST_OK) return rc;
+    if (!bias) return QUEST_ERR_NULL_POINTER;
+    if (!aligned(bias, 16)) return QUEST_ERR_ALIGNMENT;
+    return launch_e2m3<kEpiBias>(dtype, mat_d, (const uint8_t *)a_tiles, (const uint8_t *)b_tiles, vec_a_mul, vec_b_mul, size_m,
+                                 size_k, size_n, (hipStream_t)stream, RopeArgs{nullptr, 1, 0, 2, (const uint16_t *)bias});
 }
 
 extern "C" int quest_fused_matmul_dequantize_rope_e2m3(void *mat_d, const void *a_tiles, const void *b_tiles, const void *vec_a_mul,
@@ -567,7 +618,7 @@ extern "C" int quest_fused_matmul_dequantize_rope_e2m3(void *mat_d, const void *
         return QUEST_ERR_BAD_SHAPE;
     if (!aligned(freqs_cis, 16)) return QUEST_ERR_ALIGNMENT;
     return launch_e2m3<kEpiRope>(dtype, mat_d, (const uint8_t *)a_tiles, (const uint8_t *)b_tiles, vec_a_mul, vec_b_mul, size_m,
-                                       size_k, size_n, device_cu_count((hipStream_t)stream), (hipStream_t)stream,
+                                       size_k, size_n, (hipStream_t)stream,
                                        RopeArgs{freqs_cis, seq_len, rot_cols, head_dim});
 }
 
@@ -589,5 +640,5 @@ extern "C" int quest_fused_matmul_dequantize_swiglu_e2m3(void *mat_d, const void
     if (rc != QUEST_OK) return rc;
     if (size_n & 7) return QUEST_ERR_BAD_SHAPE;
     return launch_e2m3<kEpiGlu>(dtype, mat_d, (const uint8_t *)a_tiles, (const uint8_t *)b_tiles, vec_a_mul, vec_b_mul, size_m,
-                             size_k, size_n, device_cu_count((hipStream_t)stream), (hipStream_t)stream);
+                             size_k, size_n, (hipStream_t)stream);
 }

@@ -39,12 +39,14 @@ __device__ __forceinline__ void wait_vmcnt_imm() {
 // first rot_cols channels of the output -- q and k of a fused QKV projection -- applied to the rounded product before it
 // is stored: channels are heads of head_dim, a head is (re, im) pairs, pair i of a head at position t = row % seq_len
 // turns by freqs[t][i] = (cos, sin); fp32 products and sums in the reference's order, one more rounding to dtype.  The
-// arithmetic of rope_kernel (rowops.hip).
-enum { kEpiPlain = 0, kEpiGlu = 1, kEpiAdd = 2, kEpiRope = 3 };
+// arithmetic of rope_kernel (rowops.hip).  kEpiBias: the layer's bias added to the rounded product, dtype(dtype(product) + bias),
+// the two roundings of `y += bias`.
+enum { kEpiPlain = 0, kEpiGlu = 1, kEpiAdd = 2, kEpiRope = 3, kEpiBias = 4 };
 
 struct RopeArgs {
     const float *freqs;                  // (seq_len, head_dim / 2, 2) fp32, 16-byte aligned
     int seq_len, rot_cols, head_dim;     // seq_len >= 32, head_dim % 32 == 0, rot_cols % head_dim == 0
+    const uint16_t *bias = nullptr;      // kEpiBias: one value per channel
 };
 
 // Where a lane's angles lie: its first token row's position in its sequence (row % seq_len: one division per tile; the
@@ -86,6 +88,16 @@ __device__ __forceinline__ uint4 rope_turn(const uint4 &o, const float4 (&cs)[2]
         return pack2_rounded_products<DT>(out_re, out_im);
     };
     return make_uint4(turn(o.x, cs[0].x, cs[0].y), turn(o.y, cs[0].z, cs[0].w), turn(o.z, cs[1].x, cs[1].y), turn(o.w, cs[1].z, cs[1].w));
+}
+
+// dtype(x + y) of packed pairs, and of eight channels
+template <int DT>
+__device__ __forceinline__ uint32_t add_pair(uint32_t x, uint32_t y) {
+    return pack2_rounded_products<DT>(__fadd_rn(lo_f32<DT>(x), lo_f32<DT>(y)), __fadd_rn(hi_f32<DT>(x), hi_f32<DT>(y)));
+}
+template <int DT>
+__device__ __forceinline__ uint4 add_eight(const uint4 &x, const uint4 &y) {
+    return make_uint4(add_pair<DT>(x.x, y.x), add_pair<DT>(x.y, y.y), add_pair<DT>(x.z, y.z), add_pair<DT>(x.w, y.w));
 }
 
 // 16 packed bytes -> the int8 vectors 16 * (even-k nibbles) and 16 * (odd-k nibbles), both sign-correct

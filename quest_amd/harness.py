@@ -18,11 +18,12 @@ _HIP_BACKENDS = ('hip', 'triton', 'cuda')
 WEIGHT_HADAMARD_SCALE = 2. ** -3.5      # utils.py:39
 
 # Which matrix instructions the GEMM of `linear_forward` / `Linear4bit` runs on when the weight's E2M3 tiles are at
-# hand: 'fp6' = the FP6 (E2M3) kernel where it is the faster one (a few hundred tokens and more), 'int8' = always the
+# hand: 'fp6' = the FP6 (E2M3) kernels where they are the faster ones (from 33 tokens on), 'int8' = always the
 # INT8 kernels on packed nibbles.  Both give the same bits.
 MATRIX_PATH = 'fp6'
-E2M3_MIN_TILES = 66                     # 256 x 256 output tiles from which the FP6 kernel is the faster one
-E2M3_MIN_K = 2048                       # shortest rows that take it (see prefers_e2m3)
+E2M3_MIN_TOKENS = 33                    # from here on the FP6 kernels are the faster ones
+E2M3_MIN_K = 2048                       # shortest rows that take them at more than E2M3_SHORT_ROWS_TOKENS tokens (see prefers_e2m3)
+E2M3_SHORT_ROWS_TOKENS = 4096
 # Whether a producer-fused block lets the FP6 GEMM of an output projection add into the residual stream itself
 # (same bits as the addition inside the next norm kernel; one pass over the stream less).
 GEMM_ADDS_RESIDUAL = True
@@ -32,16 +33,15 @@ GEMM_ROTATES_QK = True
 
 
 def prefers_e2m3(m: int, k: int, n: int) -> bool:
-    """Whether the FP6 kernel is the faster one for an (m, k) x (n, k) layer.  Its 256 x 256 tiles need about a quarter
-    of the chip's 256 compute units busy to beat the INT8 kernels' small tiles: measured over K from 1024 to 11008, N from
-    2048 to 13824 and M from 256 to 16384, the FP6 kernel wins from 66 tiles on (M = 1536 at N = 4096, M = 512 at
-    N = 11008, M = 3072 at N = 2048) and loses below 64."""
-    tiles = ((m + 255) // 256) * ((n + 255) // 256)
-    # E2M3_MIN_K: with shorter rows the GEMM is mostly epilogue either way and the tile-writing activation kernels are a
-    # little slower than the row-writing ones (12.0 against 10.2 us at [16384, 1024]) -- measured on the 12-layer
+    """Whether the FP6 kernels are the faster ones for an (m, k) x (n, k) layer: measured over K from 1024 to 11008, N from
+    1024 to 22016 and M from 20 to 3000 they win 3 to 60 % from 33 tokens on (1.2 x on average; level or up to 8 % behind at 33 to 64
+    tokens with K = 1024, N = 11264 and K = 4096, N = 22016) and lose below, where the weights' 1.5 x bytes are the whole cost."""
+    # E2M3_MIN_K: with shorter rows and many tokens the GEMM is mostly epilogue either way and the tile-writing activation kernels
+    # are a little slower than the row-writing ones (12.0 against 10.2 us at [16384, 1024]) -- measured on the 12-layer
     # d = 1024 model at 32 x 512 tokens: 6.01 ms per forward with the FP6 path from K = 1024 on, 5.79 ms from K = 2048 on
-    # (its K = 2816 layers), 5.80 ms without it; the 1600M model (K = 2560, 6912) gains 9 %
-    return (MATRIX_PATH == 'fp6' and k % 128 == 0 and E2M3_MIN_K <= k <= 65536 and tiles >= E2M3_MIN_TILES and m * n <= (1 << 30))
+    # (its K = 2816 layers), 5.80 ms without it
+    return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and k <= 65536 and m * n <= (1 << 30)
+            and (k >= E2M3_MIN_K or m <= E2M3_SHORT_ROWS_TOKENS))
 
 
 def weight_tiles(w_int_packed: torch.Tensor) -> torch.Tensor:
@@ -221,12 +221,11 @@ class Linear4bit(nn.Module):
     def w_tiles(self) -> torch.Tensor:
         """The weight codes as E2M3 tiles (built once per content of `w_int_packed`, e.g. again after a checkpoint
         has been loaded into the buffers)."""
-        try:
-            key = (self.w_int_packed.data_ptr(), self.w_int_packed._version)
-        except RuntimeError:              # a tensor created in inference mode keeps no version counter
-            key = (self.w_int_packed.data_ptr(), None)
+        w = self.w_int_packed
+        # a tensor created in inference mode keeps no version counter (asking for it raises: 10 us a call)
+        key = (w.data_ptr(), None if w.is_inference() else w._version)
         if self._tiles is None or self._tiles_of != key:
-            self._tiles = weight_tiles(self.w_int_packed)
+            self._tiles = weight_tiles(w)
             self._tiles_of = key
         return self._tiles
 
