@@ -357,9 +357,13 @@ int quest_silu_mul_hadamard_quantize_e2m3(const void *gate_up, void *scale, void
 
 /*
  * The fused GEMM with the layer's bias (size_n, dtype) in its epilogue: mat_d = dtype(dtype(product) + bias), the two roundings of
- * `y = gemm(...); y += bias` (benchmarks/bench_e2e.py:67-69).  Arguments and limits of the plain entry
- * point; the bias 16-byte aligned.
+ * `y = gemm(...); y += bias` (benchmarks/bench_e2e.py:67-69).  Arguments and limits of the plain entry points;
+ * QUEST_ERR_UNSUPPORTED (nothing launched) for packed codes where the kernel that takes the size cannot add it (scale vectors
+ * not 4-byte or a bias not 16-byte aligned) -- make the two calls then.
  */
+int quest_fused_matmul_dequantize_bias_int4_int4t(void *mat_d, const uint8_t *mat_a, const uint8_t *mat_b, const int32_t *vec_a_add,
+                                                  const int32_t *vec_b_add, const void *vec_a_mul, const void *vec_b_mul,
+                                                  const void *bias, int size_m, int size_k, int size_n, int dtype, void *stream);
 int quest_fused_matmul_dequantize_bias_e2m3(void *mat_d, const void *a_tiles, const void *b_tiles, const void *vec_a_mul,
                                             const void *vec_b_mul, const void *bias, int size_m, int size_k, int size_n, int dtype,
                                             void *stream);

@@ -295,7 +295,8 @@ enum { OUT_BF16 = 0, OUT_FP16 = 1, OUT_INT32 = 2 };
 
 // gemm_decode.hip: the weight-streaming GEMM for M <= 64; QUEST_ERR_UNSUPPORTED when it does not apply
 int launch_gemm_decode(int out_kind, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add,
-                       const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st);
+                       const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st,
+                       const void *bias = nullptr);
 
 // ... and its split-K form for M <= 16 with a workspace (see gemm_decode.hip); gemm_decode_workspace_bytes is what it needs
 int launch_gemm_decode_splitk(int out_kind, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add,

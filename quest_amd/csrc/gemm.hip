@@ -63,7 +63,7 @@ static int gemm_launch_large(int out_kind, bool glu, void *out, const uint8_t *a
                              const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, int cus,
                              hipStream_t st, const RopeArgs *rope = nullptr, bool add = false) {
     const int small_shape = add ? 0 : small_tile_shape(M, N, cus);       // the small tiles do not add into their output
-    const int epi = add ? kEpiAdd : rope != nullptr ? kEpiRope : glu ? kEpiGlu : kEpiPlain;
+    const int epi = add ? kEpiAdd : rope != nullptr ? (rope->bias != nullptr ? kEpiBias : kEpiRope) : glu ? kEpiGlu : kEpiPlain;
     if (small_shape != 0) return launch_gemm_small(out_kind, epi, small_shape, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st, rope);
     const int units = (N + 31) / 32;
     const int per_group = units >= 8 ? units / 8 : units;
@@ -75,16 +75,20 @@ static int gemm_launch_large(int out_kind, bool glu, void *out, const uint8_t *a
 }
 
 static int gemm_launch(int out_kind, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add, const int32_t *b_add,
-                       const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st) {
+                       const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st, const void *bias = nullptr) {
+    const RopeArgs with_bias = {nullptr, 32, 0, 32, (const uint16_t *)bias};
+    const RopeArgs *args = bias != nullptr ? &with_bias : nullptr;
     // the device is asked for its CU count once per call, and only where a rule below uses it (not for a handful of tokens)
     const int cus = M > 64 ? device_cu_count(st) : 0;
     const int small_shape = small_tile_shape(M, N, cus);
-    if (small_shape != 0) return launch_gemm_small(out_kind, kEpiPlain, small_shape, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
+    if (small_shape != 0)
+        return launch_gemm_small(out_kind, args != nullptr ? kEpiBias : kEpiPlain, small_shape, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st, args);
     // a handful of tokens (unless the small tiles took the call above): the weight-streaming kernel
-    if (M <= 64) return launch_gemm_decode(out_kind, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
+    if (M <= 64) return launch_gemm_decode(out_kind, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st, bias);
     // the large-tile kernel fetches the 16-bit scale vectors two per dword: 4-byte aligned vectors
-    if (aligned(b_mul, 4) && aligned(a_mul, 4))
-        return gemm_launch_large(out_kind, false, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, cus, st);
+    if (aligned(b_mul, 4) && aligned(a_mul, 4) && aligned(bias, 16))
+        return gemm_launch_large(out_kind, false, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, cus, st, args);
+    if (bias != nullptr) return QUEST_ERR_UNSUPPORTED;
     // scale vectors at odd element offsets (a sliced tensor): the register-staged kernel reads them element by element
     return launch_gemm_staged(out_kind, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
 }
@@ -113,6 +117,19 @@ extern "C" int quest_fused_matmul_dequantize_int4_int4t(void *mat_d, const uint8
     if (!check_dtype(dtype)) return QUEST_ERR_BAD_DTYPE;
     return gemm_launch(dtype == QUEST_DTYPE_BF16 ? OUT_BF16 : OUT_FP16, mat_d, mat_a, mat_b, vec_a_add, vec_b_add, vec_a_mul,
                        vec_b_mul, size_m, size_k, size_n, (hipStream_t)stream);
+}
+
+extern "C" int quest_fused_matmul_dequantize_bias_int4_int4t(void *mat_d, const uint8_t *mat_a, const uint8_t *mat_b,
+                                                             const int32_t *vec_a_add, const int32_t *vec_b_add,
+                                                             const void *vec_a_mul, const void *vec_b_mul, const void *bias,
+                                                             int size_m, int size_k, int size_n, int dtype, void *stream) {
+    forget_stale_error();
+    const int rc = gemm_check(mat_d, mat_a, mat_b, size_m, size_k, size_n);
+    if (rc != QUEST_OK) return rc;
+    if (!vec_a_add || !vec_b_add || !vec_a_mul || !vec_b_mul || !bias) return QUEST_ERR_NULL_POINTER;
+    if (!check_dtype(dtype)) return QUEST_ERR_BAD_DTYPE;
+    return gemm_launch(dtype == QUEST_DTYPE_BF16 ? OUT_BF16 : OUT_FP16, mat_d, mat_a, mat_b, vec_a_add, vec_b_add, vec_a_mul,
+                       vec_b_mul, size_m, size_k, size_n, (hipStream_t)stream, bias);
 }
 
 extern "C" size_t quest_gemm_workspace_bytes(int size_m, int size_k, int size_n) {

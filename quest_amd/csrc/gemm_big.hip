@@ -196,8 +196,9 @@ __device__ __forceinline__ void big_tile(uint8_t *lds, Cursor &ld, Loader &ldr, 
     constexpr int DT = OUT == OUT_INT32 ? 0 : OUT;
     constexpr bool GLU = EPI == kEpiGlu;
     constexpr bool ROPE = EPI == kEpiRope;
-    constexpr bool ADD = EPI == kEpiAdd;
-    constexpr bool TAIL = EPI == kEpiPlain;      // (the other epilogues are for K % 128 == 0)
+    constexpr bool BIAS = EPI == kEpiBias;
+    constexpr bool ADD = EPI == kEpiAdd || BIAS;      // something is added to the rounded product
+    constexpr bool TAIL = EPI == kEpiPlain || BIAS;   // (the other epilogues are for K % 128 == 0)
     static_assert(EPI == kEpiPlain || OUT != OUT_INT32, "epilogues on 16-bit outputs only");
     constexpr int NAX = NA > 0 ? NA : 1;
     // Lane coordinates are derived afresh in every phase (here, in the loader's cursor step, in the epilogue): a value
@@ -379,14 +380,17 @@ __device__ __forceinline__ void big_tile(uint8_t *lds, Cursor &ld, Loader &ldr, 
             rope_fetch(rope, rl, lg_e, kTokOuter ? i : o, kTokOuter ? o : i, piece & 1, cs[par]);
         };
         if constexpr (ROPE) fetch_angles(0, 0);
-        // kEpiAdd: what the output holds under this lane's sixteen-byte pieces, fetched one piece ahead as well
+        // kEpiAdd: what the output holds under this lane's sixteen-byte pieces, fetched one piece ahead as well; kEpiBias: the
+        // bias of their channels
         uint4 res[2];
         auto fetch_res = [&](int piece, int par) {
             const int o = piece / (2 * kInner), i = (piece >> 1) % kInner, pr = piece & 1;
             const int a = kTokOuter ? i : o, b = kTokOuter ? o : i;
             const bool ok = !kGuard || (tok0 + tok_e + b * 32 + li_e < M && ch0 + (unit0 + a) * 32 + (2 * pr + lg_e) * 8 < N);
             res[par] = make_uint4(0, 0, 0, 0);
-            if (ok) res[par] = *reinterpret_cast<const uint4 *>(out_lane + ((size_t)b * 32 * n_out + a * kOutPerUnit) * kEs + (2 * pr + lg_e) * 16);
+            const uint8_t *from = BIAS ? reinterpret_cast<const uint8_t *>(rope.bias + ch0 + (unit0 + a) * 32)
+                                       : out_lane + ((size_t)b * 32 * n_out + a * kOutPerUnit) * kEs;
+            if (ok) res[par] = *reinterpret_cast<const uint4 *>(from + (2 * pr + lg_e) * 16);
         };
         if constexpr (ADD) fetch_res(0, 0);
 #pragma unroll
@@ -454,11 +458,7 @@ __device__ __forceinline__ void big_tile(uint8_t *lds, Cursor &ld, Loader &ldr, 
                                 if (ch0 + cl < rope.rot_cols) piece = rope_turn<DT>(piece, cs[pr]);
                             }
                             if constexpr (ADD) {                  // dtype(out + dtype(product)): the residual stream's addition
-                                const uint4 r = res[pr];
-                                auto add2 = [](uint32_t p, uint32_t q) {
-                                    return pack2_rounded_products<DT>(__fadd_rn(lo_f32<DT>(q), lo_f32<DT>(p)), __fadd_rn(hi_f32<DT>(q), hi_f32<DT>(p)));
-                                };
-                                piece = make_uint4(add2(piece.x, r.x), add2(piece.y, r.y), add2(piece.z, r.z), add2(piece.w, r.w));
+                                piece = add_eight<DT>(piece, res[pr]);
                             }
                             *reinterpret_cast<uint4 *>(dst + (2 * pr + lg_e) * 16) = piece;
                         }
@@ -499,7 +499,7 @@ __device__ __forceinline__ void big_tile(uint8_t *lds, Cursor &ld, Loader &ldr, 
                             const float rhs = __fmul_rn(t_half_mul, to_f32<DT>(v_mul[cl + e]));
                             uint32_t val = from_f32<DT>(__fmul_rn(lhs, rhs));
                             if constexpr (ADD) {
-                                float sum = __fadd_rn(to_f32<DT>(reinterpret_cast<uint16_t *>(out)[o]), to_f32<DT>((uint16_t)val));
+                                float sum = __fadd_rn(to_f32<DT>(BIAS ? rope.bias[ch] : reinterpret_cast<uint16_t *>(out)[o]), to_f32<DT>((uint16_t)val));
                                 asm volatile("" : "+v"(sum));
                                 val = from_f32<DT>(sum);
                             }
@@ -535,7 +535,7 @@ gemm_w4a4_big_kernel(void *__restrict__ out, const uint8_t *__restrict__ act, co
     // asm cuts the value loose from threadIdx, which would otherwise be kept (and spilled) to derive it again
     int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     asm volatile("" : "+s"(wave));
-    constexpr bool TAIL = EPI == kEpiPlain;
+    constexpr bool TAIL = EPI == kEpiPlain || EPI == kEpiBias;
     const int wc = wave & 1;                     // channel half this wave multiplies
     const int kbytes = K >> 1;
 
@@ -631,15 +631,16 @@ static int launch_shape(bool duo, void *out, const uint8_t *a, const uint8_t *b,
 int launch_gemm_big(int out_kind, int epi, bool duo, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add,
                     const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, int cus, hipStream_t st,
                     const RopeArgs *rope_args) {
-    if ((K & (epi == kEpiPlain ? 31 : 127)) != 0 || cus <= 0 || (epi != kEpiPlain && out_kind == OUT_INT32)) return QUEST_ERR_UNSUPPORTED;
-    if (epi == kEpiRope && rope_args == nullptr) return QUEST_ERR_NULL_POINTER;
-    const RopeArgs rope = epi == kEpiRope ? *rope_args : RopeArgs{nullptr, 32, 0, 32};
+    if ((K & (epi == kEpiPlain || epi == kEpiBias ? 31 : 127)) != 0 || cus <= 0 || (epi != kEpiPlain && out_kind == OUT_INT32)) return QUEST_ERR_UNSUPPORTED;
+    if ((epi == kEpiRope || epi == kEpiBias) && rope_args == nullptr) return QUEST_ERR_NULL_POINTER;
+    const RopeArgs rope = rope_args != nullptr ? *rope_args : RopeArgs{nullptr, 32, 0, 32};
 #define QUEST_BIG_EPI(E)                                                                                                            \
     (out_kind == OUT_BF16 ? launch_shape<OUT_BF16, E>(duo, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, cus, st, rope)            \
                           : launch_shape<OUT_FP16, E>(duo, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, cus, st, rope))
     if (epi == kEpiGlu) return QUEST_BIG_EPI(kEpiGlu);
     if (epi == kEpiRope) return QUEST_BIG_EPI(kEpiRope);
     if (epi == kEpiAdd) return QUEST_BIG_EPI(kEpiAdd);
+    if (epi == kEpiBias) return QUEST_BIG_EPI(kEpiBias);
     if (epi != kEpiPlain) return QUEST_ERR_UNSUPPORTED;
     if (out_kind == OUT_INT32) return launch_shape<OUT_INT32, kEpiPlain>(duo, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, cus, st, rope);
     return QUEST_BIG_EPI(kEpiPlain);

@@ -44,7 +44,8 @@ template <int OUT, int TM>
 __global__ void __launch_bounds__(64 * kWaves, TM == 1 ? 8 : TM == 2 ? 4 : 2)
 gemm_w4a4_decode_kernel(void *__restrict__ out, const uint8_t *__restrict__ act, const uint8_t *__restrict__ wgt,
                         const int32_t *__restrict__ a_add, const int32_t *__restrict__ b_add,
-                        const uint16_t *__restrict__ a_mul, const uint16_t *__restrict__ b_mul, int M, int N, int K) {
+                        const uint16_t *__restrict__ a_mul, const uint16_t *__restrict__ b_mul,
+                        const uint16_t *__restrict__ bias, int M, int N, int K) {
     __shared__ __attribute__((aligned(16))) int red[kWaves][TM][64][4];
 
     const int lane = threadIdx.x & 63;
@@ -68,6 +69,7 @@ gemm_w4a4_decode_kernel(void *__restrict__ out, const uint8_t *__restrict__ act,
     // (lane (r, g) of wave t ends up with channels ch0 + 4 g + {0..3} of token 16 t + r)
     int t_add = 0, c_add[4] = {0, 0, 0, 0};
     float t_half_mul = 0.f, c_mul[4] = {0.f, 0.f, 0.f, 0.f};
+    uint32_t c_bias[4] = {0, 0, 0, 0};
     if constexpr (OUT != OUT_INT32) {
         if (wave < TM) {
             const int tok = min(wave * 16 + r, M - 1);
@@ -78,6 +80,7 @@ gemm_w4a4_decode_kernel(void *__restrict__ out, const uint8_t *__restrict__ act,
                 const int che = min(ch0 + 4 * g + e, N - 1);
                 c_add[e] = b_add[che];
                 c_mul[e] = to_f32<OUT>(b_mul[che]);
+                if (bias != nullptr) c_bias[e] = bias[che];
             }
         }
     }
@@ -160,6 +163,10 @@ gemm_w4a4_decode_kernel(void *__restrict__ out, const uint8_t *__restrict__ act,
             const float lhs = (float)(c[e] * 2 + t_add + c_add[e]);
             const float rhs = __fmul_rn(t_half_mul, c_mul[e]);
             h[e] = from_f32<OUT>(__fmul_rn(lhs, rhs));
+            if (bias != nullptr) {                            // dtype(product + bias): the two roundings of y += bias
+                float sum = __fadd_rn(to_f32<OUT>(h[e]), to_f32<OUT>(c_bias[e]));
+                h[e] = from_f32<OUT>(sum);
+            }
         }
         uint16_t *dst = reinterpret_cast<uint16_t *>(out) + o;
         if ((N & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0) {
@@ -314,17 +321,17 @@ gemm_w4a4_decode_splitk_kernel(void *__restrict__ out, const uint8_t *__restrict
 
 template <int OUT, int TM>
 static void launch_tm(void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add, const int32_t *b_add,
-                      const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st) {
+                      const void *a_mul, const void *b_mul, const void *bias, int M, int K, int N, hipStream_t st) {
     gemm_w4a4_decode_kernel<OUT, TM><<<dim3((N + kChannels - 1) / kChannels), dim3(64 * kWaves), 0, st>>>(
-        out, a, b, a_add, b_add, (const uint16_t *)a_mul, (const uint16_t *)b_mul, M, N, K);
+        out, a, b, a_add, b_add, (const uint16_t *)a_mul, (const uint16_t *)b_mul, (const uint16_t *)bias, M, N, K);
 }
 
 template <int OUT>
 static int launch_out(void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add, const int32_t *b_add,
-                      const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st) {
-    if (M <= 16) launch_tm<OUT, 1>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
-    else if (M <= 32) launch_tm<OUT, 2>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
-    else launch_tm<OUT, 4>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
+                      const void *a_mul, const void *b_mul, const void *bias, int M, int K, int N, hipStream_t st) {
+    if (M <= 16) launch_tm<OUT, 1>(out, a, b, a_add, b_add, a_mul, b_mul, bias, M, K, N, st);
+    else if (M <= 32) launch_tm<OUT, 2>(out, a, b, a_add, b_add, a_mul, b_mul, bias, M, K, N, st);
+    else launch_tm<OUT, 4>(out, a, b, a_add, b_add, a_mul, b_mul, bias, M, K, N, st);
     return launch_status();
 }
 
@@ -377,12 +384,12 @@ int launch_gemm_decode_splitk(int out_kind, void *out, const uint8_t *a, const u
 
 // The weight-streaming kernel applies to M <= 64 and K a multiple of 32 (whole 16-byte pieces); QUEST_ERR_UNSUPPORTED otherwise.
 int launch_gemm_decode(int out_kind, void *out, const uint8_t *a, const uint8_t *b, const int32_t *a_add,
-                       const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st) {
+                       const int32_t *b_add, const void *a_mul, const void *b_mul, int M, int K, int N, hipStream_t st, const void *bias) {
     if (M > 64 || (K & 31) != 0 || !aligned(a, 16) || !aligned(b, 16)) return QUEST_ERR_UNSUPPORTED;
     switch (out_kind) {
-        case OUT_BF16: return decode::launch_out<OUT_BF16>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
-        case OUT_FP16: return decode::launch_out<OUT_FP16>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
-        default: return decode::launch_out<OUT_INT32>(out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st);
+        case OUT_BF16: return decode::launch_out<OUT_BF16>(out, a, b, a_add, b_add, a_mul, b_mul, bias, M, K, N, st);
+        case OUT_FP16: return decode::launch_out<OUT_FP16>(out, a, b, a_add, b_add, a_mul, b_mul, bias, M, K, N, st);
+        default: return decode::launch_out<OUT_INT32>(out, a, b, a_add, b_add, a_mul, b_mul, nullptr, M, K, N, st);
     }
 }
 

@@ -250,6 +250,16 @@ gemm_w4a4_small_kernel(void *__restrict__ out, const uint8_t *__restrict__ act, 
                             piece8 = rope_turn<DT>(piece8, cs);
                         }
                     }
+                    if constexpr (EPI == kEpiBias) {
+                        if ((reinterpret_cast<uintptr_t>(rope.bias) & 15) == 0)
+                            piece8 = add_eight<DT>(piece8, *reinterpret_cast<const uint4 *>(rope.bias + c));
+                        else {
+                            uint32_t bq[4];
+#pragma unroll
+                            for (int i = 0; i < 4; i++) bq[i] = rope.bias[c + 2 * i] | ((uint32_t)rope.bias[c + 2 * i + 1] << 16);
+                            piece8 = add_eight<DT>(piece8, make_uint4(bq[0], bq[1], bq[2], bq[3]));
+                        }
+                    }
                     *reinterpret_cast<uint4 *>(dst + c) = piece8;
                 }
             } else if (!GLU && tok_ok) {
@@ -258,7 +268,10 @@ gemm_w4a4_small_kernel(void *__restrict__ out, const uint8_t *__restrict__ act, 
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
                         const int c = cb + g * 8 + lg * 4 + e;
-                        if (c < N) dst[c] = (uint16_t)from_f32<DT>(v[g][e]);
+                        if (c >= N) continue;
+                        uint32_t h = from_f32<DT>(v[g][e]);
+                        if constexpr (EPI == kEpiBias) h = add_pair<DT>(h, rope.bias[c]);
+                        dst[c] = (uint16_t)h;
                     }
             }
         }
@@ -290,12 +303,14 @@ int launch_gemm_small(int out_kind, int epi, int shape, void *out, const uint8_t
                       const RopeArgs *rope_args) {
     if ((K & 31) != 0 || (shape != 64 && shape != 128) || (epi != kEpiPlain && out_kind == OUT_INT32)) return QUEST_ERR_UNSUPPORTED;
     if (epi == kEpiRope && (rope_args == nullptr || (N & 7) != 0 || !aligned(out, 16))) return QUEST_ERR_UNSUPPORTED;
-    const RopeArgs rope = epi == kEpiRope ? *rope_args : RopeArgs{nullptr, 32, 0, 32};
+    if (epi == kEpiBias && rope_args == nullptr) return QUEST_ERR_NULL_POINTER;
+    const RopeArgs rope = rope_args != nullptr ? *rope_args : RopeArgs{nullptr, 32, 0, 32};
 #define QUEST_SMALL_EPI(E)                                                                                                   \
     (out_kind == OUT_BF16 ? launch_shape<OUT_BF16, E>(shape, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st, rope)        \
                           : launch_shape<OUT_FP16, E>(shape, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st, rope))
     if (epi == kEpiGlu) return QUEST_SMALL_EPI(kEpiGlu);
     if (epi == kEpiRope) return QUEST_SMALL_EPI(kEpiRope);
+    if (epi == kEpiBias) return QUEST_SMALL_EPI(kEpiBias);
     if (epi != kEpiPlain) return QUEST_ERR_UNSUPPORTED;
     if (out_kind == OUT_INT32) return launch_shape<OUT_INT32, kEpiPlain>(shape, out, a, b, a_add, b_add, a_mul, b_mul, M, K, N, st, rope);
     return QUEST_SMALL_EPI(kEpiPlain);

@@ -129,8 +129,10 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         out = make(shape, type, args.dev);
     }
     bool add_bias = bias != nullptr;
-    if (add_bias && tiles) {                                     // in the GEMM's epilogue where the kernel can
-        rc = quest_fused_matmul_dequantize_bias_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)k, (int)n, dt, st);
+    if (add_bias) {                                              // in the GEMM's epilogue where the kernel can
+        rc = tiles ? quest_fused_matmul_dequantize_bias_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)k, (int)n, dt, st)
+                   : quest_fused_matmul_dequantize_bias_int4_int4t(out.data_ptr(), q.codes, (const uint8_t *)w->data_ptr(), q.row_sum, (const int32_t *)w_add->data_ptr(),
+                                                                   q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)k, (int)n, dt, st);
         add_bias = rc != QUEST_OK;
     }
     if (add_bias || bias == nullptr) {
