@@ -150,7 +150,7 @@ def main():
     if args.no_gemm_rope:
         harness.GEMM_ROTATES_QK = False
     if args.min_k is not None:
-        harness.E2M3_MIN_K = args.min_k
+        harness.E2M3_MIN_K = harness.E2M3_MIN_K_NARROW = args.min_k
     if args.matrix_path is not None:
         harness.MATRIX_PATH = args.matrix_path
 

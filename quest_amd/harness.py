@@ -22,7 +22,9 @@ WEIGHT_HADAMARD_SCALE = 2. ** -3.5      # utils.py:39
 # INT8 kernels on packed nibbles.  Both give the same bits.
 MATRIX_PATH = 'fp6'
 E2M3_MIN_TOKENS = 33                    # from here on the FP6 kernels are the faster ones
-E2M3_MIN_K = 2048                       # shortest rows that take them at more than E2M3_SHORT_ROWS_TOKENS tokens (see prefers_e2m3)
+E2M3_MIN_K = 1536                       # shortest rows that take them at more than E2M3_SHORT_ROWS_TOKENS tokens (see prefers_e2m3)
+E2M3_MIN_K_NARROW = 2048                # ... by a layer of fewer than E2M3_NARROW channels
+E2M3_NARROW = 1536
 E2M3_SHORT_ROWS_TOKENS = 4096
 # Whether a producer-fused block lets the FP6 GEMM of an output projection add into the residual stream itself
 # (same bits as the addition inside the next norm kernel; one pass over the stream less).
@@ -37,11 +39,12 @@ def prefers_e2m3(m: int, k: int, n: int) -> bool:
     1024 to 22016 and M from 20 to 3000 they win 3 to 60 % from 33 tokens on (1.2 x on average; level or up to 8 % behind at 33 to 64
     tokens with K = 1024, N = 11264 and K = 4096, N = 22016) and lose below, where the weights' 1.5 x bytes are the whole cost."""
     # E2M3_MIN_K: with shorter rows and many tokens the GEMM is mostly epilogue either way and the tile-writing activation kernels
-    # are a little slower than the row-writing ones (12.0 against 10.2 us at [16384, 1024]) -- measured on the 12-layer
-    # d = 1024 model at 32 x 512 tokens: 6.01 ms per forward with the FP6 path from K = 1024 on, 5.79 ms from K = 2048 on
-    # (its K = 2816 layers), 5.80 ms without it
+    # are a little slower than the row-writing ones (12.0 against 10.2 us at [16384, 1024]).  Whole layers of 4097 to 16384 tokens,
+    # INT8 / FP6 time: K = 1536 1.12 on average over N from 1500 to 22016, K = 1792 1.14, K = 1920 1.16, 0.98 at the least ((8192,
+    # 1536, 8192) 103 / 84 us, (16384, 1536, 3072) 85 / 70); K = 1024 0.85 to 1.18 ((16384, 1024, 8192) 148 / 173 us), K = 1152 to
+    # 1408 0.94 to 1.27.  Layers of 1024 channels lose 6 to 12 % at 8192 tokens up to K = 1920 (half a 256 x 256 tile per CU).
     return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and k <= 65536 and m * n <= (1 << 30)
-            and (k >= E2M3_MIN_K or m <= E2M3_SHORT_ROWS_TOKENS))
+            and (m <= E2M3_SHORT_ROWS_TOKENS or k >= (E2M3_MIN_K if n >= E2M3_NARROW else E2M3_MIN_K_NARROW)))
 
 
 def weight_tiles(w_int_packed: torch.Tensor) -> torch.Tensor:
