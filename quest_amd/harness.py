@@ -40,8 +40,8 @@ def prefers_e2m3(m: int, k: int, n: int) -> bool:
     tokens with K = 1024, N = 11264 and K = 4096, N = 22016) and lose below, where the weights' 1.5 x bytes are the whole cost."""
     # E2M3_MIN_K: with shorter rows and many tokens the GEMM is mostly epilogue either way and the tile-writing activation kernels
     # are a little slower than the row-writing ones (12.0 against 10.2 us at [16384, 1024]).  Whole layers of 4097 to 16384 tokens,
-    # INT8 / FP6 time: K = 1536 1.12 on average over N from 1500 to 22016, K = 1792 1.14, K = 1920 1.16, 0.98 at the least ((8192,
-    # 1536, 8192) 103 / 84 us, (16384, 1536, 3072) 85 / 70); K = 1024 0.85 to 1.18 ((16384, 1024, 8192) 148 / 173 us), K = 1152 to
+    # INT8 / FP6 time: K = 1536 1.12 on average over N from 1500 to 22016, K = 1792 1.14, K = 1920 1.16, 0.98 at the least ((4097,
+    # 1536, 1536) 33.7 / 27.4 us, (8192, 1536, 8192) 103 / 84, (16384, 1536, 3072) 85 / 70); K = 1024 0.85 to 1.18 ((16384, 1024, 8192) 148 / 173 us), K = 1152 to
     # 1408 0.94 to 1.27.  Layers of 1024 channels lose 6 to 12 % at 8192 tokens up to K = 1920 (half a 256 x 256 tile per CU).
     return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and k <= 65536 and m * n <= (1 << 30)
             and (m <= E2M3_SHORT_ROWS_TOKENS or k >= (E2M3_MIN_K if n >= E2M3_NARROW else E2M3_MIN_K_NARROW)))
