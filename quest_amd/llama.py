@@ -23,6 +23,7 @@ from dataclasses import dataclass
 import torch
 from torch import nn
 from torch.nn import functional as F
+from torch.nn.modules import module as _module
 
 from . import api as quest
 from . import harness
@@ -73,6 +74,12 @@ def apply_rotary_emb(q: torch.Tensor, k: torch.Tensor, freqs_cis: torch.Tensor):
         return torch.stack((re, im), dim=-1).flatten(3).to(dtype)
 
     return rot(q), rot(k)
+
+
+def _as_built(module: nn.Module, cls: type) -> bool:
+    """Whether `module` is a plain `cls` whose call is its class's `forward` and nothing else: no hook, no method of its own."""
+    return (type(module) is cls and 'forward' not in module.__dict__ and not module._forward_hooks and not module._forward_pre_hooks
+            and not _module._global_forward_hooks and not _module._global_forward_pre_hooks)
 
 
 class RMSNorm(nn.Module):
@@ -381,12 +388,21 @@ class Llama(nn.Module):
         # one position per sequence: norm and head read those rows only
         x, branch = self._stream(idx)
         norm, head = self.transformer.ln_f, self.lm_head
-        if not torch.is_grad_enabled() and type(head) is nn.Linear and head.bias is None:
+        if x.is_cuda and self._native_end():
             logits = quest.host.last_logits(x, branch, norm.weight, float(norm.eps), head.weight)
             if logits is not None:
                 return {'logits': logits}
         x = x[:, -1:, :]                               # a slice: index lists copy from the host
         return {'logits': head(norm(x if branch is None else x + branch[:, -1:, :]))}
+
+    def _native_end(self) -> bool:
+        """Whether the native norm and head may stand in for `ln_f` and `lm_head`: both still what the constructor made, nothing
+        that a call of theirs would run or record passed by, and a stream that came out of W4A4 linears -- kernels that tracing,
+        vmap and forward-mode derivatives do not see either (a dense model keeps them)."""
+        blocks = self.transformer.h
+        return (len(blocks) > 0 and isinstance(blocks[-1], LlamaBlock) and isinstance(blocks[-1].mlp.c_proj, harness.Linear4bit)
+                and not torch.is_grad_enabled() and not torch.is_autocast_enabled('cuda')
+                and _as_built(self.transformer.ln_f, RMSNorm) and _as_built(self.lm_head, nn.Linear) and self.lm_head.bias is None)
 
 
 def _pack(linear: nn.Linear, use_hadamard: bool, use_noop: bool, from_fp32: bool = False) -> harness.Linear4bit:

@@ -1,0 +1,69 @@
+"""A packed model whose parts a user has replaced, hooked or run under another mode: the native calls stand in for modules only
+where nothing is passed by."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda:0'
+
+
+def packed(seq=64, **options):
+    from quest_amd import llama
+    torch.manual_seed(21)
+    cfg = llama.LlamaConfig(n_layer=2, n_embd=256, n_head=4, vocab_size=384, sequence_length=seq)
+    model = llama.Llama(cfg).to(torch.bfloat16).to(DEV).eval()
+    ids = torch.randint(0, cfg.vocab_size, (2, 40), generator=torch.Generator().manual_seed(22)).to(DEV)
+    return llama.quantize_model(model, 'int4', **{'fuse_producers': True, **options}), ids
+
+
+@pytest.mark.parametrize('fuse', [True, False])
+@pytest.mark.parametrize('change', ['none', 'layernorm', 'identity', 'own_forward'])
+def test_last_logits_are_the_modules_own(fuse, change):
+    """The last position of all logits, which the modules themselves compute (bf16 outputs: 2^-8 of a logit each way, and a norm
+    summed in another order)."""
+    model, ids = packed(fuse_producers=fuse)
+    if change == 'layernorm':
+        model.transformer.ln_f = torch.nn.LayerNorm(256).to(DEV).bfloat16()
+        model.transformer.ln_f.bias.data.fill_(0.5)
+    elif change == 'identity':
+        model.transformer.ln_f = torch.nn.Identity()
+    elif change == 'own_forward':
+        model.lm_head.forward = lambda x: torch.nn.functional.linear(x, model.lm_head.weight) + 3
+    with torch.no_grad():
+        last, every = model(ids)['logits'], model(ids, all_logits=True)['logits']
+    want = every[:, -1:].double()
+    assert (last.double() - want).norm() <= 2. ** -7 * want.norm()
+
+
+@pytest.mark.parametrize('which', ['ln_f', 'lm_head', 'global'])
+def test_hooks_on_the_norm_and_the_head_run(which):
+    model, ids = packed()
+    seen = []
+    mods = {'ln_f': model.transformer.ln_f, 'lm_head': model.lm_head}
+    if which == 'global':
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda m, *_: seen.append(m))
+    else:
+        handle = mods[which].register_forward_hook(lambda m, i, o: seen.append(m) or o * 2)
+    try:
+        with torch.no_grad():
+            got = model(ids)['logits']
+    finally:
+        handle.remove()
+    assert all(seen.count(mods[w]) == 1 for w in mods if which in (w, 'global'))
+    if which == 'lm_head':                                   # what the hook returns is the output
+        with torch.no_grad():
+            want = 2 * model(ids)['logits'].double()
+        assert (got.double() - want).norm() <= 2. ** -7 * want.norm()
+
+
+def test_dense_model_is_traceable_under_no_grad():
+    """No tensor of the forward leaves torch's view: a trace replayed on other ids follows them."""
+    from quest_amd import llama
+    torch.manual_seed(23)
+    cfg = llama.LlamaConfig(n_layer=1, n_embd=128, n_head=2, vocab_size=64, sequence_length=16)
+    model = llama.Llama(cfg).to(torch.bfloat16).to(DEV).eval().requires_grad_(False)
+    a, b = (torch.randint(0, 64, (2, 9), generator=torch.Generator().manual_seed(s)).to(DEV) for s in (1, 2))
+    with torch.no_grad():
+        model(a)
+        traced = torch.jit.trace(lambda ids: model(ids)['logits'], (a,), check_trace=False)
+        assert torch.equal(traced(b), model(b)['logits'])

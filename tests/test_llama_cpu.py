@@ -167,3 +167,22 @@ def test_reference_checkpoint_file_loads_weights_only(tmp_path):
     other = llama.Llama(cfg)
     llama.load_reference_checkpoint(other, str(tmp_path / 'bare.pt'))
     assert torch.equal(other.lm_head.weight, donor.lm_head.weight)
+
+
+class _NoLibrary:
+    def __getattr__(self, name):
+        raise RuntimeError('the native module is not built')
+
+
+@pytest.mark.parametrize('norm', ['own', 'identity', 'layernorm'])
+def test_dense_forward_runs_its_own_norm_and_head_without_the_native_module(monkeypatch, norm):
+    """A dense model on the CPU under no_grad needs no library, whatever its final norm is: the last position of all logits."""
+    from quest_amd import api
+    monkeypatch.setattr(api, 'host', _NoLibrary())
+    model, cfg = tiny_model()
+    if norm != 'own':
+        model.transformer.ln_f = torch.nn.Identity() if norm == 'identity' else torch.nn.LayerNorm(cfg.n_embd)
+    ids = torch.randint(0, cfg.vocab_size, (2, 7), generator=torch.Generator().manual_seed(2))
+    with torch.no_grad():
+        last, every = model(ids)['logits'], model(ids, all_logits=True)['logits']
+    assert torch.allclose(last, every[:, -1:], rtol=1e-4, atol=1e-5)
