@@ -255,9 +255,9 @@ class LlamaBlock(nn.Module):
         att = None
         gemm_adds = harness.GEMM_ADDS_RESIDUAL
         o_proj = self.attn.c_proj
-        packed_adds = (isinstance(o_proj, harness.Linear4bit) and o_proj.use_hadamard and o_proj.bias is None
-                       and not o_proj.quantize_from_fp32)
-        if gemm_adds and harness.prefers_e2m3(m, c, c) and isinstance(o_proj, harness.Linear4bit) and o_proj.use_hadamard:
+        plain = _as_built(o_proj, harness.Linear4bit) and o_proj.use_hadamard         # (a hook on it wants its call, below)
+        packed_adds = plain and o_proj.bias is None and not o_proj.quantize_from_fp32
+        if gemm_adds and harness.prefers_e2m3(m, c, c) and plain:
             core = self.attn.attention_core(qkv.view(b, t, 3 * c), freqs_cis, rotated)
             o_proj.forward_tiles(*quest.hadamard_quantize_e2m3(core.view(m, c)), out=x2, add_to_out=True)
         elif gemm_adds and harness.GEMM_ADDS_RESIDUAL_PACKED and packed_adds and quest.gemm_add_fuses(m, c, c, x.device):
@@ -307,15 +307,20 @@ class LlamaBlock(nn.Module):
     def _forward_native(self, x, freqs_cis, branch, m, c, hidden):
         """`forward_fused` as one call of the native host path (the same kernels in the same order; at 37 tokens the
         twelve launches of a block cost 240 us from Python and about 50 from there).  None, with nothing launched, where
-        an option is not at its default: the statement in Python then runs."""
+        an option is not at its default or a part has been replaced or hooked: the statement in Python then runs."""
         attn, mlp = self.attn, self.mlp
+        if type(attn) is not LlamaAttention or type(mlp) is not LlamaMLP:
+            return None
         linears = (attn.c_attn, attn.c_proj, mlp.w12, mlp.c_proj)
         if not (mlp.glu is not None and attn.fused_rope and harness.GEMM_ADDS_RESIDUAL and harness.GEMM_ADDS_RESIDUAL_PACKED
-                and harness.GEMM_ROTATES_QK):
+                and harness.GEMM_ROTATES_QK and _as_built(attn.c_proj, harness.Linear4bit)):
             return None
+        for part, methods in ((attn, ('attend', 'attention_core')), (mlp, ('swiglu_quantized', 'swiglu_tiles'))):
+            if methods[0] in part.__dict__ or methods[1] in part.__dict__:
+                return None
         for w in linears:
             if not (type(w) is harness.Linear4bit and w.bias is None and w.use_hadamard and not w.use_noop
-                    and not w.quantize_from_fp32):
+                    and not w.quantize_from_fp32 and 'forward_quantized' not in w.__dict__ and 'forward_tiles' not in w.__dict__):
                 return None
         tiles = (harness.prefers_e2m3(m, c, 3 * c) | harness.prefers_e2m3(m, c, c) << 1
                  | harness.prefers_e2m3(m, c, 2 * hidden) << 2 | harness.prefers_e2m3(m, hidden, c) << 3)

@@ -67,3 +67,35 @@ def test_dense_model_is_traceable_under_no_grad():
         model(a)
         traced = torch.jit.trace(lambda ids: model(ids)['logits'], (a,), check_trace=False)
         assert torch.equal(traced(b), model(b)['logits'])
+
+
+@pytest.mark.parametrize('batch,seq', [(1, 8), (2, 40), (4, 64)])
+def test_a_hook_on_the_output_projection_is_the_blocks_output(batch, seq):
+    """The projection is called, and what the hook returns is what the stream gets: with zeros, a block without attention."""
+    model, _ = packed()
+    ids = torch.randint(0, 384, (batch, seq), generator=torch.Generator().manual_seed(24)).to(DEV)
+    calls = []
+    for block in model.transformer.h:
+        block.attn.c_proj.register_forward_hook(lambda m, i, o: calls.append(m) or torch.zeros_like(o))
+    with torch.no_grad():
+        got = model(ids, all_logits=True)['logits']
+    assert len(calls) == 2
+    for block in model.transformer.h:
+        block.attn.c_proj._forward_hooks.clear()
+        block.attn.c_proj.w_scale.zero_()
+    with torch.no_grad():
+        assert torch.equal(got, model(ids, all_logits=True)['logits'])
+
+
+@pytest.mark.parametrize('part,method', [('attn', 'attention_core'), ('mlp', 'swiglu_quantized')])
+def test_replaced_methods_of_a_fused_block_run(part, method):
+    model, ids = packed()
+    ids = ids[:1, :20]                                                 # few tokens: packed codes in front of the gated unit
+    calls = []
+    module = getattr(model.transformer.h[0], part)
+    own = getattr(module, method)
+    with torch.no_grad():
+        want = model(ids)['logits']
+        setattr(module, method, lambda *a, **k: calls.append(1) or own(*a, **k))
+        assert torch.equal(model(ids)['logits'], want)
+    assert calls
