@@ -10,6 +10,7 @@
 // caller's Python statement of the same call runs, which raises what there is to raise.  Nothing is cached between calls.
 #include <Python.h>
 
+#include <ATen/autocast_mode.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <ATen/ops/empty.h>
@@ -406,6 +407,8 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const at::Tensor *xp = args.tensor(a[0]);
     if (!args.ok || !is_half(xp->scalar_type()) || xp->dim() != 3) return declined();
     const at::ScalarType type = xp->scalar_type();
+    // (the attention below would hand back another type than the kernels after it are told)
+    if (at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) != type) return declined();
     const int64_t b = xp->size(0), t = xp->size(1), c64 = xp->size(2);
     if (!fits_int(b * t) || !fits_int(3 * c64)) return declined();
     const int m = (int)(b * t), c = (int)c64;

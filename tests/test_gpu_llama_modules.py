@@ -99,3 +99,18 @@ def test_replaced_methods_of_a_fused_block_run(part, method):
         setattr(module, method, lambda *a, **k: calls.append(1) or own(*a, **k))
         assert torch.equal(model(ids)['logits'], want)
     assert calls
+
+
+@pytest.mark.parametrize('seq', [8, 100])
+def test_fused_block_under_autocast(seq):
+    """Autocast to the model's own type keeps the logits; to the other one, the attention's output no longer has the type of the
+    weights, which is refused."""
+    model, _ = packed(seq=128)
+    ids = torch.randint(0, 384, (1, seq), generator=torch.Generator().manual_seed(25)).to(DEV)
+    with torch.no_grad():
+        want = model(ids)['logits']
+        with torch.autocast('cuda', dtype=torch.bfloat16):
+            got = model(ids)['logits']                       # (its head is torch's then: one rounding apart)
+            assert (got.double() - want.double()).norm() <= 2. ** -7 * want.double().norm()
+        with torch.autocast('cuda', dtype=torch.float16), pytest.raises(AssertionError):
+            model(ids)
