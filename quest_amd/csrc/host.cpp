@@ -113,6 +113,8 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const double had_scale = PyFloat_AsDouble(a[6]);
     const at::Tensor *given = a[7] == Py_None ? nullptr : args.matrix(a[7], type, m, n);
     if (!args.ok) return declined();
+    // (a bias whose derivative is wanted is added by torch)
+    if (bias != nullptr && ((at::GradMode::is_enabled() && bias->requires_grad()) || bias->_fw_grad(0).defined())) return declined();
 
     const c10::DeviceGuard guard(args.dev);
     void *st = stream_of(args.dev);

@@ -310,12 +310,13 @@ class Linear4bit(nn.Module):
         n = self.weight.size(0)
         if not self.use_noop and not self.quantize_from_fp32 and x.dim() > 0:
             k = x.size(-1)
-            held = self._buffers
-            tiles = self.w_tiles() if prefers_e2m3(x.numel() // max(k, 1), k, n) else None
-            y = quest.host.linear(x, held['w_int_packed'], held['w_scale'], held['w_add'], tiles, self.bias,
-                                  HADAMARD_ENTRY if self.use_hadamard else 0., None)
-            if y is not None:
-                return y
+            held = self._buffers.get                  # (not there, e.g. made a parameter: the native call declines)
+            if held('w_meta_e') is None:
+                tiles = self.w_tiles() if prefers_e2m3(x.numel() // max(k, 1), k, n) else None
+                y = quest.host.linear(x, held('w_int_packed'), held('w_scale'), held('w_add'), tiles, self.bias,
+                                      HADAMARD_ENTRY if self.use_hadamard else 0., None)
+                if y is not None:
+                    return y
         lead, n = x.shape[:-1], self.weight.size(0)
         rows = x.contiguous().view(-1, x.size(-1))
         if self.use_noop:

@@ -326,14 +326,14 @@ class LlamaBlock(nn.Module):
                  | harness.prefers_e2m3(m, c, 2 * hidden) << 2 | harness.prefers_e2m3(m, hidden, c) << 3)
         if tiles & 4 and mlp.glu_tiles is None:
             mlp.glu_tiles = harness.weight_tiles(mlp.glu[0])
-        qkv, o, both, down = (w._buffers for w in linears)
+        qkv, o, both, down = (w._buffers.get for w in linears)
         return quest.host.block(
             x, branch, freqs_cis, attn.n_head, self.ln_1.weight, float(self.ln_1.eps), self.ln_2.weight, float(self.ln_2.eps),
-            (qkv['w_int_packed'], qkv['w_scale'], qkv['w_add'], attn.c_attn.w_tiles() if tiles & 1 else None),
-            (o['w_int_packed'], o['w_scale'], o['w_add'], attn.c_proj.w_tiles() if tiles & 2 else None),
-            (both['w_int_packed'], both['w_scale'], both['w_add'], None),
+            (qkv('w_int_packed'), qkv('w_scale'), qkv('w_add'), attn.c_attn.w_tiles() if tiles & 1 else None),
+            (o('w_int_packed'), o('w_scale'), o('w_add'), attn.c_proj.w_tiles() if tiles & 2 else None),
+            (both('w_int_packed'), both('w_scale'), both('w_add'), None),
             (*mlp.glu, mlp.glu_tiles),
-            (down['w_int_packed'], down['w_scale'], down['w_add'], mlp.c_proj.w_tiles() if tiles & 8 else None),
+            (down('w_int_packed'), down('w_scale'), down('w_add'), mlp.c_proj.w_tiles() if tiles & 8 else None),
             tiles)
 
 
