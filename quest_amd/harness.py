@@ -47,6 +47,11 @@ def prefers_e2m3(m: int, k: int, n: int) -> bool:
             and (m <= E2M3_SHORT_ROWS_TOKENS or k >= (E2M3_MIN_K if n >= E2M3_NARROW else E2M3_MIN_K_NARROW)))
 
 
+def e2m3_fits(k: int, rows: int) -> bool:
+    """Whether codes of `rows` rows can be laid out as E2M3 tiles and multiplied by the FP6 kernels."""
+    return k % 128 == 0 and 0 < k <= 65536 and rows <= 32 * 65535 and (rows + 287) // 32 * (k // 64) * 1536 < 1 << 31
+
+
 def weight_tiles(w_int_packed: torch.Tensor) -> torch.Tensor:
     """The E2M3 tiles of packed weight codes (N, K/2): the FP6 kernel's operand form (1.5 x the packed bytes)."""
     return quest.int4_to_e2m3_tiles(w_int_packed)
@@ -206,9 +211,11 @@ class Linear4bit(nn.Module):
 
     def _install(self, weight: torch.Tensor, bias) -> None:
         """Pack `weight` (N, K) and keep `bias` (a tensor, a parameter or None) as a frozen parameter."""
-        packed, scale, add, _ = preprocess_weight(weight=weight, use_hadamard=self.use_hadamard,
-                                                  quantize_from_fp32=self.quantize_from_fp32)
+        with torch.inference_mode(False), torch.no_grad():           # buffers with a version counter: see _kept_tiles
+            packed, scale, add, _ = preprocess_weight(weight=weight, use_hadamard=self.use_hadamard,
+                                                      quantize_from_fp32=self.quantize_from_fp32)
         self._set_buffers(weight.shape, weight.dtype, packed, scale, add)
+        self.lay_out_tiles()
         if bias is None:
             self.bias = None
         else:
@@ -218,19 +225,60 @@ class Linear4bit(nn.Module):
         self.weight = torch.empty(shape, dtype=dtype, device='meta')
         for name, t in (('w_int_packed', packed), ('w_scale', scale), ('w_add', add), ('w_meta_e', None)):
             self.register_buffer(name, t)
-        self._tiles = None               # E2M3 tiles of w_int_packed: derived data, built on first use, not in checkpoints
-        self._tiles_of = None
+        self._tiles = None               # (E2M3 tiles, of which tensor, its address, its version): derived, not in checkpoints
+
+    def lay_out_tiles(self) -> None:
+        """Keep the weight codes as E2M3 tiles as well, the FP6 kernels' operand form (1.5 x the packed bytes on top of them).
+        Done where the buffers get their content -- packing, `load_state_dict`, a move to another device, a copy -- on the stream
+        that writes them, so whoever may read the buffers may read the tiles, and no forward call, on whatever stream or
+        under capture, has anything to build.  After writing into `w_int_packed` by hand, call it again: until then the layer runs on
+        its packed codes (the same bits).  Nothing is kept for a layer that the FP6 kernels do not take, or while MATRIX_PATH is
+        'int8'."""
+        self._tiles = None
+        w = self._buffers.get('w_int_packed')
+        if type(w) is not torch.Tensor or not w.is_cuda or w.dim() != 2 or not w.is_contiguous():
+            return
+        with torch.inference_mode(False), torch.no_grad():
+            if w.is_inference():                                     # (it would not show later writes)
+                w = self._buffers['w_int_packed'] = w.clone()
+            if MATRIX_PATH == 'fp6' and e2m3_fits(w.size(1) * 2, w.size(0)):
+                self._tiles = (weight_tiles(w), w, w.data_ptr(), w._version)
+
+    def _kept_tiles(self):
+        """The tiles of what `w_int_packed` holds now, or None."""
+        kept = self._tiles
+        if kept is None:
+            return None
+        tiles, source, address, version = kept
+        w = self._buffers.get('w_int_packed')
+        return tiles if w is source and w._version == version and w.data_ptr() == address else None
+
+    def tiles_for(self, m: int):
+        """The weight's E2M3 tiles where the FP6 kernels are the faster ones for m tokens, None where the packed codes serve."""
+        n, k = self.weight.shape
+        return self._kept_tiles() if prefers_e2m3(m, k, n) else None
 
     def w_tiles(self) -> torch.Tensor:
-        """The weight codes as E2M3 tiles (built once per content of `w_int_packed`, e.g. again after a checkpoint
-        has been loaded into the buffers)."""
-        w = self.w_int_packed
-        # a tensor created in inference mode keeps no version counter (asking for it raises: 10 us a call)
-        key = (w.data_ptr(), None if w.is_inference() else w._version)
-        if self._tiles is None or self._tiles_of != key:
-            self._tiles = weight_tiles(w)
-            self._tiles_of = key
-        return self._tiles
+        """The weight codes as E2M3 tiles: the kept ones, or a conversion of the buffer for this call."""
+        tiles = self._kept_tiles()
+        return weight_tiles(self.w_int_packed) if tiles is None else tiles
+
+    def _load_from_state_dict(self, *args, **kwargs):
+        super()._load_from_state_dict(*args, **kwargs)
+        self.lay_out_tiles()
+
+    def _apply(self, *args, **kwargs):
+        super()._apply(*args, **kwargs)
+        if self._kept_tiles() is None:
+            self.lay_out_tiles()
+        return self
+
+    def __getstate__(self):
+        return {**self.__dict__, '_tiles': None}
+
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        self.lay_out_tiles()
 
     @classmethod
     def from_weight(cls, weight: torch.Tensor, bias: torch.Tensor = None, use_hadamard: bool = False,
@@ -250,10 +298,11 @@ class Linear4bit(nn.Module):
         self = cls.__new__(cls)
         nn.Module.__init__(self)
         self._configure(use_hadamard, False)
-        self._set_buffers((out_features, in_features), dtype,
-                          torch.zeros(out_features, in_features // 2, dtype=torch.uint8, device=device),
-                          torch.zeros(out_features, 1, dtype=dtype, device=device),
-                          torch.zeros(out_features, 1, dtype=torch.int32, device=device))
+        with torch.inference_mode(False):
+            self._set_buffers((out_features, in_features), dtype,
+                              torch.zeros(out_features, in_features // 2, dtype=torch.uint8, device=device),
+                              torch.zeros(out_features, 1, dtype=dtype, device=device),
+                              torch.zeros(out_features, 1, dtype=torch.int32, device=device))
         self.bias = nn.Parameter(torch.zeros(out_features, dtype=dtype, device=device), requires_grad=False) if bias else None
         return self
 
@@ -312,7 +361,7 @@ class Linear4bit(nn.Module):
             k = x.size(-1)
             held = self._buffers.get                  # (not there, e.g. made a parameter: the native call declines)
             if held('w_meta_e') is None:
-                tiles = self.w_tiles() if prefers_e2m3(x.numel() // max(k, 1), k, n) else None
+                tiles = self._kept_tiles() if prefers_e2m3(x.numel() // max(k, 1), k, n) else None
                 y = quest.host.linear(x, held('w_int_packed'), held('w_scale'), held('w_add'), tiles, self.bias,
                                       HADAMARD_ENTRY if self.use_hadamard else 0., None)
                 if y is not None:
@@ -329,7 +378,7 @@ class Linear4bit(nn.Module):
             m, k = rows.shape
             y = linear_forward(rows, self.w_int_packed, self.w_scale, self.w_add, self.w_meta_e,
                                use_hadamard=self.use_hadamard, quantize_from_fp32=self.quantize_from_fp32,
-                               w_tiles=self.w_tiles() if prefers_e2m3(m, k, n) and not self.quantize_from_fp32 else None)
+                               w_tiles=None if self.quantize_from_fp32 else self.tiles_for(m))
         if self.bias is not None:
             y += self.bias
         return y.view(*lead, n)

@@ -104,17 +104,48 @@ class LlamaMLP(nn.Module):
         self.w2 = nn.Linear(config.n_embd, config.hidden_dim, bias=False)
         self.c_proj = nn.Linear(config.hidden_dim, config.n_embd, bias=False)
         self.w12 = None          # set by quantize_model(..., fuse_gate_up=True): one module for both
-        self.glu = None          # enable_swiglu_epilogue(): w12's packed rows in the order the gated-unit GEMM reads
-        self.glu_tiles = None
+        self.glu = None          # enable_swiglu_epilogue(): w12's packed rows in the order the gated-unit GEMM reads,
+        self.glu_tiles = None    # ... as E2M3 tiles,
+        self._glu_of = None      # ... and what they were made from
+        self.register_load_state_dict_post_hook(_renew_swiglu)
 
     def enable_swiglu_epilogue(self):
         """A second copy of the fused gate/up weights with the rows interleaved in eights (four gate rows, then the four
         up rows of the same outputs; `quest.swiglu_interleave_rows`), which lets the GEMM apply silu(gate) * up in
-        its epilogue.  Plain tensors, not buffers: they are derived data and stay out of checkpoints."""
+        its epilogue, and its E2M3 tiles in place of w12's own (`Linear4bit.lay_out_tiles` says when and why they are made).
+        Plain tensors, not buffers: they are derived data and stay out of checkpoints."""
         w = self.w12
         p = quest.swiglu_interleave_rows(w.w_int_packed.size(0) // 2, device=w.w_int_packed.device)
-        self.glu = (w.w_int_packed[p].contiguous(), w.w_scale[p].contiguous(), w.w_add[p].contiguous())
-        self.glu_tiles = None            # the interleaved rows as E2M3 tiles, built on first use
+        glu = (w.w_int_packed[p].contiguous(), w.w_scale[p].contiguous(), w.w_add[p].contiguous())
+        rows, half_k = glu[0].shape
+        fits = harness.MATRIX_PATH == 'fp6' and glu[0].is_cuda and harness.e2m3_fits(2 * half_k, rows)
+        self.glu, self.glu_tiles, self._glu_of = glu, harness.weight_tiles(glu[0]) if fits else None, self._glu_source()
+        w._tiles = None
+
+    def _glu_source(self):
+        return [(t, t.data_ptr(), None if t.is_inference() else t._version) for t in (self.w12.w_int_packed, self.w12.w_scale, self.w12.w_add)]
+
+    def kept_glu(self):
+        """`glu`, if w12 still holds what it was made from."""
+        if self.glu is None or self._glu_of is None:
+            return None
+        for (t, address, version), name in zip(self._glu_of, ('w_int_packed', 'w_scale', 'w_add')):
+            now = self.w12._buffers.get(name)
+            if now is not t or now.data_ptr() != address or (version is not None and now._version != version):
+                return None
+        return self.glu
+
+    def _apply(self, *args, **kwargs):
+        super()._apply(*args, **kwargs)
+        _renew_swiglu(self)
+        return self
+
+    def __getstate__(self):
+        return {**self.__dict__, 'glu_tiles': None, '_glu_of': None}
+
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        _renew_swiglu(self)
 
     def swiglu_quantized(self, a_scale, a_int_packed, a_int_row_sum):
         """silu(w1 x) * w2 x, (M, hidden), from the codes of x; the gated unit runs in the GEMM's epilogue when that
@@ -122,20 +153,19 @@ class LlamaMLP(nn.Module):
         m = a_int_packed.size(0)
         if self.w12.use_noop:
             return torch.zeros(m, self.c_proj.weight.size(1), dtype=a_scale.dtype, device=a_scale.device)
-        if self.glu is not None and m > 64 and a_int_packed.size(1) % 64 == 0 and self.w12.bias is None:
-            w_packed, w_scale, w_add = self.glu
+        glu = self.kept_glu()
+        if glu is not None and m > 64 and a_int_packed.size(1) % 64 == 0 and self.w12.bias is None:
+            w_packed, w_scale, w_add = glu
             return quest.fused_matmul_dequantize_swiglu_int4_int4t(a_int_packed, w_packed, a_int_row_sum, w_add, a_scale, w_scale)
         gate_up = self.w12.forward_quantized(a_scale, a_int_packed, a_int_row_sum)
         h = gate_up.size(-1) // 2
         return F.silu(gate_up[..., :h]) * gate_up[..., h:]
 
     def swiglu_tiles(self, a_scale, a_tiles):
-        """The same from the E2M3 tiles of x, on the FP6 matrix instructions (needs enable_swiglu_epilogue())."""
+        """The same from the E2M3 tiles of x, on the FP6 matrix instructions (needs enable_swiglu_epilogue() and its tiles)."""
         w_packed, w_scale, _ = self.glu
         if self.w12.use_noop:
             return torch.zeros(a_scale.numel(), self.c_proj.weight.size(1), dtype=a_scale.dtype, device=a_scale.device)
-        if self.glu_tiles is None:
-            self.glu_tiles = harness.weight_tiles(w_packed)
         return quest.fused_matmul_dequantize_e2m3(a_tiles, self.glu_tiles, a_scale, w_scale, w_packed.size(1) * 2, swiglu=True)
 
     def forward(self, x):
@@ -144,6 +174,12 @@ class LlamaMLP(nn.Module):
             h = gate_up.size(-1) // 2
             return self.c_proj(F.silu(gate_up[..., :h]) * gate_up[..., h:])
         return self.c_proj(F.silu(self.w1(x)) * self.w2(x))
+
+
+def _renew_swiglu(mlp: LlamaMLP, _incompatible_keys=None) -> None:
+    """The interleaved copy again after w12 got other content (a load, a move, a copy of the module)."""
+    if mlp.glu is not None and mlp.kept_glu() is None:
+        mlp.enable_swiglu_epilogue()
 
 
 class LlamaAttention(nn.Module):
@@ -223,7 +259,9 @@ class LlamaBlock(nn.Module):
         # each producer writes the operand form its GEMM runs fastest on: E2M3 tiles for the FP6 kernel, or packed
         # nibbles and row sums for the INT8 kernels (same codes, same output bits either way)
         rotated = False
-        if harness.prefers_e2m3(m, c, 3 * c):
+        glu = self.mlp.kept_glu()
+        qkv_tiles, o_tiles, gate_tiles, down_tiles = self._tiles_for(m, glu)
+        if qkv_tiles is not None:
             if branch is None:
                 q = quest.rmsnorm_hadamard_quantize_e2m3(x2, self.ln_1.weight, self.ln_1.eps)
             else:
@@ -257,7 +295,7 @@ class LlamaBlock(nn.Module):
         o_proj = self.attn.c_proj
         plain = _as_built(o_proj, harness.Linear4bit) and o_proj.use_hadamard         # (a hook on it wants its call, below)
         packed_adds = plain and o_proj.bias is None and not o_proj.quantize_from_fp32
-        if gemm_adds and harness.prefers_e2m3(m, c, c) and plain:
+        if gemm_adds and o_tiles is not None and plain:
             core = self.attn.attention_core(qkv.view(b, t, 3 * c), freqs_cis, rotated)
             o_proj.forward_tiles(*quest.hadamard_quantize_e2m3(core.view(m, c)), out=x2, add_to_out=True)
         elif gemm_adds and harness.GEMM_ADDS_RESIDUAL_PACKED and packed_adds and quest.gemm_add_fuses(m, c, c, x.device):
@@ -266,7 +304,6 @@ class LlamaBlock(nn.Module):
             o_proj.forward_quantized(*quest.hadamard_quantize_int4(core.view(m, c)), out=x2, add_to_out=True)
         else:
             att = self.attn.attend(qkv.view(b, t, 3 * c), freqs_cis, rotated)
-        down_tiles = harness.prefers_e2m3(m, hidden, c)
 
         def second_norm(tiles: bool):
             if att is None:
@@ -275,32 +312,24 @@ class LlamaBlock(nn.Module):
             f = quest.add_rmsnorm_hadamard_quantize_e2m3 if tiles else quest.add_rmsnorm_hadamard_quantize_int4
             return f(x2, att.view(m, c), self.ln_2.weight, self.ln_2.eps)
 
-        if harness.prefers_e2m3(m, c, 2 * hidden):
-            q = second_norm(True)
-            if self.mlp.glu is not None:
-                act = self.mlp.swiglu_tiles(*q)
-                q = quest.hadamard_quantize_e2m3(act) if down_tiles else quest.hadamard_quantize_int4(act)
-            else:
-                gate_up = self.mlp.w12.forward_tiles(*q)
-                q = quest.silu_mul_hadamard_quantize_e2m3(gate_up) if down_tiles else quest.silu_mul_hadamard_quantize_int4(gate_up)
+        on_tiles = down_tiles is not None
+        q = second_norm(gate_tiles is not None)
+        if glu is not None:
+            act = self.mlp.swiglu_tiles(*q) if gate_tiles is not None else self.mlp.swiglu_quantized(*q)
+            q = quest.hadamard_quantize_e2m3(act) if on_tiles else quest.hadamard_quantize_int4(act)
         else:
-            q = second_norm(False)
-            if self.mlp.glu is not None:
-                act = self.mlp.swiglu_quantized(*q)
-                q = quest.hadamard_quantize_e2m3(act) if down_tiles else quest.hadamard_quantize_int4(act)
-            else:
-                gate_up = self.mlp.w12.forward_quantized(*q)
-                q = quest.silu_mul_hadamard_quantize_e2m3(gate_up) if down_tiles else quest.silu_mul_hadamard_quantize_int4(gate_up)
-        if down_tiles and gemm_adds:
+            gate_up = self.mlp.w12.forward_tiles(*q) if gate_tiles is not None else self.mlp.w12.forward_quantized(*q)
+            q = quest.silu_mul_hadamard_quantize_e2m3(gate_up) if on_tiles else quest.silu_mul_hadamard_quantize_int4(gate_up)
+        if on_tiles and gemm_adds:
             # the MLP's output projection adds into the residual stream as well: nothing is left for the caller to add
             self.mlp.c_proj.forward_tiles(*q, out=x2, add_to_out=True)
             return x, None
         down = self.mlp.c_proj
-        if (not down_tiles and gemm_adds and harness.GEMM_ADDS_RESIDUAL_PACKED and isinstance(down, harness.Linear4bit) and down.use_hadamard and down.bias is None
+        if (not on_tiles and gemm_adds and harness.GEMM_ADDS_RESIDUAL_PACKED and isinstance(down, harness.Linear4bit) and down.use_hadamard and down.bias is None
                 and not down.quantize_from_fp32 and quest.gemm_add_fuses(m, hidden, c, x.device)):
             down.forward_quantized(*q, out=x2, add_to_out=True)
             return x, None
-        y = self.mlp.c_proj.forward_tiles(*q) if down_tiles else self.mlp.c_proj.forward_quantized(*q)
+        y = self.mlp.c_proj.forward_tiles(*q) if on_tiles else self.mlp.c_proj.forward_quantized(*q)
         return x, y.view(b, t, c)
 
 
@@ -312,7 +341,8 @@ class LlamaBlock(nn.Module):
         if type(attn) is not LlamaAttention or type(mlp) is not LlamaMLP:
             return None
         linears = (attn.c_attn, attn.c_proj, mlp.w12, mlp.c_proj)
-        if not (mlp.glu is not None and attn.fused_rope and harness.GEMM_ADDS_RESIDUAL and harness.GEMM_ADDS_RESIDUAL_PACKED
+        glu = mlp.kept_glu()
+        if not (glu is not None and attn.fused_rope and harness.GEMM_ADDS_RESIDUAL and harness.GEMM_ADDS_RESIDUAL_PACKED
                 and harness.GEMM_ROTATES_QK and _as_built(attn.c_proj, harness.Linear4bit)):
             return None
         for part, methods in ((attn, ('attend', 'attention_core')), (mlp, ('swiglu_quantized', 'swiglu_tiles'))):
@@ -322,19 +352,27 @@ class LlamaBlock(nn.Module):
             if not (type(w) is harness.Linear4bit and w.bias is None and w.use_hadamard and not w.use_noop
                     and not w.quantize_from_fp32 and 'forward_quantized' not in w.__dict__ and 'forward_tiles' not in w.__dict__):
                 return None
-        tiles = (harness.prefers_e2m3(m, c, 3 * c) | harness.prefers_e2m3(m, c, c) << 1
-                 | harness.prefers_e2m3(m, c, 2 * hidden) << 2 | harness.prefers_e2m3(m, hidden, c) << 3)
-        if tiles & 4 and mlp.glu_tiles is None:
-            mlp.glu_tiles = harness.weight_tiles(mlp.glu[0])
+        qkv_tiles, o_tiles, gate_tiles, down_tiles = self._tiles_for(m, glu)
         qkv, o, both, down = (w._buffers.get for w in linears)
         return quest.host.block(
             x, branch, freqs_cis, attn.n_head, self.ln_1.weight, float(self.ln_1.eps), self.ln_2.weight, float(self.ln_2.eps),
-            (qkv('w_int_packed'), qkv('w_scale'), qkv('w_add'), attn.c_attn.w_tiles() if tiles & 1 else None),
-            (o('w_int_packed'), o('w_scale'), o('w_add'), attn.c_proj.w_tiles() if tiles & 2 else None),
+            (qkv('w_int_packed'), qkv('w_scale'), qkv('w_add'), qkv_tiles),
+            (o('w_int_packed'), o('w_scale'), o('w_add'), o_tiles),
             (both('w_int_packed'), both('w_scale'), both('w_add'), None),
-            (*mlp.glu, mlp.glu_tiles),
-            (down('w_int_packed'), down('w_scale'), down('w_add'), mlp.c_proj.w_tiles() if tiles & 8 else None),
-            tiles)
+            (*glu, gate_tiles),
+            (down('w_int_packed'), down('w_scale'), down('w_add'), down_tiles),
+            (qkv_tiles is not None) | (o_tiles is not None) << 1 | (gate_tiles is not None) << 2 | (down_tiles is not None) << 3)
+
+    def _tiles_for(self, m, glu):
+        """Of the four projections (qkv, output, gate / up, down) the weight tiles that m tokens are multiplied by, None for the packed
+        codes: the one decision of both statements of the block.  glu: `mlp.kept_glu()`."""
+        def of(w):
+            return w.tiles_for(m) if isinstance(w, harness.Linear4bit) else None
+        if glu is None:
+            gate = of(self.mlp.w12)
+        else:
+            gate = self.mlp.glu_tiles if harness.prefers_e2m3(m, glu[0].size(1) * 2, glu[0].size(0)) else None
+        return of(self.attn.c_attn), of(self.attn.c_proj), gate, of(self.mlp.c_proj)
 
 
 class Llama(nn.Module):
