@@ -187,7 +187,9 @@ hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ 
             if (packed != nullptr) packed[(size_t)row * nchunks + c] = w;
         }
     };
-    if (!FP32 && quant_fast_ok(s)) {            // uniform: everything but degenerate rows
+    // A NaN shows in the RMS scale but not in a maximum; the sum of squares has it either way.
+    const bool nan_row = absmax && __syncthreads_or(sumsq != sumsq);
+    if (!FP32 && quant_fast_ok(s) && !nan_row) {            // uniform: everything but degenerate rows
         const float inv28 = quant_inv28(s);
 #pragma unroll
         for (int i = 0; i < NCHUNK; i++) {

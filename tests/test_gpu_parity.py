@@ -654,3 +654,25 @@ def test_error_codes_no_launch(quest):
         quest.find_scale_int4(torch.zeros(2, 128, dtype=torch.bfloat16))       # CPU tensor: no fallback
     with pytest.raises(NotImplementedError):
         quest.matmul_int4sp_int4t_int32(None, None, None)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('k', [128, 1000, 4096])
+@pytest.mark.parametrize('from_fp32', [False, True])
+def test_absmax_rows_with_a_nan(quest, dtype, k, from_fp32):
+    """A maximum passes a NaN by, so its row keeps a finite scale: code -8 for the NaN, as the clamp gives, and for every other
+    element the code that the row has with 0 in its place."""
+    x = torch.randn(9, k, generator=torch.Generator().manual_seed(k)).to(dtype).to(DEV)
+    at = torch.tensor([0, 1, 7, 8, k // 2, k - 9, k - 8, k - 1], device=DEV)
+    r = torch.arange(8, device=DEV)
+    x[r, at] = 0
+    clean_scale, clean, clean_sum = quest.hadamard_quantize_int4(x, hadamard_scale=0., scale_rule='absmax', from_fp32=from_fp32)
+    x[r, at] = float('nan')
+    scale, packed, total = quest.hadamard_quantize_int4(x, hadamard_scale=0., scale_rule='absmax', from_fp32=from_fp32)
+    assert torch.equal(scale, clean_scale)
+    from quest_amd import harness
+    codes = harness.unpack_int4(clean)
+    codes[r, at] = -8
+    assert torch.equal(harness.unpack_int4(packed), codes)
+    assert torch.equal(total, codes.sum(-1, keepdim=True, dtype=torch.int32))
+    assert torch.equal(total[8], clean_sum[8])
