@@ -15,6 +15,7 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/scaled_dot_product_attention.h>
+#include <ATen/ops/silu.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -380,11 +381,15 @@ void project(const Linear &w, const Codes &q, at::Tensor &dst, int m, int dt, vo
     }
 }
 
+void quantise_into(const Codes &q, const at::Tensor &x, int m, int k, int dt, void *st) {
+    launched(q.tiles ? quest_hadamard_quantize_e2m3(x.data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, k, m, kHadamardEntry, dt, st)
+                     : quest_hadamard_quantize_int4(x.data_ptr(), q.scale, q.codes, q.row_sum, nullptr, k, m, kHadamardEntry, dt, st),
+             "activation kernel");
+}
+
 Codes quantised(const at::Tensor &x, int m, int k, bool tiles, c10::Device dev, int dt, void *st) {
     Codes q(m, k, tiles, dev);
-    launched(tiles ? quest_hadamard_quantize_e2m3(x.data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, k, m, kHadamardEntry, dt, st)
-                   : quest_hadamard_quantize_int4(x.data_ptr(), q.scale, q.codes, q.row_sum, nullptr, k, m, kHadamardEntry, dt, st),
-             "activation kernel");
+    quantise_into(q, x, m, k, dt, st);
     return q;
 }
 
@@ -471,24 +476,30 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     }
     // norm -> gated unit -> its codes
     const bool down_tiles = down.tiles != nullptr;
+    // Up to 64 tokens fp16 keeps torch's silu: the kernels' fast exponential gives torch's bits for every bf16 gate, but for two
+    // fp16 ones it does not.
+    const bool torch_silu = m <= 64 && type == at::kHalf;
     Codes act(m, hidden, down_tiles, args.dev);
     {
-        const Codes q = normed(x, has_att ? &att : nullptr, *norm2, eps2, m, c, glu.tiles != nullptr, args.dev, dt, st);
+        const Codes q = normed(x, has_att ? &att : nullptr, *norm2, eps2, m, c, glu.tiles != nullptr && !torch_silu, args.dev, dt, st);
         if (!q.tiles && m <= 64) {
             // the weight-streaming GEMM has no gated epilogue: gate and up side by side, the product inside the quantiser
             at::Tensor both = make({m, 2 * hidden}, type, args.dev);
             project(gate_up, q, both, m, dt, st);
-            launched(down_tiles ? quest_silu_mul_hadamard_quantize_e2m3(both.data_ptr(), act.scale, act.codes, nullptr, hidden, m, kHadamardEntry, dt, st)
-                                : quest_silu_mul_hadamard_quantize_int4(both.data_ptr(), act.scale, act.codes, act.row_sum, nullptr, nullptr, hidden, m, kHadamardEntry, dt, st),
-                     "gated unit");
+            if (torch_silu) {
+                const at::Tensor gated = at::silu(both.narrow(1, 0, hidden)).mul_(both.narrow(1, hidden, hidden)).contiguous();
+                quantise_into(act, gated, m, hidden, dt, st);
+            } else {
+                launched(down_tiles ? quest_silu_mul_hadamard_quantize_e2m3(both.data_ptr(), act.scale, act.codes, nullptr, hidden, m, kHadamardEntry, dt, st)
+                                    : quest_silu_mul_hadamard_quantize_int4(both.data_ptr(), act.scale, act.codes, act.row_sum, nullptr, nullptr, hidden, m, kHadamardEntry, dt, st),
+                         "gated unit");
+            }
         } else {
             at::Tensor gated = make({m, hidden}, type, args.dev);
             launched(q.tiles ? quest_fused_matmul_dequantize_swiglu_e2m3(gated.data_ptr(), q.codes, glu.tiles->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st)
                              : quest_fused_matmul_dequantize_swiglu_int4_int4t(gated.data_ptr(), q.codes, (const uint8_t *)glu.packed->data_ptr(), q.row_sum, (const int32_t *)glu.add->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st),
                      "gated projection");
-            launched(down_tiles ? quest_hadamard_quantize_e2m3(gated.data_ptr(), act.scale, act.codes, nullptr, nullptr, nullptr, hidden, m, kHadamardEntry, dt, st)
-                                : quest_hadamard_quantize_int4(gated.data_ptr(), act.scale, act.codes, act.row_sum, nullptr, hidden, m, kHadamardEntry, dt, st),
-                     "activation kernel");
+            quantise_into(act, gated, m, hidden, dt, st);
         }
     }
     if (down_tiles || quest_fused_matmul_dequantize_add_available(m, hidden, c, st)) {

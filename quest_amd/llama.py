@@ -372,6 +372,8 @@ class LlamaBlock(nn.Module):
             gate = of(self.mlp.w12)
         else:
             gate = self.mlp.glu_tiles if harness.prefers_e2m3(m, glu[0].size(1) * 2, glu[0].size(0)) else None
+            if m <= 64 and glu[1].dtype == torch.float16:       # torch's silu, which the kernels' is not for every fp16 value
+                gate = None
         return of(self.attn.c_attn), of(self.attn.c_proj), gate, of(self.mlp.c_proj)
 
 

@@ -62,3 +62,25 @@ def test_declined_calls_raise_as_before():
         quest.find_scale_int4(torch.zeros(4, 12, dtype=torch.bfloat16, device=DEV))       # rows that are not whole eights
     with pytest.raises(RuntimeError):
         quest.quantize_int4(x, torch.ones(4, 1, dtype=torch.bfloat16, device='cpu'))
+
+
+@pytest.mark.parametrize('native', [True, False])
+@pytest.mark.parametrize('dtype,tokens,calls', [(torch.float16, 8, 2), (torch.float16, 48, 2), (torch.float16, 64, 2), (torch.float16, 65, 0),
+                                                (torch.bfloat16, 200, 0)])
+def test_few_fp16_tokens_take_torchs_silu(python_path, native, dtype, tokens, calls):
+    """The kernels' gated unit rounds two of the fp16 gates another way than torch: up to 64 tokens it is torch's, in both
+    statements of the block, which then agree to the bit."""
+    from quest_amd import llama
+    torch.manual_seed(6)
+    with torch.device(DEV):
+        net = llama.Llama(llama.LlamaConfig(n_layer=2, n_embd=1024, n_head=8, vocab_size=256)).to(dtype).eval()
+        ids = torch.randint(0, 256, (1, tokens))
+    net = llama.quantize_model(net, 'int4', fuse_producers=True)
+    with torch.no_grad():
+        want = net(ids, all_logits=True)['logits']
+        if not native:
+            python_path()
+        with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+            got = net(ids, all_logits=True)['logits']
+    assert sum(e.count for e in prof.key_averages() if e.key == 'aten::silu') == calls
+    assert torch.equal(got, want)
