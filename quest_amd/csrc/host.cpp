@@ -5,9 +5,11 @@
 // conversions, device context, one allocation per output) took 36 us per call, so every small call ran at the speed of the
 // interpreter.  The same checks and launches from here take 6-8 us, most of it the two launches.
 //
-// Contract of every function: either the call is the plain case -- exact torch tensors on one GPU, contiguous, right types
-// and sizes, accepted by the library -- and everything is launched, or None comes back with nothing launched and the
-// caller's Python statement of the same call runs, which raises what there is to raise.  Nothing is cached between calls.
+// Contract of every function: either the call is the plain case -- exact torch tensors on one GPU, contiguous, right types, sizes
+// and alignment, accepted by the library -- and everything is launched, or None comes back with nothing launched and the
+// caller's Python statement of the same call runs, which raises what there is to raise.  (Should a launch itself fail, `block`
+// raises, for its stream has changed; the others come back with None, and the Python statement starts over and reports it.)
+// Nothing is cached between calls.
 #include <Python.h>
 
 #include <ATen/autocast_mode.h>
@@ -19,6 +21,8 @@
 #include <c10/core/DeviceGuard.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <algorithm>
 
 #include "../../include/quest_hip.h"
 
@@ -73,6 +77,15 @@ PyObject *ref(PyObject *o) {
     return o;
 }
 int64_t up(int64_t bytes) { return (bytes + 255) & ~(int64_t)255; }
+bool at(const at::Tensor *t, unsigned bytes) { return t == nullptr || (reinterpret_cast<uintptr_t>(t->data_ptr()) & (bytes - 1)) == 0; }
+
+// What the GEMMs ask of sizes (gemm_check in gemm.hip, e2m3_gemm_check in gemm_e2m3.hip), for calls that launch something before them.
+bool gemm_takes(int64_t m, int64_t k, int64_t n, bool tiles) {
+    if (tiles)
+        return k % 128 == 0 && k <= 65536 && quest_e2m3_tiles_bytes((int)std::min<int64_t>(m + 256, 0x7fffffff), (int)k) < (1ull << 31) &&
+               quest_e2m3_tiles_bytes((int)std::min<int64_t>(n + 256, 0x7fffffff), (int)k) < (1ull << 31);
+    return k % 32 == 0 && k < 131072 && m * (k / 2) < (1ll << 31) && n * (k / 2) < (1ll << 31);
+}
 
 // One activation's codes in a single scratch allocation: packed nibbles, row sums and scales, or E2M3 tiles and scales.
 struct Codes {
@@ -108,12 +121,12 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (!fits_int(m) || !fits_int(k) || !fits_int(n)) return declined();
     const at::Tensor *w_scale = args.tensor(a[2], type, n);
     const at::Tensor *w_add = args.tensor(a[3], at::kInt, n);
-    const bool tiles = a[4] != Py_None;
+    const bool tiles = a[4] != Py_None && args.ok && at(w_scale, 4);      // (the FP6 kernels read scales two at a time)
     const at::Tensor *w_tiles = tiles ? args.tensor(a[4], at::kByte, (int64_t)quest_e2m3_tiles_bytes((int)n, (int)k)) : nullptr;
     const at::Tensor *bias = a[5] == Py_None ? nullptr : args.tensor(a[5], type, n);
     const double had_scale = PyFloat_AsDouble(a[6]);
     const at::Tensor *given = a[7] == Py_None ? nullptr : args.matrix(a[7], type, m, n);
-    if (!args.ok) return declined();
+    if (!args.ok || !gemm_takes(m, k, n, tiles) || !at(x, 16) || !at(w, 16) || !at(w_tiles, 16) || !at(given, 16)) return declined();
     // (a bias whose derivative is wanted is added by torch)
     if (bias != nullptr && ((at::GradMode::is_enabled() && bias->requires_grad()) || bias->_fw_grad(0).defined())) return declined();
 
@@ -433,8 +446,14 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         return declined();
     const int hidden = down.k;
     if (qkv.k != c || qkv.n != 3 * c || o.k != c || o.n != c || gate_up.k != c || gate_up.n != 2 * hidden || glu.k != c || glu.n != 2 * hidden ||
-        down.n != c || (c & 127) != 0 || (hidden & 127) != 0 || c > 32768 || hidden > 32768 || (hidden & 3) != 0 || (head_dim & 7) != 0)
+        down.n != c || (c & 127) != 0 || (hidden & 127) != 0 || c > 32768 || hidden > 32768 || (head_dim & 7) != 0)
         return declined();
+    // the residual stream is updated on the way, so what the kernels ask is asked here
+    if (branch == xp || !at(xp, 16) || !at(branch, 16) || !at(freqs, 16) || !at(norm1, 16) || !at(norm2, 16)) return declined();
+    for (const Linear *w : {&qkv, &o, &gate_up, &glu, &down})
+        if (!gemm_takes(m, w->k, w->n, false) || (w->tiles != nullptr && !gemm_takes(m, w->k, w->n, true)) || !at(w->packed, 16) ||
+            !at(w->tiles, 16) || !at(w->scale, 4))
+            return declined();
 
     const c10::DeviceGuard guard(args.dev);
     void *st = stream_of(args.dev);
@@ -526,7 +545,8 @@ PyObject *last_logits(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const at::Tensor *branch = a[1] == Py_None ? nullptr : args.tensor(a[1], type, x->numel());
     const at::Tensor *norm_w = args.tensor(a[2], type, c), *head = args.tensor(a[4]);
     const double eps = PyFloat_AsDouble(a[3]);
-    if (!args.ok || head->scalar_type() != type || head->dim() != 2 || head->size(1) != c || b > 64 || (c & 63) != 0 || !fits_int(head->size(0)))
+    if (!args.ok || head->scalar_type() != type || head->dim() != 2 || head->size(1) != c || b > 64 || (c & 63) != 0 || !fits_int(c) ||
+        !fits_int(head->size(0)) || !at(x, 4) || !at(branch, 4) || !at(norm_w, 4) || !at(head, 16))
         return declined();
     const c10::DeviceGuard guard(args.dev);
     void *st = stream_of(args.dev);

@@ -43,13 +43,18 @@ def prefers_e2m3(m: int, k: int, n: int) -> bool:
     # INT8 / FP6 time: K = 1536 1.12 on average over N from 1500 to 22016, K = 1792 1.14, K = 1920 1.16, 0.98 at the least ((4097,
     # 1536, 1536) 33.7 / 27.4 us, (8192, 1536, 8192) 103 / 84, (16384, 1536, 3072) 85 / 70); K = 1024 0.85 to 1.18 ((16384, 1024, 8192) 148 / 173 us), K = 1152 to
     # 1408 0.94 to 1.27.  Layers of 1024 channels lose 6 to 12 % at 8192 tokens up to K = 1920 (half a 256 x 256 tile per CU).
-    return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and k <= 65536 and m * n <= (1 << 30)
+    return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and k <= 65536 and m * n <= (1 << 30) and m * k <= (5 << 29)
             and (m <= E2M3_SHORT_ROWS_TOKENS or k >= (E2M3_MIN_K if n >= E2M3_NARROW else E2M3_MIN_K_NARROW)))
 
 
 def e2m3_fits(k: int, rows: int) -> bool:
     """Whether codes of `rows` rows can be laid out as E2M3 tiles and multiplied by the FP6 kernels."""
     return k % 128 == 0 and 0 < k <= 65536 and rows <= 32 * 65535 and (rows + 287) // 32 * (k // 64) * 1536 < 1 << 31
+
+
+def _scales_in_pairs(scale) -> bool:
+    """Whether the FP6 kernels can read a scale vector: two 16-bit values at a time."""
+    return scale is None or scale.data_ptr() % 4 == 0
 
 
 def weight_tiles(w_int_packed: torch.Tensor) -> torch.Tensor:
@@ -172,7 +177,7 @@ def linear_forward(activation, w_int_packed, w_scale, w_add, w_meta_e=None, out=
             activation, _a_scale, _a_int_packed, _a_int_row_sum, hadamard_scale=WEIGHT_HADAMARD_SCALE, from_fp32=True)
         return quest.fused_matmul_dequantize_int4_int4t_bf16(mat_a=a_int_packed, mat_b=w_int_packed, vec_a_add=a_int_row_sum,
                                                              vec_b_add=w_add, vec_a_mul=a_scale, vec_b_mul=w_scale, out=out)
-    if w_tiles is not None:
+    if w_tiles is not None and _scales_in_pairs(w_scale) and _scales_in_pairs(_a_scale):
         a_scale, a_tiles = quest.hadamard_quantize_e2m3(activation, _a_scale, _a_tiles,
                                                         hadamard_scale=HADAMARD_ENTRY if use_hadamard else 0.)
         return quest.fused_matmul_dequantize_e2m3(a_tiles, w_tiles, a_scale, w_scale, k, out)
@@ -256,7 +261,7 @@ class Linear4bit(nn.Module):
     def tiles_for(self, m: int):
         """The weight's E2M3 tiles where the FP6 kernels are the faster ones for m tokens, None where the packed codes serve."""
         n, k = self.weight.shape
-        return self._kept_tiles() if prefers_e2m3(m, k, n) else None
+        return self._kept_tiles() if prefers_e2m3(m, k, n) and _scales_in_pairs(self.w_scale) else None
 
     def w_tiles(self) -> torch.Tensor:
         """The weight codes as E2M3 tiles: the kept ones, or a conversion of the buffer for this call."""

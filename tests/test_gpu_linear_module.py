@@ -45,3 +45,36 @@ def test_sparse_metadata_is_refused_and_other_holders_of_the_buffers_work():
     del layer.w_int_packed
     layer.w_int_packed = torch.nn.Parameter(packed, requires_grad=False)
     assert torch.equal(layer(x), want)
+
+
+@pytest.mark.parametrize('m', [3, 40, 96, 200, 1000])
+@pytest.mark.parametrize('direct', [False, True])
+def test_scales_at_an_odd_element(m, direct):
+    """A slice of a longer scale vector: only some kernels read it, and a layer finds them at every size."""
+    from quest_amd import harness
+    layer, x = layer_and_input(m, 2048, 1024, bias=False)
+    want = layer(x)
+    layer.w_scale = torch.cat([layer.w_scale[:1], layer.w_scale])[1:]
+    assert layer.w_scale.data_ptr() % 4 == 2 and layer.tiles_for(m) is None
+    if direct:
+        got = harness.linear_forward(x, layer.w_int_packed, layer.w_scale, layer.w_add, use_hadamard=True, w_tiles=layer.w_tiles())
+    else:
+        got = layer(x)
+    assert torch.equal(got, want)
+    odd = torch.empty(m + 1, 1, dtype=x.dtype, device=DEV)[1:]
+    got = harness.linear_forward(x, layer.w_int_packed, layer.w_scale, layer.w_add, use_hadamard=True, w_tiles=layer.w_tiles(), _a_scale=odd)
+    assert torch.equal(got, want)
+
+
+def test_more_rows_than_tiles_can_hold():
+    """2^21 + 32 channels: no tiles are laid out, and the packed codes serve."""
+    from quest_amd import harness
+    n, k, m = 2 ** 21 + 32, 512, 70
+    g = torch.Generator(device=DEV).manual_seed(5)
+    layer = harness.Linear4bit.empty(k, n, device=DEV, dtype=torch.bfloat16, use_hadamard=True)
+    layer.w_int_packed.random_(0, 256, generator=g)
+    layer.w_scale.fill_(0.01)
+    layer.lay_out_tiles()
+    x = torch.randn(m, k, device=DEV, generator=g).bfloat16()
+    y = layer(x)
+    assert torch.equal(y[:, -40:], harness.linear_forward(x, layer.w_int_packed[-40:], layer.w_scale[-40:], layer.w_add[-40:], use_hadamard=True))

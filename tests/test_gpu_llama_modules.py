@@ -114,3 +114,20 @@ def test_fused_block_under_autocast(seq):
             assert (got.double() - want.double()).norm() <= 2. ** -7 * want.double().norm()
         with torch.autocast('cuda', dtype=torch.float16), pytest.raises(AssertionError):
             model(ids)
+
+
+@pytest.mark.parametrize('batch,seq', [(1, 8), (1, 40), (2, 100), (9, 512)])
+@pytest.mark.parametrize('which', ['c_attn', 'c_proj', 'w12', 'down'])
+def test_fused_block_with_scales_at_an_odd_element(batch, seq, which):
+    """What one projection's kernels cannot read, others can: the same logits, and no half-updated stream."""
+    from quest_amd import llama
+    torch.manual_seed(27)
+    cfg = llama.LlamaConfig(n_layer=2, n_embd=1024, n_head=8, vocab_size=64)
+    model = llama.quantize_model(llama.Llama(cfg).to(torch.bfloat16).to(DEV).eval(), 'int4', fuse_producers=True)
+    ids = torch.randint(0, 64, (batch, seq), generator=torch.Generator().manual_seed(28)).to(DEV)
+    with torch.no_grad():
+        want = model(ids)['logits']
+        for block in model.transformer.h:
+            w = {'c_attn': block.attn.c_attn, 'c_proj': block.attn.c_proj, 'w12': block.mlp.w12, 'down': block.mlp.c_proj}[which]
+            w.w_scale = torch.cat([w.w_scale[:1], w.w_scale])[1:]
+        assert torch.equal(model(ids)['logits'], want)
