@@ -322,10 +322,12 @@ PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const at::Tensor *packed = a[3] == Py_None ? nullptr : args.matrix(a[3], at::kByte, m, k / 2);
     const at::Tensor *row_sum = a[4] == Py_None ? nullptr : args.tensor(a[4], at::kInt, m);
     if (!args.ok || !fits_int(m) || !fits_int(k)) return declined();
+    const int dequantize = PyObject_IsTrue(a[5]);
+    if (dequantize < 0) return nullptr;
     const c10::DeviceGuard guard(args.dev);
     const int rc = quest_quantize_int4(x->data_ptr(), scale->data_ptr(), x_int ? (int8_t *)x_int->data_ptr() : nullptr,
                                        packed ? (uint8_t *)packed->data_ptr() : nullptr, row_sum ? (int32_t *)row_sum->data_ptr() : nullptr,
-                                       (int)k, (int)m, PyObject_IsTrue(a[5]) == 1, dtype_code(x->scalar_type()), stream_of(args.dev));
+                                       (int)k, (int)m, dequantize, dtype_code(x->scalar_type()), stream_of(args.dev));
     if (rc != QUEST_OK) return declined();
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
@@ -434,6 +436,7 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const int m = (int)(b * t), c = (int)c64;
     const at::Tensor *branch = a[1] == Py_None ? nullptr : args.tensor(a[1], type, xp->numel());
     const long n_head = PyLong_AsLong(a[3]);
+    if (n_head == -1 && PyErr_Occurred()) return nullptr;
     if (n_head <= 0 || c % n_head != 0) return declined();
     const int head_dim = (int)(c / n_head);
     const at::Tensor *freqs = args.tensor(a[2], at::kFloat, t * (head_dim / 2) * 2);

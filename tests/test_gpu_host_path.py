@@ -84,3 +84,12 @@ def test_few_fp16_tokens_take_torchs_silu(python_path, native, dtype, tokens, ca
             got = net(ids, all_logits=True)['logits']
     assert sum(e.count for e in prof.key_averages() if e.key == 'aten::silu') == calls
     assert torch.equal(got, want)
+
+
+def test_an_option_without_a_truth_value_raises_its_own_error():
+    import quest_amd as quest
+    x = torch.randn(4, 256, device=DEV).bfloat16()
+    before = x.clone()
+    with pytest.raises(RuntimeError, match='Boolean value of Tensor'):
+        quest.quantize_int4(x, torch.ones(4, 1, dtype=torch.bfloat16, device=DEV), do_dequantize=torch.ones(2))
+    assert torch.equal(x, before)
