@@ -76,6 +76,19 @@ PyObject *ref(PyObject *o) {
     Py_INCREF(o);
     return o;
 }
+// Allocations and launches run without the interpreter lock, as calls through ctypes do: a launch can wait for room in its queue.
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    Unlocked() = default;
+    Unlocked(const Unlocked &) = delete;
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+template <typename F>
+int on(c10::Device dev, F &&launch) {
+    const Unlocked unlocked;
+    const c10::DeviceGuard guard(dev);
+    return launch(stream_of(dev));
+}
 int64_t up(int64_t bytes) { return (bytes + 255) & ~(int64_t)255; }
 bool at(const at::Tensor *t, unsigned bytes) { return t == nullptr || (reinterpret_cast<uintptr_t>(t->data_ptr()) & (bytes - 1)) == 0; }
 
@@ -130,35 +143,36 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     // (a bias whose derivative is wanted is added by torch)
     if (bias != nullptr && ((at::GradMode::is_enabled() && bias->requires_grad()) || bias->_fw_grad(0).defined())) return declined();
 
-    const c10::DeviceGuard guard(args.dev);
-    void *st = stream_of(args.dev);
-    const int dt = dtype_code(type);
-    Codes q(m, k, tiles, args.dev);
-    int rc = tiles ? quest_hadamard_quantize_e2m3(x->data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, (int)k, (int)m, (float)had_scale, dt, st)
-                   : quest_hadamard_quantize_int4(x->data_ptr(), q.scale, q.codes, q.row_sum, nullptr, (int)k, (int)m, (float)had_scale, dt, st);
-    if (rc != QUEST_OK) return declined();
     at::Tensor out;
-    if (given != nullptr) {
-        out = *given;
-    } else {
-        c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
-        shape.back() = n;
-        out = make(shape, type, args.dev);
-    }
-    bool add_bias = bias != nullptr;
-    if (add_bias) {                                              // in the GEMM's epilogue where the kernel can
-        rc = tiles ? quest_fused_matmul_dequantize_bias_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)k, (int)n, dt, st)
-                   : quest_fused_matmul_dequantize_bias_int4_int4t(out.data_ptr(), q.codes, (const uint8_t *)w->data_ptr(), q.row_sum, (const int32_t *)w_add->data_ptr(),
-                                                                   q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)k, (int)n, dt, st);
-        add_bias = rc != QUEST_OK;
-    }
-    if (add_bias || bias == nullptr) {
-        rc = tiles ? quest_fused_matmul_dequantize_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), (int)m, (int)k, (int)n, dt, st)
-                   : quest_fused_matmul_dequantize_int4_int4t(out.data_ptr(), q.codes, (const uint8_t *)w->data_ptr(), q.row_sum,
-                                                              (const int32_t *)w_add->data_ptr(), q.scale, w_scale->data_ptr(), (int)m, (int)k, (int)n, dt, st);
-        if (rc != QUEST_OK) return declined();
-        if (add_bias) out.add_(*bias);
-    }
+    const int rc = on(args.dev, [&](void *st) {
+        const int dt = dtype_code(type);
+        Codes q(m, k, tiles, args.dev);
+        int rc = tiles ? quest_hadamard_quantize_e2m3(x->data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, (int)k, (int)m, (float)had_scale, dt, st)
+                   : quest_hadamard_quantize_int4(x->data_ptr(), q.scale, q.codes, q.row_sum, nullptr, (int)k, (int)m, (float)had_scale, dt, st);
+        if (rc != QUEST_OK) return rc;
+        if (given != nullptr) {
+            out = *given;
+        } else {
+            c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
+            shape.back() = n;
+            out = make(shape, type, args.dev);
+        }
+        bool add_bias = bias != nullptr;
+        if (add_bias) {                                      // in the GEMM's epilogue where the kernel can
+            rc = tiles ? quest_fused_matmul_dequantize_bias_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)k, (int)n, dt, st)
+                       : quest_fused_matmul_dequantize_bias_int4_int4t(out.data_ptr(), q.codes, (const uint8_t *)w->data_ptr(), q.row_sum, (const int32_t *)w_add->data_ptr(),
+                                                                       q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)k, (int)n, dt, st);
+            add_bias = rc != QUEST_OK;
+        }
+        if (add_bias || bias == nullptr) {
+            rc = tiles ? quest_fused_matmul_dequantize_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), (int)m, (int)k, (int)n, dt, st)
+                       : quest_fused_matmul_dequantize_int4_int4t(out.data_ptr(), q.codes, (const uint8_t *)w->data_ptr(), q.row_sum,
+                                                                  (const int32_t *)w_add->data_ptr(), q.scale, w_scale->data_ptr(), (int)m, (int)k, (int)n, dt, st);
+            if (rc == QUEST_OK && add_bias) out.add_(*bias);
+        }
+        return rc;
+    });
+    if (rc != QUEST_OK) return declined();
     return given != nullptr ? ref(a[7]) : wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
@@ -181,11 +195,13 @@ PyObject *gemm(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const at::Tensor *b_mul = args.tensor(a[5], type, n);
     const at::Tensor *given = a[6] == Py_None ? nullptr : args.matrix(a[6], type, m, n);
     if (!args.ok) return declined();
-    const c10::DeviceGuard guard(args.dev);
-    at::Tensor out = given != nullptr ? *given : make({m, n}, type, args.dev);
-    const int rc = quest_fused_matmul_dequantize_int4_int4t(out.data_ptr(), (const uint8_t *)x->data_ptr(), (const uint8_t *)w->data_ptr(),
-                                                            (const int32_t *)a_add->data_ptr(), (const int32_t *)b_add->data_ptr(),
-                                                            a_mul->data_ptr(), b_mul->data_ptr(), (int)m, (int)k, (int)n, dtype_code(type), stream_of(args.dev));
+    at::Tensor out;
+    const int rc = on(args.dev, [&](void *st) {
+        out = given != nullptr ? *given : make({m, n}, type, args.dev);
+        return quest_fused_matmul_dequantize_int4_int4t(out.data_ptr(), (const uint8_t *)x->data_ptr(), (const uint8_t *)w->data_ptr(),
+                                                        (const int32_t *)a_add->data_ptr(), (const int32_t *)b_add->data_ptr(), a_mul->data_ptr(),
+                                                        b_mul->data_ptr(), (int)m, (int)k, (int)n, dtype_code(type), st);
+    });
     if (rc != QUEST_OK) return declined();
     return given != nullptr ? ref(a[6]) : wrap(std::move(out));
     END_HANDLE_TH_ERRORS
@@ -204,10 +220,12 @@ PyObject *matmul_int32(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (!fits_int(m) || !fits_int(k) || !fits_int(n)) return declined();
     const at::Tensor *given = a[2] == Py_None ? nullptr : args.matrix(a[2], at::kInt, m, n);
     if (!args.ok) return declined();
-    const c10::DeviceGuard guard(args.dev);
-    at::Tensor out = given != nullptr ? *given : make({m, n}, at::kInt, args.dev);
-    const int rc = quest_matmul_int4_int4t_int32((int32_t *)out.data_ptr(), (const uint8_t *)x->data_ptr(), (const uint8_t *)w->data_ptr(),
-                                                 (int)m, (int)k, (int)n, stream_of(args.dev));
+    at::Tensor out;
+    const int rc = on(args.dev, [&](void *st) {
+        out = given != nullptr ? *given : make({m, n}, at::kInt, args.dev);
+        return quest_matmul_int4_int4t_int32((int32_t *)out.data_ptr(), (const uint8_t *)x->data_ptr(), (const uint8_t *)w->data_ptr(), (int)m,
+                                             (int)k, (int)n, st);
+    });
     if (rc != QUEST_OK) return declined();
     return given != nullptr ? ref(a[2]) : wrap(std::move(out));
     END_HANDLE_TH_ERRORS
@@ -231,12 +249,13 @@ PyObject *hadamard_quantize(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const double had_scale = PyFloat_AsDouble(a[4]);
     const long rule = PyLong_AsLong(a[5]);
     if (!args.ok) return declined();
-    const c10::DeviceGuard guard(args.dev);
-    if (!scale.defined()) scale = make({m, 1}, type, args.dev);
-    if (!packed.defined()) packed = make({m, k / 2}, at::kByte, args.dev);
-    if (!row_sum.defined()) row_sum = make({m, 1}, at::kInt, args.dev);
-    const int rc = quest_hadamard_quantize_int4_rule(x->data_ptr(), scale.data_ptr(), (uint8_t *)packed.data_ptr(), (int32_t *)row_sum.data_ptr(),
-                                                     nullptr, (int)k, (int)m, (float)had_scale, (int)rule, dtype_code(type), stream_of(args.dev));
+    const int rc = on(args.dev, [&](void *st) {
+        if (!scale.defined()) scale = make({m, 1}, type, args.dev);
+        if (!packed.defined()) packed = make({m, k / 2}, at::kByte, args.dev);
+        if (!row_sum.defined()) row_sum = make({m, 1}, at::kInt, args.dev);
+        return quest_hadamard_quantize_int4_rule(x->data_ptr(), scale.data_ptr(), (uint8_t *)packed.data_ptr(), (int32_t *)row_sum.data_ptr(),
+                                                 nullptr, (int)k, (int)m, (float)had_scale, (int)rule, dtype_code(type), st);
+    });
     if (rc != QUEST_OK) return declined();
     PyObject *t = PyTuple_New(3);
     if (t == nullptr) return nullptr;
@@ -257,10 +276,14 @@ PyObject *pack_weight(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const at::ScalarType type = w->scalar_type();
     const int64_t n = w->size(0), k = w->size(1);
     if (!fits_int(n) || !fits_int(k)) return declined();
-    const c10::DeviceGuard guard(args.dev);
-    at::Tensor packed = make({n, k / 2}, at::kByte, args.dev), scale = make({n, 1}, type, args.dev), add = make({n, 1}, at::kInt, args.dev);
-    const int rc = quest_pack_weight_int4(w->data_ptr(), scale.data_ptr(), (uint8_t *)packed.data_ptr(), (int32_t *)add.data_ptr(), (int)k, (int)n,
-                                          (float)PyFloat_AsDouble(a[1]), (int)PyLong_AsLong(a[2]), dtype_code(type), stream_of(args.dev));
+    const float had_scale = (float)PyFloat_AsDouble(a[1]);
+    const int rule = (int)PyLong_AsLong(a[2]);
+    at::Tensor packed, scale, add;
+    const int rc = on(args.dev, [&](void *st) {
+        packed = make({n, k / 2}, at::kByte, args.dev), scale = make({n, 1}, type, args.dev), add = make({n, 1}, at::kInt, args.dev);
+        return quest_pack_weight_int4(w->data_ptr(), scale.data_ptr(), (uint8_t *)packed.data_ptr(), (int32_t *)add.data_ptr(), (int)k, (int)n,
+                                      had_scale, rule, dtype_code(type), st);
+    });
     if (rc != QUEST_OK) return declined();
     PyObject *t = PyTuple_New(3);
     if (t == nullptr) return nullptr;
@@ -282,9 +305,11 @@ PyObject *hadamard128(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     at::Tensor out;
     if (a[1] != Py_None) out = *args.tensor(a[1], x->scalar_type(), x->numel());
     if (!args.ok || (out.defined() && out.sizes() != x->sizes()) || !fits_int(k) || !fits_int(rows)) return declined();
-    const c10::DeviceGuard guard(args.dev);
-    if (!out.defined()) out = make(x->sizes(), x->scalar_type(), args.dev);
-    const int rc = quest_hadamard128(out.data_ptr(), x->data_ptr(), (int)k, (int)rows, (float)PyFloat_AsDouble(a[2]), dtype_code(x->scalar_type()), stream_of(args.dev));
+    const float had_scale = (float)PyFloat_AsDouble(a[2]);
+    const int rc = on(args.dev, [&](void *st) {
+        if (!out.defined()) out = make(x->sizes(), x->scalar_type(), args.dev);
+        return quest_hadamard128(out.data_ptr(), x->data_ptr(), (int)k, (int)rows, had_scale, dtype_code(x->scalar_type()), st);
+    });
     if (rc != QUEST_OK) return declined();
     return a[1] != Py_None ? ref(a[1]) : wrap(std::move(out));
     END_HANDLE_TH_ERRORS
@@ -301,9 +326,10 @@ PyObject *find_scale(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     at::Tensor scale;
     if (a[1] != Py_None) scale = *args.tensor(a[1], x->scalar_type(), m);
     if (!args.ok || !fits_int(m) || !fits_int(k)) return declined();
-    const c10::DeviceGuard guard(args.dev);
-    if (!scale.defined()) scale = make({m, 1}, x->scalar_type(), args.dev);
-    const int rc = quest_find_scale_int4(scale.data_ptr(), x->data_ptr(), (int)k, (int)m, dtype_code(x->scalar_type()), stream_of(args.dev));
+    const int rc = on(args.dev, [&](void *st) {
+        if (!scale.defined()) scale = make({m, 1}, x->scalar_type(), args.dev);
+        return quest_find_scale_int4(scale.data_ptr(), x->data_ptr(), (int)k, (int)m, dtype_code(x->scalar_type()), st);
+    });
     if (rc != QUEST_OK) return declined();
     return a[1] != Py_None ? ref(a[1]) : wrap(std::move(scale));
     END_HANDLE_TH_ERRORS
@@ -324,10 +350,11 @@ PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (!args.ok || !fits_int(m) || !fits_int(k)) return declined();
     const int dequantize = PyObject_IsTrue(a[5]);
     if (dequantize < 0) return nullptr;
-    const c10::DeviceGuard guard(args.dev);
-    const int rc = quest_quantize_int4(x->data_ptr(), scale->data_ptr(), x_int ? (int8_t *)x_int->data_ptr() : nullptr,
-                                       packed ? (uint8_t *)packed->data_ptr() : nullptr, row_sum ? (int32_t *)row_sum->data_ptr() : nullptr,
-                                       (int)k, (int)m, dequantize, dtype_code(x->scalar_type()), stream_of(args.dev));
+    const int rc = on(args.dev, [&](void *st) {
+        return quest_quantize_int4(x->data_ptr(), scale->data_ptr(), x_int ? (int8_t *)x_int->data_ptr() : nullptr,
+                                   packed ? (uint8_t *)packed->data_ptr() : nullptr, row_sum ? (int32_t *)row_sum->data_ptr() : nullptr, (int)k,
+                                   (int)m, dequantize, dtype_code(x->scalar_type()), st);
+    });
     if (rc != QUEST_OK) return declined();
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
@@ -347,10 +374,12 @@ PyObject *add_mul_vv(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const at::Tensor *a_add = args.tensor(a[0], at::kInt, m), *b_add = args.tensor(a[2], at::kInt, n), *b_mul = args.tensor(a[3], type, n);
     const at::Tensor *given = a[5] == Py_None ? nullptr : args.matrix(a[5], type, m, n);
     if (!args.ok || !fits_int(m) || !fits_int(n)) return declined();
-    const c10::DeviceGuard guard(args.dev);
-    at::Tensor out = given != nullptr ? *given : make({m, n}, type, args.dev);
-    const int rc = quest_add_mul_vv(out.data_ptr(), (const int32_t *)a_add->data_ptr(), a_mul->data_ptr(), (const int32_t *)b_add->data_ptr(),
-                                    b_mul->data_ptr(), (const int32_t *)c->data_ptr(), (int)m, (int)n, dtype_code(type), stream_of(args.dev));
+    at::Tensor out;
+    const int rc = on(args.dev, [&](void *st) {
+        out = given != nullptr ? *given : make({m, n}, type, args.dev);
+        return quest_add_mul_vv(out.data_ptr(), (const int32_t *)a_add->data_ptr(), a_mul->data_ptr(), (const int32_t *)b_add->data_ptr(),
+                                b_mul->data_ptr(), (const int32_t *)c->data_ptr(), (int)m, (int)n, dtype_code(type), st);
+    });
     if (rc != QUEST_OK) return declined();
     return given != nullptr ? ref(a[5]) : wrap(std::move(out));
     END_HANDLE_TH_ERRORS
@@ -458,78 +487,80 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             !at(w->tiles, 16) || !at(w->scale, 4))
             return declined();
 
-    const c10::DeviceGuard guard(args.dev);
-    void *st = stream_of(args.dev);
-    const int dt = dtype_code(type);
-    at::Tensor x = *xp;
+    at::Tensor x = *xp, mlp;                                     // mlp: what is left to be added to x, if anything
+    on(args.dev, [&](void *st) {
+        const int dt = dtype_code(type);
 
-    // norm -> q, k, v with q and k rotated
-    at::Tensor heads = make({m, 3 * c}, type, args.dev);
-    {
-        const Codes q = normed(x, branch, *norm1, eps1, m, c, qkv.tiles != nullptr, args.dev, dt, st);
-        const float *f = (const float *)freqs->data_ptr();
-        int rc = q.tiles ? (t >= 32 && head_dim % 32 == 0
-                                ? quest_fused_matmul_dequantize_rope_e2m3(heads.data_ptr(), q.codes, qkv.tiles->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st)
-                                : QUEST_ERR_UNSUPPORTED)
-                         : quest_fused_matmul_dequantize_rope_int4_int4t(heads.data_ptr(), q.codes, (const uint8_t *)qkv.packed->data_ptr(), q.row_sum, (const int32_t *)qkv.add->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st);
-        if (rc == QUEST_ERR_UNSUPPORTED || rc == QUEST_ERR_BAD_SHAPE) {        // nothing was launched: the two calls
-            project(qkv, q, heads, m, dt, st);
-            rc = quest_rope_interleaved(heads.data_ptr(), f, m, (int)t, 3 * c, 2 * c, head_dim, dt, st);
-        }
-        launched(rc, "QKV projection");
-    }
-    // causal attention
-    const int64_t row = 3 * c64;
-    const auto part = [&](int64_t i) { return heads.as_strided({b, n_head, t, head_dim}, {t * row, head_dim, row, 1}, i * c64); };
-    const at::Tensor y = at::scaled_dot_product_attention(part(0), part(1), part(2), {}, 0.0, true);
-    const at::Tensor core = y.transpose(1, 2).contiguous();
-    // output projection: into the residual stream where its GEMM can add
-    bool has_att = false;
-    at::Tensor att;
-    {
-        const Codes q = quantised(core, m, c, o.tiles != nullptr, args.dev, dt, st);
-        if (q.tiles || quest_fused_matmul_dequantize_add_available(m, c, c, st)) {
-            project(o, q, x, m, dt, st, true);
-        } else {
-            has_att = true;
-            att = make({m, c}, type, args.dev);
-            project(o, q, att, m, dt, st);
-        }
-    }
-    // norm -> gated unit -> its codes
-    const bool down_tiles = down.tiles != nullptr;
-    // Up to 64 tokens fp16 keeps torch's silu: the kernels' fast exponential gives torch's bits for every bf16 gate, but for two
-    // fp16 ones it does not.
-    const bool torch_silu = m <= 64 && type == at::kHalf;
-    Codes act(m, hidden, down_tiles, args.dev);
-    {
-        const Codes q = normed(x, has_att ? &att : nullptr, *norm2, eps2, m, c, glu.tiles != nullptr && !torch_silu, args.dev, dt, st);
-        if (!q.tiles && m <= 64) {
-            // the weight-streaming GEMM has no gated epilogue: gate and up side by side, the product inside the quantiser
-            at::Tensor both = make({m, 2 * hidden}, type, args.dev);
-            project(gate_up, q, both, m, dt, st);
-            if (torch_silu) {
-                const at::Tensor gated = at::silu(both.narrow(1, 0, hidden)).mul_(both.narrow(1, hidden, hidden)).contiguous();
-                quantise_into(act, gated, m, hidden, dt, st);
-            } else {
-                launched(down_tiles ? quest_silu_mul_hadamard_quantize_e2m3(both.data_ptr(), act.scale, act.codes, nullptr, hidden, m, kHadamardEntry, dt, st)
-                                    : quest_silu_mul_hadamard_quantize_int4(both.data_ptr(), act.scale, act.codes, act.row_sum, nullptr, nullptr, hidden, m, kHadamardEntry, dt, st),
-                         "gated unit");
+        // norm -> q, k, v with q and k rotated
+        at::Tensor heads = make({m, 3 * c}, type, args.dev);
+        {
+            const Codes q = normed(x, branch, *norm1, eps1, m, c, qkv.tiles != nullptr, args.dev, dt, st);
+            const float *f = (const float *)freqs->data_ptr();
+            int rc = q.tiles ? (t >= 32 && head_dim % 32 == 0
+                                    ? quest_fused_matmul_dequantize_rope_e2m3(heads.data_ptr(), q.codes, qkv.tiles->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st)
+                                    : QUEST_ERR_UNSUPPORTED)
+                             : quest_fused_matmul_dequantize_rope_int4_int4t(heads.data_ptr(), q.codes, (const uint8_t *)qkv.packed->data_ptr(), q.row_sum, (const int32_t *)qkv.add->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st);
+            if (rc == QUEST_ERR_UNSUPPORTED || rc == QUEST_ERR_BAD_SHAPE) {        // nothing was launched: the two calls
+                project(qkv, q, heads, m, dt, st);
+                rc = quest_rope_interleaved(heads.data_ptr(), f, m, (int)t, 3 * c, 2 * c, head_dim, dt, st);
             }
-        } else {
-            at::Tensor gated = make({m, hidden}, type, args.dev);
-            launched(q.tiles ? quest_fused_matmul_dequantize_swiglu_e2m3(gated.data_ptr(), q.codes, glu.tiles->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st)
-                             : quest_fused_matmul_dequantize_swiglu_int4_int4t(gated.data_ptr(), q.codes, (const uint8_t *)glu.packed->data_ptr(), q.row_sum, (const int32_t *)glu.add->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st),
-                     "gated projection");
-            quantise_into(act, gated, m, hidden, dt, st);
+            launched(rc, "QKV projection");
         }
-    }
-    if (down_tiles || quest_fused_matmul_dequantize_add_available(m, hidden, c, st)) {
-        project(down, act, x, m, dt, st, true);
-        Py_RETURN_TRUE;
-    }
-    at::Tensor mlp = make({b, t, c64}, type, args.dev);
-    project(down, act, mlp, m, dt, st);
+        // causal attention
+        const int64_t row = 3 * c64;
+        const auto part = [&](int64_t i) { return heads.as_strided({b, n_head, t, head_dim}, {t * row, head_dim, row, 1}, i * c64); };
+        const at::Tensor y = at::scaled_dot_product_attention(part(0), part(1), part(2), {}, 0.0, true);
+        const at::Tensor core = y.transpose(1, 2).contiguous();
+        // output projection: into the residual stream where its GEMM can add
+        bool has_att = false;
+        at::Tensor att;
+        {
+            const Codes q = quantised(core, m, c, o.tiles != nullptr, args.dev, dt, st);
+            if (q.tiles || quest_fused_matmul_dequantize_add_available(m, c, c, st)) {
+                project(o, q, x, m, dt, st, true);
+            } else {
+                has_att = true;
+                att = make({m, c}, type, args.dev);
+                project(o, q, att, m, dt, st);
+            }
+        }
+        // norm -> gated unit -> its codes
+        const bool down_tiles = down.tiles != nullptr;
+        // Up to 64 tokens fp16 keeps torch's silu: the kernels' fast exponential gives torch's bits for every bf16 gate, but for two
+        // fp16 ones it does not.
+        const bool torch_silu = m <= 64 && type == at::kHalf;
+        Codes act(m, hidden, down_tiles, args.dev);
+        {
+            const Codes q = normed(x, has_att ? &att : nullptr, *norm2, eps2, m, c, glu.tiles != nullptr && !torch_silu, args.dev, dt, st);
+            if (!q.tiles && m <= 64) {
+                // the weight-streaming GEMM has no gated epilogue: gate and up side by side, the product inside the quantiser
+                at::Tensor both = make({m, 2 * hidden}, type, args.dev);
+                project(gate_up, q, both, m, dt, st);
+                if (torch_silu) {
+                    const at::Tensor gated = at::silu(both.narrow(1, 0, hidden)).mul_(both.narrow(1, hidden, hidden)).contiguous();
+                    quantise_into(act, gated, m, hidden, dt, st);
+                } else {
+                    launched(down_tiles ? quest_silu_mul_hadamard_quantize_e2m3(both.data_ptr(), act.scale, act.codes, nullptr, hidden, m, kHadamardEntry, dt, st)
+                                        : quest_silu_mul_hadamard_quantize_int4(both.data_ptr(), act.scale, act.codes, act.row_sum, nullptr, nullptr, hidden, m, kHadamardEntry, dt, st),
+                             "gated unit");
+                }
+            } else {
+                at::Tensor gated = make({m, hidden}, type, args.dev);
+                launched(q.tiles ? quest_fused_matmul_dequantize_swiglu_e2m3(gated.data_ptr(), q.codes, glu.tiles->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st)
+                                 : quest_fused_matmul_dequantize_swiglu_int4_int4t(gated.data_ptr(), q.codes, (const uint8_t *)glu.packed->data_ptr(), q.row_sum, (const int32_t *)glu.add->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st),
+                         "gated projection");
+                quantise_into(act, gated, m, hidden, dt, st);
+            }
+        }
+        if (down_tiles || quest_fused_matmul_dequantize_add_available(m, hidden, c, st)) {
+            project(down, act, x, m, dt, st, true);
+        } else {
+            mlp = make({b, t, c64}, type, args.dev);
+            project(down, act, mlp, m, dt, st);
+        }
+        return 0;
+    });
+    if (!mlp.defined()) Py_RETURN_TRUE;
     return wrap(std::move(mlp));
     END_HANDLE_TH_ERRORS
 }
@@ -551,13 +582,16 @@ PyObject *last_logits(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (!args.ok || head->scalar_type() != type || head->dim() != 2 || head->size(1) != c || b > 64 || (c & 63) != 0 || !fits_int(c) ||
         !fits_int(head->size(0)) || !at(x, 4) || !at(branch, 4) || !at(norm_w, 4) || !at(head, 16))
         return declined();
-    const c10::DeviceGuard guard(args.dev);
-    void *st = stream_of(args.dev);
     const int64_t v = head->size(0), last = (t - 1) * c * 2;
-    at::Tensor normed = make({b, c}, type, args.dev), logits = make({b, 1, v}, type, args.dev);
-    int rc = quest_rmsnorm_rows(normed.data_ptr(), (const uint8_t *)x->data_ptr() + last, branch ? (const uint8_t *)branch->data_ptr() + last : nullptr,
-                                norm_w->data_ptr(), (float)eps, (int)b, (long)(t * c), (int)c, dtype_code(type), st);
-    if (rc == QUEST_OK) rc = quest_dense_rows(logits.data_ptr(), normed.data_ptr(), head->data_ptr(), (int)b, (int)c, (int)v, dtype_code(type), st);
+    at::Tensor logits;
+    const int rc = on(args.dev, [&](void *st) {
+        const at::Tensor normed = make({b, c}, type, args.dev);
+        logits = make({b, 1, v}, type, args.dev);
+        const int rc = quest_rmsnorm_rows(normed.data_ptr(), (const uint8_t *)x->data_ptr() + last, branch ? (const uint8_t *)branch->data_ptr() + last : nullptr,
+                                          norm_w->data_ptr(), (float)eps, (int)b, (long)(t * c), (int)c, dtype_code(type), st);
+        if (rc != QUEST_OK) return rc;
+        return quest_dense_rows(logits.data_ptr(), normed.data_ptr(), head->data_ptr(), (int)b, (int)c, (int)v, dtype_code(type), st);
+    });
     if (rc != QUEST_OK) return declined();
     return wrap(std::move(logits));
     END_HANDLE_TH_ERRORS

@@ -1,5 +1,9 @@
 """The native host path (csrc/host.cpp) against the Python statements it stands in for: the same bits, the same errors.
 Declining every call makes the Python statements run."""
+import sys
+import threading
+import time
+
 import pytest
 import torch
 
@@ -93,3 +97,53 @@ def test_an_option_without_a_truth_value_raises_its_own_error():
     with pytest.raises(RuntimeError, match='Boolean value of Tensor'):
         quest.quantize_int4(x, torch.ones(4, 1, dtype=torch.bfloat16, device=DEV), do_dequantize=torch.ones(2))
     assert torch.equal(x, before)
+
+
+@pytest.mark.parametrize('call', ['linear', 'block', 'last_logits', 'steps'])
+def test_other_threads_run_during_native_calls(call):
+    """The interpreter lock is free while a native call allocates and launches: with a switch interval that never ends, a thread
+    that wants it gets it from there only."""
+    import quest_amd as quest
+    from quest_amd import harness, llama
+    x = torch.randn(2, 1024, device=DEV).bfloat16()
+    if call == 'linear':
+        layer = harness.Linear4bit.from_weight(torch.randn(256, 1024, device=DEV).bfloat16())
+        run = lambda: layer(x)                                                # noqa: E731
+    elif call == 'steps':
+        scale, packed = quest.find_scale_int4(x), torch.empty(2, 512, dtype=torch.uint8, device=DEV)
+        run = lambda: (quest.hadamard128(x), quest.find_scale_int4(x), quest.quantize_int4(x, scale, x_int_packed=packed),      # noqa: E731
+                       quest.matmul_int4_int4t_int32(packed, packed), quest.hadamard_quantize_int4(x))
+    else:
+        cfg = llama.LlamaConfig(n_layer=1, n_embd=1024, n_head=8, vocab_size=64)
+        net = llama.quantize_model(llama.Llama(cfg).to(DEV).bfloat16().eval(), 'int4', fuse_producers=True)
+        stream = torch.randn(2, 8, 1024, device=DEV).bfloat16()
+        freqs = net.freqs_cis[:8].to(DEV)
+        if call == 'block':
+            run = lambda: net.transformer.h[0].forward_fused(stream, freqs)   # noqa: E731
+        else:
+            run = lambda: quest.api.host.last_logits(stream, None, net.transformer.ln_f.weight, 1e-5, net.lm_head.weight)   # noqa: E731
+    with torch.no_grad():
+        run()
+        torch.cuda.synchronize()
+        turns, stop, ready = [0], threading.Event(), threading.Event()
+
+        def other():
+            ready.set()
+            while not stop.is_set():
+                turns[0] += 1
+                time.sleep(0)
+        thread = threading.Thread(target=other)
+        interval = sys.getswitchinterval()
+        thread.start()
+        ready.wait()
+        try:
+            sys.setswitchinterval(1000)
+            before = turns[0]
+            for _ in range(3000):
+                run()
+            after = turns[0]
+        finally:
+            stop.set()
+            sys.setswitchinterval(interval)
+            thread.join()
+    assert after - before > 10
