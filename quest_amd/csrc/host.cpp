@@ -92,6 +92,22 @@ int on(c10::Device dev, F &&launch) {
 int64_t up(int64_t bytes) { return (bytes + 255) & ~(int64_t)255; }
 bool at(const at::Tensor *t, unsigned bytes) { return t == nullptr || (reinterpret_cast<uintptr_t>(t->data_ptr()) & (bytes - 1)) == 0; }
 
+// Whether `t` is the tensor that something was derived from and still holds what it held: its address and version then are given.
+bool unchanged(PyObject *t, PyObject *source, PyObject *address, PyObject *version) {
+    if (t != source || !THPVariable_CheckExact(t)) return false;
+    const at::Tensor &v = THPVariable_Unpack(t);
+    return !v.is_inference() && PyLong_Check(address) && PyLong_AsVoidPtr(address) == v.data_ptr() && PyLong_Check(version) &&
+           PyLong_AsLongLong(version) == (long long)v._version();
+}
+
+// E2M3 tiles of the packed weight `packed`: a tensor of them, or (tiles, of which tensor, its address, its version) as Linear4bit keeps
+// them.  None if there are none, or if the tensor has changed since.
+PyObject *tiles_of(PyObject *kept, PyObject *packed) {
+    if (!PyTuple_Check(kept)) return kept;
+    if (PyTuple_GET_SIZE(kept) != 4 || !unchanged(packed, PyTuple_GET_ITEM(kept, 1), PyTuple_GET_ITEM(kept, 2), PyTuple_GET_ITEM(kept, 3))) return Py_None;
+    return PyTuple_GET_ITEM(kept, 0);
+}
+
 // What the GEMMs ask of sizes (gemm_check in gemm.hip, e2m3_gemm_check in gemm_e2m3.hip), for calls that launch something before them.
 bool gemm_takes(int64_t m, int64_t k, int64_t n, bool tiles) {
     if (tiles)
@@ -118,7 +134,7 @@ struct Codes {
 };
 
 // ---- linear(x, w_packed, w_scale, w_add, w_tiles, bias, had_scale, out) ---------------------------------------------
-// The W4A4 linear layer: activation kernel, GEMM, bias.  x (..., K); w_tiles: None, or the weight's E2M3 tiles when the
+// The W4A4 linear layer: activation kernel, GEMM, bias.  x (..., K); w_tiles: None, or the weight's E2M3 tiles (see tiles_of) when the
 // FP6 kernel is wanted; out: None or the (M, N) result to fill.
 PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (n_args != 8) return declined();
@@ -134,8 +150,9 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (!fits_int(m) || !fits_int(k) || !fits_int(n)) return declined();
     const at::Tensor *w_scale = args.tensor(a[2], type, n);
     const at::Tensor *w_add = args.tensor(a[3], at::kInt, n);
-    const bool tiles = a[4] != Py_None && args.ok && at(w_scale, 4);      // (the FP6 kernels read scales two at a time)
-    const at::Tensor *w_tiles = tiles ? args.tensor(a[4], at::kByte, (int64_t)quest_e2m3_tiles_bytes((int)n, (int)k)) : nullptr;
+    PyObject *const tiles_arg = tiles_of(a[4], a[1]);
+    const bool tiles = tiles_arg != Py_None && args.ok && at(w_scale, 4);      // (the FP6 kernels read scales two at a time)
+    const at::Tensor *w_tiles = tiles ? args.tensor(tiles_arg, at::kByte, (int64_t)quest_e2m3_tiles_bytes((int)n, (int)k)) : nullptr;
     const at::Tensor *bias = a[5] == Py_None ? nullptr : args.tensor(a[5], type, n);
     const double had_scale = PyFloat_AsDouble(a[6]);
     const at::Tensor *given = a[7] == Py_None ? nullptr : args.matrix(a[7], type, m, n);
@@ -385,12 +402,12 @@ PyObject *add_mul_vv(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     END_HANDLE_TH_ERRORS
 }
 
-// ---- block(x, branch, freqs, n_head, norm1, eps1, norm2, eps2, qkv, o, gate_up, glu, down, tiles) ---------------------
+// ---- block(x, branch, freqs, n_head, norm1, eps1, norm2, eps2, qkv, o, gate_up, glu, down, tiles, glu_of) -------------
 // One producer-fused decoder block (LlamaBlock.forward_fused with every option at its default): x (B, T, C) is the residual
 // stream, updated in place; branch: None, or the previous block's MLP output still to be added.  qkv, o, gate_up, glu, down:
 // (packed, scale, add, tiles or None) of the projections, glu the row-interleaved gate / up weights; tiles: which of the
-// four GEMMs (bit 0 qkv, 1 o, 2 gate_up, 3 down) run on E2M3 tiles.  Returns True, or the block's MLP output when it is
-// still to be added.
+// four GEMMs (bit 0 qkv, 1 o, 2 gate_up, 3 down) run on E2M3 tiles where there are any; glu_of: gate_up's three tensors, their
+// addresses and their versions when glu was made from them.  Returns True, or the block's MLP output when it is still to be added.
 struct Linear {
     const at::Tensor *packed, *scale, *add, *tiles;
     int n, k;
@@ -404,7 +421,8 @@ struct Linear {
         k = (int)packed->size(1) * 2;
         scale = args.tensor(PyTuple_GET_ITEM(t, 1), type, n);
         add = args.tensor(PyTuple_GET_ITEM(t, 2), at::kInt, n);
-        tiles = want_tiles ? args.tensor(PyTuple_GET_ITEM(t, 3), at::kByte, (int64_t)quest_e2m3_tiles_bytes(n, k)) : nullptr;
+        PyObject *const form = want_tiles ? tiles_of(PyTuple_GET_ITEM(t, 3), PyTuple_GET_ITEM(t, 0)) : Py_None;
+        tiles = form != Py_None ? args.tensor(form, at::kByte, (int64_t)quest_e2m3_tiles_bytes(n, k)) : nullptr;
         return args.ok;
     }
 };
@@ -452,7 +470,7 @@ Codes normed(at::Tensor &x, const at::Tensor *branch, const at::Tensor &weight, 
 }
 
 PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
-    if (n_args != 14) return declined();
+    if (n_args != 15) return declined();
     HANDLE_TH_ERRORS
     Args args;
     const at::Tensor *xp = args.tensor(a[0]);
@@ -476,6 +494,10 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (!args.ok || PyErr_Occurred() || !qkv.take(args, a[8], type, tiles & 1) || !o.take(args, a[9], type, tiles & 2) ||
         !gate_up.take(args, a[10], type, false) || !glu.take(args, a[11], type, tiles & 4) || !down.take(args, a[12], type, tiles & 8))
         return declined();
+    if (!PyTuple_Check(a[14]) || PyTuple_GET_SIZE(a[14]) != 9) return declined();
+    for (int i = 0; i < 3; i++)
+        if (!unchanged(PyTuple_GET_ITEM(a[10], i), PyTuple_GET_ITEM(a[14], i), PyTuple_GET_ITEM(a[14], 3 + i), PyTuple_GET_ITEM(a[14], 6 + i)))
+            return declined();
     const int hidden = down.k;
     if (qkv.k != c || qkv.n != 3 * c || o.k != c || o.n != c || gate_up.k != c || gate_up.n != 2 * hidden || glu.k != c || glu.n != 2 * hidden ||
         down.n != c || (c & 127) != 0 || (hidden & 127) != 0 || c > 32768 || hidden > 32768 || (head_dim & 7) != 0)

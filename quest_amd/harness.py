@@ -240,12 +240,13 @@ class Linear4bit(nn.Module):
         its packed codes (the same bits).  Nothing is kept for a layer that the FP6 kernels do not take, or while MATRIX_PATH is
         'int8'."""
         self._tiles = None
-        w = self._buffers.get('w_int_packed')
-        if type(w) is not torch.Tensor or not w.is_cuda or w.dim() != 2 or not w.is_contiguous():
-            return
         with torch.inference_mode(False), torch.no_grad():
-            if w.is_inference():                                     # (it would not show later writes)
-                w = self._buffers['w_int_packed'] = w.clone()
+            for name, t in self._buffers.items():
+                if type(t) is torch.Tensor and t.is_inference():     # (it would not show later writes)
+                    self._buffers[name] = t.clone()
+            w = self._buffers.get('w_int_packed')
+            if type(w) is not torch.Tensor or not w.is_cuda or w.dim() != 2 or not w.is_contiguous():
+                return
             if MATRIX_PATH == 'fp6' and e2m3_fits(w.size(1) * 2, w.size(0)):
                 self._tiles = (weight_tiles(w), w, w.data_ptr(), w._version)
 
@@ -254,14 +255,18 @@ class Linear4bit(nn.Module):
         kept = self._tiles
         if kept is None:
             return None
-        tiles, source, address, version = kept
+        tiles, source, address, version = kept                        # (what csrc/host.cpp asks as well: unchanged())
         w = self._buffers.get('w_int_packed')
         return tiles if w is source and w._version == version and w.data_ptr() == address else None
 
     def tiles_for(self, m: int):
         """The weight's E2M3 tiles where the FP6 kernels are the faster ones for m tokens, None where the packed codes serve."""
         n, k = self.weight.shape
-        return self._kept_tiles() if prefers_e2m3(m, k, n) and _scales_in_pairs(self.w_scale) else None
+        return self.readable_tiles() if prefers_e2m3(m, k, n) else None
+
+    def readable_tiles(self):
+        """The kept tiles, if the FP6 kernels can read the scales beside them."""
+        return self._kept_tiles() if _scales_in_pairs(self.w_scale) else None
 
     def w_tiles(self) -> torch.Tensor:
         """The weight codes as E2M3 tiles: the kept ones, or a conversion of the buffer for this call."""
@@ -366,7 +371,7 @@ class Linear4bit(nn.Module):
             k = x.size(-1)
             held = self._buffers.get                  # (not there, e.g. made a parameter: the native call declines)
             if held('w_meta_e') is None:
-                tiles = self._kept_tiles() if prefers_e2m3(x.numel() // max(k, 1), k, n) else None
+                tiles = self._tiles if prefers_e2m3(x.numel() // max(k, 1), k, n) else None
                 y = quest.host.linear(x, held('w_int_packed'), held('w_scale'), held('w_add'), tiles, self.bias,
                                       HADAMARD_ENTRY if self.use_hadamard else 0., None)
                 if y is not None:

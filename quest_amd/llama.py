@@ -123,17 +123,16 @@ class LlamaMLP(nn.Module):
         w._tiles = None
 
     def _glu_source(self):
-        return [(t, t.data_ptr(), None if t.is_inference() else t._version) for t in (self.w12.w_int_packed, self.w12.w_scale, self.w12.w_add)]
+        now = [self.w12._buffers.get(name) for name in ('w_int_packed', 'w_scale', 'w_add')]
+        return (*now, *(t.data_ptr() for t in now), *(None if t.is_inference() else t._version for t in now))
 
     def kept_glu(self):
         """`glu`, if w12 still holds what it was made from."""
-        if self.glu is None or self._glu_of is None:
+        if self.glu is None or self._glu_of is None or any(self.w12._buffers.get(n) is None for n in ('w_int_packed', 'w_scale', 'w_add')):
             return None
-        for (t, address, version), name in zip(self._glu_of, ('w_int_packed', 'w_scale', 'w_add')):
-            now = self.w12._buffers.get(name)
-            if now is not t or now.data_ptr() != address or (version is not None and now._version != version):
-                return None
-        return self.glu
+        now = self._glu_source()
+        same = all(a is b for a, b in zip(now[:3], self._glu_of)) and now[3:] == self._glu_of[3:] and None not in now[6:]
+        return self.glu if same else None
 
     def _apply(self, *args, **kwargs):
         super()._apply(*args, **kwargs)
@@ -249,18 +248,21 @@ class LlamaBlock(nn.Module):
         given, is the previous block's MLP output still to be added to it.  Returns (x, this block's MLP output or
         None): the caller adds the last one (or hands it to the next block); None when the output projection's GEMM has
         added it already."""
+        done = self._forward_native(x, freqs_cis, branch)
+        if done is not None:
+            return x, (None if done is True else done)
         b, t, c = x.shape
         m = b * t
         hidden = self.mlp.c_proj.weight.size(1)
-        done = self._forward_native(x, freqs_cis, branch, m, c, hidden)
-        if done is not None:
-            return x, (None if done is True else done)
         x2 = x.view(m, c)
         # each producer writes the operand form its GEMM runs fastest on: E2M3 tiles for the FP6 kernel, or packed
         # nibbles and row sums for the INT8 kernels (same codes, same output bits either way)
         rotated = False
         glu = self.mlp.kept_glu()
-        qkv_tiles, o_tiles, gate_tiles, down_tiles = self._tiles_for(m, glu)
+        forms = self._on_tiles(m, c, hidden, x.dtype)
+        qkv_tiles, o_tiles, down_tiles = (w.readable_tiles() if forms & bit and isinstance(w, harness.Linear4bit) else None
+                                          for w, bit in ((self.attn.c_attn, 1), (self.attn.c_proj, 2), (self.mlp.c_proj, 8)))
+        gate_tiles = None if not forms & 4 else self.mlp.w12.readable_tiles() if glu is None else self.mlp.glu_tiles
         if qkv_tiles is not None:
             if branch is None:
                 q = quest.rmsnorm_hadamard_quantize_e2m3(x2, self.ln_1.weight, self.ln_1.eps)
@@ -333,48 +335,46 @@ class LlamaBlock(nn.Module):
         return x, y.view(b, t, c)
 
 
-    def _forward_native(self, x, freqs_cis, branch, m, c, hidden):
-        """`forward_fused` as one call of the native host path (the same kernels in the same order; at 37 tokens the
-        twelve launches of a block cost 240 us from Python and about 50 from there).  None, with nothing launched, where
-        an option is not at its default or a part has been replaced or hooked: the statement in Python then runs."""
-        attn, mlp = self.attn, self.mlp
-        if type(attn) is not LlamaAttention or type(mlp) is not LlamaMLP:
+    def _forward_native(self, x, freqs_cis, branch):
+        """`forward_fused` as one call of the native host path (the same kernels in the same order, but for a gated unit of up to 64
+        tokens, which a bf16 block has in the quantiser; at 37 tokens the twelve launches of a block cost 240 us from Python
+        and about 50 from there).  None, with nothing launched, where an option is not at its default or a part has been
+        replaced or hooked: the statement in Python then runs.  (Parts are read from the modules' dictionaries, which costs a
+        third of asking the modules.)"""
+        parts = self._modules
+        attn, mlp, norm1, norm2 = parts['attn'], parts['mlp'], parts['ln_1'], parts['ln_2']
+        if type(attn) is not LlamaAttention or type(mlp) is not LlamaMLP or x.dim() != 3:
             return None
-        linears = (attn.c_attn, attn.c_proj, mlp.w12, mlp.c_proj)
-        glu = mlp.kept_glu()
-        if not (glu is not None and attn.fused_rope and harness.GEMM_ADDS_RESIDUAL and harness.GEMM_ADDS_RESIDUAL_PACKED
-                and harness.GEMM_ROTATES_QK and _as_built(attn.c_proj, harness.Linear4bit)):
+        own_a, own_m = attn.__dict__, mlp.__dict__
+        glu = own_m['glu']
+        if (glu is None or not own_a['fused_rope'] or 'attend' in own_a or 'attention_core' in own_a or 'swiglu_quantized' in own_m
+                or 'swiglu_tiles' in own_m
+                or not (harness.GEMM_ADDS_RESIDUAL and harness.GEMM_ADDS_RESIDUAL_PACKED and harness.GEMM_ROTATES_QK)):
             return None
-        for part, methods in ((attn, ('attend', 'attention_core')), (mlp, ('swiglu_quantized', 'swiglu_tiles'))):
-            if methods[0] in part.__dict__ or methods[1] in part.__dict__:
-                return None
+        linears = attn._modules.get('c_attn'), attn._modules.get('c_proj'), mlp._modules.get('w12'), mlp._modules.get('c_proj')
+        held = []
         for w in linears:
             if not (type(w) is harness.Linear4bit and w.bias is None and w.use_hadamard and not w.use_noop
                     and not w.quantize_from_fp32 and 'forward_quantized' not in w.__dict__ and 'forward_tiles' not in w.__dict__):
                 return None
-        qkv_tiles, o_tiles, gate_tiles, down_tiles = self._tiles_for(m, glu)
-        qkv, o, both, down = (w._buffers.get for w in linears)
-        return quest.host.block(
-            x, branch, freqs_cis, attn.n_head, self.ln_1.weight, float(self.ln_1.eps), self.ln_2.weight, float(self.ln_2.eps),
-            (qkv('w_int_packed'), qkv('w_scale'), qkv('w_add'), qkv_tiles),
-            (o('w_int_packed'), o('w_scale'), o('w_add'), o_tiles),
-            (both('w_int_packed'), both('w_scale'), both('w_add'), None),
-            (*glu, gate_tiles),
-            (down('w_int_packed'), down('w_scale'), down('w_add'), down_tiles),
-            (qkv_tiles is not None) | (o_tiles is not None) << 1 | (gate_tiles is not None) << 2 | (down_tiles is not None) << 3)
+            t = w._buffers.get
+            held.append((t('w_int_packed'), t('w_scale'), t('w_add'), w._tiles))
+        if not _as_built(linears[1], harness.Linear4bit):
+            return None
+        qkv, o, both, down = held
+        b, t, c = x.shape
+        return quest.host.block(x, branch, freqs_cis, attn.n_head, norm1._parameters.get('weight'), float(norm1.eps),
+                                norm2._parameters.get('weight'), float(norm2.eps), qkv, o, both, (*glu, mlp.glu_tiles), down,
+                                self._on_tiles(b * t, c, glu[0].size(0) >> 1, x.dtype), mlp._glu_of)
 
-    def _tiles_for(self, m, glu):
-        """Of the four projections (qkv, output, gate / up, down) the weight tiles that m tokens are multiplied by, None for the packed
-        codes: the one decision of both statements of the block.  glu: `mlp.kept_glu()`."""
-        def of(w):
-            return w.tiles_for(m) if isinstance(w, harness.Linear4bit) else None
-        if glu is None:
-            gate = of(self.mlp.w12)
-        else:
-            gate = self.mlp.glu_tiles if harness.prefers_e2m3(m, glu[0].size(1) * 2, glu[0].size(0)) else None
-            if m <= 64 and glu[1].dtype == torch.float16:       # torch's silu, which the kernels' is not for every fp16 value
-                gate = None
-        return of(self.attn.c_attn), of(self.attn.c_proj), gate, of(self.mlp.c_proj)
+    @staticmethod
+    def _on_tiles(m, c, hidden, dtype):
+        """Which of the four projections (bit 0 qkv, 1 output, 2 gate / up, 3 down) run on E2M3 tiles for m tokens, if there are any: the
+        one decision of both statements of the block."""
+        prefers = harness.prefers_e2m3
+        forms = prefers(m, c, 3 * c) | prefers(m, c, c) << 1 | prefers(m, c, 2 * hidden) << 2 | prefers(m, hidden, c) << 3
+        # few fp16 tokens: torch's silu, which the kernels' is not for every fp16 value
+        return forms & ~4 if m <= 64 and dtype == torch.float16 else forms
 
 
 class Llama(nn.Module):
