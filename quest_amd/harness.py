@@ -18,11 +18,11 @@ _HIP_BACKENDS = ('hip', 'triton', 'cuda')
 WEIGHT_HADAMARD_SCALE = 2. ** -3.5      # utils.py:39
 
 # Which matrix instructions the GEMM of `linear_forward` / `Linear4bit` runs on when the weight's E2M3 tiles are at
-# hand: 'fp6' = the FP6 (E2M3) kernels where they are the faster ones (from 33 tokens on), 'int8' = always the
+# hand: 'fp6' = the FP6 (E2M3) kernels where they are the faster ones, 'int8' = always the
 # INT8 kernels on packed nibbles.  Both give the same bits.
 MATRIX_PATH = 'fp6'
-E2M3_MIN_TOKENS = 33                    # from here on the FP6 kernels are the faster ones
-E2M3_MIN_K = 1536                       # shortest rows that take them at more than E2M3_SHORT_ROWS_TOKENS tokens (see prefers_e2m3)
+E2M3_MIN_TOKENS = 33                    # a fused block: from here on (see block_prefers_e2m3); a layer: see prefers_e2m3
+E2M3_MIN_K = 1536                       # shortest rows that take them at more than E2M3_SHORT_ROWS_TOKENS tokens
 E2M3_MIN_K_NARROW = 2048                # ... by a layer of fewer than E2M3_NARROW channels
 E2M3_NARROW = 1536
 E2M3_SHORT_ROWS_TOKENS = 4096
@@ -35,16 +35,50 @@ GEMM_ROTATES_QK = True
 
 
 def prefers_e2m3(m: int, k: int, n: int) -> bool:
-    """Whether the FP6 kernels are the faster ones for an (m, k) x (n, k) layer: measured over K from 1024 to 11008, N from
-    1024 to 22016 and M from 20 to 3000 they win 3 to 60 % from 33 tokens on (1.2 x on average; level or up to 8 % behind at 33 to 64
-    tokens with K = 1024, N = 11264 and K = 4096, N = 22016) and lose below, where the weights' 1.5 x bytes are the whole cost."""
-    # E2M3_MIN_K: with shorter rows and many tokens the GEMM is mostly epilogue either way and the tile-writing activation kernels
-    # are a little slower than the row-writing ones (12.0 against 10.2 us at [16384, 1024]).  Whole layers of 4097 to 16384 tokens,
-    # INT8 / FP6 time: K = 1536 1.12 on average over N from 1500 to 22016, K = 1792 1.14, K = 1920 1.16, 0.98 at the least ((4097,
-    # 1536, 1536) 33.7 / 27.4 us, (8192, 1536, 8192) 103 / 84, (16384, 1536, 3072) 85 / 70); K = 1024 0.85 to 1.18 ((16384, 1024, 8192) 148 / 173 us), K = 1152 to
-    # 1408 0.94 to 1.27.  Layers of 1024 channels lose 6 to 12 % at 8192 tokens up to K = 1920 (half a 256 x 256 tile per CU).
-    return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and k <= 65536 and m * n <= (1 << 30) and m * k <= (5 << 29)
-            and (m <= E2M3_SHORT_ROWS_TOKENS or k >= (E2M3_MIN_K if n >= E2M3_NARROW else E2M3_MIN_K_NARROW)))
+    """Whether the FP6 kernels are the faster ones for an (m, k) x (n, k) layer on its own, quantiser included, with weights that come
+    from HBM (copies of more than 300 MB in turn): 2096 sizes, K 128 to 11008, N 136 to 22016, M 33 to 4096.  The path taken is
+    within 0.8 % of the faster one on average (always FP6: 3.0 %) and, from K = 640 on, within 16 % everywhere."""
+    if MATRIX_PATH != 'fp6' or k % 128 or not _tiles_addressable(m, k, n):
+        return False
+    if m > E2M3_SHORT_ROWS_TOKENS:
+        return _enough_per_row(k, n)
+    # K < 640: as often slower as faster (K = 128: 0.83 at (2000, 22016), 1.47 at (700, 11008); K = 512: 0.88 to 1.41)
+    if m < 49 or k < 640:
+        return False
+    # Some tens of tokens: the weights are the cost, and the tiles are 1.5 x the codes' bytes.  (INT8 / FP6 time: (33, 11008, 11008)
+    # 0.72, (64, 4096, 11008) 0.88, (40, 1024, 4096) 0.96; (64, 2048, 2048) 1.06, (64, 11008, 1024) 1.27.)  More than 16384
+    # channels are a second round of the INT8 kernel's tiles: (56, 3072, 22016) 1.06.
+    if m <= 64:
+        return (n <= 4096 and k >= 1536) or (n > 16384 and 2048 <= k <= 6912)
+    # The INT8 kernels' 64 x 64 tiles: half a round of the 256 CUs or less 0.95 to 1.31 (1.08 on average), one nearly full round 0.82
+    # to 1.16 (0.92; (256, 6912, 3072) 0.87, (128, 4096, 8192) 0.87), two rounds 0.82 to 1.10 (0.96) with K >= 4096 and 0.91 to
+    # 1.12 (1.01) below, more 0.90 to 1.57 (1.10).
+    tiles = ((m + 63) >> 6) * ((n + 63) >> 6)
+    if tiles <= 512:
+        return tiles <= 128 or (tiles > 256 and k < 4096)
+    return not (m > 3000 and k < 1536 and 512 <= n <= 2048)           # (4096, 1024, 2048) 0.90, (4096, 1280, 512) 0.95
+
+
+def block_prefers_e2m3(m: int, k: int, n: int) -> bool:
+    """The same for a projection of a producer-fused block, where the FP6 kernels also save launches (the rotary embedding, the gated
+    unit and both residual additions ride in their epilogues at every size).  Whole blocks, d = 256 to 4096, 33 to 4000 tokens,
+    weights from HBM, INT8 / FP6 time: 0.97 to 1.18 ((d = 768, 1000 tokens) 0.97, (2560, 200) 0.99, (1024, 37) 1.08, (2560, 64)
+    1.14, (4096, 500) 1.17)."""
+    return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and _tiles_addressable(m, k, n)
+            and (m <= E2M3_SHORT_ROWS_TOKENS or _enough_per_row(k, n)))
+
+
+def _tiles_addressable(m: int, k: int, n: int) -> bool:
+    return k <= 65536 and m * n <= (1 << 30) and m * k <= (5 << 29)
+
+
+def _enough_per_row(k: int, n: int) -> bool:
+    # With short rows and many tokens the GEMM is mostly epilogue either way and the tile-writing activation kernels are a little
+    # slower than the row-writing ones (12.0 against 10.2 us at [16384, 1024]).  Whole layers of 4097 to 16384 tokens, INT8 / FP6
+    # time: K = 1536 1.12 on average over N from 1500 to 22016, K = 1792 1.14, K = 1920 1.16 ((4097, 1536, 1536) 33.7 / 27.4 us,
+    # (8192, 1536, 8192) 103 / 84, (16384, 1536, 3072) 85 / 70); K = 1024 0.85 to 1.18 ((16384, 1024, 8192) 148 / 173 us), K = 1152
+    # to 1408 0.94 to 1.27.  Layers of 1024 channels lose 6 to 12 % at 8192 tokens up to K = 1920 (half a 256 x 256 tile per CU).
+    return k >= (E2M3_MIN_K if n >= E2M3_NARROW else E2M3_MIN_K_NARROW)
 
 
 def e2m3_fits(k: int, rows: int) -> bool:

@@ -371,7 +371,7 @@ class LlamaBlock(nn.Module):
     def _on_tiles(m, c, hidden, dtype):
         """Which of the four projections (bit 0 qkv, 1 output, 2 gate / up, 3 down) run on E2M3 tiles for m tokens, if there are any: the
         one decision of both statements of the block."""
-        prefers = harness.prefers_e2m3
+        prefers = harness.block_prefers_e2m3
         forms = prefers(m, c, 3 * c) | prefers(m, c, c) << 1 | prefers(m, c, 2 * hidden) << 2 | prefers(m, hidden, c) << 3
         # few fp16 tokens: torch's silu, which the kernels' is not for every fp16 value
         return forms & ~4 if m <= 64 and dtype == torch.float16 else forms
