@@ -321,7 +321,10 @@ int quest_fused_matmul_dequantize_rope_e2m3(void *mat_d, const void *a_tiles, co
  * Diagnostic (host only, nothing is launched): how quest_fused_matmul_dequantize_e2m3 divides a shape among the
  * workgroups of a device with `cus` compute units.  plan[0..7] = workgroups, scheduling groups (one per XCD when 8),
  * tiles per token tile when every workgroup gets exactly one (else 0), how many ways the groups divide the token tiles
- * (0 or 1: not at all, each group takes a slice of the channel units; g: a g x groups / g grid of groups), tile rows, tile channels at most, LDS slots, k per slot.  A measured figure that depends on
+ * (0 or 1: not at all, each group takes a slice of the channel units; g: a g x groups / g grid of groups), tile rows, tile channels at most, LDS slots, k per slot.
+ * Shapes of at most half a 256 x 256 tile per compute unit run on smaller tiles, one per workgroup, dealt to the XCDs in contiguous
+ * eighths (plan[1..3] = 8, 0, 0): 128 k per slot where the waves share the tile, 64 where each has a quarter of K and slots of
+ * its own.  A measured figure that depends on
  * the schedule (HBM traffic per launch) is only valid while this plan is the one it was measured under.
  */
 int quest_e2m3_gemm_plan(int size_m, int size_k, int size_n, int cus, int *plan);

@@ -502,7 +502,9 @@ static int launch_large(int dtype, void *out, const uint8_t *a, const uint8_t *b
 // The tile shapes of the two kernels for smaller problems, with what a launch takes in us: fixed + rounds (stage K / 128 + tile) +
 // weights (per MB of weight tiles), rounds = tiles per CU, rounded up.  Fitted to 240 sizes (M from 20 to 3000, K from 1024 to 11008,
 // N from 1024 to 22016, weights rotating through several copies): the shape with the smallest estimate is within 0.9 % of
-// always picking the fastest one in total time, within 16 % on every single size.
+// always picking the fastest one in total time, within 16 % on every single size.  With weights from HBM (copies of more than 320
+// MB, 816 sizes, K from 256) it is within 1.4 % in total and 20 % on every size; on rows of 16384 to 65536, beyond the fit and its
+// negative coefficients, within 0.1 and 3 %.
 struct Shape {
     bool split;
     int tf, cf;
@@ -625,6 +627,13 @@ extern "C" int quest_fused_matmul_dequantize_rope_e2m3(void *mat_d, const void *
 extern "C" int quest_e2m3_gemm_plan(int size_m, int size_k, int size_n, int cus, int *plan) {
     if (!plan) return QUEST_ERR_NULL_POINTER;
     if (size_m <= 0 || size_n <= 0 || size_k <= 0 || (size_k & 127) || cus <= 0) return QUEST_ERR_BAD_SHAPE;
+    if (const Shape *s = smaller_shape(size_m, size_k, size_n, cus)) {
+        const int rows = 32 * s->tf, channels = 32 * s->cf;
+        const long workgroups = tile_grid((size_m + rows - 1) / rows, (size_n + channels - 1) / channels);
+        const int v[8] = {(int)workgroups, 8, 0, 0, rows, channels, s->split ? gemm_e2m3_split_slots(s->tf, s->cf) : gemm_e2m3_mid_slots(s->tf, s->cf), s->split ? 64 : 128};
+        for (int i = 0; i < 8; i++) plan[i] = v[i];
+        return QUEST_OK;
+    }
     long grid = 0;
     const Schedule sch = make_schedule(size_m, size_n, e2m3::kMaxUnits, 1, cus, &grid, e2m3::kTokSplit);
     const int v[8] = {(int)grid, sch.groups, sch.row_tiles, sch.by_tokens, e2m3::kRows, 32 * e2m3::kMaxUnits, e2m3::kStages, 64};

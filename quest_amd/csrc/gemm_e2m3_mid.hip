@@ -225,6 +225,15 @@ static int launch(void *out, const uint8_t *a, const uint8_t *b, int M, int K, i
 
 }  // namespace e2m3m
 
+#define QUEST_MID_SHAPES QUEST_MID(8, 4) QUEST_MID(4, 6) QUEST_MID(4, 4) QUEST_MID(4, 2) QUEST_MID(2, 4) QUEST_MID(2, 2)
+
+int gemm_e2m3_mid_slots(int tf, int cf) {
+#define QUEST_MID(TF, CF) if (tf == TF && cf == CF) return e2m3m::Tile<TF, CF, 2, 2>::kStages;
+    QUEST_MID_SHAPES
+#undef QUEST_MID
+    return 0;
+}
+
 int launch_gemm_e2m3_mid(int dtype, int tf, int cf, void *out, const uint8_t *a, const uint8_t *b, int M, int K, int N, const Epilogue &epi, hipStream_t st) {
 #define QUEST_MID_DT(DT, T) (epi.kind == kEpiRope ? e2m3m::launch<DT, true, T>(out, a, b, M, K, N, epi, st) : e2m3m::launch<DT, false, T>(out, a, b, M, K, N, epi, st))
 #define QUEST_MID(TF, CF)                                                                                        \
@@ -232,12 +241,7 @@ int launch_gemm_e2m3_mid(int dtype, int tf, int cf, void *out, const uint8_t *a,
         using T = e2m3m::Tile<TF, CF, 2, 2>;                                                                     \
         return dtype == QUEST_DTYPE_BF16 ? QUEST_MID_DT(0, T) : QUEST_MID_DT(1, T);                              \
     }
-    QUEST_MID(8, 4)
-    QUEST_MID(4, 6)
-    QUEST_MID(4, 4)
-    QUEST_MID(4, 2)
-    QUEST_MID(2, 4)
-    QUEST_MID(2, 2)
+    QUEST_MID_SHAPES
 #undef QUEST_MID
 #undef QUEST_MID_DT
     return QUEST_ERR_UNSUPPORTED;

@@ -226,14 +226,20 @@ static int launch(void *out, const uint8_t *a, const uint8_t *b, int M, int K, i
 
 }  // namespace e2m3s
 
+#define QUEST_SPLIT_SHAPES QUEST_SPLIT(1, 1) QUEST_SPLIT(1, 2) QUEST_SPLIT(2, 2) QUEST_SPLIT(4, 2)
+
+int gemm_e2m3_split_slots(int tf, int cf) {
+#define QUEST_SPLIT(TF, CF) if (tf == TF && cf == CF) return e2m3s::Tile<TF, CF>::kStages;
+    QUEST_SPLIT_SHAPES
+#undef QUEST_SPLIT
+    return 0;
+}
+
 int launch_gemm_e2m3_split(int dtype, int tf, int cf, void *out, const uint8_t *a, const uint8_t *b, int M, int K, int N, const Epilogue &epi, hipStream_t st) {
 #define QUEST_SPLIT_DT(DT, TF, CF) (epi.kind == kEpiRope ? e2m3s::launch<DT, true, TF, CF>(out, a, b, M, K, N, epi, st) : e2m3s::launch<DT, false, TF, CF>(out, a, b, M, K, N, epi, st))
 #define QUEST_SPLIT(TF, CF) \
-    if (tf == TF && cf == CF) return dtype == QUEST_DTYPE_BF16 ? QUEST_SPLIT_DT(0, TF, CF) : QUEST_SPLIT_DT(1, TF, CF)
-    QUEST_SPLIT(1, 1);
-    QUEST_SPLIT(1, 2);
-    QUEST_SPLIT(2, 2);
-    QUEST_SPLIT(4, 2);
+    if (tf == TF && cf == CF) return dtype == QUEST_DTYPE_BF16 ? QUEST_SPLIT_DT(0, TF, CF) : QUEST_SPLIT_DT(1, TF, CF);
+    QUEST_SPLIT_SHAPES
 #undef QUEST_SPLIT
 #undef QUEST_SPLIT_DT
     return QUEST_ERR_UNSUPPORTED;

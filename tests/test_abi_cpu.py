@@ -79,3 +79,24 @@ def test_unpack_int4_host_helper_matches_oracle():
     from quest_amd import harness
     b = torch.arange(256, dtype=torch.int32).to(torch.uint8).view(2, 128)
     assert torch.equal(harness.unpack_int4(b), qo.unpack_int4(b))
+
+
+def test_e2m3_plan_names_the_kernel_that_runs():
+    """(tile rows, tile channels, k per slot) on 256 compute units for the sizes that the GPU tests of the tile shapes use: 64 k = K
+    split over the waves, 128 k = the waves share the tile; 256 x 256 tiles otherwise."""
+    from quest_amd import _lib
+    lib = _lib.load()
+    expected = {(32, 32, 64): [(1, 128, 8), (257, 2560, 77), (97, 640, 264)], (32, 64, 64): [(33, 1024, 4100), (257, 128, 1500)],
+                (64, 64, 64): [(100, 512, 4104), (333, 128, 2056), (2100, 384, 203), (257, 4096, 3104)], (128, 64, 64): [(257, 4096, 4100), (65, 4096, 11000)],
+                (64, 64, 128): [(200, 128, 11000), (1000, 128, 2051)], (64, 128, 128): [(257, 384, 6008), (257, 2560, 10999)],
+                (128, 64, 128): [(200, 384, 4104), (1000, 2560, 1031)], (128, 128, 128): [(130, 512, 10999), (1400, 1024, 2056)],
+                (128, 192, 128): [(333, 1024, 11000), (3000, 512, 1501)], (256, 128, 128): [(2100, 128, 3099), (3000, 384, 2056)],
+                (256, 256, 64): [(4098, 256, 2104), (4096, 4096, 11008)]}
+    plan = (ctypes.c_int * 8)()
+    for (rows, channels, k), sizes in expected.items():
+        for m, size_k, n in sizes:
+            assert lib.quest_e2m3_gemm_plan(m, size_k, n, 256, plan) == 0
+            assert (plan[4], plan[5], plan[7]) == (rows, channels, k), (m, size_k, n, list(plan))
+            tiles = -(-m // rows) * -(-n // channels)
+            assert plan[6] >= 3 and (rows == 256 == channels or tiles <= plan[0] < tiles + 8)
+    assert lib.quest_e2m3_gemm_plan(200, 100, 64, 256, plan) == -2

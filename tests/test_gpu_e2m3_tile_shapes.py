@@ -7,8 +7,8 @@ pytestmark = pytest.mark.gpu
 DEV = 'cuda:0'
 SHAPES = [(1, 128, 8), (257, 2560, 77), (97, 640, 264),                    # split 1 x 1
           (33, 1024, 4100), (257, 128, 1500),                              # split 1 x 2
-          (100, 512, 4104), (333, 128, 2056), (2100, 384, 203),            # split 2 x 2
-          (257, 4096, 3104), (65, 4096, 11000),                            # split 4 x 2
+          (100, 512, 4104), (333, 128, 2056), (2100, 384, 203), (257, 4096, 3104),      # split 2 x 2
+          (257, 4096, 4100), (65, 4096, 11000),                            # split 4 x 2
           (200, 128, 11000), (1000, 128, 2051),                            # 2 x 2
           (257, 384, 6008), (257, 2560, 10999),                            # 2 x 4
           (200, 384, 4104), (1000, 2560, 1031),                            # 4 x 2
