@@ -35,7 +35,7 @@ def _run(cmd: list[str], verbose: bool) -> None:
     noise = "is not a recognized feature for this target"
     err = '\n'.join(l for l in res.stderr.splitlines() if noise not in l)
     if res.returncode != 0:
-        raise RuntimeError(f'hipcc failed ({res.returncode}):\n{err}')
+        raise RuntimeError(f'{os.path.basename(cmd[0])} failed ({res.returncode}):\n{err}')
     if verbose and err.strip():
         print(err, file=sys.stderr)
 
@@ -43,15 +43,18 @@ def _run(cmd: list[str], verbose: bool) -> None:
 def _host_command(out: str) -> list[str]:
     import torch
     root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get('ROCM_PATH', '/opt/rocm')
+    # (the ABI of torch's own std::string, or nothing that takes one would link)
     return [os.environ.get('CXX', 'g++'), '-O2', '-std=c++17', '-fPIC', '-shared', '-Wall', '-D__HIP_PLATFORM_AMD__=1', '-DUSE_ROCM=1',
-            '-isystem', os.path.join(root, 'include'), '-isystem', '/opt/rocm/include', '-isystem', sysconfig.get_paths()['include'],
+            f'-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}',
+            '-isystem', os.path.join(root, 'include'), '-isystem', os.path.join(rocm, 'include'), '-isystem', sysconfig.get_paths()['include'],
             os.path.join(CSRC, 'host.cpp'), '-o', out, '-L' + os.path.join(root, 'lib'), '-lc10', '-lc10_hip', '-ltorch_cpu',
             '-ltorch_python', '-L' + HERE, '-l:libquest_hip.so', '-Wl,-rpath,$ORIGIN']
 
 
 def build(verbose: bool = False, extra_flags: list[str] | None = None, jobs: int = 4) -> str:
     """Compiles every source to an object (up to `jobs` at a time), links the shared library, then the host module."""
-    hipcc = os.environ.get('HIPCC', '/opt/rocm/bin/hipcc')
+    hipcc = os.environ.get('HIPCC', os.path.join(os.environ.get('ROCM_PATH', '/opt/rocm'), 'bin', 'hipcc'))
     flags = [f for f in FLAGS if f != '-shared'] + list(extra_flags or [])
     with tempfile.TemporaryDirectory(prefix='quest_hip_build_') as tmp:
         objs = [os.path.join(tmp, os.path.splitext(s)[0] + '.o') for s in SOURCES]
@@ -61,6 +64,9 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None, jobs: int
                 fut.result()
         _run([hipcc, '--offload-arch=gfx950', '-shared', '-fPIC', *objs, '-o', LIB_PATH], verbose)
     _run(_host_command(HOST_PATH), verbose)
+    # (an unresolved symbol would otherwise show at the first call, as a module that seems not to be there)
+    _run([sys.executable, '-c', f'import torch, importlib.util as u; s = u.spec_from_file_location("_host", {HOST_PATH!r}); s.loader.exec_module(u.module_from_spec(s))'],
+         verbose)
     return LIB_PATH
 
 

@@ -87,3 +87,10 @@ def test_which_layers_take_the_fp6_kernels(monkeypatch):
     assert harness.block_prefers_e2m3(37, 1024, 3072) and harness.block_prefers_e2m3(64, 2560, 7680)
     monkeypatch.setattr(harness, 'MATRIX_PATH', 'int8')
     assert not any(harness.prefers_e2m3(*s) or harness.block_prefers_e2m3(*s) for s in fp6)
+
+
+def test_host_module_command_follows_torch_and_rocm(monkeypatch):
+    from quest_amd import build
+    monkeypatch.setenv('ROCM_PATH', '/some/rocm')
+    cmd = build._host_command('out.so')
+    assert f'-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}' in cmd and '/some/rocm/include' in cmd
