@@ -20,7 +20,7 @@ struct Ahead {
     uint4 v[ROPE ? 2 : 1];
 };
 
-// vec16: the output's rows are whole eights of channels (and the bias 16-byte aligned).
+// vec16: the output's rows are whole eights of channels.  (A bias is 16-byte aligned: the entry point asks for it.)
 template <int DT, bool ROPE>
 __device__ __forceinline__ void fetch_ahead(Ahead<ROPE> &a, const void *out, const Epilogue &epi, int tok, int ch, int M, int N, bool vec16) {
     const bool in = tok < M && ch < N;

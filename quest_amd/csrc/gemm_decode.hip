@@ -54,7 +54,7 @@ gemm_w4a4_decode_kernel(void *__restrict__ out, const uint8_t *__restrict__ act,
     const int g = lane >> 4;
     const int row_b = K >> 1;                          // packed bytes per row
     const int ch0 = blockIdx.x * kChannels;
-    const int n_chunks = (row_b + kChunkB - 1) / kChunkB;      // the last one may hold only its first 64 bytes
+    const int n_chunks = (row_b + kChunkB - 1) / kChunkB;      // the last one may be any number of whole 16-byte pieces
 
     // rows that do not exist get an offset beyond the buffer: such loads touch no memory and return zeros
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void *)wgt, 0, (int)((long)N * row_b), 0x00020000);

@@ -72,7 +72,7 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
             }
         }
     // ... and what the epilogue adds or rotates by
-    const bool vec16 = (N & 7) == 0 && (epi.kind != kEpiBias || (reinterpret_cast<uintptr_t>(epi.rope.bias) & 15) == 0);
+    const bool vec16 = (N & 7) == 0;
     Ahead<ROPE> ahead[kT][kC][2];
 #pragma unroll
     for (int t = 0; t < kT; t++)

@@ -67,7 +67,7 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
     const int col = (int)threadIdx.x % kCols, row0 = (int)threadIdx.x / kCols;
     const int ch = ch0 + col * 8;
     const bool works = ch < N && row0 < kRowsAtOnce;
-    const bool vec16 = (N & 7) == 0 && (epi.kind != kEpiBias || (reinterpret_cast<uintptr_t>(epi.rope.bias) & 15) == 0);
+    const bool vec16 = (N & 7) == 0;
     constexpr int kIters = (32 * S::kPartBlocks + kRowsAtOnce - 1) / kRowsAtOnce;      // rows of a thread per part
     float muls[8], t_half_mul[TF / S::kPartBlocks][kIters];
 #pragma unroll
