@@ -46,3 +46,64 @@ def test_every_tile_shape_equals_the_int8_kernels(dtype, m, k, n):
         freqs = torch.stack([torch.cos(ang), torch.sin(ang)], dim=-1).contiguous()
         turned = quest.rope_interleaved_(want.clone().view(-1, 50, n), freqs, rot, 32).view(m, n)
         assert torch.equal(quest.fused_matmul_dequantize_e2m3(ta, tb, a_mul, b_mul, k, rope=(freqs, rot, 32)), turned)
+
+
+def _operands(m, k, n, dtype):
+    import quest_amd as quest
+    g = torch.Generator(device=DEV).manual_seed(m + k + n)
+    ta, tb = (quest.int4_to_e2m3_tiles(torch.randint(0, 256, (r, k // 2), generator=g, device=DEV, dtype=torch.uint8)) for r in (m, n))
+    a_mul, b_mul = ((torch.rand(r, 1, generator=g, device=DEV) * 0.09 + 0.01).to(dtype) for r in (m, n))
+    return quest, g, ta, tb, a_mul, b_mul
+
+
+def _with_bias(quest, ta, tb, a_mul, b_mul, bias, k):
+    from quest_amd import _lib
+    m, n = a_mul.numel(), b_mul.numel()
+    out = torch.empty(m, n, dtype=a_mul.dtype, device=DEV)
+    _lib.check(_lib.load().quest_fused_matmul_dequantize_bias_e2m3(
+        out.data_ptr(), ta.data_ptr(), tb.data_ptr(), a_mul.data_ptr(), b_mul.data_ptr(), bias.data_ptr(), m, k, n, _lib.DTYPE_CODE[a_mul.dtype],
+        torch.cuda.current_stream().cuda_stream), 'bias_e2m3')
+    return out
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('m,k,n', SHAPES + [(4100, 256, 2307), (4100, 256, 4099)])
+def test_bias_epilogue_of_every_tile_shape(dtype, m, k, n):
+    quest, g, ta, tb, a_mul, b_mul = _operands(m, k, n, dtype)
+    bias = torch.randn(n, generator=g, device=DEV).to(dtype)
+    plain = quest.fused_matmul_dequantize_e2m3(ta, tb, a_mul, b_mul, k)
+    assert torch.equal(_with_bias(quest, ta, tb, a_mul, b_mul, bias, k), plain + bias)
+
+
+def _is_large(m, k, n):
+    import ctypes
+    from quest_amd import _lib
+    plan = (ctypes.c_int * 8)()
+    _lib.check(_lib.load().quest_e2m3_gemm_plan(m, k, n, torch.cuda.get_device_properties(0).multi_processor_count, plan), 'plan')
+    return list(plan[4:6]) == [256, 256]
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('m,n', [(4100, 2307), (4100, 4099), (4100, 2312), (16900, 520)])
+def test_residual_epilogue_of_the_large_tiles(dtype, m, n):
+    """Odd widths (element by element), ragged ones and ragged last token tiles."""
+    k = 256
+    assert _is_large(m, k, n)
+    quest, g, ta, tb, a_mul, b_mul = _operands(m, k, n, dtype)
+    res = (torch.randn(m, n, generator=g, device=DEV) * 30).to(dtype)
+    plain = quest.fused_matmul_dequantize_e2m3(ta, tb, a_mul, b_mul, k)
+    assert torch.equal(quest.fused_matmul_dequantize_e2m3(ta, tb, a_mul, b_mul, k, out=res.clone(), add_to_out=True), res + plain)
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('batch,seq,n,rot,head_dim', [(5, 900, 2312, 1536, 32), (5, 900, 2312, 2304, 96), (7, 611, 2088, 192, 64), (100, 41, 2304, 2304, 128)])
+def test_rotary_epilogue_of_the_large_tiles(dtype, batch, seq, n, rot, head_dim):
+    """Sequences that end inside a tile, narrow heads, a last channel tile that is partly rotated or not at all."""
+    m, k = batch * seq, 256
+    assert _is_large(m, k, n)
+    quest, g, ta, tb, a_mul, b_mul = _operands(m, k, n, dtype)
+    ang = torch.rand(seq, head_dim // 2, generator=g, device=DEV) * 6.283
+    freqs = torch.stack([torch.cos(ang), torch.sin(ang)], dim=-1).contiguous()
+    plain = quest.fused_matmul_dequantize_e2m3(ta, tb, a_mul, b_mul, k)
+    want = quest.rope_interleaved_(plain.view(batch, seq, n), freqs, rot, head_dim).view(m, n)
+    assert torch.equal(quest.fused_matmul_dequantize_e2m3(ta, tb, a_mul, b_mul, k, rope=(freqs, rot, head_dim)), want)

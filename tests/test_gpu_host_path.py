@@ -147,3 +147,97 @@ def test_other_threads_run_during_native_calls(call):
             sys.setswitchinterval(interval)
             thread.join()
     assert after - before > 10
+
+
+class _Recorder:
+    """The native module with what it returns to whom."""
+
+    def __init__(self, real):
+        self.real, self.calls = real, []
+
+    def __getattr__(self, name):
+        def call(*a):
+            self.calls.append((name, getattr(self.real, name)(*a)))
+            return self.calls[-1][1]
+        return call
+
+    def took(self):
+        return [name for name, result in self.calls if result is not None]
+
+
+@pytest.fixture
+def native(monkeypatch):
+    from quest_amd import _lib, api
+    recorder = _Recorder(_lib.host)
+    monkeypatch.setattr(api, 'host', recorder)
+    return recorder
+
+
+def _calls(m, k, n, dtype, given):
+    """Every function of the native module as a call of the package on fixed inputs: name -> function returning all outputs."""
+    import quest_amd as quest
+    from quest_amd import harness
+    g = torch.Generator(device=DEV).manual_seed(m + k + n)
+    x = torch.randn(m, k, device=DEV, generator=g).to(dtype)
+    a, b = (torch.randint(0, 256, (r, k // 2), device=DEV, generator=g, dtype=torch.uint8) for r in (m, n))
+    a_mul, b_mul = ((torch.rand(r, 1, device=DEV, generator=g) + 0.5).to(dtype) for r in (m, n))
+    a_add, b_add = (torch.randint(-99, 99, (r, 1), device=DEV, generator=g, dtype=torch.int32) for r in (m, n))
+    c = torch.randint(-9999, 9999, (m, n), device=DEV, generator=g, dtype=torch.int32)
+    out = lambda *shape, t=dtype: torch.empty(*shape, dtype=t, device=DEV) if given else None      # noqa: E731
+
+    def quantize():
+        y, outs = x.clone(), (torch.empty(m, k, dtype=torch.int8, device=DEV), torch.empty(m, k // 2, dtype=torch.uint8, device=DEV),
+                              torch.empty(m, 1, dtype=torch.int32, device=DEV))
+        return quest.quantize_int4(y, a_mul, *(outs if given else (None, outs[1], None)), do_dequantize=given)
+    return dict(
+        gemm=lambda: quest.fused_matmul_dequantize_int4_int4t_bf16(a, b, a_add, b_add, a_mul, b_mul, out(m, n)),
+        matmul_int32=lambda: quest.matmul_int4_int4t_int32(a, b, out(m, n, t=torch.int32)),
+        find_scale=lambda: quest.find_scale_int4(x, out(m, 1)),
+        quantize=quantize,
+        add_mul_vv=lambda: quest.add_mul_vv(a_add, a_mul, b_add, b_mul, c, out(m, n)),
+        hadamard128=lambda: quest.hadamard128(x, out(m, k), 2. ** -3.5),
+        hadamard_quantize=lambda: quest.hadamard_quantize_int4(x, out(m, 1), out(m, k // 2, t=torch.uint8), out(m, 1, t=torch.int32), scale_rule='absmax'),
+        pack_weight=lambda: harness.preprocess_weight(x, use_hadamard=given, w_scale_mode='absmax' if given else 'rms')[:3],
+        linear=lambda: harness.linear_forward(x, b, b_mul, b_add, use_hadamard=given, out=out(m, n)))
+
+
+NAMES = ['gemm', 'matmul_int32', 'find_scale', 'quantize', 'add_mul_vv', 'hadamard128', 'hadamard_quantize', 'pack_weight', 'linear']
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('given', [False, True])
+@pytest.mark.parametrize('m,k,n', [(37, 256, 72), (1, 384, 33), (333, 1152, 1001)])
+@pytest.mark.parametrize('name', NAMES)
+def test_every_call_goes_native_and_equals_python(native, monkeypatch, name, m, k, n, given, dtype):
+    from quest_amd import api
+    call = _calls(m, k, n, dtype, given)[name]
+    got = call()
+    assert native.took() == [name]
+    monkeypatch.setattr(api, 'host', _DeclinesAll())
+    want = call()
+    for x, y in zip(*((r if isinstance(r, tuple) else (r,)) for r in (got, want))):
+        assert (x is None and y is None) or (torch.equal(x, y) and x.shape == y.shape and x.dtype == y.dtype)
+
+
+def test_which_layers_and_blocks_go_native(native):
+    """Plain ones do, down to the last logits; a strided input and a bias of another type do not."""
+    from quest_amd import harness, llama
+    layer = harness.Linear4bit.from_weight(torch.randn(72, 256, device=DEV).bfloat16(), torch.zeros(72, device=DEV).bfloat16())
+    x = torch.randn(3, 512, device=DEV).bfloat16()
+    native.calls.clear()
+    layer(x[:, :256].contiguous())
+    assert native.took() == ['linear']
+    native.calls.clear()
+    layer(x[:, ::2])
+    assert [c for c in native.calls if c[0] == 'linear'][0][1] is None
+    native.calls.clear()
+    layer.bias = torch.nn.Parameter(layer.bias.float(), requires_grad=False)
+    layer(x[:, :256].contiguous())
+    assert [c for c in native.calls if c[0] == 'linear'][0][1] is None
+    net = llama.quantize_model(llama.Llama(llama.LlamaConfig(n_layer=3, n_embd=1024, n_head=8, vocab_size=64)).to(DEV).bfloat16().eval(), 'int4',
+                               fuse_producers=True)
+    for batch, seq in ((1, 1), (2, 37), (3, 100), (9, 500)):
+        native.calls.clear()
+        with torch.no_grad():
+            net(torch.randint(0, 64, (batch, seq), device=DEV))
+        assert native.took() == ['block'] * 3 + ['last_logits']

@@ -676,3 +676,14 @@ def test_absmax_rows_with_a_nan(quest, dtype, k, from_fp32):
     assert torch.equal(harness.unpack_int4(packed), codes)
     assert torch.equal(total, codes.sum(-1, keepdim=True, dtype=torch.int32))
     assert torch.equal(total[8], clean_sum[8])
+
+
+def test_gated_unit_has_torchs_bits_for_every_bf16_gate(quest):
+    """silu(gate) of all 65536 bit patterns, the product with 1 (exact): the kernels' fast exponential and reciprocal round as torch's
+    (NaN for NaN)."""
+    gate = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).view(512, 128).to(DEV)
+    act = torch.empty(512, 128, dtype=torch.bfloat16, device=DEV)
+    quest.silu_mul_hadamard_quantize_int4(torch.cat([gate, torch.ones_like(gate)], 1), x_act=act)
+    want = torch.nn.functional.silu(gate)
+    assert torch.equal(act.isnan(), want.isnan())
+    assert torch.equal(act.nan_to_num(7.), want.nan_to_num(7.))
