@@ -113,6 +113,14 @@ def ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
     return ctypes.c_void_p(t.data_ptr())
 
 
+def wrote(*tensors: torch.Tensor | None) -> None:
+    """Counts a kernel's write into tensors of the caller's, as torch's own in-place calls do: one may be a packed weight, whose
+    derived forms (harness.Linear4bit.lay_out_tiles) are valid by that count."""
+    for t in tensors:
+        if t is not None and not t.is_inference():
+            torch.autograd.graph.increment_version(t)
+
+
 def stream_of(t: torch.Tensor) -> ctypes.c_void_p:
     """The HIP stream torch currently launches on for the tensor's device."""
     return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)

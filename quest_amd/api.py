@@ -16,7 +16,7 @@ import ctypes
 import torch
 
 from . import _lib
-from ._lib import DTYPE_CODE, check, host, ptr, require_gpu, stream_of
+from ._lib import DTYPE_CODE, check, host, ptr, require_gpu, stream_of, wrote
 
 _FLOAT16S = (torch.bfloat16, torch.float16)
 HADAMARD_ENTRY = 181. / 2048.        # bf16(2**-3.5) == fp16(2**-3.5): what the reference's matrix holds
@@ -246,6 +246,7 @@ def find_scale_int4(
     with torch.cuda.device(dev):
         check(_lib.load().quest_find_scale_int4(ptr(scale), ptr(x), x.size(1), x.size(0), DTYPE_CODE[x.dtype],
                                                 stream_of(x)), 'find_scale_int4')
+    wrote(scale)
     return scale
 
 
@@ -275,6 +276,7 @@ def quantize_int4(
         check(_lib.load().quest_quantize_int4(ptr(x), ptr(scale), ptr(x_int), ptr(x_int_packed), ptr(x_int_row_sum),
                                               x.size(1), x.size(0), int(bool(do_dequantize)), DTYPE_CODE[x.dtype],
                                               stream_of(x)), 'quantize_int4')
+    wrote(x_int_packed, x_int_row_sum)
     return x, x_int, x_int_packed, x_int_row_sum
 
 
@@ -363,6 +365,7 @@ def hadamard_quantize_int4(
         check(_lib.load().quest_hadamard_quantize_int4_rule(ptr(x), ptr(scale), ptr(x_int_packed), ptr(x_int_row_sum),
                                                             ptr(x_had), k, m, float(hadamard_scale), rule,
                                                             DTYPE_CODE[x.dtype], stream_of(x)), 'hadamard_quantize_int4')
+    wrote(scale, x_int_packed, x_int_row_sum)
     return scale, x_int_packed, x_int_row_sum
 
 
@@ -404,6 +407,7 @@ def rmsnorm_hadamard_quantize_int4(
         check(_lib.load().quest_rmsnorm_hadamard_quantize_int4(
             ptr(x), ptr(norm_weight), float(eps), ptr(scale), ptr(x_int_packed), ptr(x_int_row_sum), ptr(x_had),
             ptr(x_norm), k, m, float(hadamard_scale), DTYPE_CODE[x.dtype], stream_of(x)), 'rmsnorm_hadamard_quantize_int4')
+    wrote(scale, x_int_packed, x_int_row_sum)
     return scale, x_int_packed, x_int_row_sum
 
 
@@ -430,6 +434,7 @@ def add_rmsnorm_hadamard_quantize_int4(
         check(_lib.load().quest_add_rmsnorm_hadamard_quantize_int4(
             ptr(x), ptr(branch), ptr(norm_weight), float(eps), ptr(scale), ptr(x_int_packed), ptr(x_int_row_sum),
             k, m, float(hadamard_scale), DTYPE_CODE[x.dtype], stream_of(x)), 'add_rmsnorm_hadamard_quantize_int4')
+    wrote(scale, x_int_packed, x_int_row_sum)
     return scale, x_int_packed, x_int_row_sum
 
 
@@ -456,6 +461,7 @@ def silu_mul_hadamard_quantize_int4(
         check(_lib.load().quest_silu_mul_hadamard_quantize_int4(
             ptr(gate_up), ptr(scale), ptr(x_int_packed), ptr(x_int_row_sum), ptr(x_had), ptr(x_act), k, m,
             float(hadamard_scale), DTYPE_CODE[gate_up.dtype], stream_of(gate_up)), 'silu_mul_hadamard_quantize_int4')
+    wrote(scale, x_int_packed, x_int_row_sum)
     return scale, x_int_packed, x_int_row_sum
 
 
@@ -587,6 +593,7 @@ def hadamard_quantize_e2m3(
         int4_to_e2m3_tiles(packed, x_tiles)
     else:
         check(rc, 'hadamard_quantize_e2m3')
+    wrote(scale, x_int_packed, x_int_row_sum)
     return scale, x_tiles
 
 
@@ -612,6 +619,7 @@ def rmsnorm_hadamard_quantize_e2m3(x, norm_weight, eps, scale=None, x_tiles=None
         check(_lib.load().quest_rmsnorm_hadamard_quantize_e2m3(
             ptr(x), ptr(norm_weight), float(eps), ptr(scale), ptr(x_tiles), ptr(x_norm), k, m, float(hadamard_scale),
             DTYPE_CODE[x.dtype], stream_of(x)), 'rmsnorm_hadamard_quantize_e2m3')
+    wrote(scale)
     return scale, x_tiles
 
 
@@ -628,6 +636,7 @@ def add_rmsnorm_hadamard_quantize_e2m3(x, branch, norm_weight, eps, scale=None, 
         check(_lib.load().quest_add_rmsnorm_hadamard_quantize_e2m3(
             ptr(x), ptr(branch), ptr(norm_weight), float(eps), ptr(scale), ptr(x_tiles), k, m, float(hadamard_scale),
             DTYPE_CODE[x.dtype], stream_of(x)), 'add_rmsnorm_hadamard_quantize_e2m3')
+    wrote(scale)
     return scale, x_tiles
 
 
@@ -644,4 +653,5 @@ def silu_mul_hadamard_quantize_e2m3(gate_up, scale=None, x_tiles=None, x_act=Non
         check(_lib.load().quest_silu_mul_hadamard_quantize_e2m3(
             ptr(gate_up), ptr(scale), ptr(x_tiles), ptr(x_act), k, m, float(hadamard_scale), DTYPE_CODE[gate_up.dtype],
             stream_of(gate_up)), 'silu_mul_hadamard_quantize_e2m3')
+    wrote(scale)
     return scale, x_tiles

@@ -92,6 +92,12 @@ int on(c10::Device dev, F &&launch) {
 int64_t up(int64_t bytes) { return (bytes + 255) & ~(int64_t)255; }
 bool at(const at::Tensor *t, unsigned bytes) { return t == nullptr || (reinterpret_cast<uintptr_t>(t->data_ptr()) & (bytes - 1)) == 0; }
 
+// Counts a write into a tensor of the caller's, as torch's own in-place calls do: `unchanged` below goes by that count, and the tensor may
+// be a layer's buffer.
+void wrote(const at::Tensor &t) {
+    if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
+}
+
 // Whether `t` is the tensor that something was derived from and still holds what it held: its address and version then are given.
 bool unchanged(PyObject *t, PyObject *source, PyObject *address, PyObject *version) {
     if (t != source || !THPVariable_CheckExact(t)) return false;
@@ -274,6 +280,7 @@ PyObject *hadamard_quantize(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
                                                  nullptr, (int)k, (int)m, (float)had_scale, (int)rule, dtype_code(type), st);
     });
     if (rc != QUEST_OK) return declined();
+    wrote(scale), wrote(packed), wrote(row_sum);
     PyObject *t = PyTuple_New(3);
     if (t == nullptr) return nullptr;
     PyTuple_SET_ITEM(t, 0, a[1] != Py_None ? ref(a[1]) : wrap(std::move(scale)));
@@ -348,6 +355,7 @@ PyObject *find_scale(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         return quest_find_scale_int4(scale.data_ptr(), x->data_ptr(), (int)k, (int)m, dtype_code(x->scalar_type()), st);
     });
     if (rc != QUEST_OK) return declined();
+    wrote(scale);
     return a[1] != Py_None ? ref(a[1]) : wrap(std::move(scale));
     END_HANDLE_TH_ERRORS
 }
@@ -373,6 +381,8 @@ PyObject *quantize(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
                                    (int)m, dequantize, dtype_code(x->scalar_type()), st);
     });
     if (rc != QUEST_OK) return declined();
+    for (const at::Tensor *t : {packed, row_sum})
+        if (t != nullptr) wrote(*t);
     Py_RETURN_TRUE;
     END_HANDLE_TH_ERRORS
 }

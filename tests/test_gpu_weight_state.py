@@ -94,6 +94,34 @@ def test_writes_into_the_buffer_show(harness, inference):
         assert layer.tiles_for(M) is not None and torch.equal(layer(rows()), want)
 
 
+@pytest.mark.parametrize('native', [True, False])
+@pytest.mark.parametrize('entry', ['quantize_int4', 'hadamard_quantize_int4', 'hadamard_quantize_e2m3'])
+def test_quantisers_write_into_the_buffers(harness, monkeypatch, entry, native):
+    """Weights packed straight into a layer's buffers by the quantisers, whose writes torch does not see by itself."""
+    api = harness.quest
+    layer, fresh = harness.Linear4bit.from_weight(weight(6), use_hadamard=False), weight(7)
+    want = on_int8(harness, harness.Linear4bit.from_weight(fresh, use_hadamard=False), rows())
+    if not native:
+        class Declines:
+            def __getattr__(self, _name):
+                return lambda *_: None
+        monkeypatch.setattr(api, 'host', Declines())
+    sums = torch.empty(N, 1, dtype=torch.int32, device=DEV)
+    before = layer.w_scale._version
+    if entry == 'quantize_int4':
+        api.find_scale_int4(fresh, layer.w_scale)
+        api.quantize_int4(fresh, layer.w_scale, x_int_packed=layer.w_int_packed, x_int_row_sum=sums)
+    elif entry == 'hadamard_quantize_int4':
+        api.hadamard_quantize_int4(fresh, layer.w_scale, layer.w_int_packed, sums, hadamard_scale=0.)
+    else:
+        api.hadamard_quantize_e2m3(fresh, layer.w_scale, None, layer.w_int_packed, sums, hadamard_scale=0.)
+    layer.w_add.copy_(sums + K // 2)
+    assert layer.w_scale._version > before
+    assert torch.equal(layer(rows()), want)
+    layer.lay_out_tiles()
+    assert layer.tiles_for(M) is not None and torch.equal(layer(rows()), want)
+
+
 def test_first_call_inside_a_capture(harness):
     """Warmed with one token only, captured at many, and called eagerly before and between the replays."""
     layer, x = harness.Linear4bit.from_weight(weight(4), use_hadamard=True), rows()
