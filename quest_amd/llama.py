@@ -143,7 +143,9 @@ class LlamaMLP(nn.Module):
         return {**self.__dict__, 'glu_tiles': None, '_glu_of': None}
 
     def __setstate__(self, state):
-        super().__setstate__(state)
+        super().__setstate__({'_glu_of': None, **state})            # (not in a module that was saved before there was one)
+        if _renew_swiglu not in self._load_state_dict_post_hooks.values():
+            self.register_load_state_dict_post_hook(_renew_swiglu)
         _renew_swiglu(self)
 
     def swiglu_quantized(self, a_scale, a_int_packed, a_int_row_sum):

@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from oracle import llama_oracle as lo
-from quest_amd import checkpoint, llama
+from quest_amd import checkpoint, harness, llama
 
 CFG = dict(n_layer=2, n_embd=256, n_head=4, vocab_size=384, sequence_length=48)
 
@@ -186,3 +186,26 @@ def test_dense_forward_runs_its_own_norm_and_head_without_the_native_module(monk
     with torch.no_grad():
         last, every = model(ids)['logits'], model(ids, all_logits=True)['logits']
     assert torch.allclose(last, every[:, -1:], rtol=1e-4, atol=1e-5)
+
+
+def test_a_module_saved_before_its_rows_were_tracked_loads():
+    """Whole modules saved when LlamaMLP had no record of what the interleaved rows were made from: restored with fresh ones, which
+    follow a later load."""
+    cfg = llama.LlamaConfig(**CFG)
+
+    def mlp(seed):
+        m = llama.LlamaMLP(cfg)
+        m.w12 = harness.Linear4bit.empty(cfg.n_embd, 2 * cfg.hidden_dim, dtype=torch.bfloat16)
+        m.w1 = m.w2 = None
+        m.w12.w_int_packed.random_(generator=torch.Generator().manual_seed(seed))
+        m.enable_swiglu_epilogue()
+        return m
+
+    old, other = mlp(1), mlp(2)
+    state = {k: v for k, v in old.__getstate__().items() if k != '_glu_of'}
+    state['_load_state_dict_post_hooks'] = type(state['_load_state_dict_post_hooks'])()
+    new = llama.LlamaMLP.__new__(llama.LlamaMLP)
+    new.__setstate__(state)
+    assert all(torch.equal(a, b) for a, b in zip(new.kept_glu(), old.glu))
+    new.load_state_dict(other.state_dict())
+    assert all(torch.equal(a, b) for a, b in zip(new.kept_glu(), other.glu))
