@@ -91,9 +91,9 @@ def _scales_in_pairs(scale) -> bool:
     return scale is None or scale.data_ptr() % 4 == 0
 
 
-def weight_tiles(w_int_packed: torch.Tensor) -> torch.Tensor:
+def weight_tiles(w_int_packed: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:
     """The E2M3 tiles of packed weight codes (N, K/2): the FP6 kernel's operand form (1.5 x the packed bytes)."""
-    return quest.int4_to_e2m3_tiles(w_int_packed)
+    return quest.int4_to_e2m3_tiles(w_int_packed, out)
 
 
 def _check_backend(backend: str) -> None:
@@ -271,9 +271,10 @@ class Linear4bit(nn.Module):
         Done where the buffers get their content -- packing, `load_state_dict`, a move to another device, a copy -- on the stream
         that writes them, so whoever may read the buffers may read the tiles, and no forward call, on whatever stream or
         under capture, has anything to build.  After writing into `w_int_packed` by hand, call it again: until then the layer runs on
-        its packed codes (the same bits).  Nothing is kept for a layer that the FP6 kernels do not take, or while MATRIX_PATH is
-        'int8'."""
-        self._tiles = None
+        its packed codes (the same bits), but for a graph captured before, which reads the tiles.  They are rewritten in place while
+        the buffer stays where it is, so that such a graph follows a reload as it does on packed codes.  Nothing is kept for a
+        layer that the FP6 kernels do not take, or while MATRIX_PATH is 'int8'."""
+        before, self._tiles = self._tiles, None
         with torch.inference_mode(False), torch.no_grad():
             for name, t in self._buffers.items():
                 if type(t) is torch.Tensor and t.is_inference():     # (it would not show later writes)
@@ -282,7 +283,8 @@ class Linear4bit(nn.Module):
             if type(w) is not torch.Tensor or not w.is_cuda or w.dim() != 2 or not w.is_contiguous():
                 return
             if MATRIX_PATH == 'fp6' and e2m3_fits(w.size(1) * 2, w.size(0)):
-                self._tiles = (weight_tiles(w), w, w.data_ptr(), w._version)
+                in_place = before is not None and before[1] is w and before[2] == w.data_ptr()
+                self._tiles = (weight_tiles(w, before[0] if in_place else None), w, w.data_ptr(), w._version)
 
     def _kept_tiles(self):
         """The tiles of what `w_int_packed` holds now, or None."""

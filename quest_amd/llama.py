@@ -112,18 +112,25 @@ class LlamaMLP(nn.Module):
     def enable_swiglu_epilogue(self):
         """A second copy of the fused gate/up weights with the rows interleaved in eights (four gate rows, then the four
         up rows of the same outputs; `quest.swiglu_interleave_rows`), which lets the GEMM apply silu(gate) * up in
-        its epilogue, and its E2M3 tiles in place of w12's own (`Linear4bit.lay_out_tiles` says when and why they are made).
-        Plain tensors, not buffers: they are derived data and stay out of checkpoints."""
+        its epilogue, and its E2M3 tiles in place of w12's own (`Linear4bit.lay_out_tiles` says when and why they are made, and when in
+        place).  Plain tensors, not buffers: they are derived data and stay out of checkpoints."""
         w = self.w12
-        p = quest.swiglu_interleave_rows(w.w_int_packed.size(0) // 2, device=w.w_int_packed.device)
-        glu = (w.w_int_packed[p].contiguous(), w.w_scale[p].contiguous(), w.w_add[p].contiguous())
-        rows, half_k = glu[0].shape
-        fits = harness.MATRIX_PATH == 'fp6' and glu[0].is_cuda and harness.e2m3_fits(2 * half_k, rows)
-        self.glu, self.glu_tiles, self._glu_of = glu, harness.weight_tiles(glu[0]) if fits else None, self._glu_source()
+        now = self._glu_source()
+        in_place = (self.glu is not None and self._glu_of is not None and all(a is b for a, b in zip(now[:3], self._glu_of))
+                    and now[3:6] == self._glu_of[3:6])
+        with torch.inference_mode(False), torch.no_grad():
+            p = quest.swiglu_interleave_rows(w.w_int_packed.size(0) // 2, device=w.w_int_packed.device)
+            glu = tuple(t[p] for t in now[:3])
+            if in_place:
+                glu = tuple(old.copy_(new) for old, new in zip(self.glu, glu))
+            rows, half_k = glu[0].shape
+            fits = harness.MATRIX_PATH == 'fp6' and glu[0].is_cuda and harness.e2m3_fits(2 * half_k, rows)
+            tiles = harness.weight_tiles(glu[0], self.glu_tiles if in_place else None) if fits else None
+        self.glu, self.glu_tiles, self._glu_of = glu, tiles, now
         w._tiles = None
 
     def _glu_source(self):
-        now = [self.w12._buffers.get(name) for name in ('w_int_packed', 'w_scale', 'w_add')]
+        now = (self.w12.w_int_packed, self.w12.w_scale, self.w12.w_add)
         return (*now, *(t.data_ptr() for t in now), *(None if t.is_inference() else t._version for t in now))
 
     def kept_glu(self):

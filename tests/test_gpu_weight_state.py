@@ -139,6 +139,35 @@ def test_first_call_inside_a_capture(harness):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize('inference', [False, True])
+def test_captured_calls_follow_a_reload(harness, inference):
+    """load_state_dict writes the packed codes in place, and so their other forms: a graph captured before it runs the new weights, for a
+    layer and for a fused model (whose gate / up rows are a copy of their own)."""
+    with torch.inference_mode(inference):
+        layer, other = (harness.Linear4bit.from_weight(weight(s), use_hadamard=True) for s in (1, 2))
+    nets, x, ids = (model(1, inference), model(2, inference)), rows(), IDS.to(DEV)
+    calls = ((layer, other, lambda m: m(x)), (*nets, lambda m: m(ids, all_logits=True)['logits']))
+    for kept, new, call in calls:
+        with torch.no_grad():
+            want = call(new).clone()
+            side = torch.cuda.Stream()
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                call(kept)
+            torch.cuda.current_stream().wait_stream(side)
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                out = call(kept)
+            for _ in range(2):                                         # (the second load writes what the first one left in place)
+                with torch.inference_mode(inference):
+                    kept.load_state_dict(new.state_dict())
+                filler = [torch.full((1 << 20,), 0x55, dtype=torch.uint8, device=DEV) for _ in range(32)]      # takes up freed memory
+                graph.replay()
+                torch.cuda.synchronize()
+                assert torch.equal(out, want) and torch.equal(call(kept), want)
+                del filler
+
+
 def test_first_calls_on_two_streams(harness):
     """Both streams wait for the packing stream only."""
     layer, x = harness.Linear4bit.from_weight(weight(5), use_hadamard=True), rows()
