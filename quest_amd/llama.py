@@ -186,8 +186,12 @@ class LlamaMLP(nn.Module):
 
 def _renew_swiglu(mlp: LlamaMLP, _incompatible_keys=None) -> None:
     """The interleaved copy again after w12 got other content (a load, a move, a copy of the module)."""
-    if mlp.glu is not None and mlp.kept_glu() is None:
+    if mlp.glu is None:
+        return
+    if mlp.kept_glu() is None:
         mlp.enable_swiglu_epilogue()
+    else:
+        mlp.w12._tiles = None            # (w12's own, laid out by a move that moved nothing: read by no call)
 
 
 class LlamaAttention(nn.Module):

@@ -168,6 +168,12 @@ def test_captured_calls_follow_a_reload(harness, inference):
                 del filler
 
 
+def test_a_move_to_where_it_is_keeps_one_copy(harness):
+    net = model(1)
+    net.to(DEV)
+    assert all(b.mlp.w12._tiles is None and b.mlp.glu_tiles is not None and b.mlp.kept_glu() is not None for b in net.transformer.h)
+
+
 def test_first_calls_on_two_streams(harness):
     """Both streams wait for the packing stream only."""
     layer, x = harness.Linear4bit.from_weight(weight(5), use_hadamard=True), rows()
