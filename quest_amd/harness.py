@@ -38,12 +38,12 @@ def prefers_e2m3(m: int, k: int, n: int) -> bool:
     """Whether the FP6 kernels are the faster ones for an (m, k) x (n, k) layer on its own, quantiser included, with weights that come
     from HBM (copies of more than 300 MB in turn): 2096 sizes, K 128 to 11008, N 136 to 22016, M 33 to 4096.  The path taken is
     within 0.8 % of the faster one on average (always FP6: 3.0 %) and, from K = 640 on, within 16 % everywhere."""
-    if MATRIX_PATH != 'fp6' or k % 128 or not _tiles_addressable(m, k, n):
+    if m < 49 or k % 128 or MATRIX_PATH != 'fp6' or not _tiles_addressable(m, k, n):      # (a few tokens first: their calls are host-bound)
         return False
     if m > E2M3_SHORT_ROWS_TOKENS:
         return _enough_per_row(k, n)
     # K < 640: as often slower as faster (K = 128: 0.83 at (2000, 22016), 1.47 at (700, 11008); K = 512: 0.88 to 1.41)
-    if m < 49 or k < 640:
+    if k < 640:
         return False
     # Some tens of tokens: the weights are the cost, and the tiles are 1.5 x the codes' bytes.  (INT8 / FP6 time: (33, 11008, 11008)
     # 0.72, (64, 4096, 11008) 0.88, (40, 1024, 4096) 0.96; (64, 2048, 2048) 1.06, (64, 11008, 1024) 1.27.)  More than 16384
