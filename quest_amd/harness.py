@@ -248,13 +248,14 @@ class Linear4bit(nn.Module):
         # codes from the fp32 transform instead of its 16-bit rounding (see linear_forward); set before packing a weight
         self.quantize_from_fp32 = getattr(self, 'quantize_from_fp32', False)
 
-    def _install(self, weight: torch.Tensor, bias) -> None:
+    def _install(self, weight: torch.Tensor, bias, lay_out: bool = True) -> None:
         """Pack `weight` (N, K) and keep `bias` (a tensor, a parameter or None) as a frozen parameter."""
         with torch.inference_mode(False), torch.no_grad():           # buffers with a version counter: see _kept_tiles
             packed, scale, add, _ = preprocess_weight(weight=weight, use_hadamard=self.use_hadamard,
                                                       quantize_from_fp32=self.quantize_from_fp32)
         self._set_buffers(weight.shape, weight.dtype, packed, scale, add)
-        self.lay_out_tiles()
+        if lay_out:
+            self.lay_out_tiles()
         if bias is None:
             self.bias = None
         else:
@@ -328,13 +329,13 @@ class Linear4bit(nn.Module):
 
     @classmethod
     def from_weight(cls, weight: torch.Tensor, bias: torch.Tensor = None, use_hadamard: bool = False,
-                    quantize_from_fp32: bool = False) -> 'Linear4bit':
-        """Pack an existing (N, K) weight instead of a random one."""
+                    quantize_from_fp32: bool = False, lay_out: bool = True) -> 'Linear4bit':
+        """Pack an existing (N, K) weight instead of a random one.  lay_out: keep its E2M3 tiles as well (`lay_out_tiles`)."""
         self = cls.__new__(cls)
         nn.Module.__init__(self)
         self.quantize_from_fp32 = bool(quantize_from_fp32)
         self._configure(use_hadamard, False)
-        self._install(weight, bias)
+        self._install(weight, bias, lay_out)
         return self
 
     @classmethod

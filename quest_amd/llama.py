@@ -463,9 +463,9 @@ class Llama(nn.Module):
                 and _as_built(self.transformer.ln_f, RMSNorm) and _as_built(self.lm_head, nn.Linear) and self.lm_head.bias is None)
 
 
-def _pack(linear: nn.Linear, use_hadamard: bool, use_noop: bool, from_fp32: bool = False) -> harness.Linear4bit:
+def _pack(linear: nn.Linear, use_hadamard: bool, use_noop: bool, from_fp32: bool = False, lay_out: bool = True) -> harness.Linear4bit:
     m = harness.Linear4bit.from_weight(linear.weight.data, bias=None if linear.bias is None else linear.bias.data,
-                                       use_hadamard=use_hadamard, quantize_from_fp32=from_fp32)
+                                       use_hadamard=use_hadamard, quantize_from_fp32=from_fp32, lay_out=lay_out)
     m.use_noop = use_noop
     return m
 
@@ -488,6 +488,12 @@ def quantize_model(model: Llama, mode: str = 'int4', use_hadamard: bool = True, 
     if mode not in ('int4', 'noop'):
         raise NotImplementedError(mode)
     noop = mode == 'noop'
+    # the producer-fused kernels exist for the Hadamard variant, rows up to 32768 and the fused gate/up layout
+    # (in no-op mode the fused blocks keep their producers -- norms, residual additions, quantisers, rotary kernel --
+    # and only the GEMMs return zeros: the twin that prices the GEMMs of the producer-fused model)
+    fused = bool(fuse_producers and use_hadamard and fuse_gate_up and
+                 model.config.n_embd <= 32768 and model.config.hidden_dim <= 32768)
+    interleaved = fused and swiglu_epilogue and model.config.hidden_dim % 4 == 0
     for block in model.transformer.h:
         block.attn.c_attn = _pack(block.attn.c_attn, use_hadamard, noop, quantize_from_fp32)
         block.attn.c_proj = _pack(block.attn.c_proj, use_hadamard, noop, quantize_from_fp32)
@@ -496,23 +502,19 @@ def quantize_model(model: Llama, mode: str = 'int4', use_hadamard: bool = True, 
             both = nn.Linear(mlp.w1.in_features, 2 * mlp.w1.out_features, bias=False, device=mlp.w1.weight.device,
                              dtype=mlp.w1.weight.dtype)
             both.weight.data = torch.cat([mlp.w1.weight.data, mlp.w2.weight.data], dim=0)
-            mlp.w12 = _pack(both, use_hadamard, noop, quantize_from_fp32)
+            mlp.w12 = _pack(both, use_hadamard, noop, quantize_from_fp32, lay_out=not interleaved)      # (see enable_swiglu_epilogue)
             mlp.w1 = mlp.w2 = None
         else:
             mlp.w1 = _pack(mlp.w1, use_hadamard, noop, quantize_from_fp32)
             mlp.w2 = _pack(mlp.w2, use_hadamard, noop, quantize_from_fp32)
         mlp.c_proj = _pack(mlp.c_proj, use_hadamard, noop, quantize_from_fp32)
-        # the producer-fused kernels exist for the Hadamard variant, rows up to 32768 and the fused gate/up layout
-        # (in no-op mode the fused blocks keep their producers -- norms, residual additions, quantisers, rotary kernel --
-        # and only the GEMMs return zeros: the twin that prices the GEMMs of the producer-fused model)
         block.attn.fused_rope = bool(fuse_producers)
-        block.fuse_producers = bool(fuse_producers and use_hadamard and fuse_gate_up and
-                                    model.config.n_embd <= 32768 and model.config.hidden_dim <= 32768)
+        block.fuse_producers = fused
         if fuse_producers and not block.fuse_producers:
             import warnings
             warnings.warn('quantize_model: fuse_producers asked for, but this configuration (no Hadamard, separate gate / up '
                           'projections or rows over 32768) has no producer-fused kernels: the blocks run with torch glue')
-        if block.fuse_producers and swiglu_epilogue and model.config.hidden_dim % 4 == 0:
+        if interleaved:
             mlp.enable_swiglu_epilogue()
     return model
 

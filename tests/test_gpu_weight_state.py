@@ -174,6 +174,14 @@ def test_a_move_to_where_it_is_keeps_one_copy(harness):
     assert all(b.mlp.w12._tiles is None and b.mlp.glu_tiles is not None and b.mlp.kept_glu() is not None for b in net.transformer.h)
 
 
+def test_packing_a_fused_model_lays_out_what_it_keeps(harness, monkeypatch):
+    made, convert = [], harness.weight_tiles
+    monkeypatch.setattr(harness, 'weight_tiles', lambda *a: made.append(convert(*a)) or made[-1])
+    net = model(1)
+    kept = [t for b in net.transformer.h for t in (b.attn.c_attn._kept_tiles(), b.attn.c_proj._kept_tiles(), b.mlp.glu_tiles, b.mlp.c_proj._kept_tiles())]
+    assert len(made) == len(kept) and {t.data_ptr() for t in made} == {t.data_ptr() for t in kept}
+
+
 def test_first_calls_on_two_streams(harness):
     """Both streams wait for the packing stream only."""
     layer, x = harness.Linear4bit.from_weight(weight(5), use_hadamard=True), rows()
