@@ -3,7 +3,8 @@
 //
 // Why: a layer at a handful of tokens is 7 us of GPU work in two launches, and its Python host path (asserts, ctypes
 // conversions, device context, one allocation per output) took 36 us per call, so every small call ran at the speed of the
-// interpreter.  The same checks and launches from here take 6-8 us, most of it the two launches.
+// interpreter.  From here a call takes 10.6 us to issue, module call included (profiles/timed_layer_calls.md): that, and not the GPU's
+// 6.3 us for both launches in a graph, still bounds one token at K = N = 4096.
 //
 // Contract of every function: either the call is the plain case -- exact torch tensors on one GPU, contiguous, right types, sizes
 // and alignment, accepted by the library -- and everything is launched, or None comes back with nothing launched and the
