@@ -394,6 +394,14 @@ int quest_rmsnorm_rows(void *out, const void *x, const void *branch, const void 
  */
 int quest_dense_rows(void *out, const void *x, const void *weight, int size_m, int size_k, int size_n, int dtype, void *stream);
 
+/*
+ * Causal attention on a fused projection's rows: qkv (batch, seq, 3 * n_head * head_dim) holds q, k and v one after the other, heads
+ * side by side; out (batch, seq, n_head * head_dim) = softmax(q k^T / sqrt(head_dim)) v over each row's own and earlier positions, in
+ * fp32 with the probabilities rounded to dtype in front of the second product (src/models/llama.py:150-163).  head_dim 64 or
+ * 128 and rows of a sequence below 2 GiB (QUEST_ERR_UNSUPPORTED otherwise, nothing launched); pointers 16-byte aligned.
+ */
+int quest_causal_attention(void *out, const void *qkv, int batch, int seq, int n_head, int head_dim, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -59,6 +59,7 @@ SIGNATURES = {
     'quest_pack_weight_int4': [_vp, _vp, _vp, _vp, _i, _i, _f, _i, _i, _vp],
     'quest_rmsnorm_rows': [_vp, _vp, _vp, _vp, _f, _i, ctypes.c_long, _i, _i, _vp],
     'quest_dense_rows': [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
+    'quest_causal_attention': [_vp, _vp, _i, _i, _i, _i, _i, _vp],
     'quest_silu_mul_hadamard_quantize_e2m3': [_vp, _vp, _vp, _vp, _i, _i, _f, _i, _vp],
 }
 # entry points that do not return an int status

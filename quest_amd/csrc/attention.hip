@@ -1,0 +1,385 @@
+// Causal attention of a decoder block on the fused QKV projection's output, head dimensions 64 and 128
+// (src/models/llama.py:150-163 of the reference, which calls torch's scaled_dot_product_attention).
+//
+// The block's next step is a 4-bit quantiser: one unit in the last place of an attention output moves a code now and then, and
+// twelve layers of such quantisers turn that into a visible change of a model's logits.  So the order of every fp32 operation is
+// fixed, and it is the order whose outputs equal torch's own kernel on this card bit for bit (tests/test_gpu_attention.py over
+// sequences of 1 to 2048): keys are taken BN at a time, s = (q k) * fp32(log2 e / sqrt(d)) with the product rounded first,
+// p = exp2(s - m), l = fma(l, alpha, sum p), p rounded to dtype for the second product, output * (1 / l).  BN and the two orders of
+// a step are chosen by the length alone (launch): a step wholly below a block of BM complete query rows ("full") sums a lane's
+// p in register order and multiplies keys in the order in which the first product leaves them; the steps on the diagonal
+// and those of an incomplete block sum the even and the odd 32-key tiles apart and multiply keys in their natural order.
+//
+// A wave owns 32 queries: S^T = K Q^T by 32 x 32 x 16 matrix instructions, so that a lane holds half of ONE query's scores (row
+// reductions stay in the lane, plus one exchange of the half-waves), P is the second product's operand after packing, and the
+// accumulators are O^T, whose columns are rescaled by a lane's own alpha.  The four waves of a workgroup share K and V tiles in LDS
+// (direct loads, two buffers, 16-byte chunks swizzled against bank conflicts; V transposed on the way out by ds_read_b64_tr_b16).
+// Tiles above the diagonal are neither multiplied nor exponentiated.  Long blocks are launched first.
+//
+// What bounds it: at 32 x 512 tokens with 16 heads of 64, a step of 64 keys is about 205 vector instructions of which 33 exponentials
+// (~1200 cycles a wave) beside 512 cycles of matrix instructions, and 133 MB move; 39 to 43 us (inputs in the Infinity Cache /
+// from HBM) where the library's kernel and its counter's fill took 137 + 5.  2 x 500 tokens with 20 heads of 128: 17.3 us (39 + 5),
+// 160 workgroups whose longest walks eight steps on one wave per SIMD; 1 x 37 with 16 heads of 64: 3.4 us (8.6 + 1.4), the chain
+// of one step.  Measured and not taken: four waves a SIMD at d = 64 (128 registers, spills: +8 %), three buffers of K and V (+2 %),
+// one wave a SIMD at d = 128 (+14 to 42 %), the accumulators' rescaling skipped where no maximum moved (copies around the branch: +8 %).
+#include "gemm_tiles.h"
+
+namespace quest {
+namespace attn {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef short v4s __attribute__((ext_vector_type(4)));
+typedef short v8s __attribute__((ext_vector_type(8)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+constexpr int kWaves = 4;
+constexpr int kQueries = 32 * kWaves;            // per workgroup
+
+struct Args {
+    const uint8_t *qkv;                          // (batch, seq, 3 * heads * d)
+    uint8_t *out;                                // (batch, seq, heads * d)
+    int seq, heads, pairs;                       // pairs: batch * heads
+    int block;                                   // BM: rows whose completeness decides the order of the steps below them
+    float scale;                                 // fp32(1 / sqrt(d)) * fp32(log2 e)
+};
+
+template <int DT>
+__device__ __forceinline__ v16f mfma32(const v4i &a, const v4i &b, const v16f &c) {
+    if constexpr (DT == QUEST_DTYPE_BF16) return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
+}
+template <int DT>
+__device__ __forceinline__ v4f mfma16(const v4i &a, const v4i &b, const v4f &c) {
+    if constexpr (DT == QUEST_DTYPE_BF16) return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
+    else return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
+}
+
+// x of this lane and of the lane in the other half-wave (or the neighbouring row of 16), in either order
+__device__ __forceinline__ auto both_halves(float x) { return __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false); }
+__device__ __forceinline__ auto both_rows(float x) { return __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false); }
+template <typename R> __device__ __forceinline__ float sum2(const R &r) { return __uint_as_float(r[0]) + __uint_as_float(r[1]); }
+template <typename R> __device__ __forceinline__ float max2(const R &r) { return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])); }
+
+// where the 16-byte chunks of a tile's row stand in LDS: chunk c at place c ^ swizzle.  K rows are read 16 at a time at one chunk
+// number; V by eight rows of 64 bytes: rows r .. r + 3 of each half-wave, which start 4 or 8 rows apart.
+template <int D> __device__ __forceinline__ int k_swizzle(int row) { return D == 64 ? (row >> 1) & 7 : row & 15; }
+template <int D> __device__ __forceinline__ int v_swizzle(int row) { return D == 64 ? (row & 3) | ((((row >> 2) ^ (row >> 3)) & 1) << 2) : (row & 3) << 2; }
+
+// One wave's share of a tile of ROWS rows (the first row number `row0`), `WAVES` waves sharing it; `column`: byte offset of the
+// tile's 2 D bytes in a row of `pitch` bytes.  Rows past the sequence lie past the buffer and arrive as zeros.
+template <int D, int ROWS, int WAVES, bool V>
+__device__ __forceinline__ void load_tile(uint8_t *dst, __amdgpu_buffer_rsrc_t src, int row0, uint32_t pitch, uint32_t column, int wave, int lane) {
+    constexpr int kChunks = D / 8, kRowsPerLoad = 64 / kChunks, kLoads = ROWS / kRowsPerLoad / WAVES;
+    static_assert(kLoads * kRowsPerLoad * WAVES == ROWS, "whole loads");
+#pragma unroll
+    for (int i = 0; i < kLoads; i++) {
+        const int first = (wave * kLoads + i) * kRowsPerLoad, row = first + lane / kChunks;
+        const int chunk = (lane % kChunks) ^ (V ? v_swizzle<D>(row) : k_swizzle<D>(row));
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(src, (__attribute__((address_space(3))) void *)(dst + first * 2 * D), 16,
+                                                 (uint32_t)(row0 + row) * pitch + column + chunk * 16, 0, 0, 0);
+    }
+}
+
+// Sixteen keys (from byte offset OFF of the tile on) of this lane's channels lane % 32, 32 + lane % 32, ...: the operands of D / 32
+// matrix instructions, eight keys a lane from two transposing reads each; `at0`, `at1`: this lane's addresses for channels 0 .. 31
+// (v_address).  The reads and the wait for them in one statement: as builtins the compiler would put a wait for the direct loads
+// of the NEXT step in front of them.
+template <int D, int OFF>
+__device__ __forceinline__ void read_v(v4i (&v)[D / 32], uint32_t at0, uint32_t at1) {
+    typedef int v2i __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int a = 0; a < D / 32; a += 2) {
+        v2i x[4];
+        asm volatile("ds_read_b64_tr_b16 %0, %4 offset:%8\n\tds_read_b64_tr_b16 %1, %5 offset:%8\n\t"
+                     "ds_read_b64_tr_b16 %2, %6 offset:%8\n\tds_read_b64_tr_b16 %3, %7 offset:%8\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3])
+                     : "v"(at0 ^ (a << 6)), "v"(at1 ^ (a << 6)), "v"(at0 ^ ((a + 1) << 6)), "v"(at1 ^ ((a + 1) << 6)), "i"(OFF) : "memory");
+        v[a] = v4i{x[0][0], x[0][1], x[1][0], x[1][1]};
+        v[a + 1] = v4i{x[2][0], x[2][1], x[3][0], x[3][1]};
+    }
+}
+// lane address of a transposing read of four keys from `row` on: sixteen lanes cover four rows of sixteen channels
+template <int D>
+__device__ __forceinline__ int v_address(int row, int lane) {
+    const int r = row + ((lane >> 2) & 3), chunk = 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+    return r * 2 * D + ((chunk ^ v_swizzle<D>(r)) << 4) + (lane & 1) * 8;
+}
+
+// O^T of one wave -> its 32 rows: a lane's sixteen values of 32 channels, scaled, are eight consecutive channels twice after
+// the half-waves have traded
+template <int DT, int D>
+__device__ __forceinline__ void store_rows(const v16f (&acc)[D / 32], float inv, uint8_t *row_out, bool ok, int g) {
+#pragma unroll
+    for (int a = 0; a < D / 32; a++)
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            uint32_t x[2][2];
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int e = 0; e < 2; e++) {
+                    const int r = (2 * c + j) * 4 + 2 * e;
+                    x[j][e] = pack2_rounded_products<DT>(__fmul_rn(acc[a][r], inv), __fmul_rn(acc[a][r + 1], inv));
+                }
+            const auto s0 = __builtin_amdgcn_permlane32_swap(x[0][0], x[1][0], false, false);
+            const auto s1 = __builtin_amdgcn_permlane32_swap(x[0][1], x[1][1], false, false);
+            if (ok) *reinterpret_cast<uint4 *>(row_out + (a * 32 + c * 16 + g * 8) * 2) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
+        }
+}
+
+__device__ __forceinline__ uint32_t lds_offset(const uint8_t *p) {
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t *)p;
+}
+
+// One step of BN keys for a wave's 32 queries.  FULL: the order of a full step (see the top); TILES: how many of its 32-key tiles
+// are not wholly above the diagonal, DIAGONAL: the last of those is on it.  (The cases are separate instances: with the tiles'
+// number at run time the accumulators are copied around every branch.)
+template <int DT, int D, bool FULL, int TILES, bool DIAGONAL>
+__device__ __forceinline__ void step(const uint8_t *k_tile, const uint8_t *v_tile, const v4i (&q)[D / 16], v16f (&acc)[D / 32], float &m, float &l,
+                                     float scale, int lane) {
+    const int li = lane & 31, g = lane >> 5;
+    v16f s[TILES];
+    const int k_row = li * 2 * D, k_chunk = g ^ k_swizzle<D>(li);
+#pragma unroll
+    for (int t = 0; t < TILES; t++) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[t][r] = 0.f;
+#pragma unroll
+        for (int c = 0; c < D / 16; c++)
+            s[t] = mfma32<DT>(*reinterpret_cast<const v4i *>(k_tile + t * 64 * D + k_row + ((k_chunk ^ (2 * c)) << 4)), q[c], s[t]);
+        if constexpr (D == 128) __builtin_amdgcn_sched_barrier(0);      // (both tiles' K fragments at once would spill)
+    }
+    float mx = -__builtin_inff();
+#pragma unroll
+    for (int t = 0; t < TILES; t++) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) s[t][r] = __fmul_rn(s[t][r], scale);
+        if (DIAGONAL && t == TILES - 1) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) s[t][r] = 8 * (r / 4) + r % 4 + 4 * g > li ? -__builtin_inff() : s[t][r];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; r++) mx = fmaxf(mx, s[t][r]);
+    }
+    const float m_new = fmaxf(m, max2(both_halves(mx)));
+    const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+    m = m_new;
+    constexpr int kSums = !FULL && TILES > 1 ? 2 : 1;
+    float part[kSums];
+    uint32_t p[TILES][8];
+#pragma unroll
+    for (int t = 0; t < TILES; t++) {
+        float &sum = part[t % kSums];
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            s[t][r] = __builtin_amdgcn_exp2f(s[t][r] - m_new);
+            sum = t < kSums && r == 0 ? s[t][r] : sum + s[t][r];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) p[t][i] = pack2_rne<DT>(s[t][2 * i], s[t][2 * i + 1]);
+    }
+    float row_sum = sum2(both_halves(part[0]));
+    if constexpr (kSums == 2) row_sum += sum2(both_halves(part[1]));
+    l = __builtin_fmaf(l, alpha, row_sum);
+#pragma unroll
+    for (int a = 0; a < D / 32; a++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[a][r] *= alpha;
+    const uint32_t at0 = lds_offset(v_tile) + v_address<D>(FULL ? 4 * g : 8 * g, lane);
+    const uint32_t at1 = lds_offset(v_tile) + v_address<D>(FULL ? 8 + 4 * g : 8 * g + 4, lane);
+#pragma unroll
+    for (int t = 0; t < TILES; t++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            v4i b = {(int)p[t][4 * h], (int)p[t][4 * h + 1], (int)p[t][4 * h + 2], (int)p[t][4 * h + 3]};
+            if constexpr (!FULL) {
+                const auto s0 = __builtin_amdgcn_permlane32_swap(b[0], b[2], false, false);
+                const auto s1 = __builtin_amdgcn_permlane32_swap(b[1], b[3], false, false);
+                b = v4i{(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
+            }
+            v4i v[D / 32];
+            if (h == 0) read_v<D, 0>(v, at0 + t * 64 * D, at1 + t * 64 * D);
+            else read_v<D, 32 * D>(v, at0 + t * 64 * D, at1 + t * 64 * D);
+#pragma unroll
+            for (int a = 0; a < D / 32; a++) acc[a] = mfma32<DT>(v[a], b, acc[a]);
+        }
+}
+
+template <int DT, int D, int BN>
+__global__ __launch_bounds__(64 * kWaves, D == 64 && BN <= 64 ? 3 : 2) void attention_kernel(Args p) {
+    constexpr int kTileB = BN * 2 * D;
+    __shared__ __attribute__((aligned(256))) uint8_t lds[2][2][kTileB];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 31, g = lane >> 5;
+    const int blocks = (p.seq + kQueries - 1) / kQueries;
+    const int pair = blockIdx.x % p.pairs, q_wg = (blocks - 1 - blockIdx.x / p.pairs) * kQueries;      // the longest first
+    const int batch = pair / p.heads, head = pair % p.heads;
+    const uint32_t width = p.heads * 2 * D, pitch = 3 * width;
+    const uint8_t *base = p.qkv + (size_t)batch * p.seq * pitch;
+    const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, p.seq * pitch, 0x00020000);
+    const uint32_t q_col = head * 2 * D;
+    const int q0 = q_wg + 32 * wave;                                                // this wave's first query
+
+    auto issue = [&](int k0, int buf) {
+        load_tile<D, BN, kWaves, false>(lds[buf][0], src, k0, pitch, q_col + width, wave, lane);
+        load_tile<D, BN, kWaves, true>(lds[buf][1], src, k0, pitch, q_col + 2 * width, wave, lane);
+    };
+    issue(0, 0);
+    v4i q[D / 16];
+#pragma unroll
+    for (int c = 0; c < D / 16; c++) q[c] = __builtin_amdgcn_raw_buffer_load_b128(src, (uint32_t)(q0 + li) * pitch + q_col + (2 * c + g) * 16, 0, 0);
+    v16f acc[D / 32];
+#pragma unroll
+    for (int a = 0; a < D / 32; a++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[a][r] = 0.f;
+    float m = -__builtin_inff(), l = 0.f;
+    const int keys = min(p.seq, q_wg + kQueries);
+    const int block0 = q0 / p.block * p.block;
+    const int full_end = block0 + p.block <= p.seq ? block0 : 0;                    // steps before this key are full ones
+    for (int k0 = 0, buf = 0; k0 < keys; k0 += BN, buf ^= 1) {
+        wait_vmcnt_imm<0>();                         // this wave's share of the step has landed ...
+        plain_barrier();                             // ... and everyone's, and nobody reads the other buffer any more
+        if (k0 + BN < keys) issue(k0 + BN, buf ^ 1);
+        if (q0 >= p.seq || k0 > q0) continue;       // (q0 and k0 are whole 32s)
+        constexpr int kTiles = BN / 32;
+        const int diagonal = (q0 - k0) / 32;         // the tile on the diagonal, if it is in this step
+        const uint8_t *k_tile = lds[buf][0], *v_tile = lds[buf][1];
+        if (k0 < full_end) step<DT, D, true, kTiles, false>(k_tile, v_tile, q, acc, m, l, p.scale, lane);
+        else if (diagonal >= kTiles) step<DT, D, false, kTiles, false>(k_tile, v_tile, q, acc, m, l, p.scale, lane);
+        else if (diagonal == 0) step<DT, D, false, 1, true>(k_tile, v_tile, q, acc, m, l, p.scale, lane);
+        else if constexpr (kTiles > 1) {
+            if (diagonal == 1) step<DT, D, false, 2, true>(k_tile, v_tile, q, acc, m, l, p.scale, lane);
+            else if constexpr (kTiles > 2) {
+                if (diagonal == 2) step<DT, D, false, 3, true>(k_tile, v_tile, q, acc, m, l, p.scale, lane);
+                else step<DT, D, false, 4, true>(k_tile, v_tile, q, acc, m, l, p.scale, lane);
+            }
+        }
+    }
+    if (q0 >= p.seq) return;
+    const int row = q0 + li;
+    store_rows<DT, D>(acc, __fdiv_rn(1.0f, l), p.out + ((size_t)batch * p.seq + row) * width + q_col, row < p.seq, g);
+}
+
+// The shortest sequences: one wave per head, sixteen keys a step on 16 x 16 x 32 (S^T of two sixteen-query tiles; a lane holds four
+// keys of a query), the second product on 32 x 32 x 16 as above.
+template <int DT, int D>
+__global__ __launch_bounds__(64) void attention_short_kernel(Args p) {
+    __shared__ __attribute__((aligned(256))) uint8_t lds[32 * 2 * D];
+    const int lane = threadIdx.x, lq = lane & 15, row4 = lane >> 4, g = lane >> 5;
+    const int batch = blockIdx.x / p.heads, head = blockIdx.x % p.heads;
+    const uint32_t width = p.heads * 2 * D, pitch = 3 * width, q_col = head * 2 * D;
+    const uint8_t *base = p.qkv + (size_t)batch * p.seq * pitch;
+    const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, p.seq * pitch, 0x00020000);
+    load_tile<D, 32, 1, true>(lds, src, 0, pitch, q_col + 2 * width, 0, lane);
+    v4i q[2][D / 32], k[2][D / 32];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int c = 0; c < D / 32; c++) {
+            const uint32_t at = (uint32_t)(16 * t + lq) * pitch + q_col + (4 * c + row4) * 16;
+            q[t][c] = __builtin_amdgcn_raw_buffer_load_b128(src, at, 0, 0);
+            k[t][c] = __builtin_amdgcn_raw_buffer_load_b128(src, at + width, 0, 0);
+        }
+    v16f acc[D / 32];
+#pragma unroll
+    for (int a = 0; a < D / 32; a++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[a][r] = 0.f;
+    float m[2] = {-__builtin_inff(), -__builtin_inff()}, l[2] = {0.f, 0.f};
+    const uint32_t at0 = lds_offset(lds) + v_address<D>(8 * g, lane), at1 = lds_offset(lds) + v_address<D>(8 * g + 4, lane);
+    wait_vmcnt_imm<0>();
+    plain_barrier();
+#pragma unroll
+    for (int kb = 0; kb < 2; kb++) {
+        if (kb * 16 >= p.seq) break;
+        uint32_t pk[2][2] = {};
+        float alpha[2] = {1.f, 1.f};
+#pragma unroll
+        for (int t = kb; t < 2; t++) {                             // (queries before the keys: p = 0)
+            v4f s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < D / 32; c++) s = mfma16<DT>(k[kb][c], q[t][c], s);
+            float mx = -__builtin_inff();
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                s[r] = __fmul_rn(s[r], p.scale);
+                if (t == kb) s[r] = 4 * row4 + r > lq ? -__builtin_inff() : s[r];
+                mx = fmaxf(mx, s[r]);
+            }
+            mx = max2(both_halves(mx));
+            const float m_new = fmaxf(m[t], max2(both_rows(mx)));
+            alpha[t] = __builtin_amdgcn_exp2f(m[t] - m_new);
+            m[t] = m_new;
+#pragma unroll
+            for (int r = 0; r < 4; r++) s[r] = __builtin_amdgcn_exp2f(s[r] - m_new);
+            const float sum = sum2(both_halves(((s[0] + s[1]) + s[2]) + s[3]));
+            l[t] = __builtin_fmaf(l[t], alpha[t], sum2(both_rows(sum)));
+            pk[t][0] = pack2_rne<DT>(s[0], s[1]);
+            pk[t][1] = pack2_rne<DT>(s[2], s[3]);
+        }
+        const auto s0 = __builtin_amdgcn_permlane16_swap(pk[0][0], pk[1][0], false, false);
+        const auto s1 = __builtin_amdgcn_permlane16_swap(pk[0][1], pk[1][1], false, false);
+        const v4i b = {(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
+        const float al = lane & 16 ? alpha[1] : alpha[0];
+        v4i v[D / 32];
+        if (kb == 0) read_v<D, 0>(v, at0, at1);
+        else read_v<D, 32 * D>(v, at0, at1);
+#pragma unroll
+        for (int a = 0; a < D / 32; a++) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[a][r] *= al;
+            acc[a] = mfma32<DT>(v[a], b, acc[a]);
+        }
+    }
+    const int row = lane & 31;
+    store_rows<DT, D>(acc, __fdiv_rn(1.0f, lane & 16 ? l[1] : l[0]), p.out + ((size_t)batch * p.seq + row) * width + q_col, row < p.seq, g);
+}
+
+// The length chooses the step (see the top).
+template <int DT, int D>
+void launch(Args p, hipStream_t st) {
+    constexpr bool kFp16x64 = DT == QUEST_DTYPE_FP16 && D == 64;
+    if (p.seq <= (kFp16x64 ? 16 : 32)) {
+        attention_short_kernel<DT, D><<<dim3(p.pairs), dim3(64), 0, st>>>(p);
+        return;
+    }
+    p.block = p.seq <= 128 ? 64 : 128;
+    const dim3 grid(p.pairs * ((p.seq + kQueries - 1) / kQueries)), threads(64 * kWaves);
+    if constexpr (kFp16x64) {
+        if (p.seq <= 32) {
+            attention_kernel<DT, D, 32><<<grid, threads, 0, st>>>(p);
+            return;
+        }
+    }
+    if constexpr (D == 64) {
+        if (p.seq > 128 && p.seq <= 256) {
+            attention_kernel<DT, D, 128><<<grid, threads, 0, st>>>(p);
+            return;
+        }
+    }
+    attention_kernel<DT, D, 64><<<grid, threads, 0, st>>>(p);
+}
+
+}  // namespace attn
+}  // namespace quest
+
+using namespace quest;
+
+extern "C" int quest_causal_attention(void *out, const void *qkv, int batch, int seq, int n_head, int head_dim, int dtype, void *stream) {
+    forget_stale_error();
+    if (!out || !qkv) return QUEST_ERR_NULL_POINTER;
+    if (!check_dtype(dtype)) return QUEST_ERR_BAD_DTYPE;
+    if (batch <= 0 || seq <= 0 || n_head <= 0 || head_dim <= 0) return QUEST_ERR_BAD_SHAPE;
+    // 32-bit byte offsets inside one sequence, 128 rows past its end included; one block index per head and 128 queries
+    const int64_t pitch = (int64_t)6 * n_head * head_dim, groups = (int64_t)batch * n_head * ((seq + attn::kQueries - 1) / attn::kQueries);
+    if ((head_dim != 64 && head_dim != 128) || pitch * ((int64_t)seq + 256) > 0x7fffffff || groups > 0x7fffffff) return QUEST_ERR_UNSUPPORTED;
+    if (!aligned(out, 16) || !aligned(qkv, 16)) return QUEST_ERR_ALIGNMENT;
+    attn::Args p = {(const uint8_t *)qkv, (uint8_t *)out, seq, n_head, batch * n_head, 0, 0.f};
+    p.scale = (float)(1.0 / __builtin_sqrt((double)head_dim)) * 1.44269504088896340736f;
+    hipStream_t st = (hipStream_t)stream;
+    if (dtype == QUEST_DTYPE_BF16) head_dim == 64 ? attn::launch<0, 64>(p, st) : attn::launch<0, 128>(p, st);
+    else head_dim == 64 ? attn::launch<1, 64>(p, st) : attn::launch<1, 128>(p, st);
+    return launch_status();
+}

@@ -13,6 +13,7 @@
 // Nothing is cached between calls.
 #include <Python.h>
 
+#include <ATen/Context.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -539,11 +540,17 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             }
             launched(rc, "QKV projection");
         }
-        // causal attention
-        const int64_t row = 3 * c64;
-        const auto part = [&](int64_t i) { return heads.as_strided({b, n_head, t, head_dim}, {t * row, head_dim, row, 1}, i * c64); };
-        const at::Tensor y = at::scaled_dot_product_attention(part(0), part(1), part(2), {}, 0.0, true);
-        const at::Tensor core = y.transpose(1, 2).contiguous();
+        // causal attention: the library's where ours does not take the heads or the caller has switched off the library kernel whose bits ours gives
+        at::Tensor core = make({m, c64}, type, args.dev);
+        const int rc = at::globalContext().userEnabledFlashSDP()
+                           ? quest_causal_attention(core.data_ptr(), heads.data_ptr(), (int)b, (int)t, (int)n_head, head_dim, dt, st) : QUEST_ERR_UNSUPPORTED;
+        if (rc == QUEST_ERR_UNSUPPORTED) {
+            const int64_t row = 3 * c64;
+            const auto part = [&](int64_t i) { return heads.as_strided({b, n_head, t, head_dim}, {t * row, head_dim, row, 1}, i * c64); };
+            core = at::scaled_dot_product_attention(part(0), part(1), part(2), {}, 0.0, true).transpose(1, 2).contiguous();
+        } else {
+            launched(rc, "attention");
+        }
         // output projection: into the residual stream where its GEMM can add
         bool has_att = false;
         at::Tensor att;
