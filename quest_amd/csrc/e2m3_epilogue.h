@@ -89,6 +89,11 @@ inline long tile_grid(int tiles_t, int tiles_c) { return ((long)tiles_t * tiles_
 // gemm_e2m3_mid.hip / gemm_e2m3_split.hip: tiles of 32 tf x 32 cf; QUEST_ERR_UNSUPPORTED for a shape that is not built
 int launch_gemm_e2m3_mid(int dtype, int tf, int cf, void *out, const uint8_t *a, const uint8_t *b, int M, int K, int N, const Epilogue &epi, hipStream_t st);
 int launch_gemm_e2m3_split(int dtype, int tf, int cf, void *out, const uint8_t *a, const uint8_t *b, int M, int K, int N, const Epilogue &epi, hipStream_t st);
+// gemm_e2m3_resident.hip: K from 256 to kResidentMaxK, whole eights of channels, at least eight CUs.  The plan's estimated time in us; `plan` (or
+// null): as quest_e2m3_gemm_plan reports it.
+constexpr int kResidentMaxK = 1664;
+int launch_gemm_e2m3_resident(int dtype, void *out, const uint8_t *a, const uint8_t *b, int M, int K, int N, int cus, const Epilogue &epi, hipStream_t st);
+float gemm_e2m3_resident_plan(int M, int K, int N, int cus, int *plan);
 // LDS slots of a shape's pipeline (the split kernel's: per wave); 0 for a shape that is not built
 int gemm_e2m3_mid_slots(int tf, int cf);
 int gemm_e2m3_split_slots(int tf, int cf);

@@ -25,6 +25,7 @@ E2M3_MIN_TOKENS = 33                    # a fused block: from here on (see block
 E2M3_MIN_K = 1536                       # shortest rows that take them at more than E2M3_SHORT_ROWS_TOKENS tokens
 E2M3_MIN_K_NARROW = 2048                # ... by a layer of fewer than E2M3_NARROW channels
 E2M3_NARROW = 1536
+E2M3_RESIDENT_MAX_K = 1664              # longest rows of the FP6 kernel that keeps a channel tile's weights in LDS
 E2M3_SHORT_ROWS_TOKENS = 4096
 # Whether a producer-fused block lets the FP6 GEMM of an output projection add into the residual stream itself
 # (same bits as the addition inside the next norm kernel; one pass over the stream less).
@@ -63,9 +64,11 @@ def block_prefers_e2m3(m: int, k: int, n: int) -> bool:
     """The same for a projection of a producer-fused block, where the FP6 kernels also save launches (the rotary embedding, the gated
     unit and both residual additions ride in their epilogues at every size).  Whole blocks, d = 256 to 4096, 33 to 4000 tokens,
     weights from HBM, INT8 / FP6 time: 0.97 to 1.18 ((d = 768, 1000 tokens) 0.97, (2560, 200) 0.99, (1024, 37) 1.08, (2560, 64)
-    1.14, (4096, 500) 1.17)."""
+    1.14, (4096, 500) 1.17).  Many tokens with short rows have a kernel of their own (gemm_e2m3_resident.hip), INT8 / FP6 time of
+    the GEMM: (16384, 1024) x 1024 with the residual 1.28, x 3072 rotary 1.35, x 5632 gated 1.55; (16384, 768) x 1024 1.24; (8192,
+    768) x 5632 1.36."""
     return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and _tiles_addressable(m, k, n)
-            and (m <= E2M3_SHORT_ROWS_TOKENS or _enough_per_row(k, n)))
+            and (m <= E2M3_SHORT_ROWS_TOKENS or _enough_per_row(k, n) or (768 <= k <= E2M3_RESIDENT_MAX_K and n % 16 == 0)))
 
 
 def _tiles_addressable(m: int, k: int, n: int) -> bool:
