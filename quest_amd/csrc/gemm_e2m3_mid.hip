@@ -10,6 +10,11 @@
 // What bounds it: the LDS port, which a stage's bytes cross once on their way in and twice on their way to the waves that share them
 // (72 KiB per stage of a 128 x 128 tile: 576 cycles at 128 bytes a cycle, 600 measured, against 256 of matrix work), and with one
 // tile per CU the trip to memory before the first stage and the epilogue after the last, together 5 us.
+// 128 x 96 tiles (KS = 2) share K between the waves of a pair: each multiplies 64 x 96 of one of a stage's two 64-k steps, so that 51 KiB instead
+// of 69 cross the port per stage (waves of 32 x 96 would read 48 KiB, as for 128 x 128), and at the end they trade a token block of sums each
+// (96 KiB through LDS).  They fill 216 of 256 CUs where 128 x 128 has 160 tiles: (1000, 6912, 2560) 22.7 -> 20.5 us, (516, 1152, 3695)
+// 15.9 -> 14.1, (197, 9600, 8324) 37.6 -> 34.2.  128 x 128 by pairs is 1 to 4 % slower than 2 x 2 waves: a stage's fragments are all read behind
+// its one barrier.
 // Measured against the kernels that took these sizes before (weights rotating through four copies): (200, 4096, 11008) 15.5 against
 // 19.9 us, (1000, 6912, 2560) 22.2 against 27.6, (1400, 2560, 2560) 12.9 against 26.9, (1400, 6912, 2560) 24.2 against 54.3.
 #include "e2m3_epilogue.h"
@@ -17,6 +22,7 @@
 namespace quest {
 namespace e2m3m {
 
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v8i __attribute__((ext_vector_type(8)));
@@ -24,11 +30,13 @@ typedef int v8i __attribute__((ext_vector_type(8)));
 constexpr int kWaves = 4;
 constexpr int kFragB = 1536;
 
-template <int TF_, int CF_, int WT_, int WC_>
+template <int TF_, int CF_, int WT_, int WC_, int KS_ = 1>
 struct Tile {
-    static constexpr int TF = TF_, CF = CF_, WT = WT_, WC = WC_;
-    static_assert(WT * WC == kWaves && TF % WT == 0 && CF % WC == 0, "whole fragments per wave");
+    static constexpr int TF = TF_, CF = CF_, WT = WT_, WC = WC_, KS = KS_;
+    static_assert(WT * WC * KS == kWaves && TF % WT == 0 && CF % WC == 0, "whole fragments per wave");
     static constexpr int kT = TF / WT, kC = CF / WC;                   // fragments per wave
+    static constexpr int kDone = kT / KS;                              // token blocks that a wave finishes
+    static_assert(KS == 1 || (KS == 2 && kT == 2), "a pair's waves finish one token block each");
     static constexpr int kTok = 32 * TF, kChn = 32 * CF;
     static constexpr int kSlotB = 3072 * (TF + CF);
     static constexpr int kLoads = (3 * (TF + CF) + kWaves - 1) / kWaves;       // direct loads per wave and stage
@@ -37,6 +45,7 @@ struct Tile {
     static constexpr int kFit = ((160 / kWgPerCu) * 1024 - 1024) / kSlotB;
     static constexpr int kStages = kFit < 8 ? kFit : 8;
     static_assert(kStages >= 3 && kLoads * (kStages - 2) < 64, "stages in flight");
+    static_assert(KS == 1 || kWaves * kC * 4096 <= kStages * kSlotB, "the partial sums that pairs trade");
     // (loads past the tile's last touch no memory but do write zeros: into a KiB of their own)
     static constexpr bool kSpare = 3 * (TF + CF) % kWaves != 0;
     static constexpr int kLdsB = kStages * kSlotB + (kSpare ? 1024 : 0);
@@ -45,17 +54,19 @@ struct Tile {
 template <int DT, bool ROPE, typename S>
 __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const uint8_t *__restrict__ act, const uint8_t *__restrict__ wgt,
                                      int M, int N, int K, int tok0, int ch0, const Epilogue &epi) {
-    constexpr int TF = S::TF, CF = S::CF, kT = S::kT, kC = S::kC, D = S::kStages;
+    constexpr int TF = S::TF, CF = S::CF, kT = S::kT, kC = S::kC, D = S::kStages, kDone = S::kDone;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int lane = (int)threadIdx.x & 63, li = lane & 31, lg = lane >> 5;
-    const int tf0 = (wave / S::WC) * kT, cf0 = (wave % S::WC) * kC;      // the wave's fragments of the tile
+    const int part = wave / S::KS, half = wave % S::KS;                  // (half: which 64-k step of every stage, if each wave has one)
+    const int tf0 = (part / S::WC) * kT, cf0 = (part % S::WC) * kC;      // the wave's fragments of the tile
+    const int done0 = tf0 + half * kDone;                                // the token blocks that it finishes
 
     // the epilogue's scale values set out first: a lane finishes token li of each of its token blocks and, of each channel unit,
     // channels 8 q + 4 lg ... + 3
-    float t_half_mul[kT];
+    float t_half_mul[kDone];
     uint32_t c_mul[kC][8];
 #pragma unroll
-    for (int t = 0; t < kT; t++) t_half_mul[t] = __fmul_rn(0.5f, to_f32<DT>(epi.a_mul[min(tok0 + 32 * (tf0 + t) + li, M - 1)]));
+    for (int t = 0; t < kDone; t++) t_half_mul[t] = __fmul_rn(0.5f, to_f32<DT>(epi.a_mul[min(tok0 + 32 * (done0 + t) + li, M - 1)]));
 #pragma unroll
     for (int c = 0; c < kC; c++)
 #pragma unroll
@@ -73,14 +84,14 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
         }
     // ... and what the epilogue adds or rotates by
     const bool vec16 = (N & 7) == 0;
-    Ahead<ROPE> ahead[kT][kC][2];
+    Ahead<ROPE> ahead[kDone][kC][2];
 #pragma unroll
-    for (int t = 0; t < kT; t++)
+    for (int t = 0; t < kDone; t++)
 #pragma unroll
         for (int c = 0; c < kC; c++)
 #pragma unroll
             for (int pr = 0; pr < 2; pr++)
-                fetch_ahead<DT>(ahead[t][c][pr], out, epi, tok0 + 32 * (tf0 + t) + li, ch0 + 32 * (cf0 + c) + (2 * pr + lg) * 8, M, N, vec16);
+                fetch_ahead<DT>(ahead[t][c][pr], out, epi, tok0 + 32 * (done0 + t) + li, ch0 + 32 * (cf0 + c) + (2 * pr + lg) * 8, M, N, vec16);
 
     const int nk = K / 128;                                      // stages
     const int pitch = (K / 64) * kFragB;                         // bytes per row block
@@ -130,9 +141,8 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
     };
     Frags u0, u1;
     // one stage, the MFMAs one by one with the rest of the pipeline between them, the order pinned
-    auto stage_step = [&](int stage, int slot) {
-        const int next_slot = slot + 1 == D ? 0 : slot + 1;
-        constexpr int kReads = kT + kC;
+    constexpr int kReads = kT + kC;
+    auto first_step = [&](int slot) {
 #pragma unroll
         for (int i = 0; i < kMfmas; i++) {                       // first step; the second one's fragments
             mfma(u0, i);
@@ -140,10 +150,13 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
             for (int e = i * kReads / kMfmas; e < (i + 1) * kReads / kMfmas; e++) read_one(u1, slot, 1, e);
             __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    auto last_step = [&](const Frags &now, Frags &then, int stage, int slot) {      // the only step of a wave that has one per stage
+        const int next_slot = slot + 1 == D ? 0 : slot + 1;
         constexpr int kEvents = S::kLoads + kReads;
 #pragma unroll
-        for (int i = 0; i < kMfmas; i++) {                       // second step
-            mfma(u1, i);                                         // (waits for its fragments: the slot has been read)
+        for (int i = 0; i < kMfmas; i++) {
+            mfma(now, i);                                        // (waits for its fragments: the slot has been read)
             if (i == 0) {
                 __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4) | (0 << 8));      // lgkmcnt(0): all of them
                 wait_vmcnt_imm<S::kLoads * (D - 2)>();           // this wave's loads of the next stage have landed ...
@@ -152,7 +165,7 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
             // the next stage's first fragments, then the loads into the slot
 #pragma unroll
             for (int e = i * kEvents / kMfmas; e < (i + 1) * kEvents / kMfmas; e++) {
-                if (e < kReads) read_one(u0, next_slot, 0, e); else load_one(slot, stage + D, e - kReads);
+                if (e < kReads) read_one(then, next_slot, half, e); else load_one(slot, stage + D, e - kReads);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -164,19 +177,61 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
     wait_vmcnt_imm<S::kLoads * (D - 1)>();
     plain_barrier();
 #pragma unroll
-    for (int f = 0; f < kT + kC; f++) read_one(u0, 0, 0, f);
+    for (int f = 0; f < kT + kC; f++) read_one(u0, 0, half, f);
     int slot = 0;
-    for (int stage = 0; stage < nk; stage++) {
-        stage_step(stage, slot);
-        slot = slot + 1 == D ? 0 : slot + 1;
+    auto on = [](int x) { return x + 1 == D ? 0 : x + 1; };
+    if constexpr (S::KS == 1) {
+        for (int stage = 0; stage < nk; stage++, slot = on(slot)) {
+            first_step(slot);
+            last_step(u1, u0, stage, slot);
+        }
+    } else {
+        int stage = 0;
+        for (; stage + 2 <= nk; stage += 2) {
+            last_step(u0, u1, stage, slot);
+            slot = on(slot);
+            last_step(u1, u0, stage + 1, slot);
+            slot = on(slot);
+        }
+        if (stage < nk) last_step(u0, u1, stage, slot);
     }
     wait_vmcnt_imm<0>();                                         // no direct load may outlive the workgroup's LDS allocation
+
+    // ---- a pair's waves trade the token blocks that they do not finish, a KiB of four registers at a time
+    if constexpr (S::KS == 2) {
+        __builtin_amdgcn_s_waitcnt(0);
+        plain_barrier();                                         // nobody reads or loads a slot any more
+        if (half == 1) {
+#pragma unroll
+            for (int c = 0; c < kC; c++) {
+                const v16f x = acc[0][c];
+                acc[0][c] = acc[1][c];
+                acc[1][c] = x;
+            }
+        }
+        v4f *const give = reinterpret_cast<v4f *>(lds) + wave * (kC * 256) + lane;
+        const v4f *const take = reinterpret_cast<const v4f *>(lds) + (wave ^ 1) * (kC * 256) + lane;
+#pragma unroll
+        for (int c = 0; c < kC; c++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) give[(4 * c + q) * 64] = v4f{acc[1][c][4 * q], acc[1][c][4 * q + 1], acc[1][c][4 * q + 2], acc[1][c][4 * q + 3]};
+        __builtin_amdgcn_s_waitcnt(0);
+        plain_barrier();
+#pragma unroll
+        for (int c = 0; c < kC; c++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const v4f x = take[(4 * c + q) * 64];
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[0][c][4 * q + e] += x[e];
+            }
+    }
 
     // ---- epilogue: register r of lane (li, lg) of block (t, c) is token 32 t + li, channel 32 c + 8 (r / 4) + 4 lg + r % 4; the
     // half-waves trade register groups, so that a lane holds eight consecutive channels
 #pragma unroll
-    for (int t = 0; t < kT; t++) {
-        const int tok = tok0 + 32 * (tf0 + t) + li;
+    for (int t = 0; t < kDone; t++) {
+        const int tok = tok0 + 32 * (done0 + t) + li;
 #pragma unroll
         for (int c = 0; c < kC; c++) {
             const int cu = ch0 + 32 * (cf0 + c);
@@ -225,10 +280,11 @@ static int launch(void *out, const uint8_t *a, const uint8_t *b, int M, int K, i
 
 }  // namespace e2m3m
 
-#define QUEST_MID_SHAPES QUEST_MID(8, 4) QUEST_MID(4, 6) QUEST_MID(4, 4) QUEST_MID(4, 2) QUEST_MID(2, 4) QUEST_MID(2, 2)
+#define QUEST_MID_SHAPES QUEST_MID(8, 4, 2, 2, 1) QUEST_MID(4, 6, 2, 2, 1) QUEST_MID(4, 4, 2, 2, 1) QUEST_MID(4, 3, 2, 1, 2) QUEST_MID(4, 2, 2, 2, 1) \
+    QUEST_MID(2, 4, 2, 2, 1) QUEST_MID(2, 2, 2, 2, 1)
 
 int gemm_e2m3_mid_slots(int tf, int cf) {
-#define QUEST_MID(TF, CF) if (tf == TF && cf == CF) return e2m3m::Tile<TF, CF, 2, 2>::kStages;
+#define QUEST_MID(TF, CF, WT, WC, KS) if (tf == TF && cf == CF) return e2m3m::Tile<TF, CF, WT, WC, KS>::kStages;
     QUEST_MID_SHAPES
 #undef QUEST_MID
     return 0;
@@ -236,9 +292,9 @@ int gemm_e2m3_mid_slots(int tf, int cf) {
 
 int launch_gemm_e2m3_mid(int dtype, int tf, int cf, void *out, const uint8_t *a, const uint8_t *b, int M, int K, int N, const Epilogue &epi, hipStream_t st) {
 #define QUEST_MID_DT(DT, T) (epi.kind == kEpiRope ? e2m3m::launch<DT, true, T>(out, a, b, M, K, N, epi, st) : e2m3m::launch<DT, false, T>(out, a, b, M, K, N, epi, st))
-#define QUEST_MID(TF, CF)                                                                                        \
+#define QUEST_MID(TF, CF, WT, WC, KS)                                                                                    \
     if (tf == TF && cf == CF) {                                                                                  \
-        using T = e2m3m::Tile<TF, CF, 2, 2>;                                                                     \
+        using T = e2m3m::Tile<TF, CF, WT, WC, KS>;                                                               \
         return dtype == QUEST_DTYPE_BF16 ? QUEST_MID_DT(0, T) : QUEST_MID_DT(1, T);                              \
     }
     QUEST_MID_SHAPES
