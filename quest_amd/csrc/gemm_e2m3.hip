@@ -505,7 +505,7 @@ static int launch_large(int dtype, void *out, const uint8_t *a, const uint8_t *b
 // always picking the fastest one in total time, within 16 % on every single size.  With weights from HBM (copies of more than 320
 // MB, 816 sizes, K from 256) it is within 1.4 % in total and 20 % on every size; on rows of 16384 to 65536, beyond the fit and its
 // negative coefficients, within 0.1 and 3 %.  {4, 3}'s line is {4, 4}'s and the difference of the two measured at 44 sizes (one tile per CU,
-// K from 1024 to 9600: 0.65 + 0.031 K / 128 us less).
+// K from 1152 to 9600: 0.65 + 0.031 K / 128 us less).
 struct Shape {
     bool split;
     int tf, cf;
@@ -524,6 +524,7 @@ static const Shape *smaller_shape(int M, int K, int N, int cus, float &best_us) 
     if (2L * ((M + 255) / 256) * ((N + 255) / 256) > cus) return nullptr;
     const Shape *best = nullptr;
     for (const Shape &s : kShapes) {
+        if (s.cf == 3 && K < 1152) continue;        // (measured for longer rows; 0.3 to 1.8 us at K = 1024 to 1152)
         const long tiles = (long)((M + 32 * s.tf - 1) / (32 * s.tf)) * ((N + 32 * s.cf - 1) / (32 * s.cf));
         const float us = s.fixed + (float)((tiles + cus - 1) / cus) * (s.stage * (float)(K / 128) + s.tile) + s.weights * 0.75e-6f * (float)N * (float)K;
         if (best == nullptr || us < best_us) { best = &s; best_us = us; }
