@@ -16,6 +16,10 @@
 // (direct loads, two buffers, 16-byte chunks swizzled against bank conflicts; V transposed on the way out by ds_read_b64_tr_b16).
 // Tiles above the diagonal are neither multiplied nor exponentiated.  Long blocks are launched first.
 //
+// Scores of -inf count as that library's do: a row's running maximum starts at the lowest finite value, so that a step (or a whole
+// row) of nothing else adds nothing, and a row of nothing else is zero.  A NaN or an infinity in a query, key or value shows in the rows
+// that attend to it and, as 0 * inf, in the earlier rows of the same 32 keys (the library's: of the same step).
+//
 // What bounds it: at 32 x 512 tokens with 16 heads of 64, a step of 64 keys is about 205 vector instructions of which 33 exponentials
 // (~1200 cycles a wave) beside 512 cycles of matrix instructions, and 133 MB move; 39 to 43 us (inputs in the Infinity Cache /
 // from HBM) where the library's kernel and its counter's fill took 137 + 5.  2 x 500 tokens with 20 heads of 128: 17.3 us (39 + 5),
@@ -36,6 +40,7 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int kWaves = 4;
 constexpr int kQueries = 32 * kWaves;            // per workgroup
+constexpr float kLowest = -3.4028234663852886e38f;
 
 struct Args {
     const uint8_t *qkv;                          // (batch, seq, 3 * heads * d)
@@ -128,6 +133,9 @@ __device__ __forceinline__ void store_rows(const v16f (&acc)[D / 32], float inv,
             if (ok) *reinterpret_cast<uint4 *>(row_out + (a * 32 + c * 16 + g * 8) * 2) = make_uint4(s0[0], s1[0], s0[1], s1[1]);
         }
 }
+
+// 1 / l; 0 for a row whose scores are all -inf (any other has a p of 1)
+__device__ __forceinline__ float inverse(float l) { return l == 0.f ? 0.f : __fdiv_rn(1.0f, l); }
 
 __device__ __forceinline__ uint32_t lds_offset(const uint8_t *p) {
     return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t *)p;
@@ -234,7 +242,7 @@ __global__ __launch_bounds__(64 * kWaves, D == 64 && BN <= 64 ? 3 : 2) void atte
     for (int a = 0; a < D / 32; a++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[a][r] = 0.f;
-    float m = -__builtin_inff(), l = 0.f;
+    float m = kLowest, l = 0.f;
     const int keys = min(p.seq, q_wg + kQueries);
     const int block0 = q0 / p.block * p.block;
     const int full_end = block0 + p.block <= p.seq ? block0 : 0;                    // steps before this key are full ones
@@ -259,7 +267,7 @@ __global__ __launch_bounds__(64 * kWaves, D == 64 && BN <= 64 ? 3 : 2) void atte
     }
     if (q0 >= p.seq) return;
     const int row = q0 + li;
-    store_rows<DT, D>(acc, __fdiv_rn(1.0f, l), p.out + ((size_t)batch * p.seq + row) * width + q_col, row < p.seq, g);
+    store_rows<DT, D>(acc, inverse(l), p.out + ((size_t)batch * p.seq + row) * width + q_col, row < p.seq, g);
 }
 
 // The shortest sequences: one wave per head, sixteen keys a step on 16 x 16 x 32 (S^T of two sixteen-query tiles; a lane holds four
@@ -287,7 +295,7 @@ __global__ __launch_bounds__(64) void attention_short_kernel(Args p) {
     for (int a = 0; a < D / 32; a++)
 #pragma unroll
         for (int r = 0; r < 16; r++) acc[a][r] = 0.f;
-    float m[2] = {-__builtin_inff(), -__builtin_inff()}, l[2] = {0.f, 0.f};
+    float m[2] = {kLowest, kLowest}, l[2] = {0.f, 0.f};
     const uint32_t at0 = lds_offset(lds) + v_address<D>(8 * g, lane), at1 = lds_offset(lds) + v_address<D>(8 * g + 4, lane);
     wait_vmcnt_imm<0>();
     plain_barrier();
@@ -334,7 +342,7 @@ __global__ __launch_bounds__(64) void attention_short_kernel(Args p) {
         }
     }
     const int row = lane & 31;
-    store_rows<DT, D>(acc, __fdiv_rn(1.0f, lane & 16 ? l[1] : l[0]), p.out + ((size_t)batch * p.seq + row) * width + q_col, row < p.seq, g);
+    store_rows<DT, D>(acc, inverse(lane & 16 ? l[1] : l[0]), p.out + ((size_t)batch * p.seq + row) * width + q_col, row < p.seq, g);
 }
 
 // The length chooses the step (see the top).

@@ -73,6 +73,23 @@ def test_nothing_crosses_a_sequence_end(t, d):
     assert out[t:2 * t].isnan().all() and (out[3 * t:] == 7).all()
 
 
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('d', [64, 128])
+@pytest.mark.parametrize('t', [1, 5, 16, 30, 64, 127, 200, 300, 500])
+def test_scores_of_minus_infinity_add_nothing(t, d, dtype):
+    """The first half of the keys score -inf for every query: whole steps, and whole rows, of nothing else.  The rows behind them are
+    those of the other keys, whichever order they are summed in; the first ones are zero, as the library's are."""
+    qkv = inputs(1, t, 1, d, dtype, 1.0, t)
+    half = (t + 1) // 2
+    qkv[0, :, 0] = qkv[0, :, 0].abs() + 0.1
+    qkv[0, :half, d:2 * d] = 0
+    qkv[0, :half, d] = float('-inf')
+    q, k, v = parts(qkv, 1)
+    want = F.scaled_dot_product_attention(q, k, v, is_causal=True).transpose(1, 2).reshape(1, t, d)
+    got = attend(qkv, 1)
+    assert torch.equal(got, want) and not got[0, :half].any() and got.isfinite().all()
+
+
 def test_refused_calls():
     lib, qkv = _lib.load(), torch.zeros(1, 8, 3 * 96, dtype=torch.bfloat16, device='cuda')
     out = torch.zeros(1, 8, 96, dtype=torch.bfloat16, device='cuda')
