@@ -400,7 +400,10 @@ int quest_dense_rows(void *out, const void *x, const void *weight, int size_m, i
  * side by side; out (batch, seq, n_head * head_dim) = softmax(q k^T / sqrt(head_dim)) v over each row's own and earlier positions, in
  * fp32 with the probabilities rounded to dtype in front of the second product (src/models/llama.py:150-163).  head_dim 64 or
  * 128 and rows of a sequence below 2 GiB (QUEST_ERR_UNSUPPORTED otherwise, nothing launched); pointers 16-byte aligned.
+ * Up to QUEST_ATTENTION_SAME_BITS rows of a sequence the outputs are those of torch's own kernel (torch 2.10 on gfx950) bit for bit; beyond,
+ * that kernel sums in another order and the two differ by rounding.
  */
+#define QUEST_ATTENTION_SAME_BITS(head_dim) ((head_dim) == 64 ? 4096 : 2048)
 int quest_causal_attention(void *out, const void *qkv, int batch, int seq, int n_head, int head_dim, int dtype, void *stream);
 
 #ifdef __cplusplus

@@ -3,8 +3,9 @@
 //
 // The block's next step is a 4-bit quantiser: one unit in the last place of an attention output moves a code now and then, and
 // twelve layers of such quantisers turn that into a visible change of a model's logits.  So the order of every fp32 operation is
-// fixed, and it is the order whose outputs equal torch's own kernel on this card bit for bit (tests/test_gpu_attention.py over
-// sequences of 1 to 2048): keys are taken BN at a time, s = (q k) * fp32(log2 e / sqrt(d)) with the product rounded first,
+// fixed, and it is the order whose outputs equal torch's own kernel on this card bit for bit (tests/test_gpu_attention.py), up to
+// 4096 rows with heads of 64 and 2048 with heads of 128 (beyond, 1e-5 of the outputs and from 4097 rows on a sixth of them differ by
+// rounding, and fused blocks call the library): keys are taken BN at a time, s = (q k) * fp32(log2 e / sqrt(d)) with the product rounded first,
 // p = exp2(s - m), l = fma(l, alpha, sum p), p rounded to dtype for the second product, output * (1 / l).  BN and the two orders of
 // a step are chosen by the length alone (launch): a step wholly below a block of BM complete query rows ("full") sums a lane's
 // p in register order and multiplies keys in the order in which the first product leaves them; the steps on the diagonal

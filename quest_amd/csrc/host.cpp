@@ -540,9 +540,10 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             }
             launched(rc, "QKV projection");
         }
-        // causal attention: the library's where ours does not take the heads or the caller has switched off the library kernel whose bits ours gives
+        // causal attention: the library's where ours does not take the heads, gives other bits (a 4-bit quantiser follows) or the caller has
+        // switched off the library kernel whose bits ours gives
         at::Tensor core = make({m, c64}, type, args.dev);
-        const int rc = at::globalContext().userEnabledFlashSDP()
+        const int rc = at::globalContext().userEnabledFlashSDP() && t <= QUEST_ATTENTION_SAME_BITS(head_dim)
                            ? quest_causal_attention(core.data_ptr(), heads.data_ptr(), (int)b, (int)t, (int)n_head, head_dim, dt, st) : QUEST_ERR_UNSUPPORTED;
         if (rc == QUEST_ERR_UNSUPPORTED) {
             const int64_t row = 3 * c64;

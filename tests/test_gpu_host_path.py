@@ -55,6 +55,30 @@ def test_block_native_equals_python(python_path, batch, seq):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize('head_dim,seq,ours', [(64, 4096, True), (64, 4097, False), (64, 4200, False), (128, 2048, True), (128, 2049, False), (128, 4200, False)])
+def test_sequences_beyond_the_pinned_bits_go_to_the_library(python_path, head_dim, seq, ours):
+    """Where the attention kernel's bits are not the library's any more, a native block calls the library."""
+    from quest_amd import llama
+    torch.manual_seed(4)
+    with torch.device(DEV):
+        net = llama.Llama(llama.LlamaConfig(n_layer=1, n_embd=512, n_head=512 // head_dim, vocab_size=256, sequence_length=seq)).to(torch.bfloat16).eval()
+        ids = torch.randint(0, 256, (1, seq))
+    net = llama.quantize_model(net, 'int4', fuse_producers=True)
+    with torch.no_grad():
+        got, calls = _attention_calls(lambda: net(ids, all_logits=True)['logits'])
+        assert calls == (0 if ours else 1)
+        python_path()
+        want = net(ids, all_logits=True)['logits']
+    assert torch.equal(got, want)
+
+
+def _attention_calls(call):
+    """The call's result and how often it went to the library's attention."""
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        result = call()
+    return result, sum(e.count for e in prof.key_averages() if e.key == 'aten::scaled_dot_product_attention')
+
+
 def test_declined_calls_raise_as_before():
     import quest_amd as quest
     x = torch.zeros(4, 256, dtype=torch.bfloat16, device=DEV)
