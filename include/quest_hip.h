@@ -403,7 +403,7 @@ int quest_dense_rows(void *out, const void *x, const void *weight, int size_m, i
  * Up to QUEST_ATTENTION_SAME_BITS rows of a sequence the outputs are those of torch's own kernel (torch 2.10 on gfx950) bit for bit; beyond,
  * that kernel sums in another order and the two differ by rounding.
  */
-#define QUEST_ATTENTION_SAME_BITS(head_dim) ((head_dim) == 64 ? 4096 : 2048)
+#define QUEST_ATTENTION_SAME_BITS(head_dim) ((head_dim) == 64 ? 4096 : (head_dim) == 128 ? 2048 : 0)
 int quest_causal_attention(void *out, const void *qkv, int batch, int seq, int n_head, int head_dim, int dtype, void *stream);
 
 #ifdef __cplusplus

@@ -481,6 +481,13 @@ Codes normed(at::Tensor &x, const at::Tensor *branch, const at::Tensor &weight, 
     return q;
 }
 
+// whether scaled_dot_product_attention would run the flash kernel whose bits ours gives: not switched off, no backend put before it
+// (sdpa_kernel's set_priority), no other flash library preferred
+bool default_flash_attention() {
+    at::Context &ctx = at::globalContext();
+    return ctx.userEnabledFlashSDP() && ctx.sDPPriorityOrder()[0] == at::SDPBackend::flash_attention && ctx.getROCmFAPreferredBackend() != at::ROCmFABackend::Ck;
+}
+
 PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (n_args != 15) return declined();
     HANDLE_TH_ERRORS
@@ -540,11 +547,14 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             }
             launched(rc, "QKV projection");
         }
-        // causal attention: the library's where ours does not take the heads, gives other bits (a 4-bit quantiser follows) or the caller has
-        // switched off the library kernel whose bits ours gives
-        at::Tensor core = make({m, c64}, type, args.dev);
-        const int rc = at::globalContext().userEnabledFlashSDP() && t <= QUEST_ATTENTION_SAME_BITS(head_dim)
-                           ? quest_causal_attention(core.data_ptr(), heads.data_ptr(), (int)b, (int)t, (int)n_head, head_dim, dt, st) : QUEST_ERR_UNSUPPORTED;
+        // causal attention: the library's where ours does not take the heads, gives other bits (a 4-bit quantiser follows) or is not in the
+        // place of the library kernel that the caller's choice of backends names
+        at::Tensor core;
+        int rc = QUEST_ERR_UNSUPPORTED;
+        if (t <= QUEST_ATTENTION_SAME_BITS(head_dim) && default_flash_attention()) {
+            core = make({m, c64}, type, args.dev);
+            rc = quest_causal_attention(core.data_ptr(), heads.data_ptr(), (int)b, (int)t, (int)n_head, head_dim, dt, st);
+        }
         if (rc == QUEST_ERR_UNSUPPORTED) {
             const int64_t row = 3 * c64;
             const auto part = [&](int64_t i) { return heads.as_strided({b, n_head, t, head_dim}, {t * row, head_dim, row, 1}, i * c64); };

@@ -72,6 +72,32 @@ def test_sequences_beyond_the_pinned_bits_go_to_the_library(python_path, head_di
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('head_dim,backends,ours', [
+    (64, None, True), (128, None, True), (32, None, False), (96, None, False), (64, ['EFFICIENT_ATTENTION'], False), (128, ['EFFICIENT_ATTENTION'], False),
+    (64, ['EFFICIENT_ATTENTION', 'FLASH_ATTENTION'], False), (64, ['FLASH_ATTENTION', 'EFFICIENT_ATTENTION'], True), (64, ['FLASH_ATTENTION'], True)])
+def test_attention_is_the_one_that_the_caller_chose(python_path, head_dim, backends, ours, dtype):
+    """Heads that the attention kernel does not take, and any choice of backends in which flash is not the first, go to the library, with
+    the bits of the Python statements.  (Never the math backend: its batched products on transposed operands have faulted.)"""
+    import contextlib
+
+    from torch.nn.attention import SDPBackend, sdpa_kernel
+
+    from quest_amd import llama
+    torch.manual_seed(5)
+    with torch.device(DEV):
+        net = llama.Llama(llama.LlamaConfig(n_layer=2, n_embd=384, n_head=384 // head_dim, vocab_size=256)).to(dtype).eval()
+        ids = torch.randint(0, 256, (2, 100))
+    net = llama.quantize_model(net, 'int4', fuse_producers=True)
+    chosen = lambda: contextlib.nullcontext() if backends is None else sdpa_kernel([getattr(SDPBackend, b) for b in backends], set_priority=True)      # noqa: E731
+    with torch.no_grad(), chosen():
+        got, calls = _attention_calls(lambda: net(ids, all_logits=True)['logits'])
+        assert calls == (0 if ours else 2)
+        python_path()
+        want = net(ids, all_logits=True)['logits']
+    assert torch.equal(got, want)
+
+
 def _attention_calls(call):
     """The call's result and how often it went to the library's attention."""
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
