@@ -517,8 +517,8 @@ static constexpr Shape kShapes[] = {
     {true, 1, 1, 2.31f, 0.0568f, 1.10f, 0.044f},   {true, 1, 2, 2.28f, 0.0772f, 1.13f, 0.053f},   {true, 2, 2, 2.22f, 0.1246f, 1.30f, 0.018f},
     {true, 4, 2, 0.37f, 0.1900f, 4.62f, -0.014f}};
 
-// Up to half a 256 x 256 tile per CU the smaller tiles are the faster ones (1.01 to 4 x at all of those sizes); from 129 tiles on the
-// 256 x 256 kernel is, by 5 to 40 %.
+// Up to half a 256 x 256 tile per CU the smaller tiles are faster than those (1.01 to 4 x at all of those sizes); from 129 tiles on
+// they are slower, by 5 to 40 %.
 static const Shape *smaller_shape(int M, int K, int N, int cus, float &best_us) {
     best_us = 0.f;
     if (2L * ((M + 255) / 256) * ((N + 255) / 256) > cus) return nullptr;
@@ -534,11 +534,22 @@ static const Shape *smaller_shape(int M, int K, int N, int cus, float &best_us) 
 
 // Whether the kernel that keeps a channel tile's weights in LDS takes a size: rows that fit (K <= kResidentMaxK), outputs in whole 16-byte
 // pieces, and an estimate below the smaller tiles' (106 sizes, K 512 to 1536, 512 to 5500 tokens: up to 1.5 x faster than the kernel
-// before; (1000, 3072) at K = 1024 11.5 us against 9.5 stays with the smaller tiles).  Larger sizes all gain, 1.05 to 1.5 x.  Below 512 tokens
-// or elements of K one tile's weights cost more than its products.
+// before; (1000, 3072) at K = 1024 11.5 us against 9.5 stays with the smaller tiles).  Below 512 tokens or elements of K one tile's weights
+// cost more than its products.  Where 256 x 256 tiles are the alternative (1040 sizes, hot weights and weights from HBM), two plans are not
+// the faster ones.  One workgroup per tile leaves the others idle: with 21 of 32 busy 0.98 to 1.8 x the speed, with fewer (more than 16384
+// channels) 0.91 to 1.3 ((700, 1664, 16640) 25.3 against 22.9 us, (2048, 1024, 16640) 42.8 against 39.0).  Even runs have every XCD
+// fetch all weights, which few tokens do not hide: 0.81 to 0.97 up to 4096 tokens ((3000, 1536, 16640) 89.8 against 73.1, (3769, 1664, 2096)
+// 20.8 against 17.8), with many channels up to 4864 ((4827, 1280, 17536) 110.5 against 103.2, (4650, 1280, 10416) 63.7 against 59.3);
+// 0.97 to 1.8 beyond.
 static bool resident_takes(int M, int K, int N, int cus, float smaller_us, int epi) {
     if (M < 512 || K < 512 || K > kResidentMaxK || (N & (epi == kEpiGlu ? 15 : 7)) != 0 || cus < 8) return false;
-    return smaller_us == 0.f || gemm_e2m3_resident_plan(M, K, N, cus, nullptr) < smaller_us;
+    int plan[8];
+    const float us = gemm_e2m3_resident_plan(M, K, N, cus, plan);
+    if (smaller_us != 0.f) return us < smaller_us;
+    const int per_tile = plan[2], ways_t = plan[3], channels = plan[5];
+    if (per_tile == 0) return M > (N <= 8192 ? 4096 : 4864);
+    const int tiles = ((N + channels - 1) / channels * ways_t + 7) / 8;      // of an XCD
+    return 20 * tiles * per_tile >= 13 * (cus / 8);                          // 21 of 32
 }
 
 template <int EPI>

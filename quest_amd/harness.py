@@ -25,8 +25,10 @@ E2M3_MIN_TOKENS = 33                    # a fused block: from here on (see block
 E2M3_MIN_K = 1536                       # shortest rows that take them at more than E2M3_SHORT_ROWS_TOKENS tokens
 E2M3_MIN_K_NARROW = 2048                # ... by a layer of fewer than E2M3_NARROW channels
 E2M3_NARROW = 1536
-E2M3_RESIDENT_MAX_K = 1664              # longest rows of the FP6 kernel that keeps a channel tile's weights in LDS
 E2M3_SHORT_ROWS_TOKENS = 4096
+E2M3_RESIDENT_MAX_K = 1664              # longest rows of the FP6 kernel that keeps a channel tile's weights in LDS
+E2M3_RESIDENT_WIDE = 16384              # ... which takes more channels only at more than
+E2M3_RESIDENT_WIDE_TOKENS = 4864        # so many tokens (and, at fewer, some that the INT8 kernels keep)
 # Whether a producer-fused block lets the FP6 GEMM of an output projection add into the residual stream itself
 # (same bits as the addition inside the next norm kernel; one pass over the stream less).
 GEMM_ADDS_RESIDUAL = True
@@ -68,7 +70,8 @@ def block_prefers_e2m3(m: int, k: int, n: int) -> bool:
     the GEMM: (16384, 1024) x 1024 with the residual 1.28, x 3072 rotary 1.35, x 5632 gated 1.55; (16384, 768) x 1024 1.24; (8192,
     768) x 5632 1.36."""
     return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and _tiles_addressable(m, k, n)
-            and (m <= E2M3_SHORT_ROWS_TOKENS or _enough_per_row(k, n) or (768 <= k <= E2M3_RESIDENT_MAX_K and n % 16 == 0)))
+            and (m <= E2M3_SHORT_ROWS_TOKENS or _enough_per_row(k, n) or
+                 (768 <= k <= E2M3_RESIDENT_MAX_K and n % 16 == 0 and (n <= E2M3_RESIDENT_WIDE or m > E2M3_RESIDENT_WIDE_TOKENS))))
 
 
 def _tiles_addressable(m: int, k: int, n: int) -> bool:

@@ -100,3 +100,21 @@ def test_e2m3_plan_names_the_kernel_that_runs():
             tiles = -(-m // rows) * -(-n // channels)
             assert plan[6] >= 3 and (rows == 256 == channels or tiles <= plan[0] < tiles + 8)
     assert lib.quest_e2m3_gemm_plan(200, 100, 64, 256, plan) == -2
+
+
+def test_e2m3_short_rows_take_the_resident_kernel_where_it_is_the_faster_one():
+    """Rows of 512 to 1664 elements on 256 compute units: 256 x 256 tiles where the kernel that keeps a channel tile in LDS would leave
+    workgroups idle or fetch all weights eight times for few tokens (measured 3 to 19 % slower there)."""
+    from quest_amd import _lib, harness
+    lib = _lib.load()
+    plan = (ctypes.c_int * 8)()
+    large = [(512, 1408, 16640), (700, 1664, 16640), (658, 1408, 16832), (700, 1664, 19584), (2048, 1024, 16640), (2048, 1536, 18112),
+             (3000, 1536, 16640), (3000, 640, 18112), (4000, 1024, 18112), (3913, 1536, 17712), (4827, 1280, 17536),
+             (3769, 1664, 2096), (4061, 1536, 2104), (4650, 1280, 10416)]
+    resident = [(563, 1024, 22016), (1022, 1024, 22016), (3000, 1024, 22016), (5000, 1536, 16640), (8192, 1024, 18112), (1000, 1536, 11264), (6000, 1024, 13824),
+                (4227, 1536, 3192), (4542, 1664, 1808), (5003, 1024, 10448)]
+    for sizes, rows in ((large, 256), (resident, 64)):
+        for m, k, n in sizes:
+            assert lib.quest_e2m3_gemm_plan(m, k, n, 256, plan) == 0 and plan[4] == rows, (m, k, n, list(plan))
+    # a fused block goes back to the INT8 kernels with it
+    assert not harness.block_prefers_e2m3(4200, 1024, 17536) and harness.block_prefers_e2m3(5000, 1024, 17536) and harness.block_prefers_e2m3(4200, 1024, 11264)
