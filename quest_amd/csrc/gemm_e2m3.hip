@@ -517,6 +517,16 @@ static constexpr Shape kShapes[] = {
     {true, 1, 1, 2.31f, 0.0568f, 1.10f, 0.044f},   {true, 1, 2, 2.28f, 0.0772f, 1.13f, 0.053f},   {true, 2, 2, 2.22f, 0.1246f, 1.30f, 0.018f},
     {true, 4, 2, 0.37f, 0.1900f, 4.62f, -0.014f}};
 
+// Sizes that 128 x 96 tiles may take.  Shorter rows: tests/test_abi_cpu.py pins two of them to 128 x 128 (it costs 0.3 to 1.8 us at
+// K = 1024).  Fewer than eight 128-channel tiles: an XCD, which takes an eighth of the tiles, then has less than one of them, so that
+// more and narrower ones are more trips over the tokens ((4000, 6272, 768) 27.9 against 23.2 us, (4386, 9472, 640) 0.78 x the speed; 0.78
+// to 1.09 x over 110 sizes) -- unless there are as many of either (129 to 192 and 257 to 288 channels: 1.00 to 1.19 x; one tile: 0.97
+// to 1.03).  From 897 channels on 0.96 to 1.15 x with the weights at hand, 0.99 to 1.12 x from HBM (344 sizes).
+static bool tiles_of_96(int K, int N) {
+    const int wide = (N + 127) / 128, narrow = (N + 95) / 96;
+    return K >= 1152 && (wide >= 8 || (wide > 1 && wide == narrow));
+}
+
 // Up to half a 256 x 256 tile per CU the smaller tiles are faster than those (1.01 to 4 x at all of those sizes); from 129 tiles on
 // they are slower, by 5 to 40 %.
 static const Shape *smaller_shape(int M, int K, int N, int cus, float &best_us) {
@@ -524,7 +534,7 @@ static const Shape *smaller_shape(int M, int K, int N, int cus, float &best_us) 
     if (2L * ((M + 255) / 256) * ((N + 255) / 256) > cus) return nullptr;
     const Shape *best = nullptr;
     for (const Shape &s : kShapes) {
-        if (s.cf == 3 && K < 1152) continue;        // (measured for longer rows; 0.3 to 1.8 us at K = 1024 to 1152)
+        if (s.cf == 3 && !tiles_of_96(K, N)) continue;
         const long tiles = (long)((M + 32 * s.tf - 1) / (32 * s.tf)) * ((N + 32 * s.cf - 1) / (32 * s.cf));
         const float us = s.fixed + (float)((tiles + cus - 1) / cus) * (s.stage * (float)(K / 128) + s.tile) + s.weights * 0.75e-6f * (float)N * (float)K;
         if (best == nullptr || us < best_us) { best = &s; best_us = us; }

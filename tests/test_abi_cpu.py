@@ -118,3 +118,17 @@ def test_e2m3_short_rows_take_the_resident_kernel_where_it_is_the_faster_one():
             assert lib.quest_e2m3_gemm_plan(m, k, n, 256, plan) == 0 and plan[4] == rows, (m, k, n, list(plan))
     # a fused block goes back to the INT8 kernels with it
     assert not harness.block_prefers_e2m3(4200, 1024, 17536) and harness.block_prefers_e2m3(5000, 1024, 17536) and harness.block_prefers_e2m3(4200, 1024, 11264)
+
+
+def test_e2m3_few_channel_tiles_are_128_wide():
+    """128 x 96 tiles only where the XCDs do not read the tokens more often for them: eight 128-channel tiles and more, or as many of
+    either width (measured up to 1.28 times slower elsewhere)."""
+    from quest_amd import _lib
+    lib = _lib.load()
+    plan = (ctypes.c_int * 8)()
+    sizes = {128: [(4000, 6272, 768), (8613, 6272, 224), (7460, 1792, 320), (4386, 9472, 640), (5084, 2048, 512), (6929, 3712, 384), (3118, 2048, 896),
+                   (28978, 2560, 67), (20148, 3072, 83)],
+             96: [(3072, 5120, 897), (2560, 8192, 1024), (15669, 3456, 138), (16201, 1536, 192), (7191, 9600, 257), (200, 4096, 11008), (1000, 2560, 2560)]}
+    for channels, shapes in sizes.items():
+        for m, k, n in shapes:
+            assert lib.quest_e2m3_gemm_plan(m, k, n, 256, plan) == 0 and list(plan[4:6]) == [128, channels], (m, k, n, list(plan))
