@@ -15,7 +15,7 @@ reference takes it):
   noop            no-op linears (they still rotate their input), torch glue   (reference: noop)
   fused           int4_had with the producer-fused blocks: norm / residual / SwiGLU inside the quantisers, rotary kernel
   fused_noop      the same blocks with the GEMMs returning zeros (an output projection that would add into the residual
-                  stream leaves it untouched): what of `fused` is not GEMM time
+                  stream leaves it untouched), with the attention kernel of the fused ones: what of `fused` is not GEMM time
 
     python -m quest_amd.bench_e2e [--model 1600m|213m] [--batch-sizes 1 2 4 8] [--matrix-path fp6|int8] [--json F] [--markdown F]
 
@@ -29,7 +29,8 @@ import json
 
 import torch
 
-from . import harness, llama
+from . import _lib, harness, llama
+from . import api as quest
 
 MODELS = {
     # gemm-quest/benchmarks/config_1600M.json
@@ -58,8 +59,26 @@ def build(mode: str, cfg: llama.LlamaConfig, device) -> llama.Llama:
     if mode == 'fused':
         return llama.quantize_model(model, 'int4', use_hadamard=True, fuse_gate_up=True, fuse_producers=True)
     if mode == 'fused_noop':
-        return llama.quantize_model(model, 'noop', use_hadamard=True, fuse_gate_up=True, fuse_producers=True)
+        model = llama.quantize_model(model, 'noop', use_hadamard=True, fuse_gate_up=True, fuse_producers=True)
+        for block in model.transformer.h:
+            block.attn.attention_core = _attention_of_fused_blocks(block.attn.n_head)
+        return model
     raise NotImplementedError(mode)
+
+
+def _attention_of_fused_blocks(n_head: int):
+    """No-op linears take a block's statement in Python, whose attention is torch's: the kernel that `fused` runs in its place, without
+    which the difference of the two would hold that of the two kernels."""
+    def core(qkv, freqs_cis, rotated=False):
+        b, t, c3 = qkv.shape
+        c = c3 // 3
+        if not rotated:
+            quest.rope_interleaved_(qkv, freqs_cis.contiguous(), 2 * c, c // n_head)
+        out = torch.empty(b, t, c, dtype=qkv.dtype, device=qkv.device)
+        _lib.check(_lib.load().quest_causal_attention(out.data_ptr(), qkv.data_ptr(), b, t, n_head, c // n_head, _lib.DTYPE_CODE[qkv.dtype],
+                                                      torch.cuda.current_stream().cuda_stream), 'causal_attention')
+        return out
+    return core
 
 
 @torch.inference_mode()

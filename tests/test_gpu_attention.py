@@ -100,3 +100,16 @@ def test_refused_calls():
     assert call(out.data_ptr(), qkv.data_ptr(), 1, 0, 1, 64) != 0 and call(out.data_ptr(), qkv.data_ptr(), 1, 1 << 30, 1, 64) != 0
     torch.cuda.synchronize()
     assert not out.any()
+
+
+@pytest.mark.parametrize('name', ['213m', '1600m'])
+def test_both_twins_of_the_sweep_run_the_same_attention(name):
+    """Fused blocks minus the same with no-op GEMMs prices the GEMMs: neither may run the library's attention."""
+    from quest_amd import bench_e2e, llama
+    cfg = llama.LlamaConfig(**{**bench_e2e.MODELS[name], 'n_layer': 1, 'vocab_size': 256})
+    ids = torch.randint(0, 256, (2, 70), device='cuda')
+    for mode in ('fused', 'fused_noop'):
+        net = bench_e2e.build(mode, cfg, torch.device('cuda'))
+        with torch.inference_mode(), torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+            assert net.hidden_states(ids).isfinite().all()
+        assert not [e.key for e in prof.key_averages() if 'scaled_dot_product' in e.key]
