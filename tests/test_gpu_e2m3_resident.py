@@ -7,7 +7,9 @@ import torch
 
 pytestmark = pytest.mark.gpu
 DEV = 'cuda:0'
-SHAPES = [(800, 512, 11008), (600, 640, 11024), (3000, 1024, 2056), (5503, 1664, 2056), (8200, 768, 3080), (2111, 1536, 5648), (16500, 1152, 6160)]
+# (the gated epilogue takes outputs in whole 16-byte pieces too: channels in whole sixteens)
+SHAPES = [(800, 512, 11008), (600, 640, 11024), (3000, 1024, 2064), (5503, 1664, 2064), (8200, 768, 3088), (2111, 1536, 5648), (16500, 1152, 6160)]
+EIGHTS = [(3000, 1024, 2056), (5503, 1664, 2056), (8200, 768, 3080)]        # ... and these run the gated epilogue on other kernels
 
 
 def _plan(m, k, n):
@@ -18,7 +20,7 @@ def _plan(m, k, n):
 
 
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize('m,k,n', SHAPES)
+@pytest.mark.parametrize('m,k,n', SHAPES + EIGHTS)
 def test_every_epilogue_equals_the_int8_kernels(dtype, m, k, n):
     import quest_amd as quest
     from quest_amd import _lib, harness
@@ -57,6 +59,12 @@ def test_every_epilogue_equals_the_int8_kernels(dtype, m, k, n):
         freqs = torch.stack([torch.cos(ang), torch.sin(ang)], dim=-1).contiguous()
         turned = quest.rope_interleaved_(want[:rows].clone().view(-1, seq, n), freqs, rot, head_dim).view(rows, n)
         assert torch.equal(quest.fused_matmul_dequantize_e2m3(quest.int4_to_e2m3_tiles(a[:rows].contiguous()), tb, a_mul[:rows], b_mul, k, rope=(freqs, rot, head_dim)), turned)
+
+
+def test_the_shapes_take_both_kinds_of_plan():
+    """One or several workgroups per channel tile, and even runs over an XCD's tiles; every shape also gated."""
+    shared = [_plan(*s)[2] for s in SHAPES]
+    assert 0 in shared and 1 < max(shared) and all(n % 16 == 0 for _, _, n in SHAPES)
 
 
 def test_scales_at_the_edge_of_the_range():
