@@ -495,7 +495,7 @@ def bench_small_layer_gpu(quest, dev):
         quest.fused_matmul_dequantize_int4_int4t_bf16(packed, wp, row_sum, wa, scale, ws, out)
 
     ms = launches_ms(layer, 100, 10)
-    # the checker: activation codes of this workload against the full CPU oracle pipeline on the same x (the
+    # checked: activation codes of this workload against the full CPU oracle pipeline on the same x (the
     # reference's F.linear Hadamard, torch-CPU scale, quantiser), and the layer output against the oracle's
     from oracle import quest_oracle as qo
     _, o_scale, o_packed, _ = qo.hadamard_quantize_int4(x.cpu(), hadamard='matmul')

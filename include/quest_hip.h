@@ -325,7 +325,8 @@ int quest_fused_matmul_dequantize_rope_e2m3(void *mat_d, const void *a_tiles, co
  * Shapes of at most half a 256 x 256 tile per compute unit run on smaller tiles, one per workgroup, dealt to the XCDs in contiguous
  * eighths (plan[1..3] = 8, 0, 0): 128 k per slot where the waves share the tile, 64 where each has a quarter of K and slots of
  * its own.  Rows of 512 to 1664 elements whose channel tiles stay in LDS report 64 x 128 and k per slot = size_k; plan[2] is then
- * how many workgroups of an XCD share a channel tile (0: they divide its tiles into even runs).  A measured figure that depends on
+ * how many workgroups of an XCD share a channel tile (0: they divide its tiles into even runs).  The plan is that of the plain epilogue; every
+ * other one has the same, but for the gated one with size_n % 16 != 0, which rows of 512 to 1664 elements run on the tiles named first.  A measured figure that depends on
  * the schedule (HBM traffic per launch) is only valid while this plan is the one it was measured under.
  */
 int quest_e2m3_gemm_plan(int size_m, int size_k, int size_n, int cus, int *plan);

@@ -1,5 +1,5 @@
-// The epilogue that the two smaller-tile FP6 GEMM kernels (gemm_e2m3_mid.hip, gemm_e2m3_split.hip) share: eight consecutive
-// channels of one token row, rounded to the dtype, on their way to memory.
+// What the FP6 GEMM kernels beside gemm_e2m3.hip share: the description of an epilogue and their entry points, and for the two
+// smaller-tile kernels (gemm_e2m3_mid.hip, gemm_e2m3_split.hip) the way of eight consecutive channels of one token row, rounded to the dtype, to memory.
 #pragma once
 #include "gemm_tiles.h"
 

@@ -504,8 +504,8 @@ static int launch_large(int dtype, void *out, const uint8_t *a, const uint8_t *b
 // N from 1024 to 22016, weights rotating through several copies): the shape with the smallest estimate is within 0.9 % of
 // always picking the fastest one in total time, within 16 % on every single size.  With weights from HBM (copies of more than 320
 // MB, 816 sizes, K from 256) it is within 1.4 % in total and 20 % on every size; on rows of 16384 to 65536, beyond the fit and its
-// negative coefficients, within 0.1 and 3 %.  {4, 3}'s line is {4, 4}'s and the difference of the two measured at 44 sizes (one tile per CU,
-// K from 1152 to 9600: 0.65 + 0.031 K / 128 us less).
+// negative coefficients, within 0.1 and 3 %.  (All of this for the ten other shapes.)  {4, 3} was not fitted: its line is {4, 4}'s and the
+// difference of the two measured at 44 sizes (one tile per CU, K from 1024 to 9600: 0.65 + 0.031 K / 128 us less); see tiles_of_96.
 struct Shape {
     bool split;
     int tf, cf;

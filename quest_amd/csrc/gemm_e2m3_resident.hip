@@ -11,7 +11,7 @@
 // two one after the other.  Hence the doubled products (one addition per output less), four channels' scales unpacked once for both
 // row blocks, and stores of 64 bytes per row (32 rows x 32 bytes at a power-of-two pitch meet in one L2 channel: rotary 55.2, now 50.3 us).
 // Against the 256 x 256 kernel and the INT8 one, us, weights rotating through copies of 400 MB, K = 1024: (16384, 3072) rotary 50 / 62 / 68,
-// (16384, 1024) residual 20 / 25 / 26, (16384, 5632) gated 68 / 99 / 105, (3000, 2048) 9.8 / 13.8 / 15.0; (9000, 1536, 4096) 36 / 48 / 58.
+// (16384, 1024) residual 21 / 25 / 27, (16384, 5632) gated 73 / 105 / 103 (71 / 110 / 105 with the weights at hand), (3000, 2048) 9.8 / 13.8 / 15.0; (9000, 1536, 4096) 36 / 48 / 58.
 // Stores past the caches (nt) take twice to three times as long, write-through ones a fifth longer.
 #include "e2m3_epilogue.h"
 
@@ -315,7 +315,8 @@ gemm_e2m3_resident_kernel(void *__restrict__ out, const uint8_t *__restrict__ ac
 // Of the ways to divide the output among the XCDs and their workgroups the one with the least estimated time, in us: 2.5 for the launch, for
 // every four blocks of a workgroup (one per SIMD) 3.2 of epilogue and 1.9 per 1024 k of products, 3 for every channel tile that it loads, 0.1 per
 // MB that the XCDs fetch.  Whole tiles per workgroup, or, where every XCD has an eighth of the tokens, even runs over its tiles (its L2 then
-// holds its tokens; with a quarter of them, (16384, 1024, 5632) gated takes 79.8 instead of 73.8 us).  The estimate orders the
+// holds its tokens; a quarter of them and half the channels is no faster on the whole: (16384, 1024, 5632) gated 70 us against 73, (16384, 1024, 3072)
+// rotary 53 / 52, (16384, 1024, 1024) residual 23 / 21).  The estimate orders the
 // eight plans of thirteen sizes as measured but for differences of 5 %; for one to three rounds it is within 15 % of the time itself.
 static Plan make_plan(int M, int K, int N, int cus, float *us_out) {
     const int groups_t = (M + kRows - 1) / kRows, tiles_c = (N + kChannels - 1) / kChannels, per = cus / 8;

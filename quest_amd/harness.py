@@ -39,13 +39,15 @@ GEMM_ROTATES_QK = True
 
 def prefers_e2m3(m: int, k: int, n: int) -> bool:
     """Whether the FP6 kernels are the faster ones for an (m, k) x (n, k) layer on its own, quantiser included, with weights that come
-    from HBM (copies of more than 300 MB in turn): 2096 sizes, K 128 to 11008, N 136 to 22016, M 33 to 4096.  The path taken is
-    within 0.8 % of the faster one on average (always FP6: 3.0 %) and, from K = 640 on, within 16 % everywhere."""
+    from HBM (copies of more than 300 MB in turn).  The lines were drawn over 2096 sizes, K 128 to 11008, N 136 to 22016, M 33 to 4096,
+    with the FP6 kernels before gemm_e2m3_resident.hip, and have not been drawn again.  With today's kernels the path taken is 2.9 % behind
+    the faster one on average over 220 sizes of these ranges (always FP6: 1.2 %), and 10 % over 260 sizes with rows of 640 to 1664
+    elements and 512 tokens and more (0.5 %), most at more than 4096 tokens with K < 1536 ((6618, 1280, 9712) 1.69)."""
     if m < 49 or k % 128 or MATRIX_PATH != 'fp6' or not _tiles_addressable(m, k, n):      # (a few tokens first: their calls are host-bound)
         return False
     if m > E2M3_SHORT_ROWS_TOKENS:
         return _enough_per_row(k, n)
-    # K < 640: as often slower as faster (K = 128: 0.83 at (2000, 22016), 1.47 at (700, 11008); K = 512: 0.88 to 1.41)
+    # K < 640: as often slower as faster (K = 128: 0.86 at (2000, 22016), 1.49 at (700, 11008); K = 512: 0.88 to 1.42)
     if k < 640:
         return False
     # Some tens of tokens: the weights are the cost, and the tiles are 1.5 x the codes' bytes.  (INT8 / FP6 time: (33, 11008, 11008)
@@ -59,7 +61,7 @@ def prefers_e2m3(m: int, k: int, n: int) -> bool:
     tiles = ((m + 63) >> 6) * ((n + 63) >> 6)
     if tiles <= 512:
         return tiles <= 128 or (tiles > 256 and k < 4096)
-    return not (m > 3000 and k < 1536 and 512 <= n <= 2048)           # (4096, 1024, 2048) 0.90, (4096, 1280, 512) 0.95
+    return not (m > 3000 and k < 1536 and 512 <= n <= 2048)           # (4096, 1280, 512) 0.96; (4096, 1024, 2048) 1.11 by now
 
 
 def block_prefers_e2m3(m: int, k: int, n: int) -> bool:
@@ -67,8 +69,8 @@ def block_prefers_e2m3(m: int, k: int, n: int) -> bool:
     unit and both residual additions ride in their epilogues at every size).  Whole blocks, d = 256 to 4096, 33 to 4000 tokens,
     weights from HBM, INT8 / FP6 time: 0.97 to 1.18 ((d = 768, 1000 tokens) 0.97, (2560, 200) 0.99, (1024, 37) 1.08, (2560, 64)
     1.14, (4096, 500) 1.17).  Many tokens with short rows have a kernel of their own (gemm_e2m3_resident.hip), INT8 / FP6 time of
-    the GEMM: (16384, 1024) x 1024 with the residual 1.28, x 3072 rotary 1.35, x 5632 gated 1.55; (16384, 768) x 1024 1.24; (8192,
-    768) x 5632 1.36."""
+    the GEMM: (16384, 1024) x 1024 with the residual 1.28, x 3072 rotary 1.35, x 5632 gated 1.40; (16384, 768) x 1024 1.26; (8192,
+    768) x 5632 1.45."""
     return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and _tiles_addressable(m, k, n)
             and (m <= E2M3_SHORT_ROWS_TOKENS or _enough_per_row(k, n) or
                  (768 <= k <= E2M3_RESIDENT_MAX_K and n % 16 == 0 and (n <= E2M3_RESIDENT_WIDE or m > E2M3_RESIDENT_WIDE_TOKENS))))
@@ -81,9 +83,10 @@ def _tiles_addressable(m: int, k: int, n: int) -> bool:
 def _enough_per_row(k: int, n: int) -> bool:
     # With short rows and many tokens the GEMM is mostly epilogue either way and the tile-writing activation kernels are a little
     # slower than the row-writing ones (12.0 against 10.2 us at [16384, 1024]).  Whole layers of 4097 to 16384 tokens, INT8 / FP6
-    # time: K = 1536 1.12 on average over N from 1500 to 22016, K = 1792 1.14, K = 1920 1.16 ((4097, 1536, 1536) 33.7 / 27.4 us,
-    # (8192, 1536, 8192) 103 / 84, (16384, 1536, 3072) 85 / 70); K = 1024 0.85 to 1.18 ((16384, 1024, 8192) 148 / 173 us), K = 1152
-    # to 1408 0.94 to 1.27.  Layers of 1024 channels lose 6 to 12 % at 8192 tokens up to K = 1920 (half a 256 x 256 tile per CU).
+    # time on the 256 x 256 tiles: K = 1792 1.14, K = 1920 1.16; K = 1024 0.85 to 1.18, K = 1152 to 1408 0.94 to 1.27.  Layers of 1024
+    # channels lose 6 to 12 % at 8192 tokens up to K = 1920 (half a 256 x 256 tile per CU).  The resident channel tile has changed that up
+    # to K = 1664 ((4097, 1536, 1536) 32.8 / 24.1 us, (8192, 1536, 8192) 120 / 78, (16384, 1536, 3072) 92 / 71): K = 640 to 1408 1.0 to 1.69 but for
+    # less than 1024 channels ((16384, 1024, 8192) 164 / 117; (7883, 640, 904) 0.81).  Fused blocks follow it, layers on their own not yet.
     return k >= (E2M3_MIN_K if n >= E2M3_NARROW else E2M3_MIN_K_NARROW)
 
 
