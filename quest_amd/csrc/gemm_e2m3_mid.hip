@@ -6,7 +6,9 @@
 // direct loads of 1 KiB per row block (the heads of its two fragments, then both tails), laid out in LDS as they come, so that a
 // fragment is one ds_read_b128 and one ds_read_b64 at lane-linear addresses.  While one 64-k step is multiplied from registers the
 // next one's fragments are read; one barrier per stage, in the second step, tells that the next stage has landed everywhere and
-// that this stage's slot is free for the loads of the stage kStages further on.  A tile's scale values are fetched at its start.
+// that this stage's slot is free for the loads of the stage kStages further on.  A tile's scale values are fetched at its start, as buffer
+// loads whose range check stands for the matrix' edges: with a branch per value the first stage's loads set out 0.3 to 0.8 us later ((1000,
+// 512, 3072) 7.7 -> 7.0 us, (1200, 896, 2304) 8.6 -> 7.8, (333, 1024, 11000) 11.7 -> 10.8, (1000, 2560, 7680) 21.6 -> 20.3).
 // What bounds it: the LDS port, which a stage's bytes cross once on their way in and twice on their way to the waves that share them
 // (72 KiB per stage of a 128 x 128 tile: 576 cycles at 128 bytes a cycle, 600 measured, against 256 of matrix work), and with one
 // tile per CU the trip to memory before the first stage and the epilogue after the last, together 5 us.
@@ -15,6 +17,8 @@
 // (96 KiB through LDS).  They fill 216 of 256 CUs where 128 x 128 has 160 tiles: (1000, 6912, 2560) 22.7 -> 20.5 us, (516, 1152, 3695)
 // 15.9 -> 14.1, (197, 9600, 8324) 37.6 -> 34.2.  128 x 128 by pairs is 1 to 4 % slower than 2 x 2 waves: a stage's fragments are all read behind
 // its one barrier.
+// Token fragments straight into registers (no two waves of the pairs need the same ones: 27 KiB a stage through the port) with the channels'
+// read a stage ahead are no faster (0.97 to 1.03 x over 12 sizes): what is left of a stage is its bytes into the CU.
 // Measured against the kernels that took these sizes before (weights rotating through four copies): (200, 4096, 11008) 15.5 against
 // 19.9 us, (1000, 6912, 2560) 22.2 against 27.6, (1400, 2560, 2560) 12.9 against 26.9, (1400, 6912, 2560) 24.2 against 54.3.
 #include "e2m3_epilogue.h"
@@ -62,36 +66,29 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
     const int done0 = tf0 + half * kDone;                                // the token blocks that it finishes
 
     // the epilogue's scale values set out first: a lane finishes token li of each of its token blocks and, of each channel unit,
-    // channels 8 q + 4 lg ... + 3
-    float t_half_mul[kDone];
-    uint32_t c_mul[kC][8];
+    // channels 8 q + 4 lg ... + 3 (values past the vectors' ends read as zeros: their outputs are not stored)
+    const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc((void *)epi.a_mul, 0, M * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc((void *)epi.b_mul, 0, (N * 2 + 2) & ~3, 0x00020000);
+    uint16_t t_mul[kDone];
+    v2i c_mul[kC][4];
 #pragma unroll
-    for (int t = 0; t < kDone; t++) t_half_mul[t] = __fmul_rn(0.5f, to_f32<DT>(epi.a_mul[min(tok0 + 32 * (done0 + t) + li, M - 1)]));
+    for (int t = 0; t < kDone; t++) t_mul[t] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(ar, (tok0 + 32 * (done0 + t) + li) * 2, 0, 0);
 #pragma unroll
     for (int c = 0; c < kC; c++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int ch = ch0 + 32 * (cf0 + c) + 8 * q + 4 * lg;
-            if (ch + 3 < N) {
-                const uint32_t *p = reinterpret_cast<const uint32_t *>(epi.b_mul + ch);
-                c_mul[c][2 * q] = p[0];
-                c_mul[c][2 * q + 1] = p[1];
-            } else {
-#pragma unroll
-                for (int e = 0; e < 2; e++)
-                    c_mul[c][2 * q + e] = epi.b_mul[min(ch + 2 * e, N - 1)] | ((uint32_t)epi.b_mul[min(ch + 2 * e + 1, N - 1)] << 16);
-            }
-        }
+        for (int q = 0; q < 4; q++) c_mul[c][q] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(br, (ch0 + 32 * (cf0 + c) + 8 * q + 4 * lg) * 2, 0, 0));
     // ... and what the epilogue adds or rotates by
     const bool vec16 = (N & 7) == 0;
     Ahead<ROPE> ahead[kDone][kC][2];
+    if (ROPE || epi.kind == kEpiAdd || epi.kind == kEpiBias) {                      // uniform
 #pragma unroll
-    for (int t = 0; t < kDone; t++)
+        for (int t = 0; t < kDone; t++)
 #pragma unroll
-        for (int c = 0; c < kC; c++)
+            for (int c = 0; c < kC; c++)
 #pragma unroll
-            for (int pr = 0; pr < 2; pr++)
-                fetch_ahead<DT>(ahead[t][c][pr], out, epi, tok0 + 32 * (done0 + t) + li, ch0 + 32 * (cf0 + c) + (2 * pr + lg) * 8, M, N, vec16);
+                for (int pr = 0; pr < 2; pr++)
+                    fetch_ahead<DT>(ahead[t][c][pr], out, epi, tok0 + 32 * (done0 + t) + li, ch0 + 32 * (cf0 + c) + (2 * pr + lg) * 8, M, N, vec16);
+    }
 
     const int nk = K / 128;                                      // stages
     const int pitch = (K / 64) * kFragB;                         // bytes per row block
@@ -232,6 +229,7 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
 #pragma unroll
     for (int t = 0; t < kDone; t++) {
         const int tok = tok0 + 32 * (done0 + t) + li;
+        const float t_half_mul = __fmul_rn(0.5f, to_f32<DT>(t_mul[t]));
 #pragma unroll
         for (int c = 0; c < kC; c++) {
             const int cu = ch0 + 32 * (cf0 + c);
@@ -242,8 +240,8 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     const float s = acc[t][c][4 * q + e];
-                    const uint32_t m2 = c_mul[c][2 * q + (e >> 1)];
-                    v[e] = __fmul_rn(__fadd_rn(s, s), __fmul_rn(t_half_mul[t], e & 1 ? hi_f32<DT>(m2) : lo_f32<DT>(m2)));
+                    const uint32_t m2 = (uint32_t)c_mul[c][q][e >> 1];
+                    v[e] = __fmul_rn(__fadd_rn(s, s), __fmul_rn(t_half_mul, e & 1 ? hi_f32<DT>(m2) : lo_f32<DT>(m2)));
                 }
                 x[q][0] = pack2_rounded_products<DT>(v[0], v[1]);
                 x[q][1] = pack2_rounded_products<DT>(v[2], v[3]);

@@ -75,17 +75,23 @@ __device__ __forceinline__ void tile(uint8_t *lds, void *__restrict__ out, const
 #pragma unroll
         for (int i = 0; i < kIters; i++)
             t_half_mul[part][i] = __fmul_rn(0.5f, to_f32<DT>(epi.a_mul[min(tok0 + 32 * S::kPartBlocks * part + row0 + i * kRowsAtOnce, M - 1)]));
+    {   // (channels past the vector's end read as zeros: their outputs are not stored)
+        const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc((void *)epi.b_mul, 0, (N * 2 + 2) & ~3, 0x00020000);
+        const v4i m = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(br, ch * 2, 0, 0));
 #pragma unroll
-    for (int i = 0; i < 8; i++) muls[i] = to_f32<DT>(epi.b_mul[ch + i < N ? ch + i : N - 1]);
+        for (int i = 0; i < 8; i++) muls[i] = i & 1 ? hi_f32<DT>((uint32_t)m[i >> 1]) : lo_f32<DT>((uint32_t)m[i >> 1]);
+    }
     // ... and what the epilogue adds or rotates by
     Ahead<ROPE> ahead[TF / S::kPartBlocks][kIters];
+    if (ROPE || epi.kind == kEpiAdd || epi.kind == kEpiBias) {   // uniform
 #pragma unroll
-    for (int part = 0; part < TF / S::kPartBlocks; part++)
+        for (int part = 0; part < TF / S::kPartBlocks; part++)
 #pragma unroll
-        for (int i = 0; i < kIters; i++) {
-            const int row = row0 + i * kRowsAtOnce;
-            fetch_ahead<DT>(ahead[part][i], out, epi, tok0 + 32 * S::kPartBlocks * part + row, works && row < 32 * S::kPartBlocks ? ch : N, M, N, vec16);
-        }
+            for (int i = 0; i < kIters; i++) {
+                const int row = row0 + i * kRowsAtOnce;
+                fetch_ahead<DT>(ahead[part][i], out, epi, tok0 + 32 * S::kPartBlocks * part + row, works && row < 32 * S::kPartBlocks ? ch : N, M, N, vec16);
+            }
+    }
     // tails: lanes 0-31 bring fragment 2 j's 512 bytes, lanes 32-63 those of 2 j + 1 of the same matrix (or nothing)
     uint32_t tail_at[S::kTailLoads];
 #pragma unroll
