@@ -89,6 +89,17 @@ int quest_fused_matmul_dequantize_int4_int4t(void *mat_d, const uint8_t *mat_a, 
                                              int size_m, int size_k, int size_n, int dtype, void *stream);
 
 /*
+ * A whole W4A4 linear layer on a few tokens in one launch: out (size_m, size_n) dtype = what quest_hadamard_quantize_int4 (with had_scale) and
+ * quest_fused_matmul_dequantize_int4_int4t (with `bias`, or NULL) give one after the other, bit for bit, without scratch memory.  x
+ * (size_m, size_k) dtype, w_packed (size_n, size_k / 2), w_add and w_scale (size_n).  QUEST_ERR_UNSUPPORTED, with nothing
+ * launched, for what the two launches do better or this kernel cannot: more than 16 tokens of up to 2048 elements, 8 of up to 4096, 4 of up to
+ * 8192, 2 of up to 12288, rows of fewer than 513 or more than 12288, a had_scale that dtype does not hold.  With had_scale = 0 rows are whole 32s, else whole 128s
+ * (rows that are not whole 128s: the sum of squares runs in another order than that entry point's, so that a scale can differ by one unit in the last place).
+ */
+int quest_linear_few_tokens(void *out, const void *x, const uint8_t *w_packed, const int32_t *w_add, const void *w_scale, const void *bias,
+                            int size_m, int size_k, int size_n, float had_scale, int dtype, void *stream);
+
+/*
  * quest_fused_matmul_dequantize_int4_int4t with a caller-owned workspace, which lets a handful of tokens
  * (size_m <= 16: the decode shapes) split K across workgroups: every slice leaves its partial int32 tile in the
  * workspace and the workgroup that arrives last (a counter per channel tile, no atomics on the result) adds them --

@@ -27,38 +27,11 @@
 // two whole groups of 32 consecutive k, each output becomes the fp16 value q + 1/2 (floor of the same nudged quotient
 // the nibble path converts; the clamp is the saturation of the FP6 conversion) and v_cvt_scalef32_pk32_fp6_f16 packs
 // 32 of them into the lane's 24 bytes of its fragment.
-#include "common.h"
+#include "hadamard_unit.h"
 #include <type_traits>
 
 namespace quest {
 namespace hq {
-
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef int v4i __attribute__((ext_vector_type(4)));
-
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-
-// acc + lo(w)^2 + hi(w)^2 for a dword of two 16-bit floats (squares of 16-bit floats are exact in fp32)
-template <int DT>
-__device__ __forceinline__ float dot2_self(uint32_t w, float acc) {
-    if constexpr (DT == QUEST_DTYPE_BF16)
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, w), __builtin_bit_cast(v2bf, w), acc, false);
-    else
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(v2h, w), __builtin_bit_cast(v2h, w), acc, false);
-}
-
-template <int DT>
-__device__ __forceinline__ v16f mfma_h(const v4i &a, const v4i &b, const v16f &c) {
-    if constexpr (DT == QUEST_DTYPE_BF16)
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
-}
-
-typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
 // WPR waves share one row (32 blocks of 128 each); a workgroup holds one or two rows' worth of waves (small
 // workgroups: two-wave ones measured 3 % faster than four-wave ones for whole-wave rows, eight-wave ones 5 % slower).
@@ -88,30 +61,10 @@ struct Shape {
 //   kPreSiluMul  y = dtype(dtype(silu(gate)) * up), gate and up the two halves of a (M, 2 K) row (llama.py:117-118).
 enum { kPreNone = 0, kPreRmsNorm = 1, kPreSiluMul = 2 };
 
-// Sum over the G lanes (G a power of two, aligned) of each half-wave that hold one row, and over the two half-waves.
-template <int G>
-__device__ __forceinline__ float group_sum_f(float v) {
-    if constexpr (G >= 2) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));
-    if constexpr (G >= 4) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true));
-    if constexpr (G >= 8) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));
-    if constexpr (G >= 16) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, true));
-    if constexpr (G >= 32) v += lane_xor_f<16>(v);
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-template <int G>
-__device__ __forceinline__ int group_sum_i(int v) {
-    if constexpr (G >= 2) v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, true);
-    if constexpr (G >= 4) v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, true);
-    if constexpr (G >= 8) v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, true);
-    if constexpr (G >= 16) v += __builtin_amdgcn_update_dpp(0, v, 0x128, 0xF, 0xF, true);
-    if constexpr (G >= 32) v += lane_xor_i<16>(v);
-    const auto r = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
-    return (int)r[0] + (int)r[1];
-}
-
 // G = lanes of a half-wave per row (the row's blocks rounded up to a power of two): a wave holds 32 / G rows.
-template <int DT, int WPR, int G, int PRE, bool TL>
+// RAG: rows of whole 32s without the transform (K % 128 != 0): the last block is cut short, and tiles are those of the row with zeros behind it up
+// to a whole 128 (the FP6 zero, so that what stands there in the weights' tiles does not matter).
+template <int DT, int WPR, int G, int PRE, bool TL, bool RAG>
 __global__ void __launch_bounds__((64 * Shape<WPR, G, TL>::kWaves), (Shape<WPR, G, TL>::kMinBlocks))
 hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ norm_w,
                               uint16_t *__restrict__ scale, uint32_t *__restrict__ packed, int32_t *__restrict__ row_sum,
@@ -119,6 +72,7 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
                               uint16_t *sum_out, uint8_t *__restrict__ tiles, int xcd_chunk, int K, int M, int ldx,
                               uint32_t entry_bits, float eps, int sum_bias) {
     static_assert(WPR == 1 || G == 32, "rows shared by waves: whole waves");
+    static_assert(!RAG || PRE == kPreNone, "rows that end inside a block come from no producer");
     using Sh = Shape<WPR, G, TL>;
     constexpr int kRows = Sh::kRows;
     constexpr int kRowsPerWave = 32 / G;
@@ -135,33 +89,11 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
     const int vb = xcd_chunk > 0 ? (int)(blockIdx.x & 7) * xcd_chunk + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
     const int row = (vb * kRows + row_local) * kRowsPerWave + n / G;
     const int blk = part * 32 + n % G;         // block of the row in this column
-    const bool live = row < M && blk < (K >> 7);
+    const int n_blk = RAG ? (K + 127) >> 7 : K >> 7;
+    const bool live = row < M && blk < n_blk;
 
-    // ---- the four A fragments: +-entry with sign (-1)^(popcount(n & 7 & j) + n3 h) [* (-1)^n4] [* -1]
     v4i hv[2][2];
-    {
-        const uint32_t lane_flip = ((n >> 3) & 1) & h;
-        uint32_t base[4];
-#pragma unroll
-        for (int d = 0; d < 4; d++) {
-            uint32_t w = 0;
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const int j = 2 * d + e;
-                const uint32_t neg = (__builtin_popcount(n & 7 & j) & 1) ^ lane_flip;
-                w |= (entry_bits ^ (neg << 15)) << (16 * e);
-            }
-            base[d] = w;
-        }
-        const uint32_t s0_flip = ((n >> 4) & 1) ? 0x80008000u : 0u;
-#pragma unroll
-        for (int d = 0; d < 4; d++) {
-            hv[0][0][d] = (int)base[d];
-            hv[0][1][d] = (int)(base[d] ^ 0x80008000u);
-            hv[1][0][d] = (int)(base[d] ^ s0_flip);
-            hv[1][1][d] = (int)(base[d] ^ s0_flip ^ 0x80008000u);
-        }
-    }
+    signed_entries(hv, n, h, entry_bits);
 
     // ---- B fragments straight from HBM: chunk 2 s + h of a block is bytes [32 s + 16 h, +16) of its 256.
     // Lanes without a block get an offset beyond the buffer: such loads touch no memory and return zeros.
@@ -172,7 +104,8 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
     const uint32_t ld_off = live ? (uint32_t)(row * ldx * 2 + blk * 256 + h * 16) : dead;
     v4u bq[8];
 #pragma unroll
-    for (int s = 0; s < 8; s++) bq[s] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(ld_off + 32 * s), 0, 0);
+    for (int s = 0; s < 8; s++)
+        bq[s] = __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(!RAG || blk * 128 + 16 * s < K ? ld_off + 32 * s : dead), 0, 0);
     // all eight in flight before anything else: left alone the scheduler sinks the last two below the first MFMAs to
     // save registers, which costs every wave a second trip to memory
     __builtin_amdgcn_sched_barrier(0);
@@ -243,52 +176,8 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
         }
     }
 
-    // ---- Hadamard: 8 k-steps x 4 row tiles; then round to the dtype (the transform's output exists only in dtype) and
-    // sum the squares.  entry_bits == 0: no transform -- the loaded chunks are the outputs already and only have to
-    // change lanes: lane (n, h) loaded the chunks whose k has bit 3 equal to h and the code below wants those whose bit 2
-    // is h, so the two half-waves trade half of every chunk (nothing is multiplied: NaN and Inf stay where they are).
     uint32_t yb[4][8];                          // [mt][q * 2 + pair]: outputs 32 mt + 8 q + 4 h + {0,1} / {2,3}
-    float sumsq = 0.f;
-    if (entry_bits == 0) {                      // uniform
-#pragma unroll
-        for (int s = 0; s < 8; s++)
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                // outputs 16 s + 8 (q & 1) + 4 h + 2 p + {0, 1}: pair 2 h + p of the chunk held by the half-wave q & 1
-                const auto sw = __builtin_amdgcn_permlane32_swap(bq[s][p], bq[s][2 + p], false, false);
-#pragma unroll
-                for (int qo = 0; qo < 2; qo++) {
-                    const uint32_t w = sw[qo];
-                    yb[s >> 1][(2 * (s & 1) + qo) * 2 + p] = w;
-                    sumsq = dot2_self<DT>(w, sumsq);
-                }
-            }
-    } else {
-        v16f acc[4];
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[mt][r] = 0.f;
-#pragma unroll
-        for (int s = 0; s < 8; s++) {
-            const v4i b = __builtin_bit_cast(v4i, bq[s]);
-#pragma unroll
-            for (int mt = 0; mt < 4; mt++) {
-                const int neg = ((mt & 1) & ((s >> 1) & 1)) ^ (((mt >> 1) & 1) & ((s >> 2) & 1));
-                acc[mt] = mfma_h<DT>(hv[s & 1][neg], b, acc[mt]);
-            }
-        }
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-            for (int q = 0; q < 4; q++)
-#pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    const uint32_t w = pack2_rne<DT>(acc[mt][q * 4 + 2 * p], acc[mt][q * 4 + 2 * p + 1]);
-                    yb[mt][q * 2 + p] = w;
-                    sumsq = dot2_self<DT>(w, sumsq);            // both squares straight from the packed pair
-                }
-    }
+    const float sumsq = transform<DT>(yb, bq, hv, entry_bits);
     // lanes without a block transformed zeros: they add nothing
     float total = G == 32 ? wave_sum_dpp_f(sumsq) : group_sum_f<G>(sumsq);
     __shared__ float part_sq[Sh::kWaves];
@@ -322,7 +211,7 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
         typedef unsigned v16u __attribute__((ext_vector_type(16)));
         const float sf_t = to_f32<DT>(s16);
         const float inv = quant_inv(sf_t);
-        uint8_t *frag = tiles + ((size_t)(row >> 5) * (size_t)(K >> 6) + 2 * blk + h) * 1536;
+        uint8_t *frag = tiles + ((size_t)(row >> 5) * (size_t)(2 * n_blk) + 2 * blk + h) * 1536;
         __shared__ __attribute__((aligned(16))) uint8_t stage[Sh::kStageBytes];
         auto emit = [&](auto fast_tag) {
             constexpr bool kFast = decltype(fast_tag)::value;
@@ -347,7 +236,8 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
                         hp[4 * (j >> 1) + 2 * hh + (j & 1)] = __builtin_bit_cast(unsigned, c);
                     }
                 }
-                const v6u r = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(__builtin_bit_cast(v32h, hp), 1.0f);
+                v6u r = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(__builtin_bit_cast(v32h, hp), 1.0f);
+                if (RAG && blk * 128 + 64 * h + 32 * g >= K) r = v6u{0, 0, 0, 0, 0, 0};
                 if constexpr (TL) {
                     // position (g, h, block) of the row, this row's chunk in it
                     const int pos = (2 * g + h) * Sh::kBlocks + blk;
@@ -371,18 +261,18 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
             constexpr int kTR = Sh::kTileRows;
             const int row0 = vb * kTR;
             const int m_pad = (M + 31) & ~31;
-            const size_t frag0 = (size_t)(row0 >> 5) * (size_t)(K >> 6);
+            const size_t frag0 = (size_t)(row0 >> 5) * (size_t)(2 * n_blk);
             for (int u = threadIdx.x; u < Sh::kPositions * kTR; u += 64 * Sh::kWaves) {
                 const int pos = u / kTR, c = u % kTR;
                 const int gg = pos / (2 * Sh::kBlocks), hh = (pos / Sh::kBlocks) & 1, bb = pos % Sh::kBlocks;
-                if (bb < (K >> 7) && row0 + c < m_pad)
+                if (bb < n_blk && row0 + c < m_pad)
                     *reinterpret_cast<uint4 *>(tiles + (frag0 + 2 * bb + hh) * 1536 + (32 * gg + (row0 & 31) + c) * 16) =
                         *reinterpret_cast<const uint4 *>(stage + pos * Sh::kHeadPitch + c * 16);
             }
             for (int u = threadIdx.x; u < Sh::kPositions * kTR / 2; u += 64 * Sh::kWaves) {
                 const int pos = u / (kTR / 2), c = 2 * (u % (kTR / 2));
                 const int gg = pos / (2 * Sh::kBlocks), hh = (pos / Sh::kBlocks) & 1, bb = pos % Sh::kBlocks;
-                if (bb < (K >> 7) && row0 + c < m_pad)
+                if (bb < n_blk && row0 + c < m_pad)
                     *reinterpret_cast<uint4 *>(tiles + (frag0 + 2 * bb + hh) * 1536 + 1024 + (32 * gg + (row0 & 31) + c) * 8) =
                         *reinterpret_cast<const uint4 *>(stage + Sh::kPositions * Sh::kHeadPitch + pos * Sh::kTailPitch + c * 8);
             }
@@ -390,59 +280,28 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
     }
     if (packed == nullptr && row_sum == nullptr) return;      // uniform over the workgroup
 
-    // ---- codes.  Outputs 8 Q + 4 h + {0..3} (Q = 4 mt + q) give one half-word c3 c2 c1 c0 of two's-complement nibbles.
-    // Scales in the quantiser's fast range (everything but degenerate rows) take the clamp-free form: the code
-    // arrives in the top nibble of an integer and is shifted into the half-word by one v_alignbit per code.
-    const float sf = to_f32<DT>(s16);
-    uint32_t hw[16];
-    if (__builtin_amdgcn_ballot_w64(row < M && !quant_fast_ok(sf)) == 0) {
-        const float inv28 = quant_inv28(sf);
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const uint32_t w0 = yb[mt][q * 2], w1 = yb[mt][q * 2 + 1];
-                uint32_t g = (uint32_t)quant_top_nibble_half<DT, 1>(w1, inv28) >> 28;
-                g = push_top_nibble(g, quant_top_nibble_half<DT, 0>(w1, inv28));
-                g = push_top_nibble(g, quant_top_nibble_half<DT, 1>(w0, inv28));
-                hw[mt * 4 + q] = push_top_nibble(g, quant_top_nibble_half<DT, 0>(w0, inv28));
-            }
-    } else {
-        const float inv = quant_inv(sf);
-#pragma unroll
-        for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const uint32_t w0 = yb[mt][q * 2], w1 = yb[mt][q * 2 + 1];
-                const uint32_t c0 = (uint32_t)quant_code_inv_i(lo_f32<DT>(w0), inv) & 15u;
-                const uint32_t c1 = (uint32_t)quant_code_inv_i(hi_f32<DT>(w0), inv) & 15u;
-                const uint32_t c2 = (uint32_t)quant_code_inv_i(lo_f32<DT>(w1), inv) & 15u;
-                const uint32_t c3 = (uint32_t)quant_code_inv_i(hi_f32<DT>(w1), inv) & 15u;
-                hw[mt * 4 + q] = (((c3 * 16 + c2) * 16 + c1) * 16) + c0;
-            }
-    }
-    // lane (n, 0) ends with dwords 0..7 of the block's 64 packed bytes, lane (n, 1) with dwords 8..15: dword D is the
-    // half-word Q = D of lane (n, 0) below that of lane (n, 1).  v_permlane32_swap hands the lower lane both half-words
-    // t and the upper lane both half-words t + 8.  Every code sits in exactly one lane's dwords, so the row sum is the
-    // sum of their signed nibbles.
-    int isum = 0;
+    // every code sits in exactly one lane's dwords, so the row sum is the sum of their signed nibbles
     uint32_t dw[8];
+    nibbles<DT>(dw, yb, s16, row < M);
+    if constexpr (RAG) {
 #pragma unroll
-    for (int t = 0; t < 8; t++) {
-        const auto sw = __builtin_amdgcn_permlane32_swap(hw[t], hw[t + 8], false, false);
-        dw[t] = sw[0] | (sw[1] << 16);
-        isum = __builtin_amdgcn_sdot8((int)dw[t], 0x11111111, isum, false);
+        for (int t = 0; t < 8; t++)
+            if (blk * 128 + 64 * h + 8 * t >= K) dw[t] = 0;          // (a degenerate row's zeros need not quantise to code 0)
     }
+    int isum = 0;
+#pragma unroll
+    for (int t = 0; t < 8; t++) isum = __builtin_amdgcn_sdot8((int)dw[t], 0x11111111, isum, false);
     if (packed != nullptr && live) {
         uint32_t *dst = packed + (size_t)row * (K >> 3) + blk * 16 + h * 8;
         if ((reinterpret_cast<uintptr_t>(packed) & 15) == 0) {           // uniform; rows are whole multiples of 64 bytes
-            *reinterpret_cast<uint4 *>(dst) = make_uint4(dw[0], dw[1], dw[2], dw[3]);
-            *reinterpret_cast<uint4 *>(dst + 4) = make_uint4(dw[4], dw[5], dw[6], dw[7]);
+            if (!RAG || blk * 128 + 64 * h < K) *reinterpret_cast<uint4 *>(dst) = make_uint4(dw[0], dw[1], dw[2], dw[3]);
+            if (!RAG || blk * 128 + 64 * h + 32 < K) *reinterpret_cast<uint4 *>(dst + 4) = make_uint4(dw[4], dw[5], dw[6], dw[7]);
         } else {                                                          // a view that starts 4 bytes into an allocation
             // (volatile: kept apart from the vector stores above, which the compiler would otherwise merge with these
             // into a common, narrower sequence)
 #pragma unroll
-            for (int t = 0; t < 8; t++) *reinterpret_cast<volatile uint32_t *>(dst + t) = dw[t];
+            for (int t = 0; t < 8; t++)
+                if (!RAG || blk * 128 + 64 * h + 8 * t < K) *reinterpret_cast<volatile uint32_t *>(dst + t) = dw[t];
         }
     }
     if (row_sum != nullptr) {
@@ -461,23 +320,6 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
 
 }  // namespace hq
 
-// Whether `v` survives a round trip through the 16-bit dtype, and its bits there.
-static bool representable16(float v, int dtype, uint32_t *bits) {
-    uint32_t u;
-    __builtin_memcpy(&u, &v, 4);
-    if (dtype == QUEST_DTYPE_BF16) {
-        if (u & 0xFFFFu) return false;
-        *bits = u >> 16;
-        return true;
-    }
-    const _Float16 hf = (_Float16)v;
-    if ((float)hf != v) return false;
-    uint16_t b;
-    __builtin_memcpy(&b, &hf, 2);
-    *bits = b;
-    return true;
-}
-
 struct Args {
     const void *x, *norm_w;
     void *scale;
@@ -495,7 +337,7 @@ struct Args {
     int cus;                   // compute units of the device (only looked at when tiles are written)
 };
 
-template <int DT, int WPR, int G, int PRE, bool TL>
+template <int DT, int WPR, int G, int PRE, bool TL, bool RAG>
 static void launch_shape_as(const Args &a) {
     using Sh = hq::Shape<WPR, G, TL>;
     constexpr int rows = Sh::kTileRows;                            // rows per workgroup
@@ -504,7 +346,7 @@ static void launch_shape_as(const Args &a) {
         xcd_chunk = (grid + 7) / 8;
         grid = 8 * xcd_chunk;
     }
-    hq::hadamard_quantize_mfma_kernel<DT, WPR, G, PRE, TL><<<dim3(grid), dim3(64 * Sh::kWaves), 0, a.st>>>(
+    hq::hadamard_quantize_mfma_kernel<DT, WPR, G, PRE, TL, RAG><<<dim3(grid), dim3(64 * Sh::kWaves), 0, a.st>>>(
         (const uint16_t *)a.x, (const uint16_t *)a.norm_w, (uint16_t *)a.scale, (uint32_t *)a.packed, a.row_sum,
         (uint16_t *)a.x_had, (uint16_t *)a.pre_out, (const uint16_t *)a.add_in, (uint16_t *)a.sum_out, a.tiles, xcd_chunk,
         a.K, a.M, a.ldx, a.bits, a.eps, a.sum_bias);
@@ -514,13 +356,20 @@ static void launch_shape_as(const Args &a) {
 // such workgroups are at least two per compute unit: below that the small workgroups, which write their 16-byte pieces
 // straight to the tiles, fill the device better (bf16 rows of 4096: 4.0 against 5.9 us for 512 rows, 7.3 against 7.2 us
 // for 2048, 14.5 against 11.5 us for 4096).  Same arithmetic and same bytes either way.
-template <int DT, int WPR, int G, int PRE>
-static void launch_shape(const Args &a) {
+template <int DT, int WPR, int G, int PRE, bool RAG>
+static void launch_shape_for(const Args &a) {
     if constexpr (WPR <= 3 && G >= 8) {
         constexpr int rows = hq::Shape<WPR, G, true>::kTileRows;
-        if (a.tiles != nullptr && (a.M + rows - 1) / rows >= 2 * a.cus) return launch_shape_as<DT, WPR, G, PRE, true>(a);
+        if (a.tiles != nullptr && (a.M + rows - 1) / rows >= 2 * a.cus) return launch_shape_as<DT, WPR, G, PRE, true, RAG>(a);
     }
-    launch_shape_as<DT, WPR, G, PRE, false>(a);
+    launch_shape_as<DT, WPR, G, PRE, false, RAG>(a);
+}
+template <int DT, int WPR, int G, int PRE>
+static void launch_shape(const Args &a) {
+    if constexpr (PRE == hq::kPreNone) {
+        if (a.K & 127) return launch_shape_for<DT, WPR, G, PRE, true>(a);
+    }
+    launch_shape_for<DT, WPR, G, PRE, false>(a);
 }
 
 // rows of up to 32 blocks: one wave holds 32 / G of them
@@ -552,7 +401,7 @@ static void launch_long(int wpr, const Args &a) {
 
 template <int DT>
 static void launch_dtype(int pre, const Args &a) {
-    const int nb = a.K / 128;
+    const int nb = (a.K + 127) / 128;
     if (nb > 32) {
         const int wpr = (nb + 31) / 32;
         if (pre == hq::kPreRmsNorm) return launch_long<DT, hq::kPreRmsNorm>(wpr, a);
@@ -566,7 +415,7 @@ static void launch_dtype(int pre, const Args &a) {
     else launch_short<DT, hq::kPreNone>(g, a);
 }
 
-// Launches the matrix-core kernel when it applies (K a multiple of 128 up to 32768, a
+// Launches the matrix-core kernel when it applies (K a multiple of 128 up to 32768, or of 32 without the transform; a
 // Hadamard entry the dtype represents exactly); returns QUEST_ERR_UNSUPPORTED otherwise so that the caller can take
 // another path.  Whether it applies depends on K, the factor and the dtype only -- never on the number of rows or on
 // where the buffers lie -- so that one shape always runs the same arithmetic.
@@ -577,7 +426,8 @@ int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, fl
                                   hipStream_t st, const void *add_in, void *sum_out, uint8_t *tiles, int sum_bias) {
     uint32_t bits = 0;
     // (had_scale == 0: no transform; the kernel then only moves the chunks between lanes)
-    if (K > 32768 || (K & 127) || had_scale < 0.f || !representable16(had_scale, dtype, &bits)) return QUEST_ERR_UNSUPPORTED;
+    if (K > 32768 || had_scale < 0.f || !representable16(had_scale, dtype, &bits)) return QUEST_ERR_UNSUPPORTED;
+    if ((K & 127) != 0 && ((K & 31) != 0 || pre != 0 || had_scale != 0.f || x_had != nullptr || pre_out != nullptr)) return QUEST_ERR_UNSUPPORTED;
     const int ldx = pre == hq::kPreSiluMul ? 2 * K : K;
     if (!aligned(pre_out, 16) || !aligned(norm_w, 16)) return QUEST_ERR_UNSUPPORTED;
     if (add_in != nullptr && (pre != hq::kPreRmsNorm || sum_out == nullptr || !aligned(add_in, 16) || !aligned(sum_out, 16)))
@@ -596,7 +446,7 @@ int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, fl
         };
         const Args a = {at(x, ldx, es), norm_w, at(scale, 1, es), (uint8_t *)at(packed, K / 2, 1), (int32_t *)at(row_sum, 1, 4),
                         at(x_had, K, es), at(pre_out, K, es), at(add_in, K, es), at(sum_out, K, es),
-                        tiles == nullptr ? nullptr : tiles + (size_t)(r0 / 32) * (size_t)(K / 64) * 1536, K, rows, ldx, bits, eps, st, sum_bias, cus};
+                        tiles == nullptr ? nullptr : tiles + (size_t)(r0 / 32) * (size_t)((K + 127) / 128 * 2) * 1536, K, rows, ldx, bits, eps, st, sum_bias, cus};
         if (dtype == QUEST_DTYPE_BF16) launch_dtype<0>(pre, a);
         else launch_dtype<1>(pre, a);
     }

@@ -1,10 +1,10 @@
 // Host side of the hot calls in native code: argument checks, output and scratch allocation, stream lookup and the launches
 // of libquest_hip.so, as a CPython module over torch's C++ tensors.
 //
-// Why: a layer at a handful of tokens is 7 us of GPU work in two launches, and its Python host path (asserts, ctypes
-// conversions, device context, one allocation per output) took 36 us per call, so every small call ran at the speed of the
-// interpreter.  From here a call takes 10.6 us to issue, module call included (profiles/timed_layer_calls.md): that, and not the GPU's
-// 6.3 us for both launches in a graph, still bounds one token at K = N = 4096.
+// Why: a layer at a handful of tokens is 5 to 7 us of GPU work, and its Python host path (asserts, ctypes conversions, device
+// context, one allocation per output) took 36 us per call, so every small call ran at the speed of the interpreter.  From here a call of two
+// launches takes 10.6 us to issue, module call included, and one of a single launch (quest_linear_few_tokens) 7.3: a launch is 3.7 us of
+// it, an allocation 0.7.  That, and not the GPU, still bounds the smallest calls.
 //
 // Contract of every function: either the call is the plain case -- exact torch tensors on one GPU, contiguous, right types, sizes
 // and alignment, accepted by the library -- and everything is launched, or None comes back with nothing launched and the
@@ -169,19 +169,25 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (bias != nullptr && ((at::GradMode::is_enabled() && bias->requires_grad()) || bias->_fw_grad(0).defined())) return declined();
 
     at::Tensor out;
+    const auto result = [&]() {
+        if (given != nullptr) return *given;
+        c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
+        shape.back() = n;
+        return make(shape, type, args.dev);
+    };
     const int rc = on(args.dev, [&](void *st) {
         const int dt = dtype_code(type);
+        if (m <= 16 && !tiles) {                             // in one launch where that kernel takes it
+            out = result();
+            const int rc = quest_linear_few_tokens(out.data_ptr(), x->data_ptr(), (const uint8_t *)w->data_ptr(), (const int32_t *)w_add->data_ptr(), w_scale->data_ptr(),
+                                                   bias ? bias->data_ptr() : nullptr, (int)m, (int)k, (int)n, (float)had_scale, dt, st);
+            if (rc == QUEST_OK) return rc;
+        }
         Codes q(m, k, tiles, args.dev);
         int rc = tiles ? quest_hadamard_quantize_e2m3(x->data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, (int)k, (int)m, (float)had_scale, dt, st)
                    : quest_hadamard_quantize_int4(x->data_ptr(), q.scale, q.codes, q.row_sum, nullptr, (int)k, (int)m, (float)had_scale, dt, st);
         if (rc != QUEST_OK) return rc;
-        if (given != nullptr) {
-            out = *given;
-        } else {
-            c10::SmallVector<int64_t, 5> shape(x->sizes().begin(), x->sizes().end());
-            shape.back() = n;
-            out = make(shape, type, args.dev);
-        }
+        if (!out.defined()) out = result();
         bool add_bias = bias != nullptr;
         if (add_bias) {                                      // in the GEMM's epilogue where the kernel can
             rc = tiles ? quest_fused_matmul_dequantize_bias_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)k, (int)n, dt, st)
