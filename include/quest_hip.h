@@ -271,6 +271,14 @@ size_t quest_e2m3_tiles_bytes(int rows, int size_k);
 int quest_int4_to_e2m3_tiles(void *tiles, const uint8_t *x_int_packed, int rows, int size_k, void *stream);
 
 /*
+ * Rows that are not whole 128s (size_k % 32 == 0), without the transform: tiles of the row with zeros -- the FP6 zero, not a code -- behind
+ * it up to a whole 128, so that the GEMM entry points take them with that size_k.  (quest_e2m3_tiles_bytes of it; 65536 at most.)  The sum of squares
+ * runs in another order than quest_hadamard_quantize_int4's for such rows: a scale can differ from its by one unit in the last place.
+ */
+int quest_int4_to_e2m3_tiles_padded(void *tiles, const uint8_t *x_int_packed, int rows, int size_k, void *stream);
+int quest_quantize_e2m3_padded(const void *x, void *scale, void *x_tiles, int group_size, int batch_size, int dtype, void *stream);
+
+/*
  * mat_d (size_m, size_n) dtype = quest_fused_matmul_dequantize_int4_int4t's result for the same codes, from their
  * E2M3 tiles: dtype( f32(2 S) * (0.5f * vec_a_mul[m] * vec_b_mul[n]) ) with S = sum_k (qa + 1/2)(qb + 1/2) accumulated
  * exactly.  size_k % 128 == 0 and <= 65536; any size_m, size_n >= 1; scale vectors 4-byte aligned.

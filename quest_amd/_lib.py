@@ -43,6 +43,8 @@ SIGNATURES = {
     'quest_fused_matmul_dequantize_int4_int4t_noalloc': [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     'quest_e2m3_tiles_bytes': [_i, _i],
     'quest_int4_to_e2m3_tiles': [_vp, _vp, _i, _i, _vp],
+    'quest_int4_to_e2m3_tiles_padded': [_vp, _vp, _i, _i, _vp],
+    'quest_quantize_e2m3_padded': [_vp, _vp, _vp, _i, _i, _i, _vp],
     'quest_fused_matmul_dequantize_e2m3': [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     'quest_fused_matmul_dequantize_add_e2m3': [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     'quest_fused_matmul_dequantize_add_int4_int4t': [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],

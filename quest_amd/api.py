@@ -491,14 +491,23 @@ def e2m3_tiles_bytes(rows: int, k: int) -> int:
 def int4_to_e2m3_tiles(x_int_packed: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:
     """Packed INT4 codes (rows, K/2) uint8 -> their E2M3 tiles (flat uint8): the operand form of
     `fused_matmul_dequantize_e2m3`, each code q stored as the FP6 E2M3 value q + 1/2."""
+    return _int4_to_tiles(x_int_packed, out, x_int_packed.size(1) * 2, 'quest_int4_to_e2m3_tiles')
+
+
+def int4_to_e2m3_tiles_padded(x_int_packed: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:
+    """The same for rows of whole 32s: tiles of the row with zeros behind it up to a whole 128."""
+    return _int4_to_tiles(x_int_packed, out, (x_int_packed.size(1) * 2 + 127) // 128 * 128, 'quest_int4_to_e2m3_tiles_padded')
+
+
+def _int4_to_tiles(x_int_packed, out, tiles_k: int, entry: str) -> torch.Tensor:
     rows, k = x_int_packed.size(0), x_int_packed.size(1) * 2
     if out is None:
-        out = torch.empty(e2m3_tiles_bytes(rows, k), dtype=torch.uint8, device=x_int_packed.device)
+        out = torch.empty(e2m3_tiles_bytes(rows, tiles_k), dtype=torch.uint8, device=x_int_packed.device)
     assert x_int_packed.dtype == torch.uint8 and x_int_packed.is_contiguous() and x_int_packed.dim() == 2
-    assert out.dtype == torch.uint8 and out.is_contiguous() and out.numel() == e2m3_tiles_bytes(rows, k)
+    assert out.dtype == torch.uint8 and out.is_contiguous() and out.numel() == e2m3_tiles_bytes(rows, tiles_k)
     dev = require_gpu(x_int_packed, out)
     with torch.cuda.device(dev):
-        check(_lib.load().quest_int4_to_e2m3_tiles(ptr(out), ptr(x_int_packed), rows, k, stream_of(out)), 'int4_to_e2m3_tiles')
+        check(getattr(_lib.load(), entry)(ptr(out), ptr(x_int_packed), rows, k, stream_of(out)), entry)
     return out
 
 

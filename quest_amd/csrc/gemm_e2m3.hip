@@ -457,17 +457,17 @@ __device__ __forceinline__ uint32_t e2m3_of_nibble(uint32_t n) {             // 
 }
 
 // One thread per (row, 32 codes): 16 packed bytes in, 24 bytes out; a workgroup of 256 writes four whole fragments
-// (k-steps ks0 .. ks0 + 3 of one row block), i.e. reads one 128-byte line of each of its 32 rows.
+// (k-steps ks0 .. ks0 + 3 of one row block), i.e. reads one 128-byte line of each of its 32 rows.  nks may reach past the rows'
+// K codes (whole 32s): zeros there.
 __global__ void __launch_bounds__(256) int4_to_e2m3_tiles_kernel(uint8_t *__restrict__ tiles, const uint8_t *__restrict__ packed,
-                                                                 int rows, int K) {
-    const int nks = K / 64;
+                                                                 int rows, int K, int nks) {
     const int l = threadIdx.x & 63;
     const int ks = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int rb = blockIdx.y;
     if (ks >= nks) return;
     const int row = rb * 32 + (l & 31);
     uint32_t w[6] = {0, 0, 0, 0, 0, 0};
-    if (row < rows) {
+    if (row < rows && ks * 64 + (l >> 5) * 32 < K) {
         const uint4 p = *reinterpret_cast<const uint4 *>(packed + (size_t)row * (K / 2) + (size_t)ks * 32 + (l >> 5) * 16);
         const uint32_t src[4] = {p.x, p.y, p.z, p.w};
 #pragma unroll
@@ -576,6 +576,13 @@ static int launch_e2m3(int dtype, void *out, const uint8_t *a, const uint8_t *b,
 
 static size_t tiles_bytes(int rows, int K) { return (size_t)((rows + 31) / 32) * (size_t)(K / 64) * e2m3::kFragB; }
 
+static int int4_to_tiles(void *tiles, const uint8_t *packed, int rows, int K, int nks, hipStream_t st) {
+    const int rbs = (rows + 31) / 32;
+    if (rbs > 65535) return QUEST_ERR_UNSUPPORTED;
+    e2m3::int4_to_e2m3_tiles_kernel<<<dim3((nks + 3) / 4, rbs), dim3(256), 0, st>>>((uint8_t *)tiles, packed, rows, K, nks);
+    return launch_status();
+}
+
 static int e2m3_gemm_check(const void *out, const void *a, const void *b, const void *a_mul, const void *b_mul, int M, int K,
                            int N, int dtype) {
     if (!out || !a || !b || !a_mul || !b_mul) return QUEST_ERR_NULL_POINTER;
@@ -603,11 +610,15 @@ extern "C" int quest_int4_to_e2m3_tiles(void *tiles, const uint8_t *x_int_packed
     if (!tiles || !x_int_packed) return QUEST_ERR_NULL_POINTER;
     if (rows <= 0 || size_k <= 0 || (size_k & 63)) return QUEST_ERR_BAD_SHAPE;
     if (!aligned(tiles, 16) || !aligned(x_int_packed, 16)) return QUEST_ERR_ALIGNMENT;
-    const int nks = size_k / 64, rbs = (rows + 31) / 32;
-    if (rbs > 65535) return QUEST_ERR_UNSUPPORTED;
-    e2m3::int4_to_e2m3_tiles_kernel<<<dim3((nks + 3) / 4, rbs), dim3(256), 0, (hipStream_t)stream>>>(
-        (uint8_t *)tiles, x_int_packed, rows, size_k);
-    return launch_status();
+    return int4_to_tiles(tiles, x_int_packed, rows, size_k, size_k / 64, (hipStream_t)stream);
+}
+
+extern "C" int quest_int4_to_e2m3_tiles_padded(void *tiles, const uint8_t *x_int_packed, int rows, int size_k, void *stream) {
+    forget_stale_error();
+    if (!tiles || !x_int_packed) return QUEST_ERR_NULL_POINTER;
+    if (rows <= 0 || size_k <= 0 || size_k > 65536 || (size_k & 31)) return QUEST_ERR_BAD_SHAPE;
+    if (!aligned(tiles, 16) || !aligned(x_int_packed, 16)) return QUEST_ERR_ALIGNMENT;
+    return int4_to_tiles(tiles, x_int_packed, rows, size_k, (size_k + 127) / 128 * 2, (hipStream_t)stream);
 }
 
 extern "C" int quest_fused_matmul_dequantize_e2m3(void *mat_d, const void *a_tiles, const void *b_tiles, const void *vec_a_mul,

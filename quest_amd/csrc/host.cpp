@@ -160,11 +160,13 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const at::Tensor *w_add = args.tensor(a[3], at::kInt, n);
     PyObject *const tiles_arg = tiles_of(a[4], a[1]);
     const bool tiles = tiles_arg != Py_None && args.ok && at(w_scale, 4);      // (the FP6 kernels read scales two at a time)
-    const at::Tensor *w_tiles = tiles ? args.tensor(tiles_arg, at::kByte, (int64_t)quest_e2m3_tiles_bytes((int)n, (int)k)) : nullptr;
+    // (rows that are not whole 128s come as tiles with zeros behind them)
+    const int64_t kt = tiles ? (k + 127) / 128 * 128 : k;
+    const at::Tensor *w_tiles = tiles ? args.tensor(tiles_arg, at::kByte, (int64_t)quest_e2m3_tiles_bytes((int)n, (int)kt)) : nullptr;
     const at::Tensor *bias = a[5] == Py_None ? nullptr : args.tensor(a[5], type, n);
     const double had_scale = PyFloat_AsDouble(a[6]);
     const at::Tensor *given = a[7] == Py_None ? nullptr : args.matrix(a[7], type, m, n);
-    if (!args.ok || !gemm_takes(m, k, n, tiles) || !at(x, 16) || !at(w, 16) || !at(w_tiles, 16) || !at(given, 16)) return declined();
+    if (!args.ok || !gemm_takes(m, kt, n, tiles) || !at(x, 16) || !at(w, 16) || !at(w_tiles, 16) || !at(given, 16)) return declined();
     // (a bias whose derivative is wanted is added by torch)
     if (bias != nullptr && ((at::GradMode::is_enabled() && bias->requires_grad()) || bias->_fw_grad(0).defined())) return declined();
 
@@ -183,20 +185,21 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
                                                    bias ? bias->data_ptr() : nullptr, (int)m, (int)k, (int)n, (float)had_scale, dt, st);
             if (rc == QUEST_OK) return rc;
         }
-        Codes q(m, k, tiles, args.dev);
-        int rc = tiles ? quest_hadamard_quantize_e2m3(x->data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, (int)k, (int)m, (float)had_scale, dt, st)
-                   : quest_hadamard_quantize_int4(x->data_ptr(), q.scale, q.codes, q.row_sum, nullptr, (int)k, (int)m, (float)had_scale, dt, st);
+        Codes q(m, kt, tiles, args.dev);
+        int rc = kt != k && had_scale == 0. ? quest_quantize_e2m3_padded(x->data_ptr(), q.scale, q.codes, (int)k, (int)m, dt, st)
+                 : tiles ? quest_hadamard_quantize_e2m3(x->data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, (int)k, (int)m, (float)had_scale, dt, st)
+                         : quest_hadamard_quantize_int4(x->data_ptr(), q.scale, q.codes, q.row_sum, nullptr, (int)k, (int)m, (float)had_scale, dt, st);
         if (rc != QUEST_OK) return rc;
         if (!out.defined()) out = result();
         bool add_bias = bias != nullptr;
         if (add_bias) {                                      // in the GEMM's epilogue where the kernel can
-            rc = tiles ? quest_fused_matmul_dequantize_bias_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)k, (int)n, dt, st)
+            rc = tiles ? quest_fused_matmul_dequantize_bias_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)kt, (int)n, dt, st)
                        : quest_fused_matmul_dequantize_bias_int4_int4t(out.data_ptr(), q.codes, (const uint8_t *)w->data_ptr(), q.row_sum, (const int32_t *)w_add->data_ptr(),
                                                                        q.scale, w_scale->data_ptr(), bias->data_ptr(), (int)m, (int)k, (int)n, dt, st);
             add_bias = rc != QUEST_OK;
         }
         if (add_bias || bias == nullptr) {
-            rc = tiles ? quest_fused_matmul_dequantize_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), (int)m, (int)k, (int)n, dt, st)
+            rc = tiles ? quest_fused_matmul_dequantize_e2m3(out.data_ptr(), q.codes, w_tiles->data_ptr(), q.scale, w_scale->data_ptr(), (int)m, (int)kt, (int)n, dt, st)
                        : quest_fused_matmul_dequantize_int4_int4t(out.data_ptr(), q.codes, (const uint8_t *)w->data_ptr(), q.row_sum,
                                                                   (const int32_t *)w_add->data_ptr(), q.scale, w_scale->data_ptr(), (int)m, (int)k, (int)n, dt, st);
             if (rc == QUEST_OK && add_bias) out.add_(*bias);

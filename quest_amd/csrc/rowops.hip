@@ -616,6 +616,16 @@ extern "C" int quest_hadamard_quantize_e2m3(const void *x, void *scale, void *x_
                                          batch_size, had_scale, dtype, (hipStream_t)stream, nullptr, nullptr, (uint8_t *)x_tiles);
 }
 
+extern "C" int quest_quantize_e2m3_padded(const void *x, void *scale, void *x_tiles, int group_size, int batch_size, int dtype, void *stream) {
+    forget_stale_error();
+    if (!x || !scale || !x_tiles) return QUEST_ERR_NULL_POINTER;
+    if (!check_dtype(dtype)) return QUEST_ERR_BAD_DTYPE;
+    if (group_size <= 0 || batch_size <= 0 || (group_size & 31)) return QUEST_ERR_BAD_SHAPE;
+    if (!aligned(x, 16) || !aligned(x_tiles, 16)) return QUEST_ERR_ALIGNMENT;
+    return launch_hadamard_quantize_mfma(0, x, nullptr, 0.f, scale, nullptr, nullptr, nullptr, nullptr, group_size, batch_size, 0.f, dtype,
+                                         (hipStream_t)stream, nullptr, nullptr, (uint8_t *)x_tiles);
+}
+
 extern "C" int quest_rmsnorm_hadamard_quantize_e2m3(const void *x, const void *norm_weight, float eps, void *scale,
                                                     void *x_tiles, void *x_norm, int group_size, int batch_size,
                                                     float had_scale, int dtype, void *stream) {

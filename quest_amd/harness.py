@@ -95,6 +95,11 @@ def e2m3_fits(k: int, rows: int) -> bool:
     return k % 128 == 0 and 0 < k <= 65536 and rows <= 32 * 65535 and (rows + 287) // 32 * (k // 64) * 1536 < 1 << 31
 
 
+def tiles_k(k: int, use_hadamard: bool) -> int:
+    """The row length that a layer's tiles are laid out for: without the transform, rows of whole 32s get zeros up to a whole 128."""
+    return k if use_hadamard or k % 32 else (k + 127) // 128 * 128
+
+
 def _scales_in_pairs(scale) -> bool:
     """Whether the FP6 kernels can read a scale vector: two 16-bit values at a time."""
     return scale is None or scale.data_ptr() % 4 == 0
@@ -292,9 +297,12 @@ class Linear4bit(nn.Module):
             w = self._buffers.get('w_int_packed')
             if type(w) is not torch.Tensor or not w.is_cuda or w.dim() != 2 or not w.is_contiguous():
                 return
-            if MATRIX_PATH == 'fp6' and e2m3_fits(w.size(1) * 2, w.size(0)):
+            k = w.size(1) * 2
+            padded = tiles_k(k, self.use_hadamard)
+            if MATRIX_PATH == 'fp6' and e2m3_fits(padded, w.size(0)) and (padded == k or padded >= 640):      # (shorter ones: see prefers_e2m3)
                 in_place = before is not None and before[1] is w and before[2] == w.data_ptr()
-                self._tiles = (weight_tiles(w, before[0] if in_place else None), w, w.data_ptr(), w._version)
+                lay = weight_tiles if padded == k else quest.int4_to_e2m3_tiles_padded
+                self._tiles = (lay(w, before[0] if in_place else None), w, w.data_ptr(), w._version)
 
     def _kept_tiles(self):
         """The tiles of what `w_int_packed` holds now, or None."""
@@ -311,12 +319,12 @@ class Linear4bit(nn.Module):
         return self.readable_tiles() if prefers_e2m3(m, k, n) else None
 
     def readable_tiles(self):
-        """The kept tiles, if the FP6 kernels can read the scales beside them."""
-        return self._kept_tiles() if _scales_in_pairs(self.w_scale) else None
+        """The kept tiles, if the FP6 kernels can read the scales beside them and the rows are whole 128s."""
+        return self._kept_tiles() if _scales_in_pairs(self.w_scale) and self.weight.size(1) % 128 == 0 else None
 
     def w_tiles(self) -> torch.Tensor:
         """The weight codes as E2M3 tiles: the kept ones, or a conversion of the buffer for this call."""
-        tiles = self._kept_tiles()
+        tiles = self._kept_tiles() if self.weight.size(1) % 128 == 0 else None
         return weight_tiles(self.w_int_packed) if tiles is None else tiles
 
     def _load_from_state_dict(self, *args, **kwargs):
@@ -417,7 +425,7 @@ class Linear4bit(nn.Module):
             k = x.size(-1)
             held = self._buffers.get                  # (not there, e.g. made a parameter: the native call declines)
             if held('w_meta_e') is None:
-                tiles = self._tiles if prefers_e2m3(x.numel() // max(k, 1), k, n) else None
+                tiles = self._tiles if prefers_e2m3(x.numel() // max(k, 1), tiles_k(k, self.use_hadamard), n) else None
                 y = quest.host.linear(x, held('w_int_packed'), held('w_scale'), held('w_add'), tiles, self.bias,
                                       HADAMARD_ENTRY if self.use_hadamard else 0., None)
                 if y is not None:

@@ -1,0 +1,65 @@
+"""Rows that are not whole 128s on the FP6 path: the activation kernel's tiles with zeros behind the row, the weights' tiles, and layers
+against the INT8 kernels; every remainder, every way a row is divided over waves, small and staged tile writes."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda:0'
+
+
+def _tiles_of(x):
+    import quest_amd as quest
+    from quest_amd import _lib
+    m, k = x.shape
+    scale = torch.empty(m, 1, dtype=x.dtype, device=DEV)
+    tiles = torch.full((quest.e2m3_tiles_bytes(m, (k + 127) // 128 * 128),), 0xAA, dtype=torch.uint8, device=DEV)
+    _lib.check(_lib.load().quest_quantize_e2m3_padded(x.data_ptr(), scale.data_ptr(), tiles.data_ptr(), k, m, _lib.DTYPE_CODE[x.dtype],
+                                                      torch.cuda.current_stream().cuda_stream), 'quantize_e2m3_padded')
+    return scale, tiles
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('m,k', [(5, 32), (33, 160), (70, 224), (64, 480), (40, 992), (37, 1376), (100, 2016), (5, 4064), (9, 4128), (33, 10976),
+                                 (3, 32736), (4500, 1056), (2100, 4192), (8300, 736)])
+def test_tiles_hold_the_codes_and_zeros_behind_them(dtype, m, k):
+    import quest_amd as quest
+    from oracle import quest_oracle as qo
+    x = torch.randn(m, k, device=DEV, generator=torch.Generator(device=DEV).manual_seed(m + k)).to(dtype)
+    x[1, :] = 0
+    x[2, 3] = float('nan')
+    scale, tiles = _tiles_of(x)
+    want_scale, codes, _ = quest.hadamard_quantize_int4(x, hadamard_scale=0.)
+    same = ((scale == want_scale) | (scale.isnan() & want_scale.isnan())).flatten().cpu()
+    assert int((~same).sum()) <= 1                                   # another order of the sum of squares: one row in about ten thousand
+    values = qo.e2m3_tiles_decode(tiles.cpu(), m, (k + 127) // 128 * 128)
+    assert torch.equal(values[same, :k], qo.unpack_int4(codes.cpu()).double()[same] + 0.5)
+    assert bool((values[:, k:] == 0).all())
+
+
+@pytest.mark.parametrize('rows,k', [(1, 32), (33, 96), (100, 1376), (64, 2016), (5, 128)])
+def test_weight_tiles(rows, k):
+    import quest_amd as quest
+    from oracle import quest_oracle as qo
+    packed = torch.randint(0, 256, (rows, k // 2), dtype=torch.uint8, device=DEV, generator=torch.Generator(device=DEV).manual_seed(k))
+    values = qo.e2m3_tiles_decode(quest.api.int4_to_e2m3_tiles_padded(packed).cpu(), rows, (k + 127) // 128 * 128)
+    assert torch.equal(values[:, :k], qo.unpack_int4(packed.cpu()).double() + 0.5) and bool((values[:, k:] == 0).all())
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('m,k,n,bias', [(333, 1376, 4096, False), (100, 2016, 1031, True), (60, 4064, 2048, False), (1000, 1056, 2560, True), (4200, 1888, 2056, False)])
+def test_layers_equal_the_int8_kernels(dtype, m, k, n, bias):
+    from quest_amd import harness
+    g = torch.Generator(device=DEV).manual_seed(m + k + n)
+    layer = harness.Linear4bit.from_weight((torch.randn(n, k, device=DEV, generator=g) * .02).to(dtype), torch.randn(n, device=DEV, generator=g).to(dtype) if bias else None)
+    assert harness.prefers_e2m3(m, harness.tiles_k(k, False), n) and layer._kept_tiles() is not None and layer.readable_tiles() is None
+    x = torch.randn(m, k, device=DEV, generator=g).to(dtype)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        got = layer(x)
+        torch.cuda.synchronize()
+    assert any('e2m3' in e.key and 'gemm' in e.key for e in prof.key_averages())
+    want = harness.linear_forward(x, layer.w_int_packed, layer.w_scale, layer.w_add)
+    want = want if layer.bias is None else want + layer.bias
+    assert int((got != want).any(1).sum()) <= 1
+    layer.w_int_packed.zero_()                                       # written by hand: the packed codes serve until the tiles are laid out again
+    assert layer._kept_tiles() is None
+    assert torch.equal(layer(x), harness.linear_forward(x, layer.w_int_packed, layer.w_scale, layer.w_add) + (0 if layer.bias is None else layer.bias))
