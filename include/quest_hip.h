@@ -98,6 +98,8 @@ int quest_fused_matmul_dequantize_int4_int4t(void *mat_d, const uint8_t *mat_a, 
  */
 int quest_linear_few_tokens(void *out, const void *x, const uint8_t *w_packed, const int32_t *w_add, const void *w_scale, const void *bias,
                             int size_m, int size_k, int size_n, float had_scale, int dtype, void *stream);
+/* whether (size_m, size_k) is of the sizes that it takes (0 or 1): had_scale, alignment and size_n aside */
+int quest_linear_few_tokens_available(int size_m, int size_k);
 
 /*
  * quest_fused_matmul_dequantize_int4_int4t with a caller-owned workspace, which lets a handful of tokens

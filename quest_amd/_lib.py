@@ -59,6 +59,7 @@ SIGNATURES = {
     'quest_fused_matmul_dequantize_bias_int4_int4t': [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     'quest_fused_matmul_dequantize_bias_e2m3': [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     'quest_pack_weight_int4': [_vp, _vp, _vp, _vp, _i, _i, _f, _i, _i, _vp],
+    'quest_linear_few_tokens_available': [_i, _i],
     'quest_linear_few_tokens': [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _f, _i, _vp],
     'quest_rmsnorm_rows': [_vp, _vp, _vp, _vp, _f, _i, ctypes.c_long, _i, _i, _vp],
     'quest_dense_rows': [_vp, _vp, _vp, _i, _i, _i, _i, _vp],

@@ -290,6 +290,8 @@ static bool few_tokens_takes(int M, int K) {
 
 using namespace quest;
 
+extern "C" int quest_linear_few_tokens_available(int size_m, int size_k) { return size_m > 0 && size_k > 0 && few_tokens_takes(size_m, size_k); }
+
 extern "C" int quest_linear_few_tokens(void *out, const void *x, const uint8_t *w_packed, const int32_t *w_add, const void *w_scale, const void *bias,
                                        int size_m, int size_k, int size_n, float had_scale, int dtype, void *stream) {
     forget_stale_error();

@@ -438,7 +438,8 @@ int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, fl
     const long max_rows = (((1L << 31) - 1) / ((long)ldx * 2)) & ~31L;
     if (max_rows == 0) return QUEST_ERR_UNSUPPORTED;
     const size_t es = 2;
-    const int cus = tiles != nullptr ? device_cu_count(st) : 0;
+    // (fewer than 256 rows are fewer than two workgroups of the staged form per CU of any gfx950 partition: not worth the question)
+    const int cus = tiles != nullptr && M >= 256 ? device_cu_count(st) : 256;
     for (long r0 = 0; r0 < M; r0 += max_rows) {
         const int rows = (int)(M - r0 < max_rows ? M - r0 : max_rows);
         auto at = [&](const void *p, size_t row_elems, size_t elem) -> void * {

@@ -124,20 +124,18 @@ bool gemm_takes(int64_t m, int64_t k, int64_t n, bool tiles) {
     return k % 32 == 0 && k < 131072 && m * (k / 2) < (1ll << 31) && n * (k / 2) < (1ll << 31);
 }
 
-// One activation's codes in a single scratch allocation: packed nibbles, row sums and scales, or E2M3 tiles and scales.
+// One activation's codes in scratch memory: packed nibbles, row sums and scales, or E2M3 tiles and scales.
 struct Codes {
-    at::Tensor hold;
     uint8_t *codes = nullptr;         // packed nibbles or tiles
     int32_t *row_sum = nullptr;
     void *scale = nullptr;
     bool tiles = false;
-    Codes(int64_t m, int64_t k, bool as_tiles, c10::Device dev) : tiles(as_tiles) {
-        const int64_t body = up(as_tiles ? (int64_t)quest_e2m3_tiles_bytes((int)m, (int)k) : m * (k / 2));
-        const int64_t sums = as_tiles ? 0 : up(4 * m);
-        hold = make({body + sums + 2 * m}, at::kByte, dev);
-        codes = (uint8_t *)hold.data_ptr();
-        row_sum = as_tiles ? nullptr : (int32_t *)(codes + body);
-        scale = codes + body + sums;
+    static int64_t body(int64_t m, int64_t k, bool as_tiles) { return up(as_tiles ? (int64_t)quest_e2m3_tiles_bytes((int)m, (int)k) : m * (k / 2)); }
+    static int64_t bytes(int64_t m, int64_t k, bool as_tiles) { return body(m, k, as_tiles) + (as_tiles ? 0 : up(4 * m)) + up(2 * m); }
+    Codes(void *at, int64_t m, int64_t k, bool as_tiles) : codes((uint8_t *)at), tiles(as_tiles) {
+        const int64_t behind = body(m, k, as_tiles);
+        row_sum = as_tiles ? nullptr : (int32_t *)(codes + behind);
+        scale = codes + behind + (as_tiles ? 0 : up(4 * m));
     }
 };
 
@@ -179,13 +177,14 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     };
     const int rc = on(args.dev, [&](void *st) {
         const int dt = dtype_code(type);
-        if (m <= 16 && !tiles) {                             // in one launch where that kernel takes it
+        if (!tiles && quest_linear_few_tokens_available((int)m, (int)k)) {
             out = result();
             const int rc = quest_linear_few_tokens(out.data_ptr(), x->data_ptr(), (const uint8_t *)w->data_ptr(), (const int32_t *)w_add->data_ptr(), w_scale->data_ptr(),
                                                    bias ? bias->data_ptr() : nullptr, (int)m, (int)k, (int)n, (float)had_scale, dt, st);
             if (rc == QUEST_OK) return rc;
         }
-        Codes q(m, kt, tiles, args.dev);
+        const at::Tensor hold = make({Codes::bytes(m, kt, tiles)}, at::kByte, args.dev);
+        const Codes q(hold.data_ptr(), m, kt, tiles);
         int rc = kt != k && had_scale == 0. ? quest_quantize_e2m3_padded(x->data_ptr(), q.scale, q.codes, (int)k, (int)m, dt, st)
                  : tiles ? quest_hadamard_quantize_e2m3(x->data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, (int)k, (int)m, (float)had_scale, dt, st)
                          : quest_hadamard_quantize_int4(x->data_ptr(), q.scale, q.codes, q.row_sum, nullptr, (int)k, (int)m, (float)had_scale, dt, st);
@@ -453,41 +452,42 @@ void launched(int rc, const char *what) {
 }
 
 // the GEMM of a projection on quantised activations: dst = product, or dst += product with the two roundings of x + y
-void project(const Linear &w, const Codes &q, at::Tensor &dst, int m, int dt, void *st, bool add_to_dst = false) {
+void project(const Linear &w, const Codes &q, void *dst, int m, int dt, void *st, bool add_to_dst = false) {
     if (q.tiles) {
         auto *f = add_to_dst ? quest_fused_matmul_dequantize_add_e2m3 : quest_fused_matmul_dequantize_e2m3;
-        launched(f(dst.data_ptr(), q.codes, w.tiles->data_ptr(), q.scale, w.scale->data_ptr(), m, w.k, w.n, dt, st), "projection");
+        launched(f(dst, q.codes, w.tiles->data_ptr(), q.scale, w.scale->data_ptr(), m, w.k, w.n, dt, st), "projection");
     } else {
         auto *f = add_to_dst ? quest_fused_matmul_dequantize_add_int4_int4t : quest_fused_matmul_dequantize_int4_int4t;
-        launched(f(dst.data_ptr(), q.codes, (const uint8_t *)w.packed->data_ptr(), q.row_sum, (const int32_t *)w.add->data_ptr(),
+        launched(f(dst, q.codes, (const uint8_t *)w.packed->data_ptr(), q.row_sum, (const int32_t *)w.add->data_ptr(),
                    q.scale, w.scale->data_ptr(), m, w.k, w.n, dt, st), "projection");
     }
 }
 
-void quantise_into(const Codes &q, const at::Tensor &x, int m, int k, int dt, void *st) {
-    launched(q.tiles ? quest_hadamard_quantize_e2m3(x.data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, k, m, kHadamardEntry, dt, st)
-                     : quest_hadamard_quantize_int4(x.data_ptr(), q.scale, q.codes, q.row_sum, nullptr, k, m, kHadamardEntry, dt, st),
+void quantise_into(const Codes &q, const void *x, int m, int k, int dt, void *st) {
+    launched(q.tiles ? quest_hadamard_quantize_e2m3(x, q.scale, q.codes, nullptr, nullptr, nullptr, k, m, kHadamardEntry, dt, st)
+                     : quest_hadamard_quantize_int4(x, q.scale, q.codes, q.row_sum, nullptr, k, m, kHadamardEntry, dt, st),
              "activation kernel");
 }
 
-Codes quantised(const at::Tensor &x, int m, int k, bool tiles, c10::Device dev, int dt, void *st) {
-    Codes q(m, k, tiles, dev);
-    quantise_into(q, x, m, k, dt, st);
-    return q;
+// a projection of x without tiles on so few tokens that quantiser and GEMM are one launch; false: nothing was launched
+bool project_few(const Linear &w, const void *x, void *dst, int m, int dt, void *st) {
+    if (w.tiles != nullptr || !quest_linear_few_tokens_available(m, w.k)) return false;
+    const int rc = quest_linear_few_tokens(dst, x, (const uint8_t *)w.packed->data_ptr(), (const int32_t *)w.add->data_ptr(), w.scale->data_ptr(), nullptr, m, w.k, w.n,
+                                           kHadamardEntry, dt, st);
+    if (rc == QUEST_ERR_UNSUPPORTED) return false;
+    launched(rc, "projection");
+    return true;
 }
 
-Codes normed(at::Tensor &x, const at::Tensor *branch, const at::Tensor &weight, double eps, int m, int k, bool tiles, c10::Device dev,
-             int dt, void *st) {
-    Codes q(m, k, tiles, dev);
+void norm_into(const Codes &q, at::Tensor &x, const void *branch, const at::Tensor &weight, double eps, int m, int k, int dt, void *st) {
     int rc;
     if (branch == nullptr)
-        rc = tiles ? quest_rmsnorm_hadamard_quantize_e2m3(x.data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, nullptr, k, m, kHadamardEntry, dt, st)
-                   : quest_rmsnorm_hadamard_quantize_int4(x.data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, q.row_sum, nullptr, nullptr, k, m, kHadamardEntry, dt, st);
+        rc = q.tiles ? quest_rmsnorm_hadamard_quantize_e2m3(x.data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, nullptr, k, m, kHadamardEntry, dt, st)
+                     : quest_rmsnorm_hadamard_quantize_int4(x.data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, q.row_sum, nullptr, nullptr, k, m, kHadamardEntry, dt, st);
     else
-        rc = tiles ? quest_add_rmsnorm_hadamard_quantize_e2m3(x.data_ptr(), branch->data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, k, m, kHadamardEntry, dt, st)
-                   : quest_add_rmsnorm_hadamard_quantize_int4(x.data_ptr(), branch->data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, q.row_sum, k, m, kHadamardEntry, dt, st);
+        rc = q.tiles ? quest_add_rmsnorm_hadamard_quantize_e2m3(x.data_ptr(), branch, weight.data_ptr(), (float)eps, q.scale, q.codes, k, m, kHadamardEntry, dt, st)
+                     : quest_add_rmsnorm_hadamard_quantize_int4(x.data_ptr(), branch, weight.data_ptr(), (float)eps, q.scale, q.codes, q.row_sum, k, m, kHadamardEntry, dt, st);
     launched(rc, "norm kernel");
-    return q;
 }
 
 // whether scaled_dot_product_attention would run the flash kernel whose bits ours gives: not switched off, no backend put before it
@@ -541,82 +541,90 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     on(args.dev, [&](void *st) {
         const int dt = dtype_code(type);
 
+        // One scratch allocation for the block: the codes that the GEMMs read one after the other; the heads, and where they were the gated
+        // unit's outputs; the attention's outputs and, where no GEMM adds them, the output projection's; the down projection's codes.
+        // Up to 64 tokens fp16 keeps torch's silu: the kernels' fast exponential gives torch's bits for every bf16 gate, but for two
+        // fp16 ones it does not.
+        const bool torch_silu = m <= 64 && type == at::kHalf, glu_tiles = glu.tiles != nullptr && !torch_silu, down_tiles = down.tiles != nullptr;
+        const int64_t codes_b = std::max({Codes::bytes(m, c, qkv.tiles != nullptr), Codes::bytes(m, c, o.tiles != nullptr), Codes::bytes(m, c, glu_tiles)});
+        const int64_t wide_b = up(2 * m * std::max<int64_t>(3 * c64, !glu_tiles && m <= 64 ? 2 * (int64_t)hidden : hidden)), core_b = up(2 * m * c64);
+        const at::Tensor scratch = make({codes_b + wide_b + 2 * core_b + Codes::bytes(m, hidden, down_tiles)}, at::kByte, args.dev);
+        uint8_t *const codes = (uint8_t *)scratch.data_ptr(), *const wide = codes + codes_b, *const core = wide + wide_b, *const att = core + core_b;
+        const Codes act(att + core_b, m, hidden, down_tiles);
+
         // norm -> q, k, v with q and k rotated
-        at::Tensor heads = make({m, 3 * c}, type, args.dev);
         {
-            const Codes q = normed(x, branch, *norm1, eps1, m, c, qkv.tiles != nullptr, args.dev, dt, st);
+            const Codes q(codes, m, c, qkv.tiles != nullptr);
+            norm_into(q, x, branch ? branch->data_ptr() : nullptr, *norm1, eps1, m, c, dt, st);
             const float *f = (const float *)freqs->data_ptr();
             int rc = q.tiles ? (t >= 32 && head_dim % 32 == 0
-                                    ? quest_fused_matmul_dequantize_rope_e2m3(heads.data_ptr(), q.codes, qkv.tiles->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st)
+                                    ? quest_fused_matmul_dequantize_rope_e2m3(wide, q.codes, qkv.tiles->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st)
                                     : QUEST_ERR_UNSUPPORTED)
-                             : quest_fused_matmul_dequantize_rope_int4_int4t(heads.data_ptr(), q.codes, (const uint8_t *)qkv.packed->data_ptr(), q.row_sum, (const int32_t *)qkv.add->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st);
+                             : quest_fused_matmul_dequantize_rope_int4_int4t(wide, q.codes, (const uint8_t *)qkv.packed->data_ptr(), q.row_sum, (const int32_t *)qkv.add->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st);
             if (rc == QUEST_ERR_UNSUPPORTED || rc == QUEST_ERR_BAD_SHAPE) {        // nothing was launched: the two calls
-                project(qkv, q, heads, m, dt, st);
-                rc = quest_rope_interleaved(heads.data_ptr(), f, m, (int)t, 3 * c, 2 * c, head_dim, dt, st);
+                project(qkv, q, wide, m, dt, st);
+                rc = quest_rope_interleaved(wide, f, m, (int)t, 3 * c, 2 * c, head_dim, dt, st);
             }
             launched(rc, "QKV projection");
         }
         // causal attention: the library's where ours does not take the heads, gives other bits (a 4-bit quantiser follows) or is not in the
         // place of the library kernel that the caller's choice of backends names
-        at::Tensor core;
+        const void *attended = core;
+        at::Tensor theirs;
         int rc = QUEST_ERR_UNSUPPORTED;
-        if (t <= QUEST_ATTENTION_SAME_BITS(head_dim) && default_flash_attention()) {
-            core = make({m, c64}, type, args.dev);
-            rc = quest_causal_attention(core.data_ptr(), heads.data_ptr(), (int)b, (int)t, (int)n_head, head_dim, dt, st);
-        }
+        if (t <= QUEST_ATTENTION_SAME_BITS(head_dim) && default_flash_attention())
+            rc = quest_causal_attention(core, wide, (int)b, (int)t, (int)n_head, head_dim, dt, st);
         if (rc == QUEST_ERR_UNSUPPORTED) {
             const int64_t row = 3 * c64;
-            const auto part = [&](int64_t i) { return heads.as_strided({b, n_head, t, head_dim}, {t * row, head_dim, row, 1}, i * c64); };
-            core = at::scaled_dot_product_attention(part(0), part(1), part(2), {}, 0.0, true).transpose(1, 2).contiguous();
+            const at::Tensor heads = scratch.narrow(0, codes_b, 2 * m * row).view(type);
+            const auto part = [&](int64_t i) { return heads.as_strided({b, n_head, t, head_dim}, {t * row, head_dim, row, 1}, heads.storage_offset() + i * c64); };
+            theirs = at::scaled_dot_product_attention(part(0), part(1), part(2), {}, 0.0, true).transpose(1, 2).contiguous();
+            attended = theirs.data_ptr();
         } else {
             launched(rc, "attention");
         }
         // output projection: into the residual stream where its GEMM can add
-        bool has_att = false;
-        at::Tensor att;
-        {
-            const Codes q = quantised(core, m, c, o.tiles != nullptr, args.dev, dt, st);
-            if (q.tiles || quest_fused_matmul_dequantize_add_available(m, c, c, st)) {
-                project(o, q, x, m, dt, st, true);
-            } else {
-                has_att = true;
-                att = make({m, c}, type, args.dev);
-                project(o, q, att, m, dt, st);
-            }
+        bool has_att = project_few(o, attended, att, m, dt, st);
+        if (!has_att) {
+            const Codes q(codes, m, c, o.tiles != nullptr);
+            quantise_into(q, attended, m, c, dt, st);
+            has_att = !q.tiles && !quest_fused_matmul_dequantize_add_available(m, c, c, st);
+            project(o, q, has_att ? (void *)att : x.data_ptr(), m, dt, st, !has_att);
         }
-        // norm -> gated unit -> its codes
-        const bool down_tiles = down.tiles != nullptr;
-        // Up to 64 tokens fp16 keeps torch's silu: the kernels' fast exponential gives torch's bits for every bf16 gate, but for two
-        // fp16 ones it does not.
-        const bool torch_silu = m <= 64 && type == at::kHalf;
-        Codes act(m, hidden, down_tiles, args.dev);
+        // norm -> gated unit -> its codes, or, few tokens, its outputs in `gated`
+        const void *gated = nullptr;
+        at::Tensor torchs;
         {
-            const Codes q = normed(x, has_att ? &att : nullptr, *norm2, eps2, m, c, glu.tiles != nullptr && !torch_silu, args.dev, dt, st);
+            const Codes q(codes, m, c, glu_tiles);
+            norm_into(q, x, has_att ? att : nullptr, *norm2, eps2, m, c, dt, st);
             if (!q.tiles && m <= 64) {
                 // the weight-streaming GEMM has no gated epilogue: gate and up side by side, the product inside the quantiser
-                at::Tensor both = make({m, 2 * hidden}, type, args.dev);
-                project(gate_up, q, both, m, dt, st);
+                project(gate_up, q, wide, m, dt, st);
                 if (torch_silu) {
-                    const at::Tensor gated = at::silu(both.narrow(1, 0, hidden)).mul_(both.narrow(1, hidden, hidden)).contiguous();
-                    quantise_into(act, gated, m, hidden, dt, st);
+                    const at::Tensor both = scratch.narrow(0, codes_b, 4 * (int64_t)m * hidden).view(type).view({m, 2 * hidden});
+                    torchs = at::silu(both.narrow(1, 0, hidden)).mul_(both.narrow(1, hidden, hidden)).contiguous();
+                    gated = torchs.data_ptr();
                 } else {
-                    launched(down_tiles ? quest_silu_mul_hadamard_quantize_e2m3(both.data_ptr(), act.scale, act.codes, nullptr, hidden, m, kHadamardEntry, dt, st)
-                                        : quest_silu_mul_hadamard_quantize_int4(both.data_ptr(), act.scale, act.codes, act.row_sum, nullptr, nullptr, hidden, m, kHadamardEntry, dt, st),
+                    launched(down_tiles ? quest_silu_mul_hadamard_quantize_e2m3(wide, act.scale, act.codes, nullptr, hidden, m, kHadamardEntry, dt, st)
+                                        : quest_silu_mul_hadamard_quantize_int4(wide, act.scale, act.codes, act.row_sum, nullptr, nullptr, hidden, m, kHadamardEntry, dt, st),
                              "gated unit");
                 }
             } else {
-                at::Tensor gated = make({m, hidden}, type, args.dev);
-                launched(q.tiles ? quest_fused_matmul_dequantize_swiglu_e2m3(gated.data_ptr(), q.codes, glu.tiles->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st)
-                                 : quest_fused_matmul_dequantize_swiglu_int4_int4t(gated.data_ptr(), q.codes, (const uint8_t *)glu.packed->data_ptr(), q.row_sum, (const int32_t *)glu.add->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st),
+                launched(q.tiles ? quest_fused_matmul_dequantize_swiglu_e2m3(wide, q.codes, glu.tiles->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st)
+                                 : quest_fused_matmul_dequantize_swiglu_int4_int4t(wide, q.codes, (const uint8_t *)glu.packed->data_ptr(), q.row_sum, (const int32_t *)glu.add->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st),
                          "gated projection");
-                quantise_into(act, gated, m, hidden, dt, st);
+                gated = wide;
             }
         }
         if (down_tiles || quest_fused_matmul_dequantize_add_available(m, hidden, c, st)) {
-            project(down, act, x, m, dt, st, true);
+            if (gated != nullptr) quantise_into(act, gated, m, hidden, dt, st);
+            project(down, act, x.data_ptr(), m, dt, st, true);
         } else {
             mlp = make({b, t, c64}, type, args.dev);
-            project(down, act, mlp, m, dt, st);
+            if (gated == nullptr || !project_few(down, gated, mlp.data_ptr(), m, dt, st)) {
+                if (gated != nullptr) quantise_into(act, gated, m, hidden, dt, st);
+                project(down, act, mlp.data_ptr(), m, dt, st);
+            }
         }
         return 0;
     });
