@@ -281,6 +281,33 @@ int quest_int4_to_e2m3_tiles_padded(void *tiles, const uint8_t *x_int_packed, in
 int quest_quantize_e2m3_padded(const void *x, void *scale, void *x_tiles, int group_size, int batch_size, int dtype, void *stream);
 
 /*
+ * The activation kernel in front of a GEMM, with a producer of the activation or without, which reads memory ahead for that GEMM meanwhile:
+ * the codes, sums and scales of quest_[add_][rmsnorm_ | silu_mul_]hadamard_quantize_int4 or, where `tiles` is given, the tiles of their _e2m3
+ * forms (QUEST_PRODUCER_NONE without the transform: of quest_quantize_e2m3_padded).  QUEST_ERR_UNSUPPORTED, with nothing launched, where only the
+ * butterfly kernel takes the row.  next: NULL, or next_blocks pieces next_pitch bytes apart of which the first next_bytes are
+ * read and dropped, all inside one allocation.  The outputs do not depend on it.
+ */
+enum { QUEST_PRODUCER_NONE = 0, QUEST_PRODUCER_RMSNORM = 1, QUEST_PRODUCER_SILU_MUL = 2 };
+typedef struct quest_activation {
+    int producer;
+    const void *x;                /* with `branch`: replaced by x + branch */
+    const void *branch;           /* NULL, or (RMSNorm) what is added to x first */
+    const void *norm_weight;
+    float eps;
+    void *scale;
+    uint8_t *x_int_packed;        /* with x_int_row_sum, where tiles is NULL */
+    int32_t *x_int_row_sum;
+    void *tiles;
+    int size_k, size_m;
+    float had_scale;
+    int dtype;
+    const void *next;
+    size_t next_pitch, next_bytes;
+    int next_blocks;
+} quest_activation;
+int quest_activation_before_gemm(const quest_activation *a, void *stream);
+
+/*
  * mat_d (size_m, size_n) dtype = quest_fused_matmul_dequantize_int4_int4t's result for the same codes, from their
  * E2M3 tiles: dtype( f32(2 S) * (0.5f * vec_a_mul[m] * vec_b_mul[n]) ) with S = sum_k (qa + 1/2)(qb + 1/2) accumulated
  * exactly.  size_k % 128 == 0 and <= 65536; any size_m, size_n >= 1; scale vectors 4-byte aligned.

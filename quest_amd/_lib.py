@@ -44,6 +44,7 @@ SIGNATURES = {
     'quest_e2m3_tiles_bytes': [_i, _i],
     'quest_int4_to_e2m3_tiles': [_vp, _vp, _i, _i, _vp],
     'quest_int4_to_e2m3_tiles_padded': [_vp, _vp, _i, _i, _vp],
+    'quest_activation_before_gemm': [_vp, _vp],
     'quest_quantize_e2m3_padded': [_vp, _vp, _vp, _i, _i, _i, _vp],
     'quest_fused_matmul_dequantize_e2m3': [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
     'quest_fused_matmul_dequantize_add_e2m3': [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp],
@@ -69,6 +70,13 @@ SIGNATURES = {
 # entry points that do not return an int status
 _RESTYPES = {'quest_status_string': ctypes.c_char_p, 'quest_e2m3_tiles_bytes': ctypes.c_size_t,
              'quest_gemm_workspace_bytes': ctypes.c_size_t, 'quest_gemm_noalloc_scratch_bytes': ctypes.c_size_t}
+
+
+class Activation(ctypes.Structure):
+    _fields_ = [('producer', _i), ('x', _vp), ('branch', _vp), ('norm_weight', _vp), ('eps', _f), ('scale', _vp), ('x_int_packed', _vp), ('x_int_row_sum', _vp),
+                ('tiles', _vp), ('size_k', _i), ('size_m', _i), ('had_scale', _f), ('dtype', _i), ('next', _vp), ('next_pitch', ctypes.c_size_t),
+                ('next_bytes', ctypes.c_size_t), ('next_blocks', _i)]
+
 
 _lib = None
 

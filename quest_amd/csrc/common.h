@@ -310,12 +310,19 @@ int launch_gemm_decode_splitk(int out_kind, void *out, const uint8_t *a, const u
                               size_t workspace_bytes, hipStream_t st);
 size_t gemm_decode_workspace_bytes(int K, int N);
 
+// Memory that the kernel after this one will read first: the leading `bytes_of_each` bytes of `row_blocks` pieces `pitch` bytes apart, all whole 16s.
+struct NextWeights {
+    const void *at = nullptr;
+    size_t pitch = 0, bytes_of_each = 0;
+    int row_blocks = 0;
+};
+
 // hadamard_mfma.hip: the matrix-core fused activation kernel, optionally with the producer of the activation in
 // front (pre: 0 none, 1 RMSNorm, 2 SiLU(gate) * up); sum_bias is added to every row sum.  QUEST_ERR_UNSUPPORTED when it does
 // not apply
 int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, float eps, void *scale, uint8_t *packed,
                                   int32_t *row_sum, void *x_had, void *pre_out, int K, int M, float had_scale, int dtype,
-                                  hipStream_t st, const void *add_in = nullptr, void *sum_out = nullptr, uint8_t *tiles = nullptr, int sum_bias = 0);
+                                  hipStream_t st, const void *add_in = nullptr, void *sum_out = nullptr, uint8_t *tiles = nullptr, int sum_bias = 0, const NextWeights &next = {});
 
 inline int check_dtype(int dtype) { return dtype == QUEST_DTYPE_BF16 || dtype == QUEST_DTYPE_FP16; }
 inline int aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0; }

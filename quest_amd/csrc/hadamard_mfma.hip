@@ -61,16 +61,46 @@ struct Shape {
 //   kPreSiluMul  y = dtype(dtype(silu(gate)) * up), gate and up the two halves of a (M, 2 K) row (llama.py:117-118).
 enum { kPreNone = 0, kPreRmsNorm = 1, kPreSiluMul = 2 };
 
+// The workgroups behind the kernel's own (from number `first` on, a multiple of 8; 0: there are none) read what the next kernel starts on: the
+// activation kernel leaves memory idle, and a GEMM of few tokens is mostly the wait for its first weights (NextWeights in common.h).  XCD x takes
+// the x-th eighth of the pieces, as the smaller-tile GEMMs deal their channels.  What a GEMM gains, weights from HBM: (37, 1024, 3072) 0.8 us of 4, (200,
+// 4096, 11008) 2.8 of 21, (1000, 6912, 2560) 3.9 of 25; from the Infinity Cache 0.2 to 0.5.  Models: 1600M at 2 x 500 tokens 2953 -> 2822 us, 12 layers
+// at 32 x 512 3600 -> 3530, at 1 x 37 515 -> 502.
+struct Ahead {
+    const uint8_t *at;
+    unsigned pitch16, each16;       // 16-byte units
+    int pieces, first;
+};
+__device__ __forceinline__ void read_ahead(const Ahead &a) {
+    const int p = (int)blockIdx.x - a.first, xcd = p & 7, rank = p >> 3, ranks = ((int)gridDim.x - a.first) >> 3;
+    const unsigned lo = (unsigned)((long)a.pieces * xcd / 8), hi = (unsigned)((long)a.pieces * (xcd + 1) / 8), total = (hi - lo) * a.each16;
+    constexpr unsigned kEach = 4;
+    for (unsigned i = (unsigned)rank * blockDim.x * kEach + threadIdx.x; i < total; i += (unsigned)ranks * blockDim.x * kEach) {
+        uint4 v[kEach];
+#pragma unroll
+        for (unsigned u = 0; u < kEach; u++) {
+            const unsigned j = min(i + u * blockDim.x, total - 1), piece = j / a.each16;
+            v[u] = *reinterpret_cast<const uint4 *>(a.at + ((size_t)(lo + piece) * a.pitch16 + (j - piece * a.each16)) * 16);
+        }
+#pragma unroll
+        for (unsigned u = 0; u < kEach; u++) asm volatile("" ::"v"(v[u].x), "v"(v[u].y), "v"(v[u].z), "v"(v[u].w));
+    }
+}
+
 // G = lanes of a half-wave per row (the row's blocks rounded up to a power of two): a wave holds 32 / G rows.
 // RAG: rows of whole 32s without the transform (K % 128 != 0): the last block is cut short, and tiles are those of the row with zeros behind it up
 // to a whole 128 (the FP6 zero, so that what stands there in the weights' tiles does not matter).
-template <int DT, int WPR, int G, int PRE, bool TL, bool RAG>
+// AHEAD: with workgroups that read ahead (a kernel of its own: the question alone costs the others 0.3 us of 16 at bf16 [8192, 4096]).
+template <int DT, int WPR, int G, int PRE, bool TL, bool RAG, bool AHEAD>
 __global__ void __launch_bounds__((64 * Shape<WPR, G, TL>::kWaves), (Shape<WPR, G, TL>::kMinBlocks))
 hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ norm_w,
                               uint16_t *__restrict__ scale, uint32_t *__restrict__ packed, int32_t *__restrict__ row_sum,
                               uint16_t *__restrict__ x_had, uint16_t *__restrict__ pre_out, const uint16_t *add_in,
                               uint16_t *sum_out, uint8_t *__restrict__ tiles, int xcd_chunk, int K, int M, int ldx,
-                              uint32_t entry_bits, float eps, int sum_bias) {
+                              uint32_t entry_bits, float eps, int sum_bias, Ahead ahead) {
+    if constexpr (AHEAD) {
+        if ((int)blockIdx.x >= ahead.first) return read_ahead(ahead);                       // uniform: the whole workgroup
+    }
     static_assert(WPR == 1 || G == 32, "rows shared by waves: whole waves");
     static_assert(!RAG || PRE == kPreNone, "rows that end inside a block come from no producer");
     using Sh = Shape<WPR, G, TL>;
@@ -335,9 +365,10 @@ struct Args {
     hipStream_t st;
     int sum_bias;
     int cus;                   // compute units of the device (only looked at when tiles are written)
+    NextWeights next;
 };
 
-template <int DT, int WPR, int G, int PRE, bool TL, bool RAG>
+template <int DT, int WPR, int G, int PRE, bool TL, bool RAG, bool AHEAD>
 static void launch_shape_as(const Args &a) {
     using Sh = hq::Shape<WPR, G, TL>;
     constexpr int rows = Sh::kTileRows;                            // rows per workgroup
@@ -346,30 +377,40 @@ static void launch_shape_as(const Args &a) {
         xcd_chunk = (grid + 7) / 8;
         grid = 8 * xcd_chunk;
     }
-    hq::hadamard_quantize_mfma_kernel<DT, WPR, G, PRE, TL, RAG><<<dim3(grid), dim3(64 * Sh::kWaves), 0, a.st>>>(
+    hq::Ahead ahead = {(const uint8_t *)a.next.at, (unsigned)(a.next.pitch / 16), (unsigned)(a.next.bytes_of_each / 16), a.next.row_blocks, 0};
+    if constexpr (AHEAD) {
+        const size_t per_workgroup = 2 * 4 * 16 * 64 * Sh::kWaves;                          // two turns of read_ahead
+        const size_t more = (a.next.row_blocks * a.next.bytes_of_each + per_workgroup - 1) / per_workgroup;
+        ahead.first = (grid + 7) & ~7;
+        grid = ahead.first + (int)((more < 4096 ? more : 4096) + 7) / 8 * 8;
+    }
+    hq::hadamard_quantize_mfma_kernel<DT, WPR, G, PRE, TL, RAG, AHEAD><<<dim3(grid), dim3(64 * Sh::kWaves), 0, a.st>>>(
         (const uint16_t *)a.x, (const uint16_t *)a.norm_w, (uint16_t *)a.scale, (uint32_t *)a.packed, a.row_sum,
         (uint16_t *)a.x_had, (uint16_t *)a.pre_out, (const uint16_t *)a.add_in, (uint16_t *)a.sum_out, a.tiles, xcd_chunk,
-        a.K, a.M, a.ldx, a.bits, a.eps, a.sum_bias);
+        a.K, a.M, a.ldx, a.bits, a.eps, a.sum_bias, ahead);
 }
 
 // Tiles go through the workgroup's LDS where a workgroup of eight (four) rows fits -- rows of 8 to 96 blocks -- and where
 // such workgroups are at least two per compute unit: below that the small workgroups, which write their 16-byte pieces
 // straight to the tiles, fill the device better (bf16 rows of 4096: 4.0 against 5.9 us for 512 rows, 7.3 against 7.2 us
 // for 2048, 14.5 against 11.5 us for 4096).  Same arithmetic and same bytes either way.
-template <int DT, int WPR, int G, int PRE, bool RAG>
+template <int DT, int WPR, int G, int PRE, bool RAG, bool AHEAD>
 static void launch_shape_for(const Args &a) {
     if constexpr (WPR <= 3 && G >= 8) {
         constexpr int rows = hq::Shape<WPR, G, true>::kTileRows;
-        if (a.tiles != nullptr && (a.M + rows - 1) / rows >= 2 * a.cus) return launch_shape_as<DT, WPR, G, PRE, true, RAG>(a);
+        if (a.tiles != nullptr && (a.M + rows - 1) / rows >= 2 * a.cus) return launch_shape_as<DT, WPR, G, PRE, true, RAG, AHEAD>(a);
     }
-    launch_shape_as<DT, WPR, G, PRE, false, RAG>(a);
+    launch_shape_as<DT, WPR, G, PRE, false, RAG, AHEAD>(a);
 }
 template <int DT, int WPR, int G, int PRE>
 static void launch_shape(const Args &a) {
     if constexpr (PRE == hq::kPreNone) {
-        if (a.K & 127) return launch_shape_for<DT, WPR, G, PRE, true>(a);
+        if (a.K & 127) return launch_shape_for<DT, WPR, G, PRE, true, false>(a);
     }
-    launch_shape_for<DT, WPR, G, PRE, false>(a);
+    if constexpr (WPR <= 3 && G >= 8) {
+        if (a.next.at != nullptr && a.next.row_blocks > 0 && a.next.bytes_of_each >= 16) return launch_shape_for<DT, WPR, G, PRE, false, true>(a);
+    }
+    launch_shape_for<DT, WPR, G, PRE, false, false>(a);
 }
 
 // rows of up to 32 blocks: one wave holds 32 / G of them
@@ -423,7 +464,7 @@ static void launch_dtype(int pre, const Args &a) {
 // with x a (M, 2 K) tensor.  tiles: the codes as E2M3 tiles (M rows; besides or instead of packed nibbles).
 int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, float eps, void *scale, uint8_t *packed,
                                   int32_t *row_sum, void *x_had, void *pre_out, int K, int M, float had_scale, int dtype,
-                                  hipStream_t st, const void *add_in, void *sum_out, uint8_t *tiles, int sum_bias) {
+                                  hipStream_t st, const void *add_in, void *sum_out, uint8_t *tiles, int sum_bias, const NextWeights &next) {
     uint32_t bits = 0;
     // (had_scale == 0: no transform; the kernel then only moves the chunks between lanes)
     if (K > 32768 || had_scale < 0.f || !representable16(had_scale, dtype, &bits)) return QUEST_ERR_UNSUPPORTED;
@@ -447,7 +488,7 @@ int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, fl
         };
         const Args a = {at(x, ldx, es), norm_w, at(scale, 1, es), (uint8_t *)at(packed, K / 2, 1), (int32_t *)at(row_sum, 1, 4),
                         at(x_had, K, es), at(pre_out, K, es), at(add_in, K, es), at(sum_out, K, es),
-                        tiles == nullptr ? nullptr : tiles + (size_t)(r0 / 32) * (size_t)((K + 127) / 128 * 2) * 1536, K, rows, ldx, bits, eps, st, sum_bias, cus};
+                        tiles == nullptr ? nullptr : tiles + (size_t)(r0 / 32) * (size_t)((K + 127) / 128 * 2) * 1536, K, rows, ldx, bits, eps, st, sum_bias, cus, r0 == 0 ? next : NextWeights{}};
         if (dtype == QUEST_DTYPE_BF16) launch_dtype<0>(pre, a);
         else launch_dtype<1>(pre, a);
     }

@@ -139,6 +139,54 @@ struct Codes {
     }
 };
 
+// One projection's weights.
+struct Linear {
+    const at::Tensor *packed, *scale, *add, *tiles;
+    int n, k;
+    bool take(Args &args, PyObject *t, at::ScalarType type, bool want_tiles) {
+        if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 4) return args.ok = false;
+        packed = args.tensor(PyTuple_GET_ITEM(t, 0));
+        if (!args.ok || packed->scalar_type() != at::kByte || packed->dim() != 2 || !fits_int(packed->size(0)) ||
+            !fits_int(packed->size(1) * 2))
+            return args.ok = false;
+        n = (int)packed->size(0);
+        k = (int)packed->size(1) * 2;
+        scale = args.tensor(PyTuple_GET_ITEM(t, 1), type, n);
+        add = args.tensor(PyTuple_GET_ITEM(t, 2), at::kInt, n);
+        PyObject *const form = want_tiles ? tiles_of(PyTuple_GET_ITEM(t, 3), PyTuple_GET_ITEM(t, 0)) : Py_None;
+        tiles = form != Py_None ? args.tensor(form, at::kByte, (int64_t)quest_e2m3_tiles_bytes(n, k)) : nullptr;
+        return args.ok;
+    }
+};
+
+// The activation kernel for a GEMM on w: codes of x, of its norm (x + branch first where there is one, in place), or of silu(gate) * up.  It
+// reads ahead for the GEMM.
+struct Producer {
+    int kind = QUEST_PRODUCER_NONE;
+    const void *branch = nullptr, *norm_weight = nullptr;
+    double eps = 0.;
+};
+// How much of the weights: what memory gives while the kernel runs (1600M model at 2 x 500 tokens 2953 us without, 2822 to 2828 with 4 to 40 MB).
+// Many tokens: nothing of weights that are more than that, for their GEMM is long and the memory busy (layers of 3065 to 11837 tokens x 10000 x 13000
+// read 30 to 100 MB ahead and were 1.5 to 3.7 % slower).  A layer on its own gains from 64 to 512 tokens ((91, 1664, 20608) 14.0 -> 13.3 us); fewer
+// are bound by the host, more by their products.
+size_t read_ahead_bytes(int64_t m, size_t weights) {
+    const size_t most = 8000000 + 8000 * (size_t)std::min<int64_t>(m, 2048);
+    return m > 2048 && weights > most ? 0 : std::min(weights, most);
+}
+int quantise_for(const Linear &w, const Codes &q, const void *x, const Producer &p, int m, int k, float had_scale, int dt, void *st) {
+    quest_activation a = {};
+    a.producer = p.kind, a.x = x, a.branch = p.branch, a.norm_weight = p.norm_weight, a.eps = (float)p.eps;
+    a.scale = q.scale, a.x_int_packed = q.tiles ? nullptr : q.codes, a.x_int_row_sum = q.row_sum, a.tiles = q.tiles ? q.codes : nullptr;
+    a.size_k = k, a.size_m = m, a.had_scale = had_scale, a.dtype = dt;
+    // row blocks of 32 channels: so much of the start of each that the kernel is not kept waiting by it
+    a.next_blocks = q.tiles ? (w.n + 31) / 32 : w.n / 32;
+    a.next = q.tiles ? w.tiles->data_ptr() : w.packed->data_ptr();
+    a.next_pitch = q.tiles ? quest_e2m3_tiles_bytes(32, (k + 127) / 128 * 128) : (size_t)k * 16;
+    a.next_bytes = a.next_blocks > 0 ? read_ahead_bytes(m, a.next_pitch * a.next_blocks) / a.next_blocks : 0;
+    return quest_activation_before_gemm(&a, st);
+}
+
 // ---- linear(x, w_packed, w_scale, w_add, w_tiles, bias, had_scale, out) ---------------------------------------------
 // The W4A4 linear layer: activation kernel, GEMM, bias.  x (..., K); w_tiles: None, or the weight's E2M3 tiles (see tiles_of) when the
 // FP6 kernel is wanted; out: None or the (M, N) result to fill.
@@ -186,6 +234,7 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         const at::Tensor hold = make({Codes::bytes(m, kt, tiles)}, at::kByte, args.dev);
         const Codes q(hold.data_ptr(), m, kt, tiles);
         int rc = kt != k && had_scale == 0. ? quest_quantize_e2m3_padded(x->data_ptr(), q.scale, q.codes, (int)k, (int)m, dt, st)
+                 : tiles && m >= 64 && m <= 512 ? quantise_for({w, w_scale, w_add, w_tiles, (int)n, (int)k}, q, x->data_ptr(), {}, (int)m, (int)k, (float)had_scale, dt, st)
                  : tiles ? quest_hadamard_quantize_e2m3(x->data_ptr(), q.scale, q.codes, nullptr, nullptr, nullptr, (int)k, (int)m, (float)had_scale, dt, st)
                          : quest_hadamard_quantize_int4(x->data_ptr(), q.scale, q.codes, q.row_sum, nullptr, (int)k, (int)m, (float)had_scale, dt, st);
         if (rc != QUEST_OK) return rc;
@@ -428,25 +477,6 @@ PyObject *add_mul_vv(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
 // (packed, scale, add, tiles or None) of the projections, glu the row-interleaved gate / up weights; tiles: which of the
 // four GEMMs (bit 0 qkv, 1 o, 2 gate_up, 3 down) run on E2M3 tiles where there are any; glu_of: gate_up's three tensors, their
 // addresses and their versions when glu was made from them.  Returns True, or the block's MLP output when it is still to be added.
-struct Linear {
-    const at::Tensor *packed, *scale, *add, *tiles;
-    int n, k;
-    bool take(Args &args, PyObject *t, at::ScalarType type, bool want_tiles) {
-        if (!PyTuple_Check(t) || PyTuple_GET_SIZE(t) != 4) return args.ok = false;
-        packed = args.tensor(PyTuple_GET_ITEM(t, 0));
-        if (!args.ok || packed->scalar_type() != at::kByte || packed->dim() != 2 || !fits_int(packed->size(0)) ||
-            !fits_int(packed->size(1) * 2))
-            return args.ok = false;
-        n = (int)packed->size(0);
-        k = (int)packed->size(1) * 2;
-        scale = args.tensor(PyTuple_GET_ITEM(t, 1), type, n);
-        add = args.tensor(PyTuple_GET_ITEM(t, 2), at::kInt, n);
-        PyObject *const form = want_tiles ? tiles_of(PyTuple_GET_ITEM(t, 3), PyTuple_GET_ITEM(t, 0)) : Py_None;
-        tiles = form != Py_None ? args.tensor(form, at::kByte, (int64_t)quest_e2m3_tiles_bytes(n, k)) : nullptr;
-        return args.ok;
-    }
-};
-
 void launched(int rc, const char *what) {
     TORCH_CHECK(rc == QUEST_OK, what, " failed with status ", rc, ": ", quest_status_string(rc));
 }
@@ -463,10 +493,9 @@ void project(const Linear &w, const Codes &q, void *dst, int m, int dt, void *st
     }
 }
 
-void quantise_into(const Codes &q, const void *x, int m, int k, int dt, void *st) {
-    launched(q.tiles ? quest_hadamard_quantize_e2m3(x, q.scale, q.codes, nullptr, nullptr, nullptr, k, m, kHadamardEntry, dt, st)
-                     : quest_hadamard_quantize_int4(x, q.scale, q.codes, q.row_sum, nullptr, k, m, kHadamardEntry, dt, st),
-             "activation kernel");
+void quantise_into(const Linear &w, const Codes &q, const void *x, int m, int k, int dt, void *st) {
+    int rc = quantise_for(w, q, x, {}, m, k, kHadamardEntry, dt, st);
+    launched(rc, "activation kernel");
 }
 
 // a projection of x without tiles on so few tokens that quantiser and GEMM are one launch; false: nothing was launched
@@ -479,15 +508,8 @@ bool project_few(const Linear &w, const void *x, void *dst, int m, int dt, void 
     return true;
 }
 
-void norm_into(const Codes &q, at::Tensor &x, const void *branch, const at::Tensor &weight, double eps, int m, int k, int dt, void *st) {
-    int rc;
-    if (branch == nullptr)
-        rc = q.tiles ? quest_rmsnorm_hadamard_quantize_e2m3(x.data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, nullptr, k, m, kHadamardEntry, dt, st)
-                     : quest_rmsnorm_hadamard_quantize_int4(x.data_ptr(), weight.data_ptr(), (float)eps, q.scale, q.codes, q.row_sum, nullptr, nullptr, k, m, kHadamardEntry, dt, st);
-    else
-        rc = q.tiles ? quest_add_rmsnorm_hadamard_quantize_e2m3(x.data_ptr(), branch, weight.data_ptr(), (float)eps, q.scale, q.codes, k, m, kHadamardEntry, dt, st)
-                     : quest_add_rmsnorm_hadamard_quantize_int4(x.data_ptr(), branch, weight.data_ptr(), (float)eps, q.scale, q.codes, q.row_sum, k, m, kHadamardEntry, dt, st);
-    launched(rc, "norm kernel");
+void norm_into(const Linear &w, const Codes &q, at::Tensor &x, const void *branch, const at::Tensor &weight, double eps, int m, int k, int dt, void *st) {
+    launched(quantise_for(w, q, x.data_ptr(), {QUEST_PRODUCER_RMSNORM, branch, weight.data_ptr(), eps}, m, k, kHadamardEntry, dt, st), "norm kernel");
 }
 
 // whether scaled_dot_product_attention would run the flash kernel whose bits ours gives: not switched off, no backend put before it
@@ -555,7 +577,7 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         // norm -> q, k, v with q and k rotated
         {
             const Codes q(codes, m, c, qkv.tiles != nullptr);
-            norm_into(q, x, branch ? branch->data_ptr() : nullptr, *norm1, eps1, m, c, dt, st);
+            norm_into(qkv, q, x, branch ? branch->data_ptr() : nullptr, *norm1, eps1, m, c, dt, st);
             const float *f = (const float *)freqs->data_ptr();
             int rc = q.tiles ? (t >= 32 && head_dim % 32 == 0
                                     ? quest_fused_matmul_dequantize_rope_e2m3(wide, q.codes, qkv.tiles->data_ptr(), q.scale, qkv.scale->data_ptr(), m, c, 3 * c, dt, f, (int)t, 2 * c, head_dim, st)
@@ -587,7 +609,7 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         bool has_att = project_few(o, attended, att, m, dt, st);
         if (!has_att) {
             const Codes q(codes, m, c, o.tiles != nullptr);
-            quantise_into(q, attended, m, c, dt, st);
+            quantise_into(o, q, attended, m, c, dt, st);
             has_att = !q.tiles && !quest_fused_matmul_dequantize_add_available(m, c, c, st);
             project(o, q, has_att ? (void *)att : x.data_ptr(), m, dt, st, !has_att);
         }
@@ -596,7 +618,7 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         at::Tensor torchs;
         {
             const Codes q(codes, m, c, glu_tiles);
-            norm_into(q, x, has_att ? att : nullptr, *norm2, eps2, m, c, dt, st);
+            norm_into(q.tiles || m > 64 ? glu : gate_up, q, x, has_att ? att : nullptr, *norm2, eps2, m, c, dt, st);
             if (!q.tiles && m <= 64) {
                 // the weight-streaming GEMM has no gated epilogue: gate and up side by side, the product inside the quantiser
                 project(gate_up, q, wide, m, dt, st);
@@ -605,9 +627,7 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
                     torchs = at::silu(both.narrow(1, 0, hidden)).mul_(both.narrow(1, hidden, hidden)).contiguous();
                     gated = torchs.data_ptr();
                 } else {
-                    launched(down_tiles ? quest_silu_mul_hadamard_quantize_e2m3(wide, act.scale, act.codes, nullptr, hidden, m, kHadamardEntry, dt, st)
-                                        : quest_silu_mul_hadamard_quantize_int4(wide, act.scale, act.codes, act.row_sum, nullptr, nullptr, hidden, m, kHadamardEntry, dt, st),
-                             "gated unit");
+                    launched(quantise_for(down, act, wide, {QUEST_PRODUCER_SILU_MUL}, m, hidden, kHadamardEntry, dt, st), "gated unit");
                 }
             } else {
                 launched(q.tiles ? quest_fused_matmul_dequantize_swiglu_e2m3(wide, q.codes, glu.tiles->data_ptr(), q.scale, glu.scale->data_ptr(), m, c, 2 * hidden, dt, st)
@@ -617,12 +637,12 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             }
         }
         if (down_tiles || quest_fused_matmul_dequantize_add_available(m, hidden, c, st)) {
-            if (gated != nullptr) quantise_into(act, gated, m, hidden, dt, st);
+            if (gated != nullptr) quantise_into(down, act, gated, m, hidden, dt, st);
             project(down, act, x.data_ptr(), m, dt, st, true);
         } else {
             mlp = make({b, t, c64}, type, args.dev);
             if (gated == nullptr || !project_few(down, gated, mlp.data_ptr(), m, dt, st)) {
-                if (gated != nullptr) quantise_into(act, gated, m, hidden, dt, st);
+                if (gated != nullptr) quantise_into(down, act, gated, m, hidden, dt, st);
                 project(down, act, mlp.data_ptr(), m, dt, st);
             }
         }

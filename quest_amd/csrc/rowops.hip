@@ -616,6 +616,22 @@ extern "C" int quest_hadamard_quantize_e2m3(const void *x, void *scale, void *x_
                                          batch_size, had_scale, dtype, (hipStream_t)stream, nullptr, nullptr, (uint8_t *)x_tiles);
 }
 
+extern "C" int quest_activation_before_gemm(const quest_activation *a, void *stream) {
+    forget_stale_error();
+    if (!a || !a->x || !a->scale || (!a->tiles && (!a->x_int_packed || !a->x_int_row_sum))) return QUEST_ERR_NULL_POINTER;
+    if (a->producer < QUEST_PRODUCER_NONE || a->producer > QUEST_PRODUCER_SILU_MUL || (a->producer != QUEST_PRODUCER_RMSNORM && a->branch)) return QUEST_ERR_UNSUPPORTED;
+    if (a->producer == QUEST_PRODUCER_RMSNORM && !a->norm_weight) return QUEST_ERR_NULL_POINTER;
+    if (!check_dtype(a->dtype)) return QUEST_ERR_BAD_DTYPE;
+    const bool padded = a->producer == QUEST_PRODUCER_NONE && a->had_scale == 0.f && a->tiles;
+    if (a->size_k <= 0 || a->size_m <= 0 || (a->size_k & (padded ? 31 : 127))) return QUEST_ERR_BAD_SHAPE;
+    if (!aligned(a->x, 16) || !aligned(a->branch, 16) || !aligned(a->norm_weight, 16) || !aligned(a->x_int_packed, 16) || !aligned(a->tiles, 16)) return QUEST_ERR_ALIGNMENT;
+    NextWeights next;
+    if (a->next != nullptr && aligned(a->next, 16) && a->next_pitch % 16 == 0 && a->next_bytes <= a->next_pitch)
+        next = {a->next, a->next_pitch, a->next_bytes & ~(size_t)15, a->next_blocks};
+    return launch_hadamard_quantize_mfma(a->producer, a->x, a->norm_weight, a->eps, a->scale, a->tiles ? nullptr : a->x_int_packed, a->tiles ? nullptr : a->x_int_row_sum, nullptr, nullptr, a->size_k, a->size_m,
+                                         a->had_scale, a->dtype, (hipStream_t)stream, a->branch, a->branch ? (void *)a->x : nullptr, (uint8_t *)a->tiles, 0, next);
+}
+
 extern "C" int quest_quantize_e2m3_padded(const void *x, void *scale, void *x_tiles, int group_size, int batch_size, int dtype, void *stream) {
     forget_stale_error();
     if (!x || !scale || !x_tiles) return QUEST_ERR_NULL_POINTER;
