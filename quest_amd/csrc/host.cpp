@@ -216,6 +216,9 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     // (a bias whose derivative is wanted is added by torch)
     if (bias != nullptr && ((at::GradMode::is_enabled() && bias->requires_grad()) || bias->_fw_grad(0).defined())) return declined();
 
+    // (a single launch writes outputs while rows of x are still being read)
+    const auto begins = [](const at::Tensor &t) { return reinterpret_cast<uintptr_t>(t.data_ptr()); };
+    const bool apart = given == nullptr || begins(*given) + given->nbytes() <= begins(*x) || begins(*x) + x->nbytes() <= begins(*given);
     at::Tensor out;
     const auto result = [&]() {
         if (given != nullptr) return *given;
@@ -225,7 +228,7 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     };
     const int rc = on(args.dev, [&](void *st) {
         const int dt = dtype_code(type);
-        if (!tiles && quest_linear_few_tokens_available((int)m, (int)k)) {
+        if (apart && !tiles && quest_linear_few_tokens_available((int)m, (int)k)) {
             out = result();
             const int rc = quest_linear_few_tokens(out.data_ptr(), x->data_ptr(), (const uint8_t *)w->data_ptr(), (const int32_t *)w_add->data_ptr(), w_scale->data_ptr(),
                                                    bias ? bias->data_ptr() : nullptr, (int)m, (int)k, (int)n, (float)had_scale, dt, st);

@@ -74,3 +74,16 @@ def test_graph_replays():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
+
+
+@pytest.mark.parametrize('m,k', [(8, 4096), (16, 1024), (40, 1024)])
+def test_output_in_the_place_of_the_input(m, k):
+    from quest_amd import harness
+    x, w, add, scale, _ = _operands(m, k, k, torch.bfloat16)
+    x = torch.randn(m, k, device=DEV).bfloat16()
+    for tiles in (None, harness.weight_tiles(w)):
+        want = harness.linear_forward(x, w, scale, add, use_hadamard=True, w_tiles=tiles)
+        for _ in range(5):
+            both = x.clone()
+            got = harness.linear_forward(both, w, scale, add, use_hadamard=True, w_tiles=tiles, out=both)
+            assert got is both and torch.equal(got, want)
