@@ -308,6 +308,28 @@ typedef struct quest_activation {
 int quest_activation_before_gemm(const quest_activation *a, void *stream);
 
 /*
+ * quest_[rmsnorm_]hadamard_quantize_e2m3 (without norm and transform: quest_quantize_e2m3_padded) and the _e2m3 GEMM behind it with one of its
+ * epilogues, the same bits, in one launch, for sizes where that is the faster way: some tens of tokens of more than 512 and up to 2048 elements.
+ * QUEST_ERR_UNSUPPORTED, with nothing launched, for others.  out must not overlap x.
+ */
+enum { QUEST_EPILOGUE_PLAIN = 0, QUEST_EPILOGUE_SWIGLU = 1, QUEST_EPILOGUE_ADD = 2, QUEST_EPILOGUE_ROPE = 3, QUEST_EPILOGUE_BIAS = 4 };
+typedef struct quest_fused_linear {
+    void *out;
+    const void *x;                /* (size_m, size_k) */
+    const void *norm_weight;      /* NULL, or the RMSNorm in front */
+    float eps;
+    const void *w_tiles, *w_scale;
+    int epilogue;
+    const void *bias;             /* QUEST_EPILOGUE_BIAS */
+    const float *freqs_cis;       /* QUEST_EPILOGUE_ROPE, with the three behind it: as for quest_fused_matmul_dequantize_rope_e2m3, any seq_len */
+    int seq_len, rot_cols, head_dim;
+    int size_m, size_k, size_n;
+    float had_scale;
+    int dtype;
+} quest_fused_linear;
+int quest_linear_e2m3_fused(const quest_fused_linear *layer, void *stream);
+
+/*
  * mat_d (size_m, size_n) dtype = quest_fused_matmul_dequantize_int4_int4t's result for the same codes, from their
  * E2M3 tiles: dtype( f32(2 S) * (0.5f * vec_a_mul[m] * vec_b_mul[n]) ) with S = sum_k (qa + 1/2)(qb + 1/2) accumulated
  * exactly.  size_k % 128 == 0 and <= 65536; any size_m, size_n >= 1; scale vectors 4-byte aligned.

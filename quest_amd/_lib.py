@@ -62,6 +62,7 @@ SIGNATURES = {
     'quest_pack_weight_int4': [_vp, _vp, _vp, _vp, _i, _i, _f, _i, _i, _vp],
     'quest_linear_few_tokens_available': [_i, _i],
     'quest_linear_few_tokens': [_vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _f, _i, _vp],
+    'quest_linear_e2m3_fused': [_vp, _vp],
     'quest_rmsnorm_rows': [_vp, _vp, _vp, _vp, _f, _i, ctypes.c_long, _i, _i, _vp],
     'quest_dense_rows': [_vp, _vp, _vp, _i, _i, _i, _i, _vp],
     'quest_causal_attention': [_vp, _vp, _i, _i, _i, _i, _i, _vp],
@@ -76,6 +77,11 @@ class Activation(ctypes.Structure):
     _fields_ = [('producer', _i), ('x', _vp), ('branch', _vp), ('norm_weight', _vp), ('eps', _f), ('scale', _vp), ('x_int_packed', _vp), ('x_int_row_sum', _vp),
                 ('tiles', _vp), ('size_k', _i), ('size_m', _i), ('had_scale', _f), ('dtype', _i), ('next', _vp), ('next_pitch', ctypes.c_size_t),
                 ('next_bytes', ctypes.c_size_t), ('next_blocks', _i)]
+
+
+class FusedLinear(ctypes.Structure):
+    _fields_ = [('out', _vp), ('x', _vp), ('norm_weight', _vp), ('eps', _f), ('w_tiles', _vp), ('w_scale', _vp), ('epilogue', _i), ('bias', _vp), ('freqs_cis', _vp),
+                ('seq_len', _i), ('rot_cols', _i), ('head_dim', _i), ('size_m', _i), ('size_k', _i), ('size_n', _i), ('had_scale', _f), ('dtype', _i)]
 
 
 _lib = None

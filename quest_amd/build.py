@@ -18,7 +18,7 @@ LIB_PATH = os.path.join(HERE, 'libquest_hip.so')
 HOST_PATH = os.path.join(HERE, '_host.so')
 SOURCES = ['rowops.hip', 'hadamard_mfma.hip', 'gemm.hip', 'gemm_big.hip', 'gemm_small.hip', 'gemm_staged.hip',
            'gemm_decode.hip', 'gemm_decode_fused.hip', 'gemm_e2m3.hip', 'gemm_e2m3_mid.hip', 'gemm_e2m3_resident.hip',
-           'gemm_e2m3_split.hip', 'dense_rows.hip', 'attention.hip', 'capi.hip']
+           'gemm_e2m3_split.hip', 'gemm_e2m3_fused.hip', 'dense_rows.hip', 'attention.hip', 'capi.hip']
 
 FLAGS = [
     '--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-shared',

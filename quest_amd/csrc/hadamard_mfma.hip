@@ -178,16 +178,7 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
 #pragma unroll
             for (int w = 0; w < WPR; w++) ss_row += part_pre[row_local * WPR + w];
         }
-        const float mean_sq = __fmul_rn(ss_row, __fdiv_rn(1.0f, (float)K));
-        const float r = __frsqrt_rn(__fadd_rn(mean_sq, eps));
-#pragma unroll
-        for (int s = 0; s < 8; s++)
-#pragma unroll
-            for (int d = 0; d < 4; d++) {
-                const uint32_t y = pack2_rounded_products<DT>(__fmul_rn(lo_f32<DT>(bq[s][d]), r), __fmul_rn(hi_f32<DT>(bq[s][d]), r));
-                bq[s][d] = pack2_rounded_products<DT>(__fmul_rn(lo_f32<DT>(y), lo_f32<DT>(wq[s][d])),
-                                                      __fmul_rn(hi_f32<DT>(y), hi_f32<DT>(wq[s][d])));
-            }
+        normalise<DT>(bq, wq, ss_row, K, eps);
     }
     if constexpr (PRE == kPreSiluMul) {
         v4u uq[8];
@@ -235,10 +226,6 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
     // ---- codes as E2M3 tiles.  Rounded outputs 32 mt + 8 q + 4 h + {0..3} sit in lane (n, h); after the exchange lane
     // (n, h) holds all 32 outputs of the groups mt = 2 h and 2 h + 1: k-step 2 blk + h of the row, both halves.
     if (tiles != nullptr) {
-        typedef _Float16 v32h __attribute__((ext_vector_type(32)));
-        typedef _Float16 v2hh __attribute__((ext_vector_type(2)));
-        typedef unsigned v6u __attribute__((ext_vector_type(6)));
-        typedef unsigned v16u __attribute__((ext_vector_type(16)));
         const float sf_t = to_f32<DT>(s16);
         const float inv = quant_inv(sf_t);
         uint8_t *frag = tiles + ((size_t)(row >> 5) * (size_t)(2 * n_blk) + 2 * blk + h) * 1536;
@@ -247,26 +234,7 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
             constexpr bool kFast = decltype(fast_tag)::value;
 #pragma unroll
             for (int g = 0; g < 2; g++) {
-                v16u hp;                            // dword d = 4 q + 2 h' + p: outputs 8 q + 4 h' + 2 p + {0, 1} of the group
-#pragma unroll
-                for (int j = 0; j < 8; j++) {       // j = 2 q + p
-                    const auto sw = __builtin_amdgcn_permlane32_swap(yb[g][j], yb[g + 2][j], false, false);
-#pragma unroll
-                    for (int hh = 0; hh < 2; hh++) {
-                        float f0, f1;
-                        if constexpr (kFast) {
-                            f0 = quant_floor_half<DT, 0>(sw[hh], inv);
-                            f1 = quant_floor_half<DT, 1>(sw[hh], inv);
-                        } else {
-                            f0 = quant_code_inv(lo_f32<DT>(sw[hh]), inv);
-                            f1 = quant_code_inv(hi_f32<DT>(sw[hh]), inv);
-                        }
-                        // to fp16 (round towards zero saturates at +-65504 instead of overflowing), then + 1/2
-                        const v2hh c = __builtin_bit_cast(v2hh, __builtin_amdgcn_cvt_pkrtz(f0, f1)) + v2hh{(_Float16)0.5f, (_Float16)0.5f};
-                        hp[4 * (j >> 1) + 2 * hh + (j & 1)] = __builtin_bit_cast(unsigned, c);
-                    }
-                }
-                v6u r = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(__builtin_bit_cast(v32h, hp), 1.0f);
+                v6u r = e2m3_group<DT, kFast>(yb, g, inv);
                 if (RAG && blk * 128 + 64 * h + 32 * g >= K) r = v6u{0, 0, 0, 0, 0, 0};
                 if constexpr (TL) {
                     // position (g, h, block) of the row, this row's chunk in it

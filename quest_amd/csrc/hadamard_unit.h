@@ -1,6 +1,6 @@
 // One wave's share of the fused activation kernel -- up to 32 blocks of 128 of a row, or of several short ones -- in the register layout that
-// hadamard_mfma.hip describes at its top.  Shared by that kernel and by gemm_decode_fused.hip, which quantises a few tokens inside the GEMM's
-// workgroups: one sequence of operations, so that both give the same bits.
+// hadamard_mfma.hip describes at its top.  Shared by that kernel and by gemm_decode_fused.hip and gemm_e2m3_fused.hip, which quantise a few
+// tokens inside the GEMM's workgroups: one sequence of operations, so that both give the same bits.
 #pragma once
 #include "common.h"
 
@@ -172,6 +172,50 @@ __device__ __forceinline__ void nibbles(uint32_t (&dw)[8], const uint32_t (&yb)[
         const auto sw = __builtin_amdgcn_permlane32_swap(hw[t], hw[t + 8], false, false);
         dw[t] = sw[0] | (sw[1] << 16);
     }
+}
+
+// ---- RMSNorm in front of the transform: dtype(dtype(f32(x) * rsqrt(mean(x^2) + eps)) * w), ss_row the sum of the row's squares
+template <int DT>
+__device__ __forceinline__ void normalise(v4u (&bq)[8], const v4u (&wq)[8], float ss_row, int K, float eps) {
+    const float mean_sq = __fmul_rn(ss_row, __fdiv_rn(1.0f, (float)K));
+    const float r = __frsqrt_rn(__fadd_rn(mean_sq, eps));
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            const uint32_t y = pack2_rounded_products<DT>(__fmul_rn(lo_f32<DT>(bq[s][d]), r), __fmul_rn(hi_f32<DT>(bq[s][d]), r));
+            bq[s][d] = pack2_rounded_products<DT>(__fmul_rn(lo_f32<DT>(y), lo_f32<DT>(wq[s][d])),
+                                                  __fmul_rn(hi_f32<DT>(y), hi_f32<DT>(wq[s][d])));
+        }
+}
+
+// ---- codes as E2M3: lane (n, h)'s 24 bytes of half g of the block's k-step h, inv = quant_inv of the row's scale.  FAST: the scale is in the
+// quantiser's fast range.
+typedef _Float16 v32h __attribute__((ext_vector_type(32)));
+typedef unsigned v6u __attribute__((ext_vector_type(6)));
+typedef unsigned v16u __attribute__((ext_vector_type(16)));
+template <int DT, bool FAST>
+__device__ __forceinline__ v6u e2m3_group(const uint32_t (&yb)[4][8], int g, float inv) {
+    v16u hp;                                    // dword d = 4 q + 2 h' + p: outputs 8 q + 4 h' + 2 p + {0, 1} of the group
+#pragma unroll
+    for (int j = 0; j < 8; j++) {               // j = 2 q + p
+        const auto sw = __builtin_amdgcn_permlane32_swap(yb[g][j], yb[g + 2][j], false, false);
+#pragma unroll
+        for (int hh = 0; hh < 2; hh++) {
+            float f0, f1;
+            if constexpr (FAST) {
+                f0 = quant_floor_half<DT, 0>(sw[hh], inv);
+                f1 = quant_floor_half<DT, 1>(sw[hh], inv);
+            } else {
+                f0 = quant_code_inv(lo_f32<DT>(sw[hh]), inv);
+                f1 = quant_code_inv(hi_f32<DT>(sw[hh]), inv);
+            }
+            // to fp16 (round towards zero saturates at +-65504 instead of overflowing), then + 1/2
+            const v2h c = __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_pkrtz(f0, f1)) + v2h{(_Float16)0.5f, (_Float16)0.5f};
+            hp[4 * (j >> 1) + 2 * hh + (j & 1)] = __builtin_bit_cast(unsigned, c);
+        }
+    }
+    return __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(__builtin_bit_cast(v32h, hp), 1.0f);
 }
 
 }  // namespace hq

@@ -187,6 +187,14 @@ int quantise_for(const Linear &w, const Codes &q, const void *x, const Producer 
     return quest_activation_before_gemm(&a, st);
 }
 
+// a layer on tiles in one launch, for sizes where the library has that
+quest_fused_linear fused(void *out, const void *x, const void *w_tiles, const void *w_scale, int64_t m, int64_t k, int64_t n, float had_scale, int dt) {
+    quest_fused_linear l = {};
+    l.out = out, l.x = x, l.w_tiles = w_tiles, l.w_scale = w_scale;
+    l.size_m = (int)m, l.size_k = (int)k, l.size_n = (int)n, l.had_scale = had_scale, l.dtype = dt;
+    return l;
+}
+
 // ---- linear(x, w_packed, w_scale, w_add, w_tiles, bias, had_scale, out) ---------------------------------------------
 // The W4A4 linear layer: activation kernel, GEMM, bias.  x (..., K); w_tiles: None, or the weight's E2M3 tiles (see tiles_of) when the
 // FP6 kernel is wanted; out: None or the (M, N) result to fill.
@@ -232,6 +240,13 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             out = result();
             const int rc = quest_linear_few_tokens(out.data_ptr(), x->data_ptr(), (const uint8_t *)w->data_ptr(), (const int32_t *)w_add->data_ptr(), w_scale->data_ptr(),
                                                    bias ? bias->data_ptr() : nullptr, (int)m, (int)k, (int)n, (float)had_scale, dt, st);
+            if (rc == QUEST_OK) return rc;
+        }
+        if (apart && tiles) {
+            out = result();
+            quest_fused_linear l = fused(out.data_ptr(), x->data_ptr(), w_tiles->data_ptr(), w_scale->data_ptr(), m, k, n, (float)had_scale, dt);
+            if (bias != nullptr) l.epilogue = QUEST_EPILOGUE_BIAS, l.bias = bias->data_ptr();
+            const int rc = at(bias, 16) ? quest_linear_e2m3_fused(&l, st) : QUEST_ERR_UNSUPPORTED;
             if (rc == QUEST_OK) return rc;
         }
         const at::Tensor hold = make({Codes::bytes(m, kt, tiles)}, at::kByte, args.dev);
@@ -511,6 +526,19 @@ bool project_few(const Linear &w, const void *x, void *dst, int m, int dt, void 
     return true;
 }
 
+// a projection of x, through the norm if there is one, on tiles in one launch; false: nothing was launched
+bool project_fused(const Linear &w, const void *x, void *dst, int m, int dt, void *st, int epilogue, const at::Tensor *norm = nullptr, double eps = 0.,
+                   const quest_fused_linear &rope = {}) {
+    if (w.tiles == nullptr) return false;
+    quest_fused_linear l = fused(dst, x, w.tiles->data_ptr(), w.scale->data_ptr(), m, w.k, w.n, kHadamardEntry, dt);
+    l.epilogue = epilogue, l.eps = (float)eps, l.norm_weight = norm ? norm->data_ptr() : nullptr;
+    l.freqs_cis = rope.freqs_cis, l.seq_len = rope.seq_len, l.rot_cols = rope.rot_cols, l.head_dim = rope.head_dim;
+    const int rc = quest_linear_e2m3_fused(&l, st);
+    if (rc == QUEST_ERR_UNSUPPORTED || rc == QUEST_ERR_BAD_SHAPE) return false;
+    launched(rc, "projection");
+    return true;
+}
+
 void norm_into(const Linear &w, const Codes &q, at::Tensor &x, const void *branch, const at::Tensor &weight, double eps, int m, int k, int dt, void *st) {
     launched(quantise_for(w, q, x.data_ptr(), {QUEST_PRODUCER_RMSNORM, branch, weight.data_ptr(), eps}, m, k, kHadamardEntry, dt, st), "norm kernel");
 }
@@ -578,7 +606,9 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         const Codes act(att + core_b, m, hidden, down_tiles);
 
         // norm -> q, k, v with q and k rotated
-        {
+        quest_fused_linear rope = {};
+        rope.freqs_cis = (const float *)freqs->data_ptr(), rope.seq_len = (int)t, rope.rot_cols = 2 * c, rope.head_dim = head_dim;
+        if (branch != nullptr || !project_fused(qkv, x.data_ptr(), wide, m, dt, st, QUEST_EPILOGUE_ROPE, norm1, eps1, rope)) {
             const Codes q(codes, m, c, qkv.tiles != nullptr);
             norm_into(qkv, q, x, branch ? branch->data_ptr() : nullptr, *norm1, eps1, m, c, dt, st);
             const float *f = (const float *)freqs->data_ptr();
@@ -610,7 +640,7 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         }
         // output projection: into the residual stream where its GEMM can add
         bool has_att = project_few(o, attended, att, m, dt, st);
-        if (!has_att) {
+        if (!has_att && !project_fused(o, attended, x.data_ptr(), m, dt, st, QUEST_EPILOGUE_ADD)) {
             const Codes q(codes, m, c, o.tiles != nullptr);
             quantise_into(o, q, attended, m, c, dt, st);
             has_att = !q.tiles && !quest_fused_matmul_dequantize_add_available(m, c, c, st);
@@ -619,7 +649,9 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         // norm -> gated unit -> its codes, or, few tokens, its outputs in `gated`
         const void *gated = nullptr;
         at::Tensor torchs;
-        {
+        if (glu_tiles && !has_att && project_fused(glu, x.data_ptr(), wide, m, dt, st, QUEST_EPILOGUE_SWIGLU, norm2, eps2)) {
+            gated = wide;
+        } else {
             const Codes q(codes, m, c, glu_tiles);
             norm_into(q.tiles || m > 64 ? glu : gate_up, q, x, has_att ? att : nullptr, *norm2, eps2, m, c, dt, st);
             if (!q.tiles && m <= 64) {
@@ -639,7 +671,8 @@ PyObject *block(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
                 gated = wide;
             }
         }
-        if (down_tiles || quest_fused_matmul_dequantize_add_available(m, hidden, c, st)) {
+        if (gated != nullptr && project_fused(down, gated, x.data_ptr(), m, dt, st, QUEST_EPILOGUE_ADD)) {
+        } else if (down_tiles || quest_fused_matmul_dequantize_add_available(m, hidden, c, st)) {
             if (gated != nullptr) quantise_into(down, act, gated, m, hidden, dt, st);
             project(down, act, x.data_ptr(), m, dt, st, true);
         } else {

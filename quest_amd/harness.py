@@ -43,7 +43,13 @@ def prefers_e2m3(m: int, k: int, n: int) -> bool:
     with the FP6 kernels before gemm_e2m3_resident.hip, and have not been drawn again.  With today's kernels the path taken is 2.9 % behind
     the faster one on average over 220 sizes of these ranges (always FP6: 1.2 %), and 10 % over 260 sizes with rows of 640 to 1664
     elements and 512 tokens and more (0.5 %), most at more than 4096 tokens with K < 1536 ((6618, 1280, 9712) 1.69)."""
-    if m < 49 or k % 128 or MATRIX_PATH != 'fp6' or not _tiles_addressable(m, k, n):      # (a few tokens first: their calls are host-bound)
+    if m < 49 and (m < 9 or k > 2048):                # (a few tokens first: their calls are host-bound)
+        return False
+    if k % 128 or MATRIX_PATH != 'fp6' or not _tiles_addressable(m, k, n):
+        return False
+    if m <= 64 and one_launch_on_tiles(m, k, n):
+        return True
+    if m < 49:
         return False
     if m > E2M3_SHORT_ROWS_TOKENS:
         return _enough_per_row(k, n)
@@ -62,6 +68,13 @@ def prefers_e2m3(m: int, k: int, n: int) -> bool:
     if tiles <= 512:
         return tiles <= 128 or (tiles > 256 and k < 4096)
     return not (m > 3000 and k < 1536 and 512 <= n <= 2048)           # (4096, 1280, 512) 0.96; (4096, 1024, 2048) 1.11 by now
+
+
+def one_launch_on_tiles(m: int, k: int, n: int) -> bool:
+    """Whether the FP6 layer is one launch (gemm_e2m3_fused.hip) at sizes where the INT8 kernels, one launch themselves up to 16 tokens, are the
+    slower ones on the GPU too: 1.0 to 1.6 times from 9 to 64 tokens, (8, 1024, 3072) the same.  That file has the exact rule; what is let through here
+    and not there takes two launches, which are no slower than INT8's at these sizes."""
+    return 512 < k <= 2048 and m <= 64 and m * n <= (360000 if k <= 1024 else 131072)
 
 
 def block_prefers_e2m3(m: int, k: int, n: int) -> bool:

@@ -385,7 +385,12 @@ class LlamaBlock(nn.Module):
         """Which of the four projections (bit 0 qkv, 1 output, 2 gate / up, 3 down) run on E2M3 tiles for m tokens, if there are any: the
         one decision of both statements of the block."""
         prefers = harness.block_prefers_e2m3
-        forms = prefers(m, c, 3 * c) | prefers(m, c, c) << 1 | prefers(m, c, 2 * hidden) << 2 | prefers(m, hidden, c) << 3
+        if m < harness.E2M3_MIN_TOKENS:          # few tokens of short rows: a launch for each of the projections on tiles, norm, rotation and all
+            takes = harness.one_launch_on_tiles
+            short = harness.MATRIX_PATH == 'fp6' and c % 128 == 0 and hidden % 128 == 0 and takes(m, c, 3 * c) and takes(m, c, 2 * hidden)
+            forms = 15 if short else 0
+        else:
+            forms = prefers(m, c, 3 * c) | prefers(m, c, c) << 1 | prefers(m, c, 2 * hidden) << 2 | prefers(m, hidden, c) << 3
         # few fp16 tokens: torch's silu, which the kernels' is not for every fp16 value
         return forms & ~4 if m <= 64 and dtype == torch.float16 else forms
 
