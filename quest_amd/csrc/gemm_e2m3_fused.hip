@@ -7,13 +7,13 @@
 // price is the quantiser's arithmetic in every workgroup, so a tile has few tokens and a workgroup several channel tiles.
 //
 // G waves per workgroup for rows of up to G blocks of 128 (G = 8, 16): a wave quantises 32 / G rows (at most half of them have any: sixteen rows cost what
-// eight do, 32 another 1.7 us of vector ALU, 3.2 with the norm) and multiplies the 64-k steps w and w + G of every channel tile: its token fragments
-// stay in registers, its weight fragments come straight from memory, two tiles ahead (the first tile's wait in LDS, where the wave's sums will be: the
-// transform needs the registers).  The G partial sums meet in LDS, and the first wave finishes a tile.
-// What bounds it: the chain -- launch, rows, transform and quantiser, products, sums -- of 4.6 us (K = 1024; 5.6 with the norm in front), then 0.8 us per
-// further channel tile, two barriers around one wave's epilogue.  GPU us in a graph against the two launches (which read ahead) and the INT8 ones, weights
-// from the Infinity Cache: (37, 1024, 1024) 4.6 / 6.9 / 7.2, with the norm (37, 1024, 3072) 6.7 / 8.6 / 8.5 and (37, 1024, 5632) 7.8 / 8.9 / 9.2, (16, 1024,
-// 22016) 7.8 / 10.3 / 9.9, (16, 2048, 6144) 7.3 / 8.3 / 8.1.  The 12-layer model at 1 x 37 tokens 493 -> 434 us.
+// eight do, 32 another 1.7 us of vector ALU, 3.2 with the norm).  Then CT channel tiles at a time are multiplied by G / CT waves each, the 64-k steps dealt
+// to them in turn: a wave's token fragments stay in registers, its weight fragments come straight from memory, two rounds ahead (the first round's wait in
+// LDS, where the wave's sums will be: the transform needs the registers).  The partial sums meet in LDS, and a tile's first wave finishes it.
+// What bounds it: the chain -- launch, rows, transform and quantiser, products, sums -- of 4.6 us (K = 1024; 5.6 with the norm in front), then 0.8 to 1.0 us
+// per further round, two barriers around the epilogue.  GPU us in a graph against the two launches (which read ahead) and the INT8 ones, weights from the
+// Infinity Cache: (37, 1024, 1024) 4.7 / 6.9 / 7.2, with the norm (37, 1024, 3072) 6.2 / 8.7 / 8.6 and (37, 1024, 5632) 7.2 / 9.0 / 9.3, (16, 1024,
+// 22016) 8.1 / 10.2 / 9.9, (16, 2048, 6144) 7.3 / 8.3 / 8.1.
 #include "e2m3_epilogue.h"
 #include "hadamard_unit.h"
 
@@ -33,11 +33,13 @@ constexpr int kTailAt = 2 * kMaxRows * 16;         // of a token fragment in LDS
 constexpr int kFragPitch = kTailAt + 2 * kMaxRows * 8 + 64;      // the blocks of a row, two fragments apart, on different banks
 constexpr int kSumPitch = kChn + 4;                // floats per token row, as in gemm_e2m3_split.hip
 
-template <int G>
+template <int G, int CT>
 struct Shape {
     static constexpr int kWaves = G, kRowsPerWave = 32 / G, kSteps = 2 * G;
+    static constexpr int kShare = G / CT, kMine = 2 * CT;        // waves of a channel tile, steps of one of them
+    static_assert(G % CT == 0, "whole waves per channel tile");
     static constexpr int kStageB = 32 * 256;       // a wave's rows as they come, 32 blocks
-    static constexpr int kSumsAt = kSteps * kFragPitch, kWaveB = 2 * kFragB;             // of a wave's sums, and of its first weights
+    static constexpr int kSumsAt = kSteps * kFragPitch, kWaveB = kMine * kFragB;         // of a wave's sums, and of its first weights
     static constexpr int kRowsAt = kSumsAt + kWaves * kWaveB;
     static constexpr int kNormAt = kRowsAt + kMaxRows / kRowsPerWave * kStageB, kScalesAt = kNormAt + G * 256;
     static constexpr int kLdsB = kScalesAt + kMaxRows * 2;
@@ -48,7 +50,7 @@ struct Args {
     void *out;
     const uint16_t *x, *norm_w;
     const uint8_t *wgt;
-    int M, N, K, tiles_t, tiles_c;
+    int M, N, K, tiles_t, tiles_c;                 // (tiles_c: of CT channel tiles)
     int rows, ways;                                // tokens of a tile; workgroups of an XCD per token tile
     uint32_t entry_bits;
     float eps;
@@ -61,9 +63,10 @@ __device__ __forceinline__ void lds_barrier() {
     plain_barrier();
 }
 
-template <int DT, int G, bool NORM, bool ROPE>
+// CT: channel tiles that the waves share
+template <int DT, int G, int CT, bool NORM, bool ROPE>
 __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Args p) {
-    using S = Shape<G>;
+    using S = Shape<G, CT>;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[S::kLdsB];
     float *const sums = reinterpret_cast<float *>(lds + S::kSumsAt);
     uint16_t *const scales = reinterpret_cast<uint16_t *>(lds + S::kScalesAt);
@@ -81,28 +84,31 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
     // ---- weights: the wave's two steps of a channel tile; steps past the row's end and tiles past the last touch no memory and are zeros
     const int nk = (K + 127) / 128 * 2, pitch = nk * kFragB;     // (rows of whole 32s, without the transform, have tiles with zeros behind them)
     const uint32_t dead = 0x80000000u;
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void *)p.wgt, 0, p.tiles_c * pitch, 0x00020000);
+    const int blocks_c = (N + kChn - 1) / kChn, share = wave % S::kShare, mine_c = wave / S::kShare;
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void *)p.wgt, 0, blocks_c * pitch, 0x00020000);
     struct Frag { v4u head; v2u tail; };
     auto step_at = [&](int tile, int i) {
-        const int step = wave + G * i;
-        return tile < ct_end && step < nk ? (uint32_t)(tile * pitch + step * kFragB) : dead;
+        const int step = share + S::kShare * i, block = tile * CT + mine_c;
+        return tile < ct_end && block < blocks_c && step < nk ? (uint32_t)(block * pitch + step * kFragB) : dead;
     };
-    auto load_weights = [&](Frag (&w)[2], int tile) {
+    auto load_weights = [&](Frag (&w)[S::kMine], int tile) {
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
+        for (int i = 0; i < S::kMine; i++) {
             const uint32_t at = step_at(tile, i);
             w[i].head = __builtin_amdgcn_raw_buffer_load_b128(wr, (int)(at + lane * 16), 0, 0);
             w[i].tail = __builtin_amdgcn_raw_buffer_load_b64(wr, (int)(at + 1024 + lane * 8), 0, 0);
         }
     };
     uint8_t *const first = lds + S::kSumsAt + wave * S::kWaveB;
-    auto load_first = [&]() {                      // both heads, then lanes 0-31 bring the first step's tail, lanes 32-63 the second's
+    auto load_first = [&]() {                      // the heads, then two steps' tails at a time, one by lanes 0-31
         auto to_lds = [&](uint32_t at, int dst) {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (__attribute__((address_space(3))) void *)(first + dst), 16, at, 0, 0, 0);
         };
-        to_lds(step_at(ct, 0) + lane * 16, 0);
-        to_lds(step_at(ct, 1) + lane * 16, 1024);
-        to_lds((lane < 32 ? step_at(ct, 0) : step_at(ct, 1)) + 1024 + (lane & 31) * 16, 2048);
+#pragma unroll
+        for (int i = 0; i < S::kMine; i++) to_lds(step_at(ct, i) + lane * 16, i * 1024);
+#pragma unroll
+        for (int i = 0; i < S::kMine; i += 2)
+            to_lds((lane < 32 ? step_at(ct, i) : step_at(ct, i + 1)) + 1024 + (lane & 31) * 16, S::kMine * 1024 + i * 512);
     };
 
     // ---- the wave's token rows (register layout: hadamard_unit.h)
@@ -133,16 +139,17 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
     load_first();
     __builtin_amdgcn_sched_barrier(0);             // all of these are in flight before anything is waited for
 
-    // ---- what the first 64 threads finish a tile with: eight channels of a token each
-    const int col = (int)threadIdx.x & 3, t_row = (int)threadIdx.x >> 2;
-    const bool finishes = t_row < kMaxRows;        // uniform in the wave
+    // ---- what a channel tile's first wave finishes it with: eight channels of a token per lane
+    const int col = lane & 3, t_row = lane >> 2;
+    static_assert(kMaxRows * kChn == 8 * 64, "a lane's share");
+    const bool finishes = share == 0;              // uniform in the wave
     const bool vec16 = (N & 7) == 0;
     const __amdgpu_buffer_rsrc_t br = __builtin_amdgcn_make_buffer_rsrc((void *)p.epi.b_mul, 0, (N * 2 + 2) & ~3, 0x00020000);
     v4u muls[2];                                   // of this channel tile and the next
     Ahead<ROPE> ahead[2];
     auto fetch_channels = [&](v4u &muls, Ahead<ROPE> &ahead, int tile) {          // (channels past the vector's end read as zeros: their outputs are not stored)
         if (!finishes || tile >= ct_end) return;
-        const int ch = tile * kChn + col * 8;
+        const int ch = (tile * CT + mine_c) * kChn + col * 8;
         muls = __builtin_amdgcn_raw_buffer_load_b128(br, ch * 2, 0, 0);
         if (ROPE || p.epi.kind == kEpiAdd || p.epi.kind == kEpiBias) fetch_ahead<DT>(ahead, p.out, p.epi, tok0 + t_row, ch, tok_end, N, vec16);
     };
@@ -150,7 +157,7 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
     if (busy) {
         v4i hv[2][2];
         hq::signed_entries(hv, n, h, p.entry_bits);
-        wait_vmcnt_imm<3>();                       // the rows (and the norm's weights) are here, the first weights need not be
+        wait_vmcnt_imm<3 * CT>();                     // the rows (and the norm's weights) are here, the first weights need not be
         asm volatile("" ::: "memory");
         v4u bq[8];
 #pragma unroll
@@ -191,7 +198,7 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
         fetch_channels(muls[0], ahead[0], ct);
     }
     wait_vmcnt_imm<0>();                           // the first weights are in LDS
-    Frag w[2][2];                                  // of this channel tile and the next
+    Frag w[2][S::kMine];                                // of this channel tile and the next
     load_weights(w[1], ct + p.ways);
     fetch_channels(muls[1], ahead[1], ct + p.ways);
     lds_barrier();
@@ -203,16 +210,16 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
         f[5] = (int)b[1];
         return f;
     };
-    v8i tok[2];
+    v8i tok[S::kMine];
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
+    for (int i = 0; i < S::kMine; i++) {
         w[0][i].head = *reinterpret_cast<const v4u *>(first + i * 1024 + lane * 16);
-        w[0][i].tail = *reinterpret_cast<const v2u *>(first + 2048 + i * 512 + lane * 8);
-        const uint8_t *f = lds + (wave + G * i) * kFragPitch;
+        w[0][i].tail = *reinterpret_cast<const v2u *>(first + S::kMine * 1024 + i * 512 + lane * 8);
+        const uint8_t *f = lds + (share + S::kShare * i) * kFragPitch;
         const int slot = kMaxRows * h + n % kMaxRows;
         tok[i] = fragment(*reinterpret_cast<const v4u *>(f + slot * 16), *reinterpret_cast<const v2u *>(f + kTailAt + slot * 8));
     }
-    const float t_half_mul = __fmul_rn(0.5f, to_f32<DT>(scales[t_row % kMaxRows]));
+    const float t_half_mul = __fmul_rn(0.5f, to_f32<DT>(scales[t_row]));
     float *const mine = sums + wave * (S::kWaveB / 4) + n * kSumPitch + 4 * h;
     while (true) {
 #pragma unroll
@@ -221,7 +228,7 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
 #pragma unroll
             for (int r = 0; r < 16; r++) acc[r] = 0.f;
 #pragma unroll
-            for (int i = 0; i < 2; i++) acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fragment(w[u][i].head, w[u][i].tail), tok[i], acc, 2, 2, 0, 0, 0, 0);
+            for (int i = 0; i < S::kMine; i++) acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fragment(w[u][i].head, w[u][i].tail), tok[i], acc, 2, 2, 0, 0, 0, 0);
             load_weights(w[u], ct + 2 * p.ways);
             // register r of lane (li, lg) is token li, channel 8 (r / 4) + 4 lg + r % 4
             if (n < kMaxRows) {
@@ -230,13 +237,13 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
             }
             lds_barrier();
             if (finishes) {
-                const int ch = ct * kChn + col * 8;
+                const int ch = (ct * CT + mine_c) * kChn + col * 8;
                 float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
-                for (int v = 0; v < G; v++)
+                for (int v = 0; v < S::kShare; v++)
 #pragma unroll
                     for (int i = 0; i < 2; i++) {
-                        const float4 s = *reinterpret_cast<const float4 *>(sums + v * (S::kWaveB / 4) + t_row * kSumPitch + col * 8 + 4 * i);
+                        const float4 s = *reinterpret_cast<const float4 *>(sums + (wave + v) * (S::kWaveB / 4) + t_row * kSumPitch + col * 8 + 4 * i);
                         sum[4 * i] += s.x; sum[4 * i + 1] += s.y; sum[4 * i + 2] += s.z; sum[4 * i + 3] += s.w;
                     }
                 if (tok0 + t_row < tok_end && ch < N) {
@@ -258,35 +265,47 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
     }
 }
 
-template <int DT, int G>
-static int launch(const Args &a, bool norm, hipStream_t st) {
+template <int DT, int G, int CT>
+static int launch_as(const Args &a, bool norm, hipStream_t st) {
     const dim3 grid((unsigned)(8 * a.ways * a.tiles_t)), block(64 * G);
     const bool rope = a.epi.kind == kEpiRope;
-    if (norm && rope) linear_e2m3_fused_kernel<DT, G, true, true><<<grid, block, 0, st>>>(a);
-    else if (norm) linear_e2m3_fused_kernel<DT, G, true, false><<<grid, block, 0, st>>>(a);
-    else if (rope) linear_e2m3_fused_kernel<DT, G, false, true><<<grid, block, 0, st>>>(a);
-    else linear_e2m3_fused_kernel<DT, G, false, false><<<grid, block, 0, st>>>(a);
+    if (norm && rope) linear_e2m3_fused_kernel<DT, G, CT, true, true><<<grid, block, 0, st>>>(a);
+    else if (norm) linear_e2m3_fused_kernel<DT, G, CT, true, false><<<grid, block, 0, st>>>(a);
+    else if (rope) linear_e2m3_fused_kernel<DT, G, CT, false, true><<<grid, block, 0, st>>>(a);
+    else linear_e2m3_fused_kernel<DT, G, CT, false, false><<<grid, block, 0, st>>>(a);
     return launch_status();
 }
 
-// Tokens per tile and workgroups, one per CU, and whether that is the faster way.  A launch is its first round of channel tiles -- 4.6 to 5.4 us with
-// rows of up to 1024, 5.6 (eight rows a tile) or 6.8 (sixteen) beyond, with the norm 1.0, 1.3 or 2.2 more -- and 0.8 or 1.1 us for each further one; the two
-// launches take 6.7 to 8 us up to 8192 channels, 10 to 13 at 22016, with the norm 1.1 more.  So many rounds as are the faster ones, GPU us in a graph against the
-// two launches: K = 1024, 64 tokens, 8192 channels, four rounds, 7.7 / 8.0, 96 tokens, seven, 10.2 / 8.9; 22016 channels, 32 tokens, six, 9.9 / 10.5, 37, nine,
-// 12.3 / 10.5; K = 2048, 6144 channels, 16 tokens, two, 7.3 / 8.3, 32, three, 8.4 / 8.3; 22016, 16 tokens, three of sixteen rows, 11.4 / 13.4; K = 2048, 128
-// tokens, 1024 channels, one of sixteen, 6.9 / 8.1.
-static bool plan(Args &a, bool norm, int cus) {
-    const int per_xcd = (a.tiles_c + 7) / 8, extra = a.N / 8192;
+// Tokens and channel tiles that a workgroup has at a time, and workgroups, one per CU; 0 where the two launches are the faster way, else the channel
+// tiles.  A launch is its first round -- 4.6 to 5.4 us with rows of up to 1024, half a microsecond more with two channel tiles, 5.6 (eight rows) or 6.8
+// (sixteen) with longer rows, with the norm 1.0, 1.3 or 2.2 more -- and for each further round 0.8 us, with two channel tiles 1.0, with longer rows 1.1.  The
+// two launches take 6.7 to 8 us up to 8192 channels, 10 to 13 at 22016, with the norm 1.1 more.  So: one round of one channel tile where that is all, else
+// two (K = 1024, with the norm, (37, 3072) 6.2 / 6.8, (37, 5632) 7.2 / 7.8, (128, 5632) 8.3 / 10.4; four are slower, (37, 5632) 7.4, but for 96 tokens on
+// 22016 channels), and so many rounds as are faster, GPU us in a graph against the two launches.  K = 1024: (128, 8192), four rounds, 8.7 / 9.0, (192,
+// 5632) with the norm, six, 11.2 / 10.9; 22016 channels, 37 tokens, five, 10.1 / 10.5, 64, six, 11.2 / 10.8.  K = 2048: (16, 6144), two, 7.3 / 8.3, (32, 6144),
+// three, 8.4 / 8.3, (16, 22016), three of sixteen rows, 11.4 / 13.4, (128, 1024), one of sixteen, 6.9 / 8.1.
+static int plan(Args &a, bool norm, int cus) {
+    const int blocks = (a.N + kChn - 1) / kChn;
     const bool is_short = a.K <= 1024;
-    int best = 0;
-    for (int rows = 8; rows <= kMaxRows; rows += 8) {
-        const int tiles_t = (a.M + rows - 1) / rows, room = cus / (8 * tiles_t);
-        if (room < 1) continue;
-        const int rounds = (per_xcd + room - 1) / room, most = is_short ? 4 : rows == 8 ? 2 : norm ? 0 : 1;
-        if (rounds > most + (most > 0 ? extra : 0) || (best != 0 && rounds + (is_short ? 0 : 1) >= best)) continue;
-        best = rounds, a.rows = rows, a.tiles_t = tiles_t, a.ways = per_xcd < room ? per_xcd : room;
+    for (int ct = 1; ct <= (is_short ? 2 : 1); ct++) {
+        int best = 0;
+        for (int rows = 8; rows <= kMaxRows; rows += 8) {
+            const int tiles_t = (a.M + rows - 1) / rows, room = cus / (8 * tiles_t), per_xcd = ((blocks + ct - 1) / ct + 7) / 8;
+            if (room < 1) continue;
+            const int rounds = (per_xcd + room - 1) / room;
+            const int most = is_short ? (ct == 1 ? 1 : 4 + a.N / 16384) : rows == 8 ? 2 + a.N / 8192 : norm ? 0 : 1 + a.N / 8192;
+            if (rounds > most || (best != 0 && rounds + (is_short ? 0 : 1) >= best)) continue;
+            best = rounds, a.rows = rows, a.tiles_t = tiles_t, a.tiles_c = (blocks + ct - 1) / ct, a.ways = per_xcd < room ? per_xcd : room;
+        }
+        if (best != 0) return ct;
     }
-    return best != 0;
+    return 0;
+}
+
+template <int DT>
+static int launch(int ct, const Args &a, bool norm, hipStream_t st) {
+    if (a.K > 1024) return launch_as<DT, 16, 1>(a, norm, st);
+    return ct == 1 ? launch_as<DT, 8, 1>(a, norm, st) : launch_as<DT, 8, 2>(a, norm, st);
 }
 
 }  // namespace e2m3f
@@ -316,9 +335,9 @@ extern "C" int quest_linear_e2m3_fused(const quest_fused_linear *l, void *stream
     if (l->had_scale < 0.f || !representable16(l->had_scale, l->dtype, &bits) || ((long)n + 31) / 32 * ((k + 127) / 128 * 2) * e2m3f::kFragB >= (1L << 31)) return QUEST_ERR_UNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     const RopeArgs rope = {l->freqs_cis, l->seq_len, l->rot_cols, l->head_dim, (const uint16_t *)l->bias};
-    e2m3f::Args a = {l->out, (const uint16_t *)l->x, (const uint16_t *)l->norm_weight, (const uint8_t *)l->w_tiles, m, n, k, 0, (n + 31) / 32, 0, 0, bits,
+    e2m3f::Args a = {l->out, (const uint16_t *)l->x, (const uint16_t *)l->norm_weight, (const uint8_t *)l->w_tiles, m, n, k, 0, 0, 0, 0, bits,
                      l->eps, {l->epilogue, nullptr, (const uint16_t *)l->w_scale, rope}};
-    if (!e2m3f::plan(a, norm, device_cu_count(st))) return QUEST_ERR_UNSUPPORTED;
-    if (l->dtype == QUEST_DTYPE_BF16) return k <= 1024 ? e2m3f::launch<0, 8>(a, norm, st) : e2m3f::launch<0, 16>(a, norm, st);
-    return k <= 1024 ? e2m3f::launch<1, 8>(a, norm, st) : e2m3f::launch<1, 16>(a, norm, st);
+    const int ct = e2m3f::plan(a, norm, device_cu_count(st));
+    if (ct == 0) return QUEST_ERR_UNSUPPORTED;
+    return l->dtype == QUEST_DTYPE_BF16 ? e2m3f::launch<0>(ct, a, norm, st) : e2m3f::launch<1>(ct, a, norm, st);
 }

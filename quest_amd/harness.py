@@ -47,7 +47,7 @@ def prefers_e2m3(m: int, k: int, n: int) -> bool:
         return False
     if k % 128 or MATRIX_PATH != 'fp6' or not _tiles_addressable(m, k, n):
         return False
-    if m <= 64 and one_launch_on_tiles(m, k, n):
+    if m <= 128 and one_launch_on_tiles(m, k, n):
         return True
     if m < 49:
         return False
@@ -72,9 +72,9 @@ def prefers_e2m3(m: int, k: int, n: int) -> bool:
 
 def one_launch_on_tiles(m: int, k: int, n: int) -> bool:
     """Whether the FP6 layer is one launch (gemm_e2m3_fused.hip) at sizes where the INT8 kernels, one launch themselves up to 16 tokens, are the
-    slower ones on the GPU too: 1.0 to 1.6 times from 9 to 64 tokens, (8, 1024, 3072) the same.  That file has the exact rule; what is let through here
+    slower ones on the GPU too: 1.0 to 1.6 times from 9 to 128 tokens, (8, 1024, 3072) the same.  That file has the exact rule; what is let through here
     and not there takes two launches, which are no slower than INT8's at these sizes."""
-    return 512 < k <= 2048 and m <= 64 and m * n <= (360000 if k <= 1024 else 131072)
+    return 512 < k <= 2048 and m * n <= (820000 if k <= 1024 else 131072)
 
 
 def block_prefers_e2m3(m: int, k: int, n: int) -> bool:

@@ -1,5 +1,5 @@
 """The FP6 layer in one launch against the activation kernel and the GEMM one after the other: both forms of the workgroup (rows of 5 to 8 and of 9 to
-16 blocks), the edges of token and channel tiles, more tiles than workgroups, the norm in front, every epilogue, degenerate rows."""
+16 blocks), one channel tile at a time and two, the edges of token and channel tiles, more tiles than workgroups, the norm in front, every epilogue, degenerate rows."""
 import ctypes
 
 import pytest
@@ -9,9 +9,9 @@ pytestmark = pytest.mark.gpu
 DEV = 'cuda:0'
 PLAIN, SWIGLU, ADD, ROPE, BIAS = range(5)
 SIZES = [(37, 1024, 3072), (1, 640, 32), (32, 1024, 1024), (33, 1152, 40), (12, 2048, 5632), (128, 2048, 1000), (5, 768, 4100), (13, 896, 22016), (256, 1024, 8),
-         (31, 1920, 4096), (65, 1664, 264), (8, 1280, 22000)]
+         (31, 1920, 4096), (65, 1664, 264), (8, 1280, 22000), (128, 1024, 8136), (37, 1024, 22016), (70, 768, 5670)]
 RAGGED = [(9, 1376, 4096), (40, 672, 300), (64, 2016, 96), (17, 544, 5000)]                     # whole 32s, without norm and transform
-REFUSED = [(257, 1024, 512), (8, 512, 512), (8, 2176, 512), (96, 1024, 8192), (64, 2048, 6144)]
+REFUSED = [(257, 1024, 512), (8, 512, 512), (8, 2176, 512), (160, 1024, 8192), (64, 2048, 6144)]
 
 
 def _call(l):
@@ -103,7 +103,7 @@ def test_other_sizes_are_refused(m, k, n):
 
 
 @pytest.mark.parametrize('m,k,n,hadamard,bias', [(9, 1024, 3072, True, False), (16, 2048, 8192, False, True), (37, 1376, 1000, False, True), (64, 1024, 5600, True, True),
-                                                 (64, 1920, 2052, True, False), (30, 640, 12000, False, False), (48, 1536, 9, True, False)])
+                                                 (64, 1920, 2052, True, False), (30, 640, 12000, False, False), (48, 1536, 9, True, False), (128, 1024, 6400, True, True)])
 def test_layer_equals_the_int8_path(monkeypatch, m, k, n, hadamard, bias):
     from quest_amd import harness
     g = torch.Generator(device=DEV).manual_seed(m + k + n)
