@@ -170,6 +170,8 @@ struct Producer {
 // Many tokens: nothing of weights that are more than that, for their GEMM is long and the memory busy (layers of 3065 to 11837 tokens x 10000 x 13000
 // read 30 to 100 MB ahead and were 1.5 to 3.7 % slower).  A layer on its own gains from 64 to 512 tokens ((91, 1664, 20608) 14.0 -> 13.3 us); fewer
 // are bound by the host, more by their products.
+// Packed weights of up to 64 tokens: nothing, for that GEMM streams them at once with all its workgroups (1600M model at 1 x 8 tokens 1062 us with, 1032
+// without, at 1 x 1 971 and 955, at 1 x 30 1201 and 1174).
 size_t read_ahead_bytes(int64_t m, size_t weights) {
     const size_t most = 8000000 + 8000 * (size_t)std::min<int64_t>(m, 2048);
     return m > 2048 && weights > most ? 0 : std::min(weights, most);
@@ -183,7 +185,7 @@ int quantise_for(const Linear &w, const Codes &q, const void *x, const Producer 
     a.next_blocks = q.tiles ? (w.n + 31) / 32 : w.n / 32;
     a.next = q.tiles ? w.tiles->data_ptr() : w.packed->data_ptr();
     a.next_pitch = q.tiles ? quest_e2m3_tiles_bytes(32, (k + 127) / 128 * 128) : (size_t)k * 16;
-    a.next_bytes = a.next_blocks > 0 ? read_ahead_bytes(m, a.next_pitch * a.next_blocks) / a.next_blocks : 0;
+    a.next_bytes = a.next_blocks > 0 && (q.tiles || m > 64) ? read_ahead_bytes(m, a.next_pitch * a.next_blocks) / a.next_blocks : 0;
     return quest_activation_before_gemm(&a, st);
 }
 
