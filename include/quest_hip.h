@@ -93,8 +93,7 @@ int quest_fused_matmul_dequantize_int4_int4t(void *mat_d, const uint8_t *mat_a, 
  * quest_fused_matmul_dequantize_int4_int4t (with `bias`, or NULL) give one after the other, bit for bit, without scratch memory.  x
  * (size_m, size_k) dtype, w_packed (size_n, size_k / 2), w_add and w_scale (size_n).  QUEST_ERR_UNSUPPORTED, with nothing
  * launched, for what the two launches do better or this kernel cannot: more than 16 tokens of up to 2048 elements, 8 of up to 4096, 4 of up to
- * 8192, 2 of up to 12288, rows of fewer than 513 or more than 12288, a had_scale that dtype does not hold.  With had_scale = 0 rows are whole 32s, else whole 128s
- * (rows that are not whole 128s: the sum of squares runs in another order than that entry point's, so that a scale can differ by one unit in the last place).
+ * 8192, 2 of up to 12288, rows of fewer than 513 or more than 12288, a had_scale that dtype does not hold.  With had_scale = 0 rows are whole 32s, else whole 128s.
  */
 int quest_linear_few_tokens(void *out, const void *x, const uint8_t *w_packed, const int32_t *w_add, const void *w_scale, const void *bias,
                             int size_m, int size_k, int size_n, float had_scale, int dtype, void *stream);
@@ -158,7 +157,7 @@ int quest_hadamard128(void *y, const void *x, int group_size, int batch_size, fl
  * lie: a had_scale the dtype holds exactly (181/2048) with group_size <= 32768 is the product with the +-had_scale
  * matrix on the matrix cores, fp32 accumulation, as the reference states the activation transform; any other factor
  * (2^-3.5, the weight-side one), and rows over 32768, are fp32 butterflies followed by one multiplication.  Without a
- * transform (had_scale == 0) rows of whole blocks of 128 up to 32768 run on the same matrix-core kernel with the
+ * transform (had_scale == 0) rows of whole 32s up to 32768 run on the same matrix-core kernel with the
  * multiplications left out (the values only change lanes), other rows on the row kernel; the two differ in the order
  * of the fp32 sum of squares only (the scale may come out one ulp apart on rare rows).  The two transforms
  * agree to fp32 summation noise (<= 1e-3 relative, the transform's stated bar), so that a value on a rounding boundary
@@ -274,8 +273,8 @@ int quest_int4_to_e2m3_tiles(void *tiles, const uint8_t *x_int_packed, int rows,
 
 /*
  * Rows that are not whole 128s (size_k % 32 == 0), without the transform: tiles of the row with zeros -- the FP6 zero, not a code -- behind
- * it up to a whole 128, so that the GEMM entry points take them with that size_k.  (quest_e2m3_tiles_bytes of it; 65536 at most.)  The sum of squares
- * runs in another order than quest_hadamard_quantize_int4's for such rows: a scale can differ from its by one unit in the last place.
+ * it up to a whole 128, so that the GEMM entry points take them with that size_k.  (quest_e2m3_tiles_bytes of it; 65536 at most, and 32768 for the
+ * activations.)  Scales and codes are those of quest_hadamard_quantize_int4 with had_scale = 0.
  */
 int quest_int4_to_e2m3_tiles_padded(void *tiles, const uint8_t *x_int_packed, int rows, int size_k, void *stream);
 int quest_quantize_e2m3_padded(const void *x, void *scale, void *x_tiles, int group_size, int batch_size, int dtype, void *stream);

@@ -219,7 +219,8 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
         for (int mt = 0; mt < 4; mt++)
 #pragma unroll
             for (int q = 0; q < 4; q++)
-                *reinterpret_cast<uint2 *>(dst + 32 * mt + 8 * q) = make_uint2(yb[mt][q * 2], yb[mt][q * 2 + 1]);
+                if (!RAG || blk * 128 + 32 * mt < K)
+                    *reinterpret_cast<uint2 *>(dst + 32 * mt + 8 * q) = make_uint2(yb[mt][q * 2], yb[mt][q * 2 + 1]);
     }
     if (writer) scale[row] = (uint16_t)s16;
 
@@ -436,7 +437,7 @@ int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, fl
     uint32_t bits = 0;
     // (had_scale == 0: no transform; the kernel then only moves the chunks between lanes)
     if (K > 32768 || had_scale < 0.f || !representable16(had_scale, dtype, &bits)) return QUEST_ERR_UNSUPPORTED;
-    if ((K & 127) != 0 && ((K & 31) != 0 || pre != 0 || had_scale != 0.f || x_had != nullptr || pre_out != nullptr)) return QUEST_ERR_UNSUPPORTED;
+    if ((K & 127) != 0 && ((K & 31) != 0 || pre != 0 || had_scale != 0.f)) return QUEST_ERR_UNSUPPORTED;
     const int ldx = pre == hq::kPreSiluMul ? 2 * K : K;
     if (!aligned(pre_out, 16) || !aligned(norm_w, 16)) return QUEST_ERR_UNSUPPORTED;
     if (add_in != nullptr && (pre != hq::kPreRmsNorm || sum_out == nullptr || !aligned(add_in, 16) || !aligned(sum_out, 16)))

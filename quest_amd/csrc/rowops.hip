@@ -522,8 +522,9 @@ static int hadamard_quantize_any(const void *x, void *scale, uint8_t *x_int_pack
     // the transform works on blocks of 128; without it (had_scale == 0) a row only has to be whole 16-byte chunks
     if (group_size <= 0 || batch_size <= 0 || (group_size & (had_scale != 0.f ? 127 : 7))) return QUEST_ERR_BAD_SHAPE;
     if (!aligned(x, 16) || !aligned(x_had, 16) || !aligned(x_int_packed, 4)) return QUEST_ERR_ALIGNMENT;
-    if (scale_rule == QUEST_SCALE_GAUSSIAN && (group_size & 127) == 0) {
-        // whole blocks, rows of up to 32768, a Hadamard entry the dtype holds exactly: matrix cores; anything else: butterflies
+    if (scale_rule == QUEST_SCALE_GAUSSIAN) {
+        // rows of up to 32768 with a Hadamard entry the dtype holds exactly, without the transform of whole 32s: matrix cores, the one order of
+        // the sum of squares that the E2M3 and the few-token kernels have too; anything else: butterflies
         const int rc = launch_hadamard_quantize_mfma(0, x, nullptr, 0.f, scale, x_int_packed, x_int_row_sum, x_had, nullptr,
                                                      group_size, batch_size, had_scale, dtype, st, nullptr, nullptr, nullptr, sum_bias);
         if (rc != QUEST_ERR_UNSUPPORTED) return rc;

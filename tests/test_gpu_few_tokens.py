@@ -46,10 +46,7 @@ def test_equals_the_two_launches(dtype, hadamard, m, k, n):
         assert rc == 0
         expected = want if b is None else want + b
         same = (got == expected) | (got.isnan() & expected.isnan())
-        if k % 128:      # another order of the sum of squares: a row's scale may be its neighbour in the dtype, about one row in ten thousand
-            assert int((~same).any(1).sum()) <= 1
-        else:
-            assert bool(same.all())
+        assert bool(same.all())
 
 
 @pytest.mark.parametrize('m,k,n', REFUSED)

@@ -113,8 +113,7 @@ def test_layer_equals_the_int8_path(monkeypatch, m, k, n, hadamard, bias):
     with torch.no_grad():
         got = layer(x)
         monkeypatch.setattr(harness, 'MATRIX_PATH', 'int8')
-        same = got == layer(x)
-    assert int((~same).any(1).sum()) <= (0 if k % 128 == 0 else 1)         # (ragged rows: another order of the sum of squares)
+        assert torch.equal(got, layer(x))
 
 
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])

@@ -29,10 +29,9 @@ def test_tiles_hold_the_codes_and_zeros_behind_them(dtype, m, k):
     x[2, 3] = float('nan')
     scale, tiles = _tiles_of(x)
     want_scale, codes, _ = quest.hadamard_quantize_int4(x, hadamard_scale=0.)
-    same = ((scale == want_scale) | (scale.isnan() & want_scale.isnan())).flatten().cpu()
-    assert int((~same).sum()) <= 1                                   # another order of the sum of squares: one row in about ten thousand
+    assert torch.equal(scale.view(torch.int16), want_scale.view(torch.int16))
     values = qo.e2m3_tiles_decode(tiles.cpu(), m, (k + 127) // 128 * 128)
-    assert torch.equal(values[same, :k], qo.unpack_int4(codes.cpu()).double()[same] + 0.5)
+    assert torch.equal(values[:, :k], qo.unpack_int4(codes.cpu()).double() + 0.5)
     assert bool((values[:, k:] == 0).all())
 
 
@@ -59,7 +58,7 @@ def test_layers_equal_the_int8_kernels(dtype, m, k, n, bias):
     assert any('e2m3' in e.key and 'gemm' in e.key for e in prof.key_averages())
     want = harness.linear_forward(x, layer.w_int_packed, layer.w_scale, layer.w_add)
     want = want if layer.bias is None else want + layer.bias
-    assert int((got != want).any(1).sum()) <= 1
+    assert torch.equal(got, want)
     layer.w_int_packed.zero_()                                       # written by hand: the packed codes serve until the tiles are laid out again
     assert layer._kept_tiles() is None
     assert torch.equal(layer(x), harness.linear_forward(x, layer.w_int_packed, layer.w_scale, layer.w_add) + (0 if layer.bias is None else layer.bias))
