@@ -197,11 +197,75 @@ quest_fused_linear fused(void *out, const void *x, const void *w_tiles, const vo
     return l;
 }
 
-// ---- linear(x, w_packed, w_scale, w_add, w_tiles, bias, had_scale, out) ---------------------------------------------
+// ---- which matrix instructions a layer on its own runs on ------------------------------------------------------------
+// sizes that the FP6 kernels address
+bool tiles_addressable(int64_t m, int64_t k, int64_t n) { return k <= 65536 && m * n <= (1ll << 30) && m * k <= (5ll << 29); }
+
+// Whether the FP6 layer is one launch (gemm_e2m3_fused.hip) at sizes where the INT8 kernels, one launch themselves up to 16 tokens, are the slower ones
+// on the GPU too: 1.0 to 1.6 times from 9 to 128 tokens, (8, 1024, 3072) the same.  That file has the exact rule; what is let through here and not there
+// takes two launches, which are no slower than INT8's at these sizes.
+bool one_launch_on_tiles(int64_t m, int64_t k, int64_t n) { return 512 < k && k <= 2048 && m * n <= (k <= 1024 ? 820000 : 131072); }
+
+// what harness.py holds under these names: from its E2M3_SHORT_ROWS_TOKENS + 1 tokens on, a layer takes the FP6 kernels with rows of E2M3_MIN_K elements and
+// more, or of E2M3_MIN_K_NARROW where it has fewer than E2M3_NARROW channels
+struct Lines {
+    int64_t min_k, min_k_narrow, narrow, short_rows_tokens;
+    bool take(PyObject *const *a) {
+        int64_t *const to[4] = {&min_k, &min_k_narrow, &narrow, &short_rows_tokens};
+        for (int i = 0; i < 4; i++)
+            if (!PyLong_Check(a[i]) || ((*to[i] = PyLong_AsLongLong(a[i])) == -1 && PyErr_Occurred())) return false;
+        return true;
+    }
+};
+
+// Whether the FP6 kernels are the faster ones for an (m, k) x (n, k) layer on its own, quantiser included, with weights that come from HBM (copies of more
+// than 300 MB in turn).  The lines were drawn over 2096 sizes, K 128 to 11008, N 136 to 22016, M 33 to 4096, with the FP6 kernels before
+// gemm_e2m3_resident.hip, and have not been drawn again.  With today's kernels the path taken is 2.9 % behind the faster one on average over 220
+// sizes of these ranges (always FP6: 1.2 %), and 10 % over 260 sizes with rows of 640 to 1664 elements and 512 tokens and more (0.5 %), most at more
+// than 4096 tokens with K < 1536 ((6618, 1280, 9712) 1.69).
+bool prefers_e2m3(int64_t m, int64_t k, int64_t n, const Lines &lines) {
+    if (m < 49 && (m < 9 || k > 2048)) return false;                 // (a few tokens first: their calls are host-bound)
+    if (k % 128 != 0 || !tiles_addressable(m, k, n)) return false;
+    if (m <= 128 && one_launch_on_tiles(m, k, n)) return true;
+    if (m < 49) return false;
+    // With short rows and many tokens the GEMM is mostly epilogue either way and the tile-writing activation kernels are a little slower than the
+    // row-writing ones: see _enough_per_row in harness.py, the same line
+    if (m > lines.short_rows_tokens) return k >= (n >= lines.narrow ? lines.min_k : lines.min_k_narrow);
+    // K < 640: as often slower as faster (K = 128: 0.86 at (2000, 22016), 1.49 at (700, 11008); K = 512: 0.88 to 1.42)
+    if (k < 640) return false;
+    // Some tens of tokens: the weights are the cost, and the tiles are 1.5 x the codes' bytes.  (INT8 / FP6 time: (33, 11008, 11008) 0.72, (64, 4096,
+    // 11008) 0.88, (40, 1024, 4096) 0.96; (64, 2048, 2048) 1.06, (64, 11008, 1024) 1.27.)  More than 16384 channels are a second round of the INT8
+    // kernel's tiles: (56, 3072, 22016) 1.06.
+    if (m <= 64) return (n <= 4096 && k >= 1536) || (n > 16384 && 2048 <= k && k <= 6912);
+    // The INT8 kernels' 64 x 64 tiles: half a round of the 256 CUs or less 0.95 to 1.31 (1.08 on average), one nearly full round 0.82 to 1.16 (0.92; (256,
+    // 6912, 3072) 0.87, (128, 4096, 8192) 0.87), two rounds 0.82 to 1.10 (0.96) with K >= 4096 and 0.91 to 1.12 (1.01) below, more 0.90 to 1.57 (1.10).
+    const int64_t tiles = ((m + 63) >> 6) * ((n + 63) >> 6);
+    if (tiles <= 512) return tiles <= 128 || (tiles > 256 && k < 4096);
+    return !(m > 3000 && k < 1536 && 512 <= n && n <= 2048);          // (4096, 1280, 512) 0.96; (4096, 1024, 2048) 1.11 by now
+}
+
+// the same for Python: three sizes, and for prefers_e2m3 the four lines behind them
+template <typename Rule>
+PyObject *ask(PyObject *const *a, Py_ssize_t n_args, Py_ssize_t wanted, Rule rule) {
+    if (n_args != wanted) return PyErr_Format(PyExc_TypeError, "%zd arguments expected, got %zd", wanted, n_args);
+    const long long m = PyLong_AsLongLong(a[0]), k = PyLong_AsLongLong(a[1]), n = PyLong_AsLongLong(a[2]);
+    if (PyErr_Occurred()) return nullptr;
+    return PyBool_FromLong(rule(m, k, n));
+}
+PyObject *py_tiles_addressable(PyObject *, PyObject *const *a, Py_ssize_t n_args) { return ask(a, n_args, 3, tiles_addressable); }
+PyObject *py_one_launch_on_tiles(PyObject *, PyObject *const *a, Py_ssize_t n_args) { return ask(a, n_args, 3, one_launch_on_tiles); }
+PyObject *py_prefers_e2m3(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
+    Lines lines;
+    if (n_args == 7 && !lines.take(a + 3)) return PyErr_Occurred() ? nullptr : PyErr_Format(PyExc_TypeError, "whole numbers expected");
+    return ask(a, n_args, 7, [&](int64_t m, int64_t k, int64_t n) { return prefers_e2m3(m, k, n, lines); });
+}
+
+// ---- linear(x, w_packed, w_scale, w_add, w_tiles, bias, had_scale, out[, lines]) -------------------------------------
 // The W4A4 linear layer: activation kernel, GEMM, bias.  x (..., K); w_tiles: None, or the weight's E2M3 tiles (see tiles_of) when the
-// FP6 kernel is wanted; out: None or the (M, N) result to fill.
+// FP6 kernel is wanted -- with the four lines behind `out`, where prefers_e2m3 says so; out: None or the (M, N) result to fill.
 PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
-    if (n_args != 8) return declined();
+    Lines lines;
+    if (n_args != 8 && (n_args != 12 || !lines.take(a + 8))) return PyErr_Occurred() ? nullptr : declined();
     HANDLE_TH_ERRORS
     Args args;
     const at::Tensor *x = args.tensor(a[0]);
@@ -214,13 +278,14 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     if (!fits_int(m) || !fits_int(k) || !fits_int(n)) return declined();
     const at::Tensor *w_scale = args.tensor(a[2], type, n);
     const at::Tensor *w_add = args.tensor(a[3], at::kInt, n);
-    PyObject *const tiles_arg = tiles_of(a[4], a[1]);
+    const double had_scale = PyFloat_AsDouble(a[6]);
+    // (rows of whole 32s that are not whole 128s come as tiles with zeros behind them, without the transform)
+    const int64_t padded = had_scale != 0. || k % 32 != 0 ? k : (k + 127) / 128 * 128;
+    PyObject *const tiles_arg = n_args == 8 || prefers_e2m3(m, padded, n, lines) ? tiles_of(a[4], a[1]) : Py_None;
     const bool tiles = tiles_arg != Py_None && args.ok && at(w_scale, 4);      // (the FP6 kernels read scales two at a time)
-    // (rows that are not whole 128s come as tiles with zeros behind them)
-    const int64_t kt = tiles ? (k + 127) / 128 * 128 : k;
+    const int64_t kt = tiles ? padded : k;
     const at::Tensor *w_tiles = tiles ? args.tensor(tiles_arg, at::kByte, (int64_t)quest_e2m3_tiles_bytes((int)n, (int)kt)) : nullptr;
     const at::Tensor *bias = a[5] == Py_None ? nullptr : args.tensor(a[5], type, n);
-    const double had_scale = PyFloat_AsDouble(a[6]);
     const at::Tensor *given = a[7] == Py_None ? nullptr : args.matrix(a[7], type, m, n);
     if (!args.ok || !gemm_takes(m, kt, n, tiles) || !at(x, 16) || !at(w, 16) || !at(w_tiles, 16) || !at(given, 16)) return declined();
     // (a bias whose derivative is wanted is added by torch)
@@ -724,9 +789,12 @@ PyObject *last_logits(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
 }
 
 PyMethodDef kMethods[] = {
-#define QUEST_FN(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
+#define QUEST_FN_AS(name, function) {#name, (PyCFunction)(void (*)(void))function, METH_FASTCALL, nullptr}
+#define QUEST_FN(name) QUEST_FN_AS(name, name)
+    QUEST_FN_AS(prefers_e2m3, py_prefers_e2m3), QUEST_FN_AS(one_launch_on_tiles, py_one_launch_on_tiles), QUEST_FN_AS(tiles_addressable, py_tiles_addressable),
     QUEST_FN(linear), QUEST_FN(gemm), QUEST_FN(matmul_int32), QUEST_FN(hadamard_quantize), QUEST_FN(pack_weight), QUEST_FN(hadamard128), QUEST_FN(find_scale), QUEST_FN(quantize), QUEST_FN(add_mul_vv), QUEST_FN(block), QUEST_FN(last_logits),
 #undef QUEST_FN
+#undef QUEST_FN_AS
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", "Native host path of quest_amd's hot calls.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -12,6 +12,7 @@ import torch
 from torch import nn
 
 from . import api as quest
+from ._lib import host as native
 from .api import HADAMARD_ENTRY
 
 _HIP_BACKENDS = ('hip', 'triton', 'cuda')
@@ -38,43 +39,14 @@ GEMM_ROTATES_QK = True
 
 
 def prefers_e2m3(m: int, k: int, n: int) -> bool:
-    """Whether the FP6 kernels are the faster ones for an (m, k) x (n, k) layer on its own, quantiser included, with weights that come
-    from HBM (copies of more than 300 MB in turn).  The lines were drawn over 2096 sizes, K 128 to 11008, N 136 to 22016, M 33 to 4096,
-    with the FP6 kernels before gemm_e2m3_resident.hip, and have not been drawn again.  With today's kernels the path taken is 2.9 % behind
-    the faster one on average over 220 sizes of these ranges (always FP6: 1.2 %), and 10 % over 260 sizes with rows of 640 to 1664
-    elements and 512 tokens and more (0.5 %), most at more than 4096 tokens with K < 1536 ((6618, 1280, 9712) 1.69)."""
-    if m < 49 and (m < 9 or k > 2048):                # (a few tokens first: their calls are host-bound)
-        return False
-    if k % 128 or MATRIX_PATH != 'fp6' or not _tiles_addressable(m, k, n):
-        return False
-    if m <= 128 and one_launch_on_tiles(m, k, n):
-        return True
-    if m < 49:
-        return False
-    if m > E2M3_SHORT_ROWS_TOKENS:
-        return _enough_per_row(k, n)
-    # K < 640: as often slower as faster (K = 128: 0.86 at (2000, 22016), 1.49 at (700, 11008); K = 512: 0.88 to 1.42)
-    if k < 640:
-        return False
-    # Some tens of tokens: the weights are the cost, and the tiles are 1.5 x the codes' bytes.  (INT8 / FP6 time: (33, 11008, 11008)
-    # 0.72, (64, 4096, 11008) 0.88, (40, 1024, 4096) 0.96; (64, 2048, 2048) 1.06, (64, 11008, 1024) 1.27.)  More than 16384
-    # channels are a second round of the INT8 kernel's tiles: (56, 3072, 22016) 1.06.
-    if m <= 64:
-        return (n <= 4096 and k >= 1536) or (n > 16384 and 2048 <= k <= 6912)
-    # The INT8 kernels' 64 x 64 tiles: half a round of the 256 CUs or less 0.95 to 1.31 (1.08 on average), one nearly full round 0.82
-    # to 1.16 (0.92; (256, 6912, 3072) 0.87, (128, 4096, 8192) 0.87), two rounds 0.82 to 1.10 (0.96) with K >= 4096 and 0.91 to
-    # 1.12 (1.01) below, more 0.90 to 1.57 (1.10).
-    tiles = ((m + 63) >> 6) * ((n + 63) >> 6)
-    if tiles <= 512:
-        return tiles <= 128 or (tiles > 256 and k < 4096)
-    return not (m > 3000 and k < 1536 and 512 <= n <= 2048)           # (4096, 1280, 512) 0.96; (4096, 1024, 2048) 1.11 by now
+    """Whether the FP6 kernels are the faster ones for an (m, k) x (n, k) layer on its own, quantiser included.  The rule is native code
+    (csrc/host.cpp, with both sides of its lines), for a layer's call asks it there: it was 0.25 us of a call in Python."""
+    return MATRIX_PATH == 'fp6' and native.prefers_e2m3(m, k, n, E2M3_MIN_K, E2M3_MIN_K_NARROW, E2M3_NARROW, E2M3_SHORT_ROWS_TOKENS)
 
 
 def one_launch_on_tiles(m: int, k: int, n: int) -> bool:
-    """Whether the FP6 layer is one launch (gemm_e2m3_fused.hip) at sizes where the INT8 kernels, one launch themselves up to 16 tokens, are the
-    slower ones on the GPU too: 1.0 to 1.6 times from 9 to 128 tokens, (8, 1024, 3072) the same.  That file has the exact rule; what is let through here
-    and not there takes two launches, which are no slower than INT8's at these sizes."""
-    return 512 < k <= 2048 and m * n <= (820000 if k <= 1024 else 131072)
+    """Whether a layer on tiles is one launch at sizes where the INT8 kernels are the slower ones on the GPU too (csrc/host.cpp)."""
+    return native.one_launch_on_tiles(m, k, n)
 
 
 def block_prefers_e2m3(m: int, k: int, n: int) -> bool:
@@ -84,13 +56,9 @@ def block_prefers_e2m3(m: int, k: int, n: int) -> bool:
     1.14, (4096, 500) 1.17).  Many tokens with short rows have a kernel of their own (gemm_e2m3_resident.hip), INT8 / FP6 time of
     the GEMM: (16384, 1024) x 1024 with the residual 1.28, x 3072 rotary 1.35, x 5632 gated 1.40; (16384, 768) x 1024 1.26; (8192,
     768) x 5632 1.45."""
-    return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and _tiles_addressable(m, k, n)
+    return (MATRIX_PATH == 'fp6' and m >= E2M3_MIN_TOKENS and k % 128 == 0 and native.tiles_addressable(m, k, n)
             and (m <= E2M3_SHORT_ROWS_TOKENS or _enough_per_row(k, n) or
                  (768 <= k <= E2M3_RESIDENT_MAX_K and n % 16 == 0 and (n <= E2M3_RESIDENT_WIDE or m > E2M3_RESIDENT_WIDE_TOKENS))))
-
-
-def _tiles_addressable(m: int, k: int, n: int) -> bool:
-    return k <= 65536 and m * n <= (1 << 30) and m * k <= (5 << 29)
 
 
 def _enough_per_row(k: int, n: int) -> bool:
@@ -433,14 +401,12 @@ class Linear4bit(nn.Module):
         return y
 
     def forward(self, x) -> torch.Tensor:
-        n = self.weight.size(0)
         if not self.use_noop and not self.quantize_from_fp32 and x.dim() > 0:
-            k = x.size(-1)
             held = self._buffers.get                  # (not there, e.g. made a parameter: the native call declines)
             if held('w_meta_e') is None:
-                tiles = self._tiles if prefers_e2m3(x.numel() // max(k, 1), tiles_k(k, self.use_hadamard), n) else None
-                y = quest.host.linear(x, held('w_int_packed'), held('w_scale'), held('w_add'), tiles, self.bias,
-                                      HADAMARD_ENTRY if self.use_hadamard else 0., None)
+                y = quest.host.linear(x, held('w_int_packed'), held('w_scale'), held('w_add'), self._tiles if MATRIX_PATH == 'fp6' else None, self.bias,
+                                      HADAMARD_ENTRY if self.use_hadamard else 0., None,
+                                      E2M3_MIN_K, E2M3_MIN_K_NARROW, E2M3_NARROW, E2M3_SHORT_ROWS_TOKENS)
                 if y is not None:
                     return y
         lead, n = x.shape[:-1], self.weight.size(0)

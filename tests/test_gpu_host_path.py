@@ -149,6 +149,36 @@ def test_an_option_without_a_truth_value_raises_its_own_error():
     assert torch.equal(x, before)
 
 
+@pytest.mark.parametrize('m,k,n', [(1, 4096, 512), (333, 1376, 4096), (2000, 1024, 512)])
+def test_a_layer_chooses_its_kernels_in_native_code(monkeypatch, m, k, n):
+    """A call that the host bounds is not kept waiting by the choice in Python (0.25 us of 12)."""
+    from quest_amd import harness
+    layer = harness.Linear4bit.from_weight((torch.randn(n, k, device=DEV) * .02).half())
+    x = torch.randn(m, k, device=DEV).half()
+    want = layer(x)
+
+    def asked(*_):
+        raise AssertionError('asked in Python')
+    for name in ('prefers_e2m3', 'one_launch_on_tiles', 'tiles_k'):
+        monkeypatch.setattr(harness, name, asked)
+    assert torch.equal(layer(x), want)
+
+
+@pytest.mark.parametrize('lines,fp6', [({}, True), ({'E2M3_MIN_K': 1664}, False), ({'E2M3_SHORT_ROWS_TOKENS': 5000, 'E2M3_MIN_K': 1664}, True), ({'MATRIX_PATH': 'int8'}, False)])
+def test_the_native_choice_follows_the_module(monkeypatch, lines, fp6):
+    from quest_amd import harness
+    layer = harness.Linear4bit.from_weight((torch.randn(1536, 1536, device=DEV) * .02).bfloat16())
+    x = torch.randn(4097, 1536, device=DEV).bfloat16()
+    want = layer(x)
+    for name, value in lines.items():
+        monkeypatch.setattr(harness, name, value)
+    assert harness.prefers_e2m3(4097, 1536, 1536) == fp6
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        got = layer(x)
+        torch.cuda.synchronize()
+    assert any('e2m3' in e.key for e in prof.key_averages()) == fp6 and torch.equal(got, want)
+
+
 @pytest.mark.parametrize('call', ['linear', 'block', 'last_logits', 'steps'])
 def test_other_threads_run_during_native_calls(call):
     """The interpreter lock is free while a native call allocates and launches: with a switch interval that never ends, a thread
