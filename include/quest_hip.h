@@ -157,9 +157,10 @@ int quest_hadamard128(void *y, const void *x, int group_size, int batch_size, fl
  * lie: a had_scale the dtype holds exactly (181/2048) with group_size <= 32768 is the product with the +-had_scale
  * matrix on the matrix cores, fp32 accumulation, as the reference states the activation transform; any other factor
  * (2^-3.5, the weight-side one), and rows over 32768, are fp32 butterflies followed by one multiplication.  Without a
- * transform (had_scale == 0) rows of whole 32s up to 32768 run on the same matrix-core kernel with the
+ * transform (had_scale == 0) rows of whole blocks of 128 up to 32768 run on the same matrix-core kernel with the
  * multiplications left out (the values only change lanes), other rows on the row kernel; the two differ in the order
- * of the fp32 sum of squares only (the scale may come out one ulp apart on rare rows).  The two transforms
+ * of the fp32 sum of squares only (a scale may differ by one ulp between the orders, on rare rows).  A row has the same order, and
+ * so the same scale and codes, in every entry point that quantises it, as tiles or inside a layer too.  The two transforms
  * agree to fp32 summation noise (<= 1e-3 relative, the transform's stated bar), so that a value on a rounding boundary
  * of the dtype may come out one ulp apart and its code one level apart: codes are reproducible for a given shape,
  * factor and dtype, not across the two.  Given the transformed tensor and the scale, codes and row sums are exactly

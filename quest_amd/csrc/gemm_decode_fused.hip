@@ -120,10 +120,15 @@ __global__ void __launch_bounds__(64 * kWaves, 1) linear_few_tokens_kernel(Args 
     uint32_t yb[4][8];
     float total = 0.f;
     if (busy) {
-        v4i hv[2][2];
-        hq::signed_entries(hv, n, h, p.entry_bits);
-        total = hq::transform<DT>(yb, bq, hv, p.entry_bits);
-        total = G == 32 ? wave_sum_dpp_f(total) : hq::group_sum_f<G>(total);
+        if constexpr (RAG) {
+            hq::spread(yb, bq);
+            total = hq::ragged_sum<DT, G>(bq);
+        } else {
+            v4i hv[2][2];
+            hq::signed_entries(hv, n, h, p.entry_bits);
+            total = hq::transform<DT>(yb, bq, hv, p.entry_bits);
+            total = G == 32 ? wave_sum_dpp_f(total) : hq::group_sum_f<G>(total);
+        }
         if (WPR > 1 && lane == 0) part_sq[wave] = total;
     }
     if constexpr (WPR > 1) {

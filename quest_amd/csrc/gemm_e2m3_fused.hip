@@ -174,9 +174,16 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
             hq::normalise<DT>(bq, nq, hq::group_sum_f<G>(ss), K, p.eps);
         }
         uint32_t yb[4][8];
-        const float sumsq = hq::transform<DT>(yb, bq, hv, p.entry_bits);
+        const bool ragged = (K & 127) != 0;        // uniform
+        float sumsq;
+        if (ragged) {
+            hq::spread(yb, bq);
+            sumsq = hq::ragged_sum<DT, G>(bq);
+        } else {
+            sumsq = hq::transform<DT>(yb, bq, hv, p.entry_bits);
+        }
         fetch_channels(muls[0], ahead[0], ct);     // (here: the transform needs the registers)
-        const float total = hq::group_sum_f<G>(sumsq);
+        const float total = ragged ? sumsq : hq::group_sum_f<G>(sumsq);
         const uint32_t s16 = from_f32<DT>(scale_from_sumsq(total, K));
         if (n % G == 0 && h == 0) scales[row] = (uint16_t)s16;
         const float sf = to_f32<DT>(s16), inv = quant_inv(sf);

@@ -198,9 +198,15 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
     }
 
     uint32_t yb[4][8];                          // [mt][q * 2 + pair]: outputs 32 mt + 8 q + 4 h + {0,1} / {2,3}
-    const float sumsq = transform<DT>(yb, bq, hv, entry_bits);
     // lanes without a block transformed zeros: they add nothing
-    float total = G == 32 ? wave_sum_dpp_f(sumsq) : group_sum_f<G>(sumsq);
+    float total;
+    if constexpr (RAG) {
+        spread(yb, bq);
+        total = ragged_sum<DT, G>(bq);
+    } else {
+        const float sumsq = transform<DT>(yb, bq, hv, entry_bits);
+        total = G == 32 ? wave_sum_dpp_f(sumsq) : group_sum_f<G>(sumsq);
+    }
     __shared__ float part_sq[Sh::kWaves];
     __shared__ int part_sum[Sh::kWaves];
     if constexpr (WPR > 1) {
@@ -219,8 +225,7 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
         for (int mt = 0; mt < 4; mt++)
 #pragma unroll
             for (int q = 0; q < 4; q++)
-                if (!RAG || blk * 128 + 32 * mt < K)
-                    *reinterpret_cast<uint2 *>(dst + 32 * mt + 8 * q) = make_uint2(yb[mt][q * 2], yb[mt][q * 2 + 1]);
+                *reinterpret_cast<uint2 *>(dst + 32 * mt + 8 * q) = make_uint2(yb[mt][q * 2], yb[mt][q * 2 + 1]);
     }
     if (writer) scale[row] = (uint16_t)s16;
 
@@ -277,30 +282,26 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
             }
         }
     }
+    if constexpr (RAG) return;                                // (packed codes of such rows: rowops.hip)
     if (packed == nullptr && row_sum == nullptr) return;      // uniform over the workgroup
 
     // every code sits in exactly one lane's dwords, so the row sum is the sum of their signed nibbles
     uint32_t dw[8];
     nibbles<DT>(dw, yb, s16, row < M);
-    if constexpr (RAG) {
-#pragma unroll
-        for (int t = 0; t < 8; t++)
-            if (blk * 128 + 64 * h + 8 * t >= K) dw[t] = 0;          // (a degenerate row's zeros need not quantise to code 0)
-    }
     int isum = 0;
 #pragma unroll
     for (int t = 0; t < 8; t++) isum = __builtin_amdgcn_sdot8((int)dw[t], 0x11111111, isum, false);
     if (packed != nullptr && live) {
         uint32_t *dst = packed + (size_t)row * (K >> 3) + blk * 16 + h * 8;
         if ((reinterpret_cast<uintptr_t>(packed) & 15) == 0) {           // uniform; rows are whole multiples of 64 bytes
-            if (!RAG || blk * 128 + 64 * h < K) *reinterpret_cast<uint4 *>(dst) = make_uint4(dw[0], dw[1], dw[2], dw[3]);
-            if (!RAG || blk * 128 + 64 * h + 32 < K) *reinterpret_cast<uint4 *>(dst + 4) = make_uint4(dw[4], dw[5], dw[6], dw[7]);
+            *reinterpret_cast<uint4 *>(dst) = make_uint4(dw[0], dw[1], dw[2], dw[3]);
+            *reinterpret_cast<uint4 *>(dst + 4) = make_uint4(dw[4], dw[5], dw[6], dw[7]);
         } else {                                                          // a view that starts 4 bytes into an allocation
             // (volatile: kept apart from the vector stores above, which the compiler would otherwise merge with these
             // into a common, narrower sequence)
 #pragma unroll
             for (int t = 0; t < 8; t++)
-                if (!RAG || blk * 128 + 64 * h + 8 * t < K) *reinterpret_cast<volatile uint32_t *>(dst + t) = dw[t];
+                *reinterpret_cast<volatile uint32_t *>(dst + t) = dw[t];
         }
     }
     if (row_sum != nullptr) {
@@ -437,7 +438,7 @@ int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, fl
     uint32_t bits = 0;
     // (had_scale == 0: no transform; the kernel then only moves the chunks between lanes)
     if (K > 32768 || had_scale < 0.f || !representable16(had_scale, dtype, &bits)) return QUEST_ERR_UNSUPPORTED;
-    if ((K & 127) != 0 && ((K & 31) != 0 || pre != 0 || had_scale != 0.f)) return QUEST_ERR_UNSUPPORTED;
+    if ((K & 127) != 0 && ((K & 31) != 0 || pre != 0 || had_scale != 0.f || x_had != nullptr || packed != nullptr || row_sum != nullptr)) return QUEST_ERR_UNSUPPORTED;
     const int ldx = pre == hq::kPreSiluMul ? 2 * K : K;
     if (!aligned(pre_out, 16) || !aligned(norm_w, 16)) return QUEST_ERR_UNSUPPORTED;
     if (add_in != nullptr && (pre != hq::kPreRmsNorm || sum_out == nullptr || !aligned(add_in, 16) || !aligned(sum_out, 16)))

@@ -36,12 +36,17 @@ typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
 // Sum over the G lanes (G a power of two, aligned) of each half-wave that hold one row, and over the two half-waves.
 template <int G>
-__device__ __forceinline__ float group_sum_f(float v) {
+__device__ __forceinline__ float lanes_sum_f(float v) {
     if constexpr (G >= 2) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));
     if constexpr (G >= 4) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true));
     if constexpr (G >= 8) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));
     if constexpr (G >= 16) v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, true));
     if constexpr (G >= 32) v += lane_xor_f<16>(v);
+    return v;
+}
+template <int G>
+__device__ __forceinline__ float group_sum_f(float v) {
+    v = lanes_sum_f<G>(v);
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
@@ -54,6 +59,42 @@ __device__ __forceinline__ int group_sum_i(int v) {
     if constexpr (G >= 32) v += lane_xor_i<16>(v);
     const auto r = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
     return (int)r[0] + (int)r[1];
+}
+
+// ---- Rows that are not whole 128s, without the transform: the sum of squares in one order, whether the row is quantised here (ragged_sum: the row, or the
+// wave's 32 blocks of it where several waves share one, in every lane of the row) or by the row kernel for packed codes (ordered_sum in rowops.hip), so
+// that its scale does not depend on that.  A chunk of eight elements is a chain of four dot products; the sixteen chunks of a block and the 32 blocks of a
+// wave are balanced trees, the chunks paired by bits 1, 3, 2 and 0 of their number (two of a lane's eight, then the half-waves).  bq[s] is chunk 2 s + h;
+// blocks past the row's end are zeros, which change no sum.
+template <int DT>
+__device__ __forceinline__ float chunk_sum(uint32_t x, uint32_t y, uint32_t z, uint32_t w) {
+    return dot2_self<DT>(w, dot2_self<DT>(z, dot2_self<DT>(y, dot2_self<DT>(x, 0.f))));
+}
+// the tree over the sixteen lanes that hold a block's chunks
+__device__ __forceinline__ float chunks_tree(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true));        // lane xor 2
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, true));       // xor 8: row_ror:8
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xF, 0xF, true));       // row_ror:4, which is xor 4 by now
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));  // xor 1
+}
+// the tree over the G lanes that hold a row's (a wave's) blocks
+template <int G>
+__device__ __forceinline__ float blocks_tree(float v) {
+    v = lanes_sum_f<(G < 16 ? G : 16)>(v);
+    if constexpr (G >= 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    return v;
+}
+template <int DT, int G>
+__device__ __forceinline__ float ragged_sum(const v4u (&bq)[8]) {
+    float c[8];
+#pragma unroll
+    for (int s = 0; s < 8; s++) c[s] = chunk_sum<DT>(bq[s][0], bq[s][1], bq[s][2], bq[s][3]);
+    const float v = ((c[0] + c[1]) + (c[4] + c[5])) + ((c[2] + c[3]) + (c[6] + c[7]));
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return blocks_tree<G>(__uint_as_float(r[0]) + __uint_as_float(r[1]));
 }
 
 // ---- the four A fragments: +-entry with sign (-1)^(popcount(n & 7 & j) + n3 h) [* (-1)^n4] [* -1]; lane (n, h)
@@ -81,27 +122,34 @@ __device__ __forceinline__ void signed_entries(v4i (&hv)[2][2], int n, int h, ui
     }
 }
 
+// ---- No transform: the loaded chunks are the outputs already and only have to change lanes: lane (n, h) loaded the chunks whose k has bit 3 equal to h
+// and the code below wants those whose bit 2 is h, so the two half-waves trade half of every chunk (nothing is multiplied: NaN and Inf stay where they are).
+// yb[mt][q * 2 + pair]: outputs 32 mt + 8 q + 4 h + {0,1} / {2,3} of block n.
+__device__ __forceinline__ void spread(uint32_t (&yb)[4][8], const v4u (&bq)[8]) {
+#pragma unroll
+    for (int s = 0; s < 8; s++)
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            // outputs 16 s + 8 (q & 1) + 4 h + 2 p + {0, 1}: pair 2 h + p of the chunk held by the half-wave q & 1
+            const auto sw = __builtin_amdgcn_permlane32_swap(bq[s][p], bq[s][2 + p], false, false);
+#pragma unroll
+            for (int qo = 0; qo < 2; qo++) yb[s >> 1][(2 * (s & 1) + qo) * 2 + p] = sw[qo];
+        }
+}
+
 // ---- Hadamard: 8 k-steps x 4 row tiles; then round to the dtype (the transform's output exists only in dtype) and sum the
-// squares.  yb[mt][q * 2 + pair]: outputs 32 mt + 8 q + 4 h + {0,1} / {2,3} of block n.  entry_bits == 0: no transform -- the loaded chunks
-// are the outputs already and only have to change lanes: lane (n, h) loaded the chunks whose k has bit 3 equal to h and the code below wants those
-// whose bit 2 is h, so the two half-waves trade half of every chunk (nothing is multiplied: NaN and Inf stay where they are).
+// squares.  yb as above.  entry_bits == 0: no transform.
 template <int DT>
 __device__ __forceinline__ float transform(uint32_t (&yb)[4][8], const v4u (&bq)[8], const v4i (&hv)[2][2], uint32_t entry_bits) {
     float sumsq = 0.f;
     if (entry_bits == 0) {                      // uniform
+        spread(yb, bq);
 #pragma unroll
         for (int s = 0; s < 8; s++)
 #pragma unroll
-            for (int p = 0; p < 2; p++) {
-                // outputs 16 s + 8 (q & 1) + 4 h + 2 p + {0, 1}: pair 2 h + p of the chunk held by the half-wave q & 1
-                const auto sw = __builtin_amdgcn_permlane32_swap(bq[s][p], bq[s][2 + p], false, false);
+            for (int p = 0; p < 2; p++)
 #pragma unroll
-                for (int qo = 0; qo < 2; qo++) {
-                    const uint32_t w = sw[qo];
-                    yb[s >> 1][(2 * (s & 1) + qo) * 2 + p] = w;
-                    sumsq = dot2_self<DT>(w, sumsq);
-                }
-            }
+                for (int qo = 0; qo < 2; qo++) sumsq = dot2_self<DT>(yb[s >> 1][(2 * (s & 1) + qo) * 2 + p], sumsq);
     } else {
         v16f acc[4];
 #pragma unroll

@@ -9,7 +9,7 @@
 //   quantise   quest/quantize_kernel.cu:120-229, benchmarks/utils.py:334-365
 //   epilogue   quest/quantize_kernel.cu:264-306, benchmarks/utils.py:535-545
 //   Hadamard   benchmarks/utils.py:17,38-39,89-90
-#include "common.h"
+#include "hadamard_unit.h"
 
 namespace quest {
 
@@ -100,6 +100,33 @@ __device__ __forceinline__ uint32_t pack_nibbles8(const float (&q)[8], int &sum)
     return w;
 }
 
+// The sum of squares of a row without the transform from its chunks' sums, in the order of the kernels that quantise such a row inside its tile or GEMM
+// (ragged_sum in hadamard_unit.h).  Thread t holds chunks t, t + BLOCK, ...: sixteen lanes a block.
+// slots: N * BLOCK / 16, one for every block
+template <int BLOCK, int N>
+__device__ __forceinline__ float ordered_sum(const float (&part)[N], int nchunks, float *slots) {
+    const int lane = threadIdx.x & 63;
+    float block[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) block[i] = hq::chunks_tree(part[i]);
+    if ((lane & 15) == 0) {
+#pragma unroll
+        for (int i = 0; i < N; i++) slots[(i * BLOCK + (int)threadIdx.x) >> 4] = block[i];
+    }
+    __syncthreads();
+    constexpr int kBlocks = N * BLOCK / 16;
+    if constexpr (kBlocks == 16) return hq::blocks_tree<16>(slots[lane & 15]);
+    float total = 0.f;
+#pragma unroll
+    for (int b = 0; b < kBlocks; b += 64) {
+        if (kBlocks > 128 && b * 16 >= nchunks) break;              // uniform
+        const float v = hq::blocks_tree<32>(slots[b + (lane & (kBlocks - 1))]);
+        total += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 0));
+        if constexpr (kBlocks > 32) total += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 32));
+    }
+    return total;
+}
+
 // ---------------------------------------------------------------------------------------------
 // Fused Hadamard + scale + quantise + pack: one workgroup per row, NCHUNK 16-byte chunks per
 // thread, the row lives in registers between its single read and its writes.
@@ -109,12 +136,13 @@ __device__ __forceinline__ uint32_t pack_nibbles8(const float (&q)[8], int &sum)
 // arithmetic of the reference's evaluation-side fake quantiser (src/eval_hswag.py:201-214), which never holds the
 // rotated tensor in 16 bits -- instead of from the dtype-rounded tensor the inference path materialises.
 // ---------------------------------------------------------------------------------------------
+// (the long rows' chunks in 128 registers: left alone they take 133, one wave of four less on every SIMD)
 template <int DT, int NCHUNK, int BLOCK, bool FP32>
-__global__ void __launch_bounds__(BLOCK)
+__global__ void __launch_bounds__((BLOCK), (NCHUNK > 4 ? 4 : 1))
 hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ scale,
                          uint32_t *__restrict__ packed, int32_t *__restrict__ row_sum,
                          uint16_t *__restrict__ x_had, int K, float had_scale, int scale_rule, int sum_bias) {
-    __shared__ float slots_f[BLOCK / 64];
+    __shared__ float slots_f[NCHUNK * (BLOCK / 16)];
     __shared__ int slots_i[BLOCK / 64];
     const int row = blockIdx.x;
     const int tid = threadIdx.x;
@@ -132,27 +160,42 @@ hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ 
     }
 
     float y[FP32 ? NCHUNK : 1][8];
-    float sumsq = 0.f, amax = 0.f;
+    float sumsq = 0.f, amax = 0.f, part[FP32 ? 1 : NCHUNK];
+    if (!FP32 && had_scale == 0.f) {            // uniform
 #pragma unroll
-    for (int i = 0; i < NCHUNK; i++) {
-        float (&v)[8] = y[FP32 ? i : 0];
-        unpack8<DT>(raw[i], v);
-        if (had_scale != 0.f) {
-            float factor;
-            fwht128_chunk(v, lane, had_scale, factor);
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = scaled(v[e], factor);
-            raw[i] = make_uint4(pack2_rounded_products<DT>(v[0], v[1]), pack2_rounded_products<DT>(v[2], v[3]),
-                                pack2_rounded_products<DT>(v[4], v[5]), pack2_rounded_products<DT>(v[6], v[7]));
-            if (!FP32) unpack8<DT>(raw[i], v);  // the transform's output exists only in dtype
-        }
-        // the squares of 16-bit floats are exact in fp32: the multiply-add rounds as multiply and add would (the fp32
-        // transform's squares are not, and stay separate)
-#pragma unroll
-        for (int e = 0; e < 8; e++) sumsq = FP32 ? sumsq + v[e] * v[e] : __builtin_fmaf(v[e], v[e], sumsq);
+        for (int i = 0; i < NCHUNK; i++) part[FP32 ? 0 : i] = hq::chunk_sum<DT>(raw[i].x, raw[i].y, raw[i].z, raw[i].w);
         if (absmax) {                           // uniform
 #pragma unroll
-            for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
+            for (int i = 0; i < NCHUNK; i++) {
+                float v[8];
+                unpack8<DT>(raw[i], v);
+                sumsq += part[FP32 ? 0 : i];    // (whether there is a NaN)
+#pragma unroll
+                for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
+            }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < NCHUNK; i++) {
+            float (&v)[8] = y[FP32 ? i : 0];
+            unpack8<DT>(raw[i], v);
+            if (had_scale != 0.f) {
+                float factor;
+                fwht128_chunk(v, lane, had_scale, factor);
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] = scaled(v[e], factor);
+                raw[i] = make_uint4(pack2_rounded_products<DT>(v[0], v[1]), pack2_rounded_products<DT>(v[2], v[3]),
+                                    pack2_rounded_products<DT>(v[4], v[5]), pack2_rounded_products<DT>(v[6], v[7]));
+                if (!FP32) unpack8<DT>(raw[i], v);  // the transform's output exists only in dtype
+            }
+            // the squares of 16-bit floats are exact in fp32: the multiply-add rounds as multiply and add would (the fp32
+            // transform's squares are not, and stay separate)
+#pragma unroll
+            for (int e = 0; e < 8; e++) sumsq = FP32 ? sumsq + v[e] * v[e] : __builtin_fmaf(v[e], v[e], sumsq);
+            if (absmax) {                       // uniform
+#pragma unroll
+                for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
+            }
         }
     }
     if (x_had != nullptr) {
@@ -171,7 +214,9 @@ hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ 
         const float m = block_max_f<BLOCK>(amax, slots_f);
         s32 = __fadd_rn(__fdiv_rn(m, 7.5f), kScaleEps);
     } else {
-        const float total = block_sum_f<BLOCK>(sumsq, slots_f);
+        float total;
+        if (!FP32 && had_scale == 0.f) total = ordered_sum<BLOCK>(part, nchunks, slots_f);
+        else total = block_sum_f<BLOCK>(sumsq, slots_f);
         s32 = scale_from_sumsq(total, K);
     }
     const uint32_t s16 = from_f32<DT>(s32);
@@ -522,9 +567,8 @@ static int hadamard_quantize_any(const void *x, void *scale, uint8_t *x_int_pack
     // the transform works on blocks of 128; without it (had_scale == 0) a row only has to be whole 16-byte chunks
     if (group_size <= 0 || batch_size <= 0 || (group_size & (had_scale != 0.f ? 127 : 7))) return QUEST_ERR_BAD_SHAPE;
     if (!aligned(x, 16) || !aligned(x_had, 16) || !aligned(x_int_packed, 4)) return QUEST_ERR_ALIGNMENT;
-    if (scale_rule == QUEST_SCALE_GAUSSIAN) {
-        // rows of up to 32768 with a Hadamard entry the dtype holds exactly, without the transform of whole 32s: matrix cores, the one order of
-        // the sum of squares that the E2M3 and the few-token kernels have too; anything else: butterflies
+    if (scale_rule == QUEST_SCALE_GAUSSIAN && (group_size & 127) == 0) {
+        // whole blocks, rows of up to 32768, a Hadamard entry the dtype holds exactly: matrix cores; anything else: the row kernel
         const int rc = launch_hadamard_quantize_mfma(0, x, nullptr, 0.f, scale, x_int_packed, x_int_row_sum, x_had, nullptr,
                                                      group_size, batch_size, had_scale, dtype, st, nullptr, nullptr, nullptr, sum_bias);
         if (rc != QUEST_ERR_UNSUPPORTED) return rc;
