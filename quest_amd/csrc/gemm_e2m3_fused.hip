@@ -28,6 +28,7 @@ typedef int v8i __attribute__((ext_vector_type(8)));
 
 constexpr int kFragB = 1536;
 constexpr int kChn = 32;                           // of a tile
+constexpr int kMostCus = 256;                      // of a whole device
 constexpr int kMaxRows = 16;                       // tokens of a tile: half of a matrix instruction's columns are idle
 constexpr int kTailAt = 2 * kMaxRows * 16;         // of a token fragment in LDS: heads, then tails, of the rows that there are
 constexpr int kFragPitch = kTailAt + 2 * kMaxRows * 8 + 64;      // the blocks of a row, two fragments apart, on different banks
@@ -344,6 +345,8 @@ extern "C" int quest_linear_e2m3_fused(const quest_fused_linear *l, void *stream
     const RopeArgs rope = {l->freqs_cis, l->seq_len, l->rot_cols, l->head_dim, (const uint16_t *)l->bias};
     e2m3f::Args a = {l->out, (const uint16_t *)l->x, (const uint16_t *)l->norm_weight, (const uint8_t *)l->w_tiles, m, n, k, 0, 0, 0, 0, bits,
                      l->eps, {l->epilogue, nullptr, (const uint16_t *)l->w_scale, rope}};
+    // (what a whole device does not take, no partition of it does: two launches follow, and the host is not kept waiting by the question for its size)
+    if (e2m3f::plan(a, norm, e2m3f::kMostCus) == 0) return QUEST_ERR_UNSUPPORTED;
     const int ct = e2m3f::plan(a, norm, device_cu_count(st));
     if (ct == 0) return QUEST_ERR_UNSUPPORTED;
     return l->dtype == QUEST_DTYPE_BF16 ? e2m3f::launch<0>(ct, a, norm, st) : e2m3f::launch<1>(ct, a, norm, st);

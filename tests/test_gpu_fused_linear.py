@@ -102,6 +102,25 @@ def test_other_sizes_are_refused(m, k, n):
     assert _call(_arguments(o, out, m, k, n, harness.HADAMARD_ENTRY, False, PLAIN)) != 0 and bool((out == 7.).all())
 
 
+def test_a_refusal_costs_the_host_little():
+    """Two launches follow it, in calls that the host bounds: no question to the runtime (0.3 us) before the sizes have been looked at."""
+    import time
+    from quest_amd import _lib, harness
+    call, stream = _lib.load().quest_linear_e2m3_fused, torch.cuda.current_stream().cuda_stream
+
+    def best(m, k, n):
+        o = _operands(m, k, n, torch.bfloat16)
+        l = _arguments(o, torch.empty(m, n, dtype=torch.bfloat16, device=DEV), m, k, n, harness.HADAMARD_ENTRY, False, PLAIN)
+        refer, times = ctypes.byref(l), []
+        for _ in range(200):
+            start = time.perf_counter()
+            for _ in range(100):
+                call(refer, stream)
+            times.append(time.perf_counter() - start)
+        return min(times)
+    assert best(160, 1024, 8192) < 1.7 * best(257, 1024, 512)            # 1.2; 2.2 with the question
+
+
 @pytest.mark.parametrize('m,k,n,hadamard,bias', [(9, 1024, 3072, True, False), (16, 2048, 8192, False, True), (37, 1376, 1000, False, True), (64, 1024, 5600, True, True),
                                                  (64, 1920, 2052, True, False), (30, 640, 12000, False, False), (48, 1536, 9, True, False), (128, 1024, 6400, True, True)])
 def test_layer_equals_the_int8_path(monkeypatch, m, k, n, hadamard, bias):
