@@ -244,6 +244,9 @@ bool prefers_e2m3(int64_t m, int64_t k, int64_t n, const Lines &lines) {
     return !(m > 3000 && k < 1536 && 512 <= n && n <= 2048);          // (4096, 1280, 512) 0.96; (4096, 1024, 2048) 1.11 by now
 }
 
+// Rows that are not whole 128s, `padded` long with the zeros behind them: as tiles up to the longest that the quantiser writes
+bool ragged_takes_tiles(int64_t padded) { return padded <= 32768; }
+
 // the same for Python: three sizes, and for prefers_e2m3 the four lines behind them
 template <typename Rule>
 PyObject *ask(PyObject *const *a, Py_ssize_t n_args, Py_ssize_t wanted, Rule rule) {
@@ -262,7 +265,7 @@ PyObject *py_prefers_e2m3(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
 
 // ---- linear(x, w_packed, w_scale, w_add, w_tiles, bias, had_scale, out[, lines]) -------------------------------------
 // The W4A4 linear layer: activation kernel, GEMM, bias.  x (..., K); w_tiles: None, or the weight's E2M3 tiles (see tiles_of) when the
-// FP6 kernel is wanted -- with the four lines behind `out`, where prefers_e2m3 says so; out: None or the (M, N) result to fill.
+// FP6 kernel is wanted -- with the four lines behind `out`, where prefers_e2m3 and ragged_takes_tiles say so; out: None or the (M, N) result to fill.
 PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     Lines lines;
     if (n_args != 8 && (n_args != 12 || !lines.take(a + 8))) return PyErr_Occurred() ? nullptr : declined();
@@ -281,7 +284,7 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const double had_scale = PyFloat_AsDouble(a[6]);
     // (rows of whole 32s that are not whole 128s come as tiles with zeros behind them, without the transform)
     const int64_t padded = had_scale != 0. || k % 32 != 0 ? k : (k + 127) / 128 * 128;
-    PyObject *const tiles_arg = n_args == 8 || prefers_e2m3(m, padded, n, lines) ? tiles_of(a[4], a[1]) : Py_None;
+    PyObject *const tiles_arg = n_args == 8 || (prefers_e2m3(m, padded, n, lines) && (padded == k || ragged_takes_tiles(padded))) ? tiles_of(a[4], a[1]) : Py_None;
     const bool tiles = tiles_arg != Py_None && args.ok && at(w_scale, 4);      // (the FP6 kernels read scales two at a time)
     const int64_t kt = tiles ? padded : k;
     const at::Tensor *w_tiles = tiles ? args.tensor(tiles_arg, at::kByte, (int64_t)quest_e2m3_tiles_bytes((int)n, (int)kt)) : nullptr;

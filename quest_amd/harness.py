@@ -280,7 +280,7 @@ class Linear4bit(nn.Module):
                 return
             k = w.size(1) * 2
             padded = tiles_k(k, self.use_hadamard)
-            if MATRIX_PATH == 'fp6' and e2m3_fits(padded, w.size(0)) and (padded == k or padded >= 640):      # (shorter ones: see prefers_e2m3)
+            if MATRIX_PATH == 'fp6' and e2m3_fits(padded, w.size(0)) and (padded == k or 640 <= padded <= 32768):      # (others: see csrc/host.cpp)
                 in_place = before is not None and before[1] is w and before[2] == w.data_ptr()
                 lay = weight_tiles if padded == k else quest.int4_to_e2m3_tiles_padded
                 self._tiles = (lay(w, before[0] if in_place else None), w, w.data_ptr(), w._version)

@@ -62,3 +62,20 @@ def test_layers_equal_the_int8_kernels(dtype, m, k, n, bias):
     layer.w_int_packed.zero_()                                       # written by hand: the packed codes serve until the tiles are laid out again
     assert layer._kept_tiles() is None
     assert torch.equal(layer(x), harness.linear_forward(x, layer.w_int_packed, layer.w_scale, layer.w_add) + (0 if layer.bias is None else layer.bias))
+
+
+def test_rows_that_are_too_long_for_the_quantiser_stay_native(monkeypatch):
+    """Packed codes, and no tiles that nothing could read: the call is not left to the Python statement."""
+    from quest_amd import harness
+    g = torch.Generator(device=DEV).manual_seed(1)
+    layer = harness.Linear4bit.from_weight((torch.randn(96, 33056, device=DEV, generator=g) * .02).half())
+    x = torch.randn(600, 33056, device=DEV, generator=g).half()
+    want = harness.linear_forward(x, layer.w_int_packed, layer.w_scale, layer.w_add)
+    assert layer._tiles is None
+
+    def declined(*_, **__):
+        raise AssertionError('the native call declined')
+    monkeypatch.setattr(harness, 'linear_forward', declined)
+    assert torch.equal(layer(x), want)
+    layer._tiles = (torch.zeros(1), layer.w_int_packed, layer.w_int_packed.data_ptr(), layer.w_int_packed._version)      # (as of a loaded object)
+    assert torch.equal(layer(x), want)
