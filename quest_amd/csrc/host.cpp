@@ -244,8 +244,13 @@ bool prefers_e2m3(int64_t m, int64_t k, int64_t n, const Lines &lines) {
     return !(m > 3000 && k < 1536 && 512 <= n && n <= 2048);          // (4096, 1280, 512) 0.96; (4096, 1024, 2048) 1.11 by now
 }
 
-// Rows that are not whole 128s, `padded` long with the zeros behind them: as tiles up to the longest that the quantiser writes
-bool ragged_takes_tiles(int64_t padded) { return padded <= 32768; }
+// What is different for rows that are not whole 128s (`padded` long with the zeros behind them): the quantiser takes no longer ones, and the INT8 side has
+// another quantiser, the row kernel, which is the faster one for few rows.  49 to 56 tokens of up to 4096 elements in two launches, INT8 / FP6 GPU time: (50,
+// 3104, 4096) 0.89, (50, 4064, 1024) 0.91, (52, 4064, 4096) 0.92, (50, 2272, 2048) 1.00 and 0.94 as a call; with longer rows, more tokens or more channels (50, 6048,
+// 1024) 1.09, (50, 4960, 4096) 1.01, (64, 2272, 4096) 1.05, (50, 4064, 18000) 1.18.
+bool ragged_takes_tiles(int64_t m, int64_t padded, int64_t n) {
+    return padded <= 32768 && (m > 56 || padded > 4096 || n > 4096 || one_launch_on_tiles(m, padded, n));
+}
 
 // the same for Python: three sizes, and for prefers_e2m3 the four lines behind them
 template <typename Rule>
@@ -284,7 +289,7 @@ PyObject *linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     const double had_scale = PyFloat_AsDouble(a[6]);
     // (rows of whole 32s that are not whole 128s come as tiles with zeros behind them, without the transform)
     const int64_t padded = had_scale != 0. || k % 32 != 0 ? k : (k + 127) / 128 * 128;
-    PyObject *const tiles_arg = n_args == 8 || (prefers_e2m3(m, padded, n, lines) && (padded == k || ragged_takes_tiles(padded))) ? tiles_of(a[4], a[1]) : Py_None;
+    PyObject *const tiles_arg = n_args == 8 || (prefers_e2m3(m, padded, n, lines) && (padded == k || ragged_takes_tiles(m, padded, n))) ? tiles_of(a[4], a[1]) : Py_None;
     const bool tiles = tiles_arg != Py_None && args.ok && at(w_scale, 4);      // (the FP6 kernels read scales two at a time)
     const int64_t kt = tiles ? padded : k;
     const at::Tensor *w_tiles = tiles ? args.tensor(tiles_arg, at::kByte, (int64_t)quest_e2m3_tiles_bytes((int)n, (int)kt)) : nullptr;

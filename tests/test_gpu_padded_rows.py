@@ -64,6 +64,13 @@ def test_layers_equal_the_int8_kernels(dtype, m, k, n, bias):
     assert torch.equal(layer(x), harness.linear_forward(x, layer.w_int_packed, layer.w_scale, layer.w_add) + (0 if layer.bias is None else layer.bias))
 
 
+def _kernels(call):
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    return [e.key for e in prof.key_averages()]
+
+
 def test_rows_that_are_too_long_for_the_quantiser_stay_native(monkeypatch):
     """Packed codes, and no tiles that nothing could read: the call is not left to the Python statement."""
     from quest_amd import harness
@@ -79,3 +86,13 @@ def test_rows_that_are_too_long_for_the_quantiser_stay_native(monkeypatch):
     assert torch.equal(layer(x), want)
     layer._tiles = (torch.zeros(1), layer.w_int_packed, layer.w_int_packed.data_ptr(), layer.w_int_packed._version)      # (as of a loaded object)
     assert torch.equal(layer(x), want)
+
+
+@pytest.mark.parametrize('m,k,n,tiles', [(49, 3104, 4096, False), (56, 4064, 1024, False), (57, 3104, 1024, True), (50, 4128, 1024, True), (50, 2272, 16416, True), (52, 1568, 1024, True)])
+def test_some_tens_of_ragged_rows(m, k, n, tiles):
+    from quest_amd import harness
+    g = torch.Generator(device=DEV).manual_seed(m + k + n)
+    layer = harness.Linear4bit.from_weight((torch.randn(n, k, device=DEV, generator=g) * .02).half())
+    x, got = torch.randn(m, k, device=DEV, generator=g).half(), []
+    assert any('e2m3' in name for name in _kernels(lambda: got.append(layer(x)))) == tiles
+    assert torch.equal(got[0], harness.linear_forward(x, layer.w_int_packed, layer.w_scale, layer.w_add))
