@@ -11,8 +11,8 @@ EPS = 1e-5
 NEXT = [(0, 0, 0), (1, 16, 16), (7, 4096, 48), (8, 1536, 1536), (129, 24576, 8000)]                  # (pieces, pitch, bytes of each)
 
 
-def _run(producer, x, branch, weight, tiles, next_):
-    from quest_amd import _lib, harness
+def _run(producer, x, branch, weight, tiles, had_scale, next_):
+    from quest_amd import _lib
     import quest_amd as quest
     m, k = x.size(0), x.size(1) // (2 if producer == 2 else 1)
     scale = torch.empty(m, 1, dtype=x.dtype, device=DEV)
@@ -21,42 +21,49 @@ def _run(producer, x, branch, weight, tiles, next_):
     pieces, pitch, each = next_
     memory = torch.zeros(max(16, pieces * pitch), dtype=torch.uint8, device=DEV)
     a = _lib.Activation(producer, x.data_ptr(), 0 if branch is None else branch.data_ptr(), weight.data_ptr(), EPS, scale.data_ptr(),
-                        0 if tiles else packed.data_ptr(), 0 if tiles else row_sum.data_ptr(), t.data_ptr() if tiles else 0, k, m, harness.HADAMARD_ENTRY,
+                        0 if tiles else packed.data_ptr(), 0 if tiles else row_sum.data_ptr(), t.data_ptr() if tiles else 0, k, m, had_scale,
                         _lib.DTYPE_CODE[x.dtype], memory.data_ptr() if pieces else 0, pitch, each, pieces)
     _lib.check(_lib.load().quest_activation_before_gemm(ctypes.byref(a), torch.cuda.current_stream().cuda_stream), 'activation_before_gemm')
     return (scale, t) if tiles else (scale, packed, row_sum)
 
 
+def _codes(tiles, m, k):
+    """The bytes of m rows' codes: a fragment is 64 lanes (row, half of the 64 elements) of sixteen bytes and then of eight, and rows past m hold anything."""
+    t = tiles.view(-1, k // 64, 1536)
+    heads, tails = (part.reshape(*t.shape[:2], 2, 32, -1) for part in (t[..., :1024], t[..., 1024:]))
+    rows = torch.cat((heads, tails), -1).permute(0, 3, 1, 2, 4).reshape(t.size(0) * 32, -1)[:m]
+    assert rows.shape == (m, k // 4 * 3)
+    return rows
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize('hadamard', [True, False])
 @pytest.mark.parametrize('tiles', [False, True])
 @pytest.mark.parametrize('producer', ['none', 'norm', 'add_norm', 'silu'])
 @pytest.mark.parametrize('m,k', [(37, 1024), (5, 1920), (100, 2816), (9, 4224), (33, 11008), (4200, 1024), (3, 512), (2, 12416)])
-def test_outputs_are_those_of_the_entry_points_without(tiles, producer, m, k):
+def test_outputs_are_those_of_the_entry_points_without(tiles, producer, m, k, hadamard, dtype):
     import quest_amd as quest
+    from quest_amd import harness
     g = torch.Generator(device=DEV).manual_seed(m + k)
-    x, other = (torch.randn(m, k * (2 if producer == 'silu' else 1), device=DEV, generator=g).bfloat16() for _ in range(2))
-    weight = torch.rand(k, device=DEV, generator=g).bfloat16()
+    x, other = (torch.randn(m, k * (2 if producer == 'silu' else 1), device=DEV, generator=g).to(dtype) for _ in range(2))
+    weight = torch.rand(k, device=DEV, generator=g).to(dtype)
     branch = other if producer == 'add_norm' else None
     kind = {'none': 0, 'norm': 1, 'add_norm': 1, 'silu': 2}[producer]
-    want, plain = None, x.clone()
+    had_scale = harness.HADAMARD_ENTRY if hadamard else 0.
+    plain = x if branch is None else x + branch
+    form = 'e2m3' if tiles else 'int4'
+    want = (getattr(quest, f'hadamard_quantize_{form}')(plain, hadamard_scale=had_scale) if kind == 0
+            else getattr(quest, f'rmsnorm_hadamard_quantize_{form}')(plain, weight, EPS, hadamard_scale=had_scale) if kind == 1
+            else getattr(quest, f'silu_mul_hadamard_quantize_{form}')(plain, hadamard_scale=had_scale))
+    if tiles:
+        want = want[0], _codes(want[1], m, k)
     for next_ in [NEXT[0], *(NEXT[1:] if (m, k) in ((37, 1024), (4200, 1024)) else NEXT[-1:])]:
         mine = x.clone()
-        got = _run(kind, mine, branch, weight, tiles, next_)
-        if want is None:
-            if producer == 'add_norm':
-                plain += branch
-            norm = {'norm_weight': weight, 'eps': EPS}
-            if tiles:
-                want = (quest.hadamard_quantize_e2m3(plain) if kind == 0 else quest.rmsnorm_hadamard_quantize_e2m3(plain, weight, EPS) if kind == 1
-                        else quest.silu_mul_hadamard_quantize_e2m3(plain))
-            else:
-                want = (quest.hadamard_quantize_int4(plain) if kind == 0 else quest.rmsnorm_hadamard_quantize_int4(plain, weight, EPS) if kind == 1
-                        else quest.silu_mul_hadamard_quantize_int4(plain))
+        got = _run(kind, mine, branch, weight, tiles, had_scale, next_)
         assert torch.equal(mine, plain)                              # (with a branch: replaced by the sum)
-        rows = m // 32 * 32
+        if tiles:
+            got = got[0], _codes(got[1], m, k)
         for a, b in zip(got, want):
-            if tiles and a.dtype == torch.uint8:                     # whole row blocks: rows past m in the last one hold anything
-                n = rows // 32 * (k // 64) * 1536
-                a, b = a[:n], b[:n]
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
 
 
