@@ -135,20 +135,26 @@ __device__ __forceinline__ float ordered_sum(const float (&part)[N], int nchunks
 // FP32 (QUEST_QUANT_FROM_FP32): scale and codes come from the transform's fp32 output and the unrounded scale -- the
 // arithmetic of the reference's evaluation-side fake quantiser (src/eval_hswag.py:201-214), which never holds the
 // rotated tensor in 16 bits -- instead of from the dtype-rounded tensor the inference path materialises.
+// PLAIN: no transform (had_scale == 0), in 16 bits; such rows can end anywhere and are summed in an order of their own.  Kernels of their own, for in one
+// kernel the transform pays for them ([11008, 4096] packed: 26.6 us alone, 27.2 with the other's code beside it) and they for its registers: [16384, 30016]
+// in 333 us with 113, 217 with 60.
 // ---------------------------------------------------------------------------------------------
-// (the long rows' chunks in 128 registers: left alone they take 133, one wave of four less on every SIMD)
-template <int DT, int NCHUNK, int BLOCK, bool FP32>
-__global__ void __launch_bounds__((BLOCK), (NCHUNK > 4 ? 4 : 1))
+// Most waves on a SIMD: plain rows of more than 8192 elements have room for eight, which is slower: bf16 [16384, 10976] 84 us, with four 78.
+constexpr int plain_waves(int nchunk) { return nchunk > 4 ? 4 : 8; }
+template <int DT, int NCHUNK, int BLOCK, bool FP32, bool PLAIN>
+__global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(1, PLAIN ? plain_waves(NCHUNK) : 8)))
 hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ scale,
                          uint32_t *__restrict__ packed, int32_t *__restrict__ row_sum,
                          uint16_t *__restrict__ x_had, int K, float had_scale, int scale_rule, int sum_bias) {
-    __shared__ float slots_f[NCHUNK * (BLOCK / 16)];
+    static_assert(!(FP32 && PLAIN));
+    __shared__ float slots_f[PLAIN ? NCHUNK * (BLOCK / 16) : BLOCK / 64];
     __shared__ int slots_i[BLOCK / 64];
     const int row = blockIdx.x;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int nchunks = K >> 3;
-    const int chunk0 = had_scale != 0.f ? fwht_chunk_of(tid) : tid;         // blocks of 16 chunks: a row holds whole ones
+    const bool had = !PLAIN && had_scale != 0.f;
+    const int chunk0 = had ? fwht_chunk_of(tid) : tid;         // blocks of 16 chunks: a row holds whole ones
     const uint4 *xr = reinterpret_cast<const uint4 *>(x + (size_t)row * K);
     const bool absmax = scale_rule == QUEST_SCALE_ABSMAX;
 
@@ -160,16 +166,16 @@ hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ 
     }
 
     float y[FP32 ? NCHUNK : 1][8];
-    float sumsq = 0.f, amax = 0.f, part[FP32 ? 1 : NCHUNK];
-    if (!FP32 && had_scale == 0.f) {            // uniform
+    float sumsq = 0.f, amax = 0.f, part[PLAIN ? NCHUNK : 1];
+    if constexpr (PLAIN) {
 #pragma unroll
-        for (int i = 0; i < NCHUNK; i++) part[FP32 ? 0 : i] = hq::chunk_sum<DT>(raw[i].x, raw[i].y, raw[i].z, raw[i].w);
+        for (int i = 0; i < NCHUNK; i++) part[i] = hq::chunk_sum<DT>(raw[i].x, raw[i].y, raw[i].z, raw[i].w);
         if (absmax) {                           // uniform
 #pragma unroll
             for (int i = 0; i < NCHUNK; i++) {
                 float v[8];
                 unpack8<DT>(raw[i], v);
-                sumsq += part[FP32 ? 0 : i];    // (whether there is a NaN)
+                sumsq += part[i];               // (whether there is a NaN)
 #pragma unroll
                 for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
             }
@@ -179,7 +185,7 @@ hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ 
         for (int i = 0; i < NCHUNK; i++) {
             float (&v)[8] = y[FP32 ? i : 0];
             unpack8<DT>(raw[i], v);
-            if (had_scale != 0.f) {
+            if (had) {
                 float factor;
                 fwht128_chunk(v, lane, had_scale, factor);
 #pragma unroll
@@ -215,7 +221,7 @@ hadamard_quantize_kernel(const uint16_t *__restrict__ x, uint16_t *__restrict__ 
         s32 = __fadd_rn(__fdiv_rn(m, 7.5f), kScaleEps);
     } else {
         float total;
-        if (!FP32 && had_scale == 0.f) total = ordered_sum<BLOCK>(part, nchunks, slots_f);
+        if constexpr (PLAIN) total = ordered_sum<BLOCK>(part, nchunks, slots_f);
         else total = block_sum_f<BLOCK>(sumsq, slots_f);
         s32 = scale_from_sumsq(total, K);
     }
@@ -396,7 +402,8 @@ static int launch_hadamard_quantize(const void *x, void *scale, uint8_t *packed,
     const int nchunks = K >> 3;
     const bool fp32 = (scale_rule & QUEST_QUANT_FROM_FP32) != 0;
 #define QUEST_HQ(NCH, BLK)                                                                              \
-    (fp32 ? hadamard_quantize_kernel<DT, NCH, BLK, true> : hadamard_quantize_kernel<DT, NCH, BLK, false>)<<<dim3(M), dim3(BLK), 0, st>>>( \
+    (fp32 ? hadamard_quantize_kernel<DT, NCH, BLK, true, false> : had_scale == 0.f ? hadamard_quantize_kernel<DT, NCH, BLK, false, true> \
+          : hadamard_quantize_kernel<DT, NCH, BLK, false, false>)<<<dim3(M), dim3(BLK), 0, st>>>( \
         (const uint16_t *)x, (uint16_t *)scale, (uint32_t *)packed, row_sum, (uint16_t *)x_had, K, had_scale, scale_rule & ~QUEST_QUANT_FROM_FP32, sum_bias)
     if (nchunks <= 256) QUEST_HQ(1, 256);
     else if (nchunks <= 512) QUEST_HQ(2, 256);
