@@ -30,8 +30,9 @@ constexpr int kRing = 3;                           // chunks of a wave's own wei
 constexpr int kSlotB = 2048;                       // two direct loads of a KiB: 16 rows x 64 bytes each
 constexpr int kRingB = kWaves * kRing * kSlotB;
 constexpr int kPad = 16;                           // behind every row of codes: a lane quarter's sixteen rows on different banks
-constexpr int kCodesB = 34 * 1024;                 // sixteen units of 2 KiB, their pads, and what the last chunk reads past the last row
 constexpr int kMaxTokens = 16;
+constexpr int kUnits = 8;                          // most units of a call (see most_tokens)
+constexpr int kCodesB = kUnits * 2048 + kMaxTokens * kPad + kChunkB;       // a unit's codes are 2 KiB; the pads; what the last chunk reads past the last row
 constexpr int kSumsAt = kRingB + kCodesB;
 constexpr int kLdsB = kSumsAt + 2048 + 4 * 64;
 static_assert(kLdsB <= 160 * 1024 && kMaxTokens <= 16 && kWaves <= 16, "LDS of a CU");
@@ -277,7 +278,6 @@ static int launch(int nb, const Args &a, int grid, hipStream_t st) {
 // on the GPU as well at every size measured (K from 1024 to 11008, N from 1024 to 22016: 0.5 to 2.6 us); with more, the quantiser's
 // arithmetic on every CU is longer than the second launch (K = N = 4096: eight tokens 7.2 against 7.6 us, twelve 8.6 against 7.7; (11008, 4096): two
 // 9.0 against 10.1, four 10.8 against 10.2), though not than what the second launch costs the host.
-constexpr int kUnits = 8;
 static int most_tokens(int nb) {
     const int rows = nb > 16 ? 1 : nb > 8 ? 2 : 4;                  // of a unit
     const int most = nb > 64 ? kUnits / 3 : nb > 32 ? kUnits / 2 : kUnits * rows;
