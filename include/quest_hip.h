@@ -284,8 +284,9 @@ int quest_quantize_e2m3_padded(const void *x, void *scale, void *x_tiles, int gr
  * The activation kernel in front of a GEMM, with a producer of the activation or without, which reads memory ahead for that GEMM meanwhile:
  * the codes, sums and scales of quest_[add_][rmsnorm_ | silu_mul_]hadamard_quantize_int4 or, where `tiles` is given, the tiles of their _e2m3
  * forms (QUEST_PRODUCER_NONE without the transform: of quest_quantize_e2m3_padded).  QUEST_ERR_UNSUPPORTED, with nothing launched, where only the
- * butterfly kernel takes the row.  next: NULL, or next_blocks pieces next_pitch bytes apart of which the first next_bytes are
- * read and dropped, all inside one allocation.  The outputs do not depend on it.
+ * row kernel takes the row.  next: NULL, or next_blocks pieces next_pitch bytes apart of which the first next_bytes are
+ * read and dropped, all inside one allocation.  A hint: the outputs do not depend on it, and rows of up to 512 or more than 12288 elements and rows that
+ * are not whole 128s do not read it.
  */
 enum { QUEST_PRODUCER_NONE = 0, QUEST_PRODUCER_RMSNORM = 1, QUEST_PRODUCER_SILU_MUL = 2 };
 typedef struct quest_activation {

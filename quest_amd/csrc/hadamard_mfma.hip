@@ -427,9 +427,11 @@ static void launch_dtype(int pre, const Args &a) {
 }
 
 // Launches the matrix-core kernel when it applies (K a multiple of 128 up to 32768, or of 32 without the transform; a
-// Hadamard entry the dtype represents exactly); returns QUEST_ERR_UNSUPPORTED otherwise so that the caller can take
-// another path.  Whether it applies depends on K, the factor and the dtype only -- never on the number of rows or on
-// where the buffers lie -- so that one shape always runs the same arithmetic.
+// Hadamard entry the dtype represents exactly; rows that are not whole 128s as tiles only); returns QUEST_ERR_UNSUPPORTED otherwise so
+// that the caller can take another path.  Whether it applies depends on K, the factor, the dtype and the form of the codes only -- never on the
+// number of rows or on where the buffers lie -- so that one shape always runs the same arithmetic (and rows that are not whole 128s in one order in
+// either form, see ragged_sum).
+// next: read ahead by rows of 5 to 96 whole blocks; others, and rows that are not whole 128s, leave it alone.
 // pre: 0 none, 1 RMSNorm (norm_w, eps; with add_in the norm of x + add_in, the sum written to sum_out), 2 SiLU(gate) * up
 // with x a (M, 2 K) tensor.  tiles: the codes as E2M3 tiles (M rows; besides or instead of packed nibbles).
 int launch_hadamard_quantize_mfma(int pre, const void *x, const void *norm_w, float eps, void *scale, uint8_t *packed,

@@ -3,8 +3,8 @@
 //
 // Why: a layer at a handful of tokens is 5 to 7 us of GPU work, and its Python host path (asserts, ctypes conversions, device
 // context, one allocation per output) took 36 us per call, so every small call ran at the speed of the interpreter.  From here a call of two
-// launches takes 10.6 us to issue, module call included, and one of a single launch (quest_linear_few_tokens) 7.3: a launch is 3.7 us of
-// it, an allocation 0.7.  That, and not the GPU, still bounds the smallest calls.
+// launches takes 8.4 to 11.7 us to issue, module call included (30 calls in a row; boxes and processes differ so much), and one of a single launch
+// (quest_linear_few_tokens) 5.1 to 7.2: a launch is about 3.5 us of it, an allocation 0.7.  That, and not the GPU, still bounds the smallest calls.
 //
 // Contract of every function: either the call is the plain case -- exact torch tensors on one GPU, contiguous, right types, sizes
 // and alignment, accepted by the library -- and everything is launched, or None comes back with nothing launched and the
@@ -248,7 +248,11 @@ bool prefers_e2m3(int64_t m, int64_t k, int64_t n, const Lines &lines) {
 // another quantiser, the row kernel, which is the faster one for few rows.  49 to 56 tokens of up to 4096 elements in two launches, INT8 / FP6 GPU time: (50,
 // 3104, 4096) 0.89, (50, 4064, 1024) 0.91, (52, 4064, 4096) 0.92, (50, 2272, 2048) 1.00 and 0.94 as a call; with longer rows, more tokens or more channels (50, 6048,
 // 1024) 1.09, (50, 4960, 4096) 1.01, (64, 2272, 4096) 1.05, (50, 4064, 18000) 1.18.
+// Channels that are not whole 8s: the FP6 epilogue stores them one by one, which short rows do not outweigh where there are few tiles, 256 tokens up (400
+// sizes, rows of 672 to 6816): (300, 672, 3319) 0.95, (300, 1376, 17003) 0.94, (500, 672, 2052) 0.83, (500, 2016, 2052) 0.90, (1000, 1376, 1031) 0.97, (2000, 672,
+// 1031) 0.94; with more of them (500, 1376, 5569) 1.04, (1000, 1376, 3319) 1.06, (2000, 1376, 2052) 1.01, or fewer tokens (200, 1376, 1031) 1.13.
 bool ragged_takes_tiles(int64_t m, int64_t padded, int64_t n) {
+    if (n % 8 != 0 && padded <= 2048 && m > 256 && (m <= 384 ? n > 2048 : m * n <= 2200000)) return false;
     return padded <= 32768 && (m > 56 || padded > 4096 || n > 4096 || one_launch_on_tiles(m, padded, n));
 }
 

@@ -39,8 +39,9 @@ GEMM_ROTATES_QK = True
 
 
 def prefers_e2m3(m: int, k: int, n: int) -> bool:
-    """Whether the FP6 kernels are the faster ones for an (m, k) x (n, k) layer on its own, quantiser included.  The rule is native code
-    (csrc/host.cpp, with both sides of its lines), for a layer's call asks it there: it was 0.25 us of a call in Python."""
+    """Whether the FP6 kernels are the faster ones for an (m, k) x (n, k) layer on its own, quantiser included, with rows of whole 128s.  The rule
+    is native code (csrc/host.cpp, with both sides of its lines, and what differs for other rows), for a layer's call asks it there: it was
+    0.25 us of a call in Python."""
     return MATRIX_PATH == 'fp6' and native.prefers_e2m3(m, k, n, E2M3_MIN_K, E2M3_MIN_K_NARROW, E2M3_NARROW, E2M3_SHORT_ROWS_TOKENS)
 
 

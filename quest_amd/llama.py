@@ -385,7 +385,11 @@ class LlamaBlock(nn.Module):
         """Which of the four projections (bit 0 qkv, 1 output, 2 gate / up, 3 down) run on E2M3 tiles for m tokens, if there are any: the
         one decision of both statements of the block."""
         prefers = harness.block_prefers_e2m3
-        if m < harness.E2M3_MIN_TOKENS:          # few tokens of short rows: a launch for each of the projections on tiles, norm, rotation and all
+        # few tokens of short rows: QKV and gate / up are a launch each on tiles, norm, rotation and all.  The down projection, where its rows are longer
+        # than that launch takes, is two launches on tiles, the second with the residual addition; on packed codes instead whole models take 2 to 22 %
+        # longer (twelve layers of d = 640 to 2048 with rows of 1792 to 5632, 1 to 32 tokens: d = 1024 347 -> 376 us at one token, 371 -> 405 at 32; d =
+        # 2048 458 -> 475 and, at 8, 482 -> 534)
+        if m < harness.E2M3_MIN_TOKENS:
             takes = harness.one_launch_on_tiles
             short = harness.MATRIX_PATH == 'fp6' and c % 128 == 0 and hidden % 128 == 0 and takes(m, c, 3 * c) and takes(m, c, 2 * hidden)
             forms = 15 if short else 0

@@ -88,8 +88,10 @@ def test_rows_that_are_too_long_for_the_quantiser_stay_native(monkeypatch):
     assert torch.equal(layer(x), want)
 
 
-@pytest.mark.parametrize('m,k,n,tiles', [(49, 3104, 4096, False), (56, 4064, 1024, False), (57, 3104, 1024, True), (50, 4128, 1024, True), (50, 2272, 16416, True), (52, 1568, 1024, True)])
-def test_some_tens_of_ragged_rows(m, k, n, tiles):
+@pytest.mark.parametrize('m,k,n,tiles', [(49, 3104, 4096, False), (56, 4064, 1024, False), (57, 3104, 1024, True), (50, 4128, 1024, True), (50, 2272, 16416, True), (52, 1568, 1024, True),
+                                           (300, 1376, 3319, False), (300, 1376, 3320, True), (300, 1376, 1031, True), (500, 2016, 2052, False), (500, 2080, 2052, True),
+                                           (1000, 1056, 2201, True), (1000, 1056, 2199, False)])
+def test_which_ragged_layers_take_tiles(m, k, n, tiles):
     from quest_amd import harness
     g = torch.Generator(device=DEV).manual_seed(m + k + n)
     layer = harness.Linear4bit.from_weight((torch.randn(n, k, device=DEV, generator=g) * .02).half())
