@@ -118,12 +118,34 @@ __global__ void __launch_bounds__(64 * kWaves, 1) linear_few_tokens_kernel(Args 
     __builtin_amdgcn_sched_barrier(0);
     if (threadIdx.x < 512) sums[threadIdx.x] = 0;
 
+    // the scales, sums and bias of the first tile that this wave finishes: its own number of the workgroup's tiles
+    const int tok = r;
+    uint32_t c_mul[4], c_bias[4] = {0, 0, 0, 0};
+    v4u c_add;
+    const __amdgpu_buffer_rsrc_t add_r = __builtin_amdgcn_make_buffer_rsrc((void *)p.b_add, 0, N * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t mul_r = __builtin_amdgcn_make_buffer_rsrc((void *)p.b_mul, 0, N * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t bias_r = __builtin_amdgcn_make_buffer_rsrc((void *)p.bias, 0, N * 2, 0x00020000);
+    auto fetch_channels = [&](int tile) {          // (channels past the last, of tiles past the last too: zeros)
+        const int ch = tile * kChannels + 4 * g;
+        c_add = __builtin_amdgcn_raw_buffer_load_b128(add_r, ch * 4, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; e++) c_mul[e] = __builtin_amdgcn_raw_buffer_load_b16(mul_r, ch * 2 + 2 * e, 0, 0);
+        if (p.bias != nullptr) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) c_bias[e] = __builtin_amdgcn_raw_buffer_load_b16(bias_r, ch * 2 + 2 * e, 0, 0);
+        }
+    };
+    // Before the rows are looked at where no transform needs the registers and few waves have a row: behind them these would take the rows' registers, and waves
+    // without a row wait for those and for the weights behind them (one token, no transform, (1760, 20672), weights from HBM: 10.9 us behind, 10.6 before; two tokens of
+    // 10976, six waves of sixteen: 8.2 and 8.4).
+    constexpr bool kEarly = RAG && WPR == 1;
+    if constexpr (kEarly) fetch_channels(blockIdx.x + wave * gridDim.x);
+
     uint32_t yb[4][8];
     float total = 0.f;
     if (busy) {
         if constexpr (RAG) {
-            hq::spread(yb, bq);
-            total = hq::ragged_sum<DT, G>(bq);
+            total = hq::ragged_sum<DT, G>(yb, bq);
         } else {
             v4i hv[2][2];
             hq::signed_entries(hv, n, h, p.entry_bits);
@@ -162,24 +184,7 @@ __global__ void __launch_bounds__(64 * kWaves, 1) linear_few_tokens_kernel(Args 
             if constexpr (WPR == 1) a_add[row] = t; else part_add[wave] = t;
         }
     }
-    // the scales, sums and bias of the first tile that this wave finishes: its own number of the workgroup's tiles
-    const int tok = r;
-    uint32_t c_mul[4], c_bias[4] = {0, 0, 0, 0};
-    int c_add[4];
-    auto fetch_channels = [&](int tile) {          // (tiles past the last: the last channel's)
-        const int ch = tile * kChannels + 4 * g;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int c = min(ch + e, N - 1);
-            c_add[e] = p.b_add[c];
-            c_mul[e] = p.b_mul[c];
-        }
-        if (p.bias != nullptr) {
-#pragma unroll
-            for (int e = 0; e < 4; e++) c_bias[e] = p.bias[min(ch + e, N - 1)];
-        }
-    };
-    fetch_channels(blockIdx.x + wave * gridDim.x);
+    if constexpr (!kEarly) fetch_channels(blockIdx.x + wave * gridDim.x);
     lds_barrier();                                 // codes, scales and sums are there
     const float t_half_mul = __fmul_rn(0.5f, to_f32<DT>(a_mul[min(tok, M - 1)]));
     int t_add = 0;
@@ -242,7 +247,7 @@ __global__ void __launch_bounds__(64 * kWaves, 1) linear_few_tokens_kernel(Args 
             uint32_t o[4];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const float lhs = (float)(c[e] * 2 + t_add + c_add[e]);
+                const float lhs = (float)(c[e] * 2 + t_add + (int)c_add[e]);
                 const float rhs = __fmul_rn(t_half_mul, to_f32<DT>(c_mul[e]));
                 o[e] = from_f32<DT>(__fmul_rn(lhs, rhs));
                 if (p.bias != nullptr) o[e] = from_f32<DT>(__fadd_rn(to_f32<DT>(o[e]), to_f32<DT>(c_bias[e])));

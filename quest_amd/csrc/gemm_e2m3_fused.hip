@@ -178,8 +178,7 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
         const bool ragged = (K & 127) != 0;        // uniform
         float sumsq;
         if (ragged) {
-            hq::spread(yb, bq);
-            sumsq = hq::ragged_sum<DT, G>(bq);
+            sumsq = hq::ragged_sum<DT, G>(yb, bq);
         } else {
             sumsq = hq::transform<DT>(yb, bq, hv, p.entry_bits);
         }
@@ -195,7 +194,7 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
             *reinterpret_cast<uint4 *>(frag + slot * 16) = make_uint4(c[0], c[1], c[2], c[3]);
             *reinterpret_cast<uint2 *>(frag + kTailAt + slot * 8) = make_uint2(c[4], c[5]);
         };
-        if (__builtin_amdgcn_ballot_w64(counts && !quant_fast_ok(sf)) == 0) {
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(counts && !quant_fast_ok(sf)) == 0, 1)) {
 #pragma unroll
             for (int g = 0; g < 2; g++) put(g, hq::e2m3_group<DT, true>(yb, g, inv));
         } else {
