@@ -12,7 +12,7 @@
 // tile in LDS, one barrier per tile, the waves finishing tiles in turn.
 // What bounds it: up to 4096 channels the chain -- launch, activations, transform and quantiser, first products, sums -- of 4.3 us (K = 1024, one
 // token) to 7.2 (K = 4096, eight); with more the weights' way from memory.  GPU time in a graph against the two launches, weights from HBM, us: (1,
-// 4096, 4096) 5.5 / 7.1, (8, 4096, 4096) 7.2 / 7.6, (1, 1024, 4096) 4.8 / 6.2, (4, 8192, 8192) 11.4 / 13.2, (1, 4096, 22016) 12.5 / 12.9, (1, 11008, 4096)
+// 4096, 4096) 5.5 / 7.1, (8, 4096, 4096) 7.1 / 7.6, (1, 1024, 4096) 4.8 / 6.2, (4, 8192, 8192) 11.3 / 13.2, (1, 4096, 22016) 12.4 / 12.9, (1, 11008, 4096)
 // 8.0 / 9.8.  As calls, which the host bounds: (1, 4096, 4096) 7.0 / 11.2, (10, 1536, 1148) 7.3 / 11.5.
 #include "gemm_tiles.h"
 #include "hadamard_unit.h"

@@ -255,7 +255,7 @@ hadamard_quantize_mfma_kernel(const uint16_t *__restrict__ x, const uint16_t *__
             }
         };
         // degenerate rows (scale zero, Inf, NaN or outside the fast range) take the clamping form, as the nibbles do
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(row < M && !quant_fast_ok(sf_t)) == 0, 1)) emit(std::true_type{}); else emit(std::false_type{});
+        if (__builtin_amdgcn_ballot_w64(row < M && !quant_fast_ok(sf_t)) == 0) emit(std::true_type{}); else emit(std::false_type{});
         if constexpr (TL) {
             // The workgroup's rows are kTileRows consecutive slots of one row block: for every position their heads are
             // one contiguous run of the fragment (128 bytes for eight rows) and their tails another, written by
