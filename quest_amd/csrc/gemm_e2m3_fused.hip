@@ -64,8 +64,8 @@ __device__ __forceinline__ void lds_barrier() {
     plain_barrier();
 }
 
-// CT: channel tiles that the waves share
-template <int DT, int G, int CT, bool NORM, bool ROPE>
+// CT: channel tiles that the waves share.  RAG: rows that are not whole 128s, without norm and transform
+template <int DT, int G, int CT, bool NORM, bool ROPE, bool RAG>
 __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Args p) {
     using S = Shape<G, CT>;
     __shared__ __attribute__((aligned(1024))) uint8_t lds[S::kLdsB];
@@ -157,7 +157,7 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
 
     if (busy) {
         v4i hv[2][2];
-        hq::signed_entries(hv, n, h, p.entry_bits);
+        if constexpr (!RAG) hq::signed_entries(hv, n, h, p.entry_bits);
         wait_vmcnt_imm<3 * CT>();                     // the rows (and the norm's weights) are here, the first weights need not be
         asm volatile("" ::: "memory");
         v4u bq[8];
@@ -175,15 +175,11 @@ __global__ void __launch_bounds__((64 * G), (G / 4)) linear_e2m3_fused_kernel(Ar
             hq::normalise<DT>(bq, nq, hq::group_sum_f<G>(ss), K, p.eps);
         }
         uint32_t yb[4][8];
-        const bool ragged = (K & 127) != 0;        // uniform
-        float sumsq;
-        if (ragged) {
-            sumsq = hq::ragged_sum<DT, G>(yb, bq);
-        } else {
-            sumsq = hq::transform<DT>(yb, bq, hv, p.entry_bits);
-        }
+        float total;
+        if constexpr (RAG) total = hq::ragged_sum<DT, G>(yb, bq);
+        else total = hq::transform<DT>(yb, bq, hv, p.entry_bits);
         fetch_channels(muls[0], ahead[0], ct);     // (here: the transform needs the registers)
-        const float total = ragged ? sumsq : hq::group_sum_f<G>(sumsq);
+        if constexpr (!RAG) total = hq::group_sum_f<G>(total);
         const uint32_t s16 = from_f32<DT>(scale_from_sumsq(total, K));
         if (n % G == 0 && h == 0) scales[row] = (uint16_t)s16;
         const float sf = to_f32<DT>(s16), inv = quant_inv(sf);
@@ -276,10 +272,13 @@ template <int DT, int G, int CT>
 static int launch_as(const Args &a, bool norm, hipStream_t st) {
     const dim3 grid((unsigned)(8 * a.ways * a.tiles_t)), block(64 * G);
     const bool rope = a.epi.kind == kEpiRope;
-    if (norm && rope) linear_e2m3_fused_kernel<DT, G, CT, true, true><<<grid, block, 0, st>>>(a);
-    else if (norm) linear_e2m3_fused_kernel<DT, G, CT, true, false><<<grid, block, 0, st>>>(a);
-    else if (rope) linear_e2m3_fused_kernel<DT, G, CT, false, true><<<grid, block, 0, st>>>(a);
-    else linear_e2m3_fused_kernel<DT, G, CT, false, false><<<grid, block, 0, st>>>(a);
+    const bool ragged = (a.K & 127) != 0;
+    if (norm && rope) linear_e2m3_fused_kernel<DT, G, CT, true, true, false><<<grid, block, 0, st>>>(a);
+    else if (norm) linear_e2m3_fused_kernel<DT, G, CT, true, false, false><<<grid, block, 0, st>>>(a);
+    else if (rope && ragged) linear_e2m3_fused_kernel<DT, G, CT, false, true, true><<<grid, block, 0, st>>>(a);
+    else if (rope) linear_e2m3_fused_kernel<DT, G, CT, false, true, false><<<grid, block, 0, st>>>(a);
+    else if (ragged) linear_e2m3_fused_kernel<DT, G, CT, false, false, true><<<grid, block, 0, st>>>(a);
+    else linear_e2m3_fused_kernel<DT, G, CT, false, false, false><<<grid, block, 0, st>>>(a);
     return launch_status();
 }
 
